@@ -256,14 +256,14 @@ int inv_laplace_trans(double *f, TAGS_COMPLEX *g, TAGS_COMPLEX *s, double tmax, 
  * ------------------------------------------------------------------------- */
 
 enum tags_precision {
-    TAGS_PREC_FP64 = 0,   /* complex128 LU throughout (the plain form) */
-    TAGS_PREC_MIXED = 1,  /* complex64 LU on MFMA + FP64 iterative refinement,
+    TAGS_PREC_FP64 = 0,   /* complex128 factors throughout (the plain form) */
+    TAGS_PREC_MIXED = 1,  /* complex64 factors on MFMA + FP64 iterative refinement,
                              automatic FP64 fallback when refinement stalls */
 };
 
 typedef struct {
     int precision_used;   /* tags_precision actually used for this sample */
-    int refine_iters;     /* refinement steps (mixed) */
+    int refine_iters;     /* refinement steps (mixed; 0 in the FP64 form) */
     int info;             /* 0, or first zero pivot (1-based) */
     double backward_err;  /* ||b - W x||_inf / (||W||_inf ||x||_inf) in FP64 (-1 when
                              not computed: the FP64 form of a sweep without
@@ -314,8 +314,7 @@ int tags_sweep_solve(tags_sweep *sw, size_t nfreq, const TAGS_COMPLEX *s,
                      tags_item_stats *stats);
 
 /* Factorisation plan of the sweep (default TAGS_PLAN_HYBRID, the fastest
- * measured: ZL_FIRST's FP64 factor, the nodal complex64 factor from the switch
- * frequency up). Every plan
+ * measured: the nodal solve by explicit symmetric inverses). Every other plan
  * but the mixed factor of GROUNDED pivots with the process's panel algorithm
  * (tags_set_panel); the structured
  * ones skip rows and columns that are exactly zero for the columns being
@@ -354,14 +353,17 @@ int tags_sweep_solve(tags_sweep *sw, size_t nfreq, const TAGS_COMPLEX *s,
  *                       incidence blocks are not treated as dense). It needs
  *                       more refinement steps toward low frequencies, where a
  *                       stalled refinement falls back to the FP64 factor;
- * TAGS_PLAN_HYBRID      stored and factored as ZL_FIRST in FP64. In a sweep's
- *                       mixed form, each sample takes NODAL's complex64 factor,
- *                       without row exchanges (Z_L, Z_T and S are complex
- *                       symmetric with a definite real or imaginary part), at
- *                       and above the switch frequency
- *                       (tags_sweep_set_nodal_above) and ZL_FIRST's below it;
- *                       tags_immittance_solve, which has no frequency, treats
- *                       it as ZL_FIRST. */
+ * TAGS_PLAN_HYBRID      a sweep keeps the impedance blocks alone (no W) and
+ *                       solves by Y_L = Z_L^-1, Y_T = Z_T^-1 and the inverse of
+ *                       the node system A^T Y_L A + B^T Y_T B, each inverted
+ *                       without row exchanges as the complex symmetric matrix
+ *                       it is, in complex128 (FP64) or complex64 (mixed), then
+ *                       refines on W with double-double residuals (both forms;
+ *                       FP64 to an estimated error of 1e-14). A sample that
+ *                       misses its acceptance rule, a sweep with a segment
+ *                       whose ends share a node and, in the mixed form, a
+ *                       sample below tags_sweep_set_nodal_above take ZL_FIRST's
+ *                       pivoted factor; so does tags_immittance_solve. */
 enum tags_plan {
     TAGS_PLAN_DENSE = 0,
     TAGS_PLAN_STRUCTURED = 1,
@@ -430,8 +432,8 @@ int tags_inv_laplace_batch(double *f, const TAGS_COMPLEX *g, const TAGS_COMPLEX 
 enum tags_formulation { TAGS_FORM_HEM = 0, TAGS_FORM_MHEM = 1 };
 int tags_sweep_set_formulation(tags_sweep *sw, int formulation);
 
-/* Refinement of nodal complex64 factors (TAGS_PLAN_HYBRID and TAGS_PLAN_NODAL,
- * mixed form): a sample at |s| / 2 pi < below_hz (default 2e4 Hz) refines by
+/* Refinement of nodal complex64 factors (TAGS_PLAN_NODAL, mixed form; the
+ * hybrid plan's nodal solve refines classically at every frequency): a sample at |s| / 2 pi < below_hz (default 2e4 Hz) refines by
  * FGMRES in FP64 right-preconditioned by the complex64 factor, `steps`
  * (1 .. 32, default 6) Arnoldi steps per refinement step (GMRES-based
  * refinement), where the classic correction from the factor alone converges
@@ -441,12 +443,11 @@ int tags_sweep_set_formulation(tags_sweep *sw, int formulation);
  * reference. Returns 0, or TAGS_ERR_ARG. */
 int tags_sweep_set_gmres(tags_sweep *sw, double below_hz, int steps);
 
-/* Switch frequency of TAGS_PLAN_HYBRID (default 0 Hz: the nodal factor at
- * every frequency, refined as tags_sweep_set_gmres sets): in the mixed form a
- * sample at |s| / 2 pi >= hz takes the nodal plan's complex64 factor, a lower
- * one ZL_FIRST's. A nodal sample that falls back to FP64 or needs more than 10
- * refinement steps raises the switch to 1.5 times its frequency for the rest
- * of that tags_sweep_solve call (each call starts from the configured switch).
+/* Switch frequency of TAGS_PLAN_HYBRID (default 0 Hz: the nodal solve at
+ * every frequency): in the mixed form a sample at |s| / 2 pi >= hz takes the
+ * nodal solve in complex64, a lower one ZL_FIRST's complex64 factor. A nodal
+ * sample that is not accepted raises the switch to 1.5 times its frequency for
+ * the rest of that tags_sweep_solve call (each call starts from the configured switch).
  * No counterpart in the reference, which factors every sample alike. Returns 0,
  * or TAGS_ERR_ARG for hz < 0. */
 int tags_sweep_set_nodal_above(tags_sweep *sw, double hz);
@@ -490,13 +491,15 @@ typedef struct {
  * sweep and installs them (tags_sweep_set_tuning). First every MFMA tile
  * variant is timed on the sweep's own trailing-update shapes (the largest
  * update of the plan's widest phase, and a 1024 x 1024 tail product) at both
- * step widths; then, by coordinate descent from the current settings, step
+ * step widths (for the hybrid plan they serve the factorisation that takes over
+ * from the nodal solve, whose own schedule is the groups and samples in
+ * flight); then, by coordinate descent from the current settings, step
  * width (with its fastest variants), update launches, solve rows, samples in
  * flight, samples per group (half and a quarter of the automatic size below
  * order 8192; 2, 3 and 4 from 8192 up, as far as the groups in flight fit in
  * 80 % of the device's memory) and, for the mixed form of
- * the hybrid plan, the nodal switch (0 or 20 kHz) and the Arnoldi steps per
- * FGMRES refinement step (6, 8, 10) are each kept when a
+ * TAGS_PLAN_NODAL, the Arnoldi steps per FGMRES refinement step (6, 8, 10) are
+ * each kept when a
  * timed solve of the `nprobe` probe samples (s, kappa, mur, inj_node as in
  * tags_sweep_solve; one untimed solve first for the allocations; for a fair
  * comparison of group sizes nprobe should be a few times the samples in
@@ -513,16 +516,18 @@ int tags_sweep_autotune(tags_sweep *sw, int precision, size_t nprobe, const TAGS
 int tags_sweep_set_tuning(tags_sweep *sw, int precision, const tags_tuning *t);
 int tags_sweep_get_tuning(const tags_sweep *sw, int precision, tags_tuning *t);
 
-/* FP64 form only: with on != 0, W is assembled again after each sample's
- * factorisation (which replaced it) and the backward error
+/* FP64 form only: with on != 0, the backward error
+ * of the refinement's last step (hybrid plan), or of W assembled again after
+ * each sample's factorisation (which replaced it),
  * ||e_inj - W x||_inf / (||W||_inf ||x||_inf) goes to the item statistics
- * (one more fill and one FP64 residual per sample; off by default, when
+ * (other plans: one more fill and one FP64 residual per sample; off by default, when
  * backward_err is -1). No counterpart in the reference. */
 int tags_sweep_set_verify(tags_sweep *sw, int on);
 
 /* Groups of frequency samples a sweep keeps in flight (1 .. 4, default 4),
- * each with its own HIP stream, W and factor work space (about 11 GB for a
- * one-sample group of the 60 x 60 m grid in the mixed form). The calling
+ * each with its own HIP stream, matrices and work space (about 3 GB for a
+ * one-sample group of the 60 x 60 m grid in the mixed form, 11 GB with W).
+ * The calling
  * thread queues a group on every slot, then finishes them in issue order,
  * queuing the next group on each slot as it frees up, so that one group's
  * trailing updates keep the GPU busy while another waits on its panel chain. Results do not depend on the count, except

@@ -1,0 +1,85 @@
+"""GPU test of the hybrid plan's nodal solve (explicit symmetric inverses with
+refinement) against the pivoted Z_L-first FP64 factor of the assembled W, at
+the sizes where its kernels change shape: segment and node counts around the
+16-row strips, the 64-row tiles and the 64- / 128-column steps (600 rows), one
+segment, and the route out of it (a zero frequency makes Z_L vanish, so the
+nodal solve cannot accept and the pivoted factor answers).
+
+Tolerances. U[inj]: the FP64 form is refined to an estimated 1e-14 and the
+mixed one to 1e-10 of |x|, so what remains is the LU's own error, taken at the
+1e-9 of the other plan comparisons in FP64 and the 1e-8 bar in the mixed form.
+The whole x, relative to its largest entry: 1e-8 (the LU's normwise error at
+cond(W) ~ 1e8)."""
+import numpy as np
+import pytest
+
+import tags_pkg
+
+T = tags_pkg.load()
+
+pytestmark = pytest.mark.gpu
+
+
+def _rod(m):
+    rc, e, nodes = T.segment_electrode([0, 0, -0.5], [0.5 * m, 0, -0.5], m, 7e-3)
+    return e, nodes
+
+
+def _grid(vx, vy, ex, ey):
+    rc, e, nodes = T.electrode_grid(vx, vy, 0.6 * ex * (vx - 1), 0.6 * ey * (vy - 1), ex, ey, 5e-3,
+                                    -0.6)
+    return e, nodes
+
+
+def _compare(e, nodes, f, groups=(0,), mhem=False):
+    s = 2j * np.pi * np.asarray(f)
+    kap = 2e-3 + s * 12.0 * T.EPS0
+    inj = len(nodes) // 2
+    sw = T.Sweep(e, nodes)
+    if mhem:
+        sw.set_formulation(T.FORM_MHEM)
+    sw.set_plan(T.PLAN_ZL_FIRST)
+    u0, _, x0 = sw.solve(s, kap, inj, T.PREC_FP64, want_x=True)
+    sw.set_plan(T.PLAN_HYBRID)
+    scale = np.abs(x0).max(axis=1, keepdims=True)
+    for g in groups:
+        sw.set_batch(g)
+        for prec, tol in ((T.PREC_FP64, 1e-9), (T.PREC_MIXED, 1e-8)):
+            u, st, x = sw.solve(s, kap, inj, prec, want_x=True)
+            assert all(q["info"] == 0 and q["precision_used"] == prec for q in st), (prec, st)
+            assert np.max(np.abs(u - u0) / np.abs(u0)) <= tol, (prec, g)
+            assert np.max(np.abs(x - x0) / scale) <= 1e-8, (prec, g)
+            assert np.array_equal(u, x[:, inj])
+    sw.close()
+
+
+@pytest.mark.parametrize("m", [1, 2, 15, 16, 17, 31, 32, 63, 64, 65, 127, 128, 129, 191])
+def test_conductors_at_tile_edges(m):
+    _compare(*_rod(m), f=[60.0, 1e4, 3e6], groups=(0, 2))
+
+
+# (segments, nodes): (10, 10), (262, 239), (635, 580), (705, 636)
+@pytest.mark.parametrize("shape", [(2, 2, 3, 2), (7, 5, 5, 4), (9, 8, 5, 5), (11, 8, 4, 5)])
+def test_grids_across_the_step_widths(shape):
+    _compare(*_grid(*shape), f=[100.0, 2e5])
+
+
+def test_mhem_blocks():
+    _compare(*_grid(4, 3, 5, 3), f=[100.0, 1e5, 2e6], mhem=True)
+
+
+def test_zero_frequency_takes_the_pivoted_factor():
+    e, nodes = _rod(20)
+    s = np.array([0.0, 2j * np.pi * 1e5])
+    kap = 2e-3 + s * 12.0 * T.EPS0
+    sw = T.Sweep(e, nodes)
+    sw.set_plan(T.PLAN_ZL_FIRST)
+    u0, st0 = sw.solve(s, kap, 0, T.PREC_FP64)
+    sw.set_plan(T.PLAN_HYBRID)
+    for prec in (T.PREC_FP64, T.PREC_MIXED):
+        u, st = sw.solve(s, kap, 0, prec)
+        assert [q["info"] for q in st] == [q["info"] for q in st0]
+        ok = np.isfinite(u0)
+        assert np.array_equal(np.isfinite(u), ok)
+        assert np.all(np.abs(u - u0)[ok] <= 1e-8 * np.abs(u0[ok]))
+    sw.close()

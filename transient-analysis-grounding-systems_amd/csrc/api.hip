@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "lu.h"
+#include "nodal.h"
 
 namespace tags {
 
@@ -1694,7 +1695,9 @@ struct SweepSlot {
     PairScalars* hsc = nullptr;  // pinned staging of dsc
     Profiler prof;
     Solver sv;
-    int cap = 0;
+    NodalSolver nd;         // the hybrid plan's solve (nodal_path)
+    bool nodal_path = false;
+    int cap = 0, sc_cap = 0;
     const tags_sweep* bound = nullptr;  // the sweep whose plans the solver holds
     int bound_kind = -1;                // and its plan kind then
     long f = -1;            // first sample of the group in flight (-1: idle)
@@ -1702,7 +1705,6 @@ struct SweepSlot {
     std::vector<tags_item_stats> stt;  // their statistics and infos, filled as they finish
     std::vector<int> info;
     std::vector<double> hz; // their frequencies |s| / 2 pi
-    bool nodal = false;     // their complex64 factor is the nodal plan's
     size_t w_cap = 0, rhs_cap = 0;  // allocated elements of W and rhs
     // items [0, static_items) of W hold the frequency-independent part (zero
     // and incidence blocks) of static_sw's layout static_kind: the mixed form
@@ -1711,10 +1713,28 @@ struct SweepSlot {
     const tags_sweep* static_sw = nullptr;
     int static_kind = -1;
     int static_items = 0;
-    int init(long N, int batch)
+    // the stream and the scalars of `batch` samples
+    int init_items(int batch)
     {
         if (!stream.s) TAGS_HIP(hipStreamCreate(&stream.s));
-        int rc;
+        nd.st = sv.st = stream.s;
+        nd.pr = sv.pr = &prof;
+        if (batch <= sc_cap) return 0;
+        hipFree(dsc.p);
+        if (hsc) hipHostFree(hsc);
+        dsc.p = nullptr;
+        hsc = nullptr;
+        sc_cap = 0;
+        int rc = dsc.alloc((size_t)batch);
+        if (rc) return rc;
+        TAGS_HIP(hipHostMalloc(&hsc, sizeof(PairScalars) * batch, 0));
+        sc_cap = batch;
+        return 0;
+    }
+    int init(long N, int batch)
+    {
+        int rc = init_items(batch);
+        if (rc) return rc;
         const size_t nw = (size_t)N * N * batch, nr = (size_t)N * batch;
         if (nw > w_cap || nr > rhs_cap || batch > cap) {
             // grow to cover every earlier request as well (a lane of a
@@ -1723,23 +1743,15 @@ struct SweepSlot {
             const int items = std::max(batch, cap);
             hipFree(W.p);
             hipFree(rhs.p);
-            hipFree(dsc.p);
-            if (hsc) hipHostFree(hsc);
             W.p = rhs.p = nullptr;
-            dsc.p = nullptr;
-            hsc = nullptr;
             cap = 0;
             w_cap = rhs_cap = 0;
             static_items = 0;
-            if ((rc = W.alloc(aw)) || (rc = rhs.alloc(ar)) || (rc = dsc.alloc((size_t)items)))
-                return rc;
-            TAGS_HIP(hipHostMalloc(&hsc, sizeof(PairScalars) * items, 0));
+            if ((rc = W.alloc(aw)) || (rc = rhs.alloc(ar))) return rc;
             cap = items;
             w_cap = aw;
             rhs_cap = ar;
         }
-        sv.st = stream.s;
-        sv.pr = &prof;
         return 0;
     }
     ~SweepSlot()
@@ -1803,11 +1815,6 @@ struct PlanDev {
     }
 };
 
-// refinement steps above which a nodal sample of a hybrid sweep counts as slow
-// (a step costs a few per cent of a factorisation, a fallback to FP64 several
-// factorisations)
-constexpr int kHybridMaxIters = 10;
-
 struct tags_sweep {
     long m = 0, n = 0, N = 0;
     int plan_kind = TAGS_PLAN_HYBRID;
@@ -1817,15 +1824,17 @@ struct tags_sweep {
     int batch = 1;         // samples per group of the current call
     tags::LUPlan plan;
     tags::LUPlan plan32;
-    // TAGS_PLAN_HYBRID: the mixed form's complex64 factor is the nodal plan's
-    // at and above nodal_above Hz, ZL_FIRST's below; a nodal sample that falls
-    // back to FP64 or needs more than kHybridMaxIters refinement steps raises
-    // the switch to 1.5 times its frequency for the rest of the sweep
-    tags::LUPlan plan_nodal;
-    // device copies of plan, plan32 and plan_nodal's row orders
-    PlanDev plan_dev[3];
+    // TAGS_PLAN_HYBRID: solved by NodalSolver where every segment has two
+    // nodes (nodal_ok), in the mixed form at and above nodal_above Hz; a sample
+    // that misses its acceptance rule is factored by ZL_FIRST and, for the rest
+    // of the call, raises the switch to 1.5 times its frequency (mixed) or
+    // turns the nodal solve off (nodal64)
+    bool nodal_ok = true, nodal64 = true;
+    int nd_batch = 1;      // samples per group of the nodal solve
+    // device copies of plan and plan32's row orders
+    PlanDev plan_dev[2];
     double nodal_above = 0.0;
-    // nodal complex64 factors below gmres_below Hz refine by FGMRES
+    // TAGS_PLAN_NODAL's complex64 factors below gmres_below Hz refine by FGMRES
     // (gmres_steps Arnoldi steps per refinement step), above it classically
     double gmres_below = 2e4;
     int gmres_steps = 6;
@@ -1896,16 +1905,43 @@ static int sweep_batch(const tags_sweep* sw, bool mixed)
     return (int)std::max(1.0, std::min((double)kBatchMax, b));
 }
 
+// Samples per group of the nodal solve, by the same rule on its own bytes.
+// A call's nfreq samples are shared out evenly among the groups it takes.
+static int sweep_nd_batch(const tags_sweep* sw, bool mixed, size_t nfreq)
+{
+    size_t lim = 1;
+    if (sw->batch_req > 0) {
+        lim = (size_t)sw->batch_req;
+    } else if (sw->N < kBatchOneAbove) {
+        const double per = (double)NodalSolver::bytes(sw->m, sw->n, !mixed, 1);
+        lim = (size_t)std::max(1.0, std::min((double)kBatchMax, std::floor(kBatchBytes / per)));
+    }
+    const size_t groups = std::max<size_t>(1, (nfreq + lim - 1) / lim);
+    return (int)std::max<size_t>(1, sw->batch_req > 0 ? std::min(lim, nfreq)
+                                                      : (nfreq + groups - 1) / groups);
+}
+
+// Whether the nodal solve takes a sample at `hz`.
+static bool sweep_nodal(const tags_sweep* sw, bool mixed, double hz)
+{
+    if (sw->plan_kind != TAGS_PLAN_HYBRID || !sw->nodal_ok) return false;
+    return mixed ? hz >= sw->nodal_above : sw->nodal64;
+}
+
 // The first k slots exist and are allocated for groups of sw->batch samples of
-// order N (precision `mixed`).
-static int sweep_slots(tags_sweep* sw, int k, bool mixed)
+// order N (precision `mixed`) of the kinds of solve in use: the nodal solve's
+// blocks, or W with the work space of its factorisation.
+static int sweep_slots(tags_sweep* sw, int k, bool mixed, bool nodal, bool dense)
 {
     while ((int)sw->slots.size() < k) sw->slots.emplace_back(new SweepSlot());
     for (int i = 0; i < k; i++) {
         SweepSlot& sl = *sw->slots[i];
-        int rc = sl.init(sw->N, sw->batch);
+        int rc = sl.init_items(std::max(sw->batch, sw->nd_batch));
         if (rc) return rc;
-        if ((rc = sl.sv.ensure((int)sw->N, mixed, sw->batch))) return rc;
+        if (nodal && (rc = sl.nd.ensure(sw->hem, !mixed, sw->nd_batch))) return rc;
+        if (dense && ((rc = sl.init(sw->N, sw->batch)) ||
+                      (rc = sl.sv.ensure((int)sw->N, mixed, sw->batch))))
+            return rc;
         sl.prof.on = sw->profiling;
     }
     return 0;
@@ -1944,10 +1980,9 @@ static int sweep_layout(tags_sweep* sw)
         sw->plan32 = LUPlan::nodal((int)m, (int)n);
         p32 = &sw->plan32;
         break;
-    case TAGS_PLAN_HYBRID:  // complex64 plan chosen per sample (sweep_issue)
+    case TAGS_PLAN_HYBRID:  // the factor of samples that the nodal solve does not take
         sw->layout = BlockLayout{n, m, 2 * m, 0, m};
         sw->plan = LUPlan::zl_first((int)m, (int)n, false);
-        sw->plan_nodal = LUPlan::nodal((int)m, (int)n, false);
         break;
     case TAGS_PLAN_BLOCK_PIVOT:
         // the FP64 form takes the fully pivoted factor: the Z_L block's weak
@@ -1963,8 +1998,7 @@ static int sweep_layout(tags_sweep* sw)
         break;
     }
     int rc;
-    if ((rc = sw->plan_dev[0].attach(sw->plan)) || (rc = sw->plan_dev[1].attach(sw->plan32)) ||
-        (rc = sw->plan_dev[2].attach(sw->plan_nodal)))
+    if ((rc = sw->plan_dev[0].attach(sw->plan)) || (rc = sw->plan_dev[1].attach(sw->plan32)))
         return rc;
     sw->bind64 = p64;
     sw->bind32 = p32;
@@ -2016,9 +2050,14 @@ static PairScalars sample_scalars(TAGS_COMPLEX s_, TAGS_COMPLEX kappa_, double m
 // one sample from `sc`, several from their scalars `dsc` in device memory.
 static int sweep_fill_items(tags_sweep* sw, c64* W, hipStream_t st, Profiler* prof, int nb,
                             const PairScalars& sc, const PairScalars* dsc,
-                            bool fill_static = true)
+                            bool fill_static = true, long ld = 0, long sW = 0)
 {
-    const long N = sw->N, sW = N * N;
+    // a compact store of the impedance blocks (ld > 0: see nodal_z_items) is
+    // addressed as a matrix of that pitch with the blocks in its first rows
+    const long N = ld > 0 ? ld : sw->N;
+    BlockLayout L = sw->layout;
+    if (ld > 0) L = BlockLayout{sw->n, sw->m, 2 * sw->m, 0, sw->m};
+    else sW = N * N;
     Timed tm(prof, FAM_FILL, st);
     int rc;
     const PairScalars* scs = nb > 1 ? dsc : nullptr;
@@ -2027,12 +2066,12 @@ static int sweep_fill_items(tags_sweep* sw, c64* W, hipStream_t st, Profiler* pr
     if (sw->formulation == TAGS_FORM_MHEM) {
         if (!sw->pot) return TAGS_ERR_ARG;
         const size_t mm = (size_t)sw->m * sw->m;
-        if ((rc = launch_fill_mhem(W, N, sw->layout, sw->e.soa(), sw->img.soa(), sw->pot,
+        if ((rc = launch_fill_mhem(W, N, L, sw->e.soa(), sw->img.soa(), sw->pot,
                                    sw->pot + mm, sw->pot + 2 * mm, sw->pot + 3 * mm, sc, st, nb,
                                    sW, scs)))
             return rc;
-    } else if ((rc = launch_fill_zblocks(W, N, sw->layout, sw->e.soa(), sw->img.soa(), sc, st, nb,
-                                         sW, scs))) {
+    } else if ((rc = launch_fill_zblocks(W, N, L, sw->e.soa(), sw->img.soa(), sc, st, nb, sW,
+                                         scs))) {
         return rc;
     }
     tm.end();
@@ -2132,6 +2171,7 @@ int tags_sweep_create(tags_sweep** out, const Electrode* electrodes, const Elect
         if (hsn[s] < 0 || hsn[s] >= n || hen[s] < 0 || hen[s] >= n) return TAGS_ERR_ARG;
         ptr[hsn[s] + 1]++;
         if (hen[s] != hsn[s]) ptr[hen[s] + 1]++;
+        else sw->nodal_ok = false;  // A 1 = 0 and B 1 = 1 need two nodes per segment
     }
     for (long u = 0; u < n; u++) ptr[u + 1] += ptr[u];
     seg.assign(ptr[n], 0);
@@ -2324,6 +2364,16 @@ __global__ void k_unit_rhs(c64* b, long N, long pos)
 
 extern "C" {
 
+// Between polls of the streams: short solves (a few hundred microseconds) are
+// polled without a pause, which a sleep's wake-up (some 70 us) would outlast.
+struct Poll {
+    int n = 0;
+    void wait()
+    {
+        if (++n > 400) std::this_thread::sleep_for(std::chrono::microseconds(20));
+    }
+};
+
 // Per-call arguments of tags_sweep_solve shared by the issue and finish steps.
 struct SweepCall {
     size_t nfreq;
@@ -2349,36 +2399,35 @@ static int sweep_issue(tags_sweep* sw, SweepSlot& sl, size_t f, const SweepCall&
         const c64 sf = from_c(c.s[q]);
         return std::hypot(sf.x, sf.y) / (2.0 * M_PI);
     };
-    const bool hybrid = sw->plan_kind == TAGS_PLAN_HYBRID && c.mixed;
     const bool nodal_plan = sw->plan_kind == TAGS_PLAN_NODAL && c.mixed;
-    // the sample's class: 0 the plan's own complex64 factor with classic
-    // refinement (the hybrid plan's Z_L-first one below its switch), 1 a nodal
-    // factor refined by FGMRES, 2 a nodal factor refined classically
+    // the sample's class: 0 the plan's own factor with classic refinement (the
+    // hybrid plan's Z_L-first one), 1 a nodal complex64 factor refined by
+    // FGMRES, 2 one refined classically, 3 the nodal solve
     auto cls = [&](size_t q) {
-        if (!hybrid && !nodal_plan) return 0;
         const double h = hz_of(q);
-        if (hybrid && h < sw->nodal_above) return 0;
-        return h < sw->gmres_below ? 1 : 2;
+        if (sweep_nodal(sw, c.mixed, h)) return 3;
+        return nodal_plan ? (h < sw->gmres_below ? 1 : 2) : 0;
     };
     const int c0 = cls(f);
-    sl.nodal = hybrid && c0 > 0;
+    sl.nodal_path = c0 == 3;
+    const int lim = sl.nodal_path ? sw->nd_batch : sw->batch;
     int cnt = 0;
     sl.hz.clear();
-    while (cnt < sw->batch && f + cnt < c.nfreq && cls(f + cnt) == c0) {
+    while (cnt < lim && f + cnt < c.nfreq && cls(f + cnt) == c0) {
         sl.hz.push_back(hz_of(f + cnt));
         cnt++;
     }
     sl.sv.gmres_k = c0 == 1 ? sw->gmres_steps : 0;
+    // a raised switch, or the nodal solve turned off: buffers made on the way
+    if (!sl.nodal_path &&
+        ((rc = sl.init(N, sw->batch)) || (rc = sl.sv.ensure((int)N, c.mixed, sw->batch))))
+        return rc;
     sl.f = (long)f;
     sl.cnt = cnt;
     sl.stt.assign(cnt, tags_item_stats{});
     for (auto& q : sl.stt)
         for (int i = 0; i < 8; i++) q.refine_hist[i] = -1.0;
     sl.info.assign(cnt, 0);
-    if (sw->plan_kind == TAGS_PLAN_HYBRID) {
-        sl.sv.plan32 = sl.nodal ? &sw->plan_nodal : nullptr;
-        sl.sv.plan32_retry = sl.nodal ? &sw->plan : nullptr;
-    }
     hipStream_t st = sl.stream.s;
     PairScalars sc0{};
     for (int z = 0; z < cnt; z++) {
@@ -2393,6 +2442,13 @@ static int sweep_issue(tags_sweep* sw, SweepSlot& sl, size_t f, const SweepCall&
     if (cnt > 1)
         TAGS_HIP(hipMemcpyAsync(sl.dsc.p, sl.hsc, sizeof(PairScalars) * cnt,
                                 hipMemcpyHostToDevice, st));
+    if (sl.nodal_path) {
+        if ((rc = sweep_fill_items(sw, sl.nd.Z, st, &sl.prof, cnt, sc0, sl.dsc.p, false, sw->m,
+                                   sl.nd.sZ)))
+            return rc;
+        rc = sl.nd.issue(cnt, (long)c.inj_node);
+        return rc ? rc : cnt;
+    }
     // the zero and incidence blocks stay from the last mixed group of this
     // sweep on this slot unless a factor in FP64 replaced W since
     const bool keep = c.mixed && sl.static_sw == sw && sl.static_kind == sw->layout_kind &&
@@ -2440,6 +2496,68 @@ static int sweep_verify64(tags_sweep* sw, SweepSlot& sl, c64* Wz, const c64* xz,
     return 0;
 }
 
+// Sample f, item q of the slot's group, that the nodal solve did not accept:
+// the Z_L-first factor of its assembled W (mixed: complex64 with refinement,
+// then complex128). Waits; its solution replaces the item's x and u.
+static int sweep_nodal_retry(tags_sweep* sw, SweepSlot& sl, int q, size_t f, const SweepCall& c,
+                             tags_item_stats* stt, int* info)
+{
+    const long N = sw->N;
+    int rc;
+    if ((rc = sl.init(N, 1)) || (rc = sl.sv.ensure((int)N, c.mixed, 1))) return rc;
+    slot_bind(sw, sl);
+    sl.static_items = 0;
+    hipStream_t st = sl.stream.s;
+    if ((rc = sweep_fill(sw, sl.W.p, st, nullptr, c.s[f], c.kappa[f], c.mur,
+                         c.gamma ? &c.gamma[f] : nullptr, c.ref_l ? &c.ref_l[f] : nullptr,
+                         c.ref_t ? &c.ref_t[f] : nullptr)))
+        return rc;
+    hipLaunchKernelGGL(k_unit_rhs, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, sl.rhs.p, N,
+                       sw->layout.node_off + (long)c.inj_node);
+    TAGS_HIP(hipGetLastError());
+    rc = c.mixed ? sl.sv.solve_mixed(sl.W.p, sl.rhs.p, stt) : sl.sv.solve64(sl.W.p, sl.rhs.p, stt);
+    if (rc < 0) return rc;
+    *info = rc;
+    if (!c.mixed && sw->verify && rc == 0 &&
+        (rc = sweep_verify64(sw, sl, sl.W.p, sl.rhs.p, f, c, stt)))
+        return rc;
+    TAGS_HIP(hipMemcpyAsync(sl.nd.x + (long)q * N, sl.rhs.p, sizeof(c64) * N,
+                            hipMemcpyDeviceToDevice, st));
+    TAGS_HIP(hipMemcpyAsync(&sl.nd.hu[q], sl.rhs.p + sw->layout.node_off + c.inj_node, sizeof(c64),
+                            hipMemcpyDeviceToHost, st));
+    TAGS_HIP(hipStreamSynchronize(st));
+    return 0;
+}
+
+// Statistics of a nodal group whose refinement has ended, and the retries.
+static int sweep_nodal_finish(tags_sweep* sw, SweepSlot& sl, const SweepCall& c)
+{
+    NodalSolver& nd = sl.nd;
+    for (int q = 0; q < sl.cnt; q++) {
+        tags_item_stats& t = sl.stt[q];
+        sl.info[q] = 0;
+        t.info = 0;
+        if (nd.accepted[q]) {
+            t.precision_used = c.mixed ? TAGS_PREC_MIXED : TAGS_PREC_FP64;
+            t.refine_iters = c.mixed ? nd.steps[q] : 0;
+            t.backward_err = c.mixed || sw->verify ? nd.berr[q] : -1.0;
+            t.forward_est = c.mixed ? nd.fwd[q] : -1.0;
+            if (c.mixed)
+                for (int i = 0; i < 8; i++) t.refine_hist[i] = nd.hist[8 * q + i];
+            continue;
+        }
+        int rc = sweep_nodal_retry(sw, sl, q, (size_t)sl.f + q, c, &t, &sl.info[q]);
+        if (rc) return rc;
+        if (c.mixed) {
+            t.refine_iters += nd.steps[q];
+            sw->nodal_above = std::max(sw->nodal_above, 1.5 * sl.hz[q]);
+        } else {
+            sw->nodal64 = false;
+        }
+    }
+    return 0;
+}
+
 // Advances the group in flight on slot `sl`, whose stream has finished what
 // was queued: the mixed form checks its refinement and may queue another step
 // (*complete false); once complete the results are written. A singular sample
@@ -2453,31 +2571,38 @@ static int sweep_advance(tags_sweep* sw, SweepSlot& sl, const SweepCall& c, bool
     std::vector<tags_item_stats>& stt = sl.stt;
     std::vector<int>& info = sl.info;
     *complete = false;
-    int rc = c.mixed ? sl.sv.advance_mixed(sl.W.p, sl.rhs.p, stt.data(), info.data(), complete)
+    int rc;
+    if (sl.nodal_path) {
+        if ((rc = sl.nd.advance(complete)) || !*complete) return rc;
+        if ((rc = sweep_nodal_finish(sw, sl, c))) return rc;
+    } else {
+        rc = c.mixed ? sl.sv.advance_mixed(sl.W.p, sl.rhs.p, stt.data(), info.data(), complete)
                      : sl.sv.finish64(stt.data(), info.data());
-    if (rc < 0) return rc;
-    if (!c.mixed) *complete = true;
-    if (!*complete) return 0;
+        if (rc < 0) return rc;
+        if (!c.mixed) *complete = true;
+        if (!*complete) return 0;
+    }
     sl.f = -1;
     hipStream_t st = sl.stream.s;
-    if (!c.mixed && sw->verify)
+    if (!sl.nodal_path && !c.mixed && sw->verify)
         for (int z = 0; z < cnt; z++)
             if (info[z] == 0 &&
                 (rc = sweep_verify64(sw, sl, sl.W.p + (long)z * N * N, sl.rhs.p + (long)z * N,
                                      f0 + z, c, &stt[z])))
                 return rc;
-    std::vector<c64> xs((size_t)N * cnt);
-    TAGS_HIP(hipMemcpyAsync(xs.data(), sl.rhs.p, sizeof(c64) * N * cnt, hipMemcpyDeviceToHost,
-                            st));
-    TAGS_HIP(hipStreamSynchronize(st));
+    // the nodal solve has already brought U[inj]
+    const bool full = !sl.nodal_path || c.x_out;
+    std::vector<c64> xs(full ? (size_t)N * cnt : 0);
+    if (full) {
+        TAGS_HIP(hipMemcpyAsync(xs.data(), sl.nodal_path ? sl.nd.x : sl.rhs.p,
+                                sizeof(c64) * N * cnt, hipMemcpyDeviceToHost, st));
+        TAGS_HIP(hipStreamSynchronize(st));
+    }
     for (int z = 0; z < cnt; z++) {
         const size_t f = f0 + z;
         if (c.stats) c.stats[f] = stt[z];
         // a fallback factored this sample's W in FP64
         if (c.mixed && stt[z].precision_used != TAGS_PREC_MIXED) sl.static_items = 0;
-        if (sl.nodal &&
-            (stt[z].precision_used != TAGS_PREC_MIXED || stt[z].refine_iters > kHybridMaxIters))
-            sw->nodal_above = std::max(sw->nodal_above, 1.5 * sl.hz[z]);
         const c64* xz = xs.data() + (size_t)z * N;
         if (info[z] > 0) {
             const c64 nan = c64{NAN, NAN};
@@ -2486,7 +2611,8 @@ static int sweep_advance(tags_sweep* sw, SweepSlot& sl, const SweepCall& c, bool
                 for (long i = 0; i < N; i++) c.x_out[f * N + i] = to_c(nan);
             continue;
         }
-        if (c.u_inj) c.u_inj[f] = to_c(xz[L.node_off + (long)c.inj_node]);
+        if (c.u_inj)
+            c.u_inj[f] = to_c(sl.nodal_path ? sl.nd.hu[z] : xz[L.node_off + (long)c.inj_node]);
         if (c.x_out) {
             // reference order [U; I_L; I_T]
             TAGS_COMPLEX* xo = c.x_out + f * N;
@@ -2517,23 +2643,36 @@ int tags_sweep_solve(tags_sweep* sw, size_t nfreq, const TAGS_COMPLEX* s,
                  sw->plan_kind == TAGS_PLAN_GROUNDED_PIVOTED) && mixed
                     ? 1
                     : sweep_batch(sw, mixed);
+    sw->nd_batch = sweep_nd_batch(sw, mixed, nfreq);
     sw->batch_req = batch_req0;
     if (lu_panel_kind() == PANEL_PARTIAL) sw->batch = 1;
-    const int k = tu && tu->inflight > 0 ? tu->inflight : sw->inflight;
-    // every configured slot is allocated up front (a warm-up call sets all of
-    // them up)
-    int rc = sweep_slots(sw, k, mixed);
-    if (rc || (rc = sweep_potentials(sw))) return rc;
-    // after the slots exist: the layout sets every slot's plans
-    if ((rc = sweep_layout(sw))) return rc;
-    const SweepCall c{nfreq, s, kappa, gamma, ref_l, ref_t, mur, inj_node, mixed, u_inj, x_out,
-                      stats};
     // the hybrid plan's switch may rise during this call; it is restored at
     // the end, so that every call starts from the configured switch
     const double nodal_above0 = sw->nodal_above;
     const int gmres_steps0 = sw->gmres_steps;
+    auto restore = [&] {
+        sw->nodal_above = nodal_above0;
+        sw->gmres_steps = gmres_steps0;
+    };
     if (tu && mixed && tu->nodal_above >= 0.0) sw->nodal_above = tu->nodal_above;
     if (tu && mixed && tu->gmres_steps > 0) sw->gmres_steps = tu->gmres_steps;
+    sw->nodal64 = true;
+    // every slot the call can use is allocated up front (a warm-up call of the
+    // same length sets all of them up)
+    int rc = sweep_layout(sw);
+    const bool nodal = sweep_nodal(sw, mixed, INFINITY);
+    const size_t per = (size_t)(nodal ? sw->nd_batch : sw->batch);
+    const int k = (int)std::min<size_t>(tu && tu->inflight > 0 ? tu->inflight : sw->inflight,
+                                        (nfreq + per - 1) / per);
+    if (!rc) rc = sweep_slots(sw, k, mixed, nodal, !sweep_nodal(sw, mixed, 0.0));
+    // after the slots exist: the layout sets every slot's plans
+    if (!rc) rc = sweep_layout(sw);
+    if (rc || (rc = sweep_potentials(sw))) {
+        restore();
+        return rc;
+    }
+    const SweepCall c{nfreq, s, kappa, gamma, ref_l, ref_t, mur, inj_node, mixed, u_inj, x_out,
+                      stats};
     size_t next = 0;
     for (int i = 0; i < k && next < nfreq; i++) {
         const int got = sweep_issue(sw, *sw->slots[i], next, c);
@@ -2544,6 +2683,7 @@ int tags_sweep_solve(tags_sweep* sw, size_t nfreq, const TAGS_COMPLEX* s,
         next += (size_t)got;
     }
     // advance whichever slot's stream is idle; refill a slot whose group is done
+    Poll poll;
     while (!rc) {
         int busy = 0, ready = -1;
         for (int i = 0; i < k; i++) {
@@ -2558,9 +2698,10 @@ int tags_sweep_solve(tags_sweep* sw, size_t nfreq, const TAGS_COMPLEX* s,
         }
         if (!busy) break;
         if (ready < 0) {
-            std::this_thread::sleep_for(std::chrono::microseconds(20));
+            poll.wait();
             continue;
         }
+        poll.n = 0;
         SweepSlot& sl = *sw->slots[ready];
         bool complete = false;
         if ((rc = sweep_advance(sw, sl, c, &complete))) break;
@@ -2574,8 +2715,7 @@ int tags_sweep_solve(tags_sweep* sw, size_t nfreq, const TAGS_COMPLEX* s,
         }
     }
     // after an error: let every queued sample end before returning
-    sw->nodal_above = nodal_above0;
-    sw->gmres_steps = gmres_steps0;
+    restore();
     for (int i = 0; i < k; i++) {
         TAGS_HIP(hipStreamSynchronize(sw->slots[i]->stream.s));
         sw->slots[i]->f = -1;
@@ -2818,10 +2958,10 @@ int tags_sweep_autotune(tags_sweep* sw, int precision, size_t nprobe, const TAGS
     // 1. tile variants on the plan's own update shapes, per step width
     int rc = sweep_layout(sw);
     if (rc) return rc;
-    const LUPlan* plan = mixed ? (sw->plan_kind == TAGS_PLAN_HYBRID ? &sw->plan_nodal
-                                  : sw->bind32                      ? sw->bind32
-                                                                    : sw->bind64)
-                               : sw->bind64;
+    // (with the nodal solve: those of the factorisation that takes over where
+    // it is not accepted; its own products have one shape)
+    const bool nodal = sweep_nodal(sw, mixed, INFINITY);
+    const LUPlan* plan = mixed && sw->bind32 ? sw->bind32 : sw->bind64;
     if (!plan || plan->phases.empty()) return TAGS_ERR_ARG;
     const LUPhase* wide = &plan->phases[0];
     auto cols = [](const LUPhase& ph) {
@@ -2899,14 +3039,14 @@ int tags_sweep_autotune(tags_sweep* sw, int precision, size_t nprobe, const TAGS
         }
         return 0;
     };
-    {
+    if (!nodal) {
         tags_tuning c = cur;
         c.step_width = widths[1 - w0];
         c.gemm_big = big[1 - w0];
         c.gemm_small = small[1 - w0];
         if ((rc = consider(c))) return fail(rc);
     }
-    {
+    if (!nodal) {
         // the runner-up of the product timings, on the probe solves (the
         // timings see two product sizes, the solves the whole factorisation)
         const int wi = cur.step_width == widths[0] ? 0 : 1;
@@ -2917,11 +3057,13 @@ int tags_sweep_autotune(tags_sweep* sw, int precision, size_t nprobe, const TAGS
         }
     }
     for (int ch : {1, 2, 8}) {
+        if (nodal) break;
         tags_tuning c = cur;
         c.update_chunks = ch;
         if ((rc = consider(c))) return fail(rc);
     }
     for (int rows : {0, 1}) {
+        if (nodal) break;
         tags_tuning c = cur;
         c.solve_rows = rows;
         if ((rc = consider(c))) return fail(rc);
@@ -2933,7 +3075,7 @@ int tags_sweep_autotune(tags_sweep* sw, int precision, size_t nprobe, const TAGS
         if ((rc = consider(c))) return fail(rc);
     }
     if (sw->N < kBatchOneAbove) {
-        const int b0 = sweep_batch(sw, mixed);
+        const int b0 = nodal ? sweep_nd_batch(sw, mixed, nprobe) : sweep_batch(sw, mixed);
         for (int b : {b0 / 2, b0 / 4}) {
             if (b < 1 || b == b0) continue;
             tags_tuning c = cur;
@@ -2947,7 +3089,8 @@ int tags_sweep_autotune(tags_sweep* sw, int precision, size_t nprobe, const TAGS
         // device's memory
         size_t mem_free = 0, mem_total = 0;
         if (hipMemGetInfo(&mem_free, &mem_total) != hipSuccess) mem_total = 0;
-        const double per = (double)sw->N * (double)sw->N * (mixed ? 24.0 : 16.0);
+        const double per = nodal ? (double)NodalSolver::bytes(sw->m, sw->n, !mixed, 1)
+                                 : (double)sw->N * (double)sw->N * (mixed ? 24.0 : 16.0);
         const int k = cur.inflight > 0 ? cur.inflight : sw->inflight;
         for (int b = 2; b <= 4; b++) {
             if ((double)b * k * per > 0.8 * (double)mem_total) break;
@@ -2956,12 +3099,7 @@ int tags_sweep_autotune(tags_sweep* sw, int precision, size_t nprobe, const TAGS
             if ((rc = consider(c))) return fail(rc);
         }
     }
-    if (mixed && sw->plan_kind == TAGS_PLAN_HYBRID) {
-        tags_tuning c = cur;
-        c.nodal_above = cur.nodal_above > 0.0 ? 0.0 : 2e4;
-        if ((rc = consider(c))) return fail(rc);
-    }
-    if (mixed && (sw->plan_kind == TAGS_PLAN_HYBRID || sw->plan_kind == TAGS_PLAN_NODAL)) {
+    if (mixed && sw->plan_kind == TAGS_PLAN_NODAL) {
         for (int k : {6, 8, 10}) {
             if (k == (cur.gmres_steps > 0 ? cur.gmres_steps : sw->gmres_steps)) continue;
             tags_tuning c = cur;
@@ -3147,6 +3285,8 @@ int tags_cases_solve(tags_cases* cs, int precision)
                      sw->plan_kind == TAGS_PLAN_GROUNDED_PIVOTED) && mixed
                         ? 1
                         : sweep_batch(sw, mixed);
+        sw->nd_batch = sweep_nd_batch(sw, mixed, d.nfreq);
+        sw->nodal64 = true;
         sw->batch_req = batch_req0;
         if (lu_panel_kind() == PANEL_PARTIAL) sw->batch = 1;
         if ((rc = sweep_potentials(sw))) return rc;
@@ -3191,13 +3331,28 @@ int tags_cases_solve(tags_cases* cs, int precision)
             SweepSlot& L = *lp;
             for (size_t c : prep) {
                 tags_sweep* sw = cs->sw[c];
+                if ((rc = L.init_items(std::max(sw->batch, sw->nd_batch)))) return rc;
+                if (sweep_nodal(sw, mixed, 0.0)) continue;
                 if ((rc = L.init(sw->N, sw->batch)) ||
                     (rc = L.sv.ensure((int)sw->N, mixed, sw->batch)))
                     return rc;
-                if (mixed && (sw->plan_kind == TAGS_PLAN_HYBRID || sw->plan_kind == TAGS_PLAN_NODAL) &&
+                if (mixed && sw->plan_kind == TAGS_PLAN_NODAL &&
                     (rc = L.sv.gm.alloc((int)sw->N, sw->gmres_steps, sw->batch)))
                     return rc;
             }
+            // the nodal solve's arena, largest layout first
+            const tags_sweep* big = nullptr;
+            size_t most = 0;
+            for (size_t c = 0; c < nc; c++) {
+                const tags_sweep* sw = cs->sw[c];
+                if (!sweep_nodal(sw, mixed, INFINITY)) continue;
+                const size_t nbytes = NodalSolver::bytes(sw->m, sw->n, !mixed, sw->nd_batch);
+                if (nbytes > most) {
+                    most = nbytes;
+                    big = sw;
+                }
+            }
+            if (big && (rc = L.nd.ensure(big->hem, !mixed, big->nd_batch))) return rc;
         }
     }
     std::vector<long> lane_case(cs->nlanes, -1);
@@ -3207,8 +3362,10 @@ int tags_cases_solve(tags_cases* cs, int precision)
         const size_t c = order[qi];
         tags_sweep* sw = cs->sw[c];
         SweepSlot& L = *cs->lanes[li];
-        int r = L.init(sw->N, sw->batch);
-        if (r || (r = L.sv.ensure((int)sw->N, mixed, sw->batch))) return r;
+        int r;
+        if (sweep_nodal(sw, mixed, INFINITY) &&
+            (r = L.nd.ensure(sw->hem, !mixed, sw->nd_batch)))
+            return r;
         L.prof.on = cs->profiling;
         slot_bind(sw, L);
         // the case's tuned tile shapes and schedule, if any
@@ -3222,6 +3379,7 @@ int tags_cases_solve(tags_cases* cs, int precision)
     rc = 0;
     for (int li = 0; li < cs->nlanes && !rc; li++) rc = issue(li);
     // finish whichever lane is done first and refill it
+    Poll poll;
     while (!rc) {
         int busy = 0, done = -1;
         for (int li = 0; li < cs->nlanes; li++) {
@@ -3238,9 +3396,10 @@ int tags_cases_solve(tags_cases* cs, int precision)
         }
         if (!busy) break;
         if (done < 0) {
-            std::this_thread::sleep_for(std::chrono::microseconds(20));
+            poll.wait();
             continue;
         }
+        poll.n = 0;
         SweepSlot& L = *cs->lanes[done];
         const size_t c = (size_t)lane_case[done];
         bool complete = false;

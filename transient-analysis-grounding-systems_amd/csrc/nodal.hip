@@ -1,0 +1,1075 @@
+// Nodal solve of the HEM immittance system from explicit symmetric inverses,
+// batched over the frequency samples of a group.
+//
+//   [ -Z_L   0    A ] [i_L]   [r_L]
+//   [   0  -Z_T   B ] [i_T] = [r_T]     A, B: incidence, two entries per row
+//   [ A^T   B^T   0 ] [ u ]   [r_U]
+//
+// is solved by Y_L = Z_L^-1, Y_T = Z_T^-1, S = A^T Y_L A + B^T Y_T B and
+//   S u = r_U + A^T Y_L r_L + B^T Y_T r_T,  i_L = Y_L (A u - r_L),  i_T alike,
+// refined on W with double-double residuals. Z_L, Z_T and S are complex
+// symmetric with a definite real or imaginary part, so no row exchanges are
+// needed; a sample whose refinement does not meet the acceptance rule is left
+// to the caller's pivoted factorisation.
+//
+// Why explicit inverses: the blocked symmetric sweep below takes 4 dim^3 real
+// operations for an inverse (half of a general one's), all of them in one
+// shape of matrix product that does not shrink from step to step; the
+// incidence products with Y are gathers of four entries; and every solve of
+// the refinement is a matrix-vector product at memory speed, where triangular
+// solves are a chain of dependent blocks. For a 60 x 60 m grid (m = 7,440,
+// n = 6,541) that is 3.7e12 operations per sample, against 8.7e12 for the
+// block elimination with the node columns carried along and 1.84e13 for the
+// pivoted elimination.
+//
+// The node system. At low frequency |Y_L| >> |Y_T|, and the constant vector,
+// which A annihilates, has in S a quadratic form far below the rounding of
+// S's entries. So S_p = S + tau 1 1^T is inverted instead (tau: the mean
+// diagonal / n, so that the constant vector's eigenvalue is of the diagonal's
+// size), and the constant part alpha of u = alpha 1 + w follows from sums that
+// A does not enter: with c = S 1 = B^T (Y_T 1) and s = 1^T S 1 = sum(Y_T 1)
+// (A 1 = 0, B 1 = 1), h = S_p^-1 c, y = S_p^-1 f and F = 1^T f,
+//   alpha = (F - c^T y) / (s - c^T h),  w = y - alpha h.
+// A u = A w is then formed without alpha. In complex64 a refinement step then
+// contracts the error by 1e-2 .. 1e-4 at every frequency from 100 Hz to 10 MHz
+// (m = 30 .. 1320), where the plain S stalled below 20 kHz.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+
+#include "mfma.h"
+#include "nodal.h"
+
+namespace tags {
+
+// Work-group index over `total` pieces of work such that each XCD (blockIdx.x
+// mod 8) takes a contiguous range, so that the pieces of one item meet in one
+// L2; -1 past the end. The grid is 8 * ceil(total / 8).
+__device__ inline long xcd_flat(long total)
+{
+    const long per = (total + 7) / 8;
+    const long f = (long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    return f < total ? f : -1;
+}
+static unsigned xcd_grid(long total) { return (unsigned)(8 * ((total + 7) / 8)); }
+
+// One family of symmetric matrices being inverted: `items` matrices of order
+// dim in ld x ld storage (ld = dim rounded up to 64, zero beyond dim), of
+// which the 64 x 64 tiles on and below the diagonal are kept.
+template <typename T>
+struct NdPhase {
+    cx<T>* A;
+    long sA;
+    int ld, dim, items;
+    cx<T>*tp, *op;  // T and O of the current step in MFMA fragment order
+    long sp;
+    cx<T>* P;       // inverse of the current diagonal block
+};
+
+// Fragment order of a ld x NB panel: a wave's MFMA operand (16 rows, 4 k) is
+// 64 consecutive complex values; complex64 keeps two k groups side by side,
+// so that every lane loads 16 bytes.
+template <typename T, int NB>
+__device__ inline long nd_pk(int i, int k)
+{
+    if constexpr (sizeof(T) == 8)
+        return ((long)(i >> 4) * (NB / 4) + (k >> 2)) * 64 + (k & 3) * 16 + (i & 15);
+    else
+        return (((long)(i >> 4) * (NB / 8) + (k >> 3)) * 64 + (k & 3) * 16 + (i & 15)) * 2 +
+               ((k >> 2) & 1);
+}
+
+// ---------------------------------------------------------------------------
+// One step of the symmetric sweep for the block K = [c0, c0 + NB):
+//   P = A_KK^-1, T = A_*K P, A_ij -= T_i A_jK^T, A_*K = T, A_KK = -P;
+// after all steps A holds -A^-1. Every matrix in between is symmetric, rows
+// before and after K are treated alike, and only tiles on and below the
+// diagonal are touched.
+// ---------------------------------------------------------------------------
+
+// P by an unblocked sweep, one work-group of 1024 threads per item: thread t
+// holds NB^2 / 1024 entries of one row in registers; per step the pivot row
+// goes through LDS (it is the pivot column too), one barrier. Latency-bound:
+// NB steps of a broadcast, a reciprocal and NB^2 / 1024 multiply-adds.
+template <typename T, int NB>
+__global__ __launch_bounds__(1024) void k_nd_diag(NdPhase<T> p, int kb)
+{
+    constexpr int TPR = 1024 / NB, E = NB / TPR;
+    const cx<T>* A = p.A + (long)blockIdx.x * p.sA;
+    cx<T>* P = p.P + (long)blockIdx.x * NB * NB;
+    const int c0 = kb * NB, kv = min(NB, p.dim - c0);
+    const int r = threadIdx.x / TPR, q = threadIdx.x % TPR;
+    __shared__ cx<T> row[2][NB];
+    cx<T> a[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int c = q + TPR * e;
+        a[e] = cx<T>{0, 0};
+        if (r < kv && c < kv) a[e] = A[(long)(c0 + max(r, c)) * p.ld + c0 + min(r, c)];
+    }
+    for (int j = 0; j < kv; j++) {
+        cx<T>* rj = row[j & 1];
+        if (r == j) {
+#pragma unroll
+            for (int e = 0; e < E; e++) rj[q + TPR * e] = a[e];
+        }
+        __syncthreads();
+        const cx<T> d = crecip_fast(rj[j]);
+        const cx<T> l = cmul(rj[r], d);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int c = q + TPR * e;
+            const cx<T> o = rj[c];
+            const cx<T> upd = cfnma(a[e], l, o);
+            const cx<T> own = cmul(o, d);
+            cx<T> nv = csel(r == j, own, csel(c == j, l, upd));
+            if (r == j && c == j) nv = cx<T>{-d.x, -d.y};
+            a[e] = nv;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int c = q + TPR * e;
+        const bool in = r < kv && c < kv;
+        P[r * NB + c] = in ? cx<T>{-a[e].x, -a[e].y} : cx<T>{0, 0};
+    }
+}
+
+// O(i, k) of the current panel: A_iK from the stored tiles (rows before K from
+// the row block, transposed).
+template <typename T>
+__device__ inline cx<T> nd_panel_at(const cx<T>* A, long ld, int i, int c, bool before)
+{
+    return before ? A[(long)c * ld + i] : A[(long)i * ld + c];
+}
+
+// T = O P for 64 rows and 64 columns of the panel, with T and O written in
+// fragment order for the update. Four waves of 16 rows; operands straight from
+// memory (O is read once per 64 columns, P stays in L2).
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int kb)
+{
+    using V4 = typename Mfma<T>::v4;
+    constexpr int YC = NB / 64;
+    const int nt = p.ld / 64;
+    const long flat = xcd_flat((long)p.items * nt * YC);
+    if (flat < 0) return;
+    const int item = (int)(flat / (nt * YC)), rem = (int)(flat % (nt * YC));
+    const int rb = rem / YC, yc = rem % YC;
+    const int c0 = kb * NB;
+    if (rb * 64 >= c0 && rb * 64 < c0 + NB) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i0 = rb * 64 + wave * 16;
+    if (i0 >= p.dim) return;
+    const bool before = rb * 64 < c0;
+    const int kv = min(NB, p.dim - c0);
+    const cx<T>* A = p.A + (long)item * p.sA;
+    const cx<T>* P = p.P + (long)item * NB * NB + yc * 64;
+    cx<T>* tp = p.tp + (long)item * p.sp;
+    cx<T>* op = p.op + (long)item * p.sp;
+    const int lr = lane & 15, lk = lane >> 4;
+    V4 re[4], im[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        re[t] = V4{0, 0, 0, 0};
+        im[t] = V4{0, 0, 0, 0};
+    }
+#pragma unroll 4
+    for (int g = 0; g < NB / 4; g++) {
+        const int k = 4 * g + lk;
+        cx<T> a{0, 0};
+        if (k < kv) a = nd_panel_at(A, p.ld, i0 + lr, c0 + k, before);
+        if (yc == 0) op[nd_pk<T, NB>(i0 + lr, k)] = a;
+        const T na = -a.y;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const cx<T> b = P[k * NB + t * 16 + lr];
+            re[t] = Mfma<T>::run(a.x, b.x, re[t]);
+            im[t] = Mfma<T>::run(a.x, b.y, im[t]);
+            re[t] = Mfma<T>::run(na, b.y, re[t]);
+            im[t] = Mfma<T>::run(a.y, b.x, im[t]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            tp[nd_pk<T, NB>(i0 + Mfma<T>::row(lane, v), yc * 64 + t * 16 + lr)] =
+                cx<T>{re[t][v], im[t][v]};
+}
+
+// row and column tile of index t of a triangle's tiles (row >= column)
+__device__ inline void tri_tile(int t, int& ti, int& tj)
+{
+    ti = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+    while ((ti + 1) * (ti + 2) / 2 <= t) ti++;
+    while (ti * (ti + 1) / 2 > t) ti--;
+    tj = t - ti * (ti + 1) / 2;
+}
+
+// Tiles of block K after the update: A_*K = T, A_KK = -P. ti, tj: 64 x 64 tile.
+template <typename T, int NB>
+__device__ inline void nd_place(const NdPhase<T>& p, cx<T>* A, int item, int c0, int ti, int tj,
+                                bool inrow, bool incol)
+{
+    const cx<T>* tp = p.tp + (long)item * p.sp;
+    const cx<T>* P = p.P + (long)item * NB * NB;
+    for (int e = threadIdx.x; e < 4096; e += 256) {
+        const int i = ti * 64 + (e >> 6), j = tj * 64 + (e & 63);
+        if (i >= p.dim || j >= p.dim) continue;
+        cx<T> t;
+        if (inrow && incol) {
+            t = P[(i - c0) * NB + j - c0];
+            t = cx<T>{-t.x, -t.y};
+        } else if (incol) {
+            t = tp[nd_pk<T, NB>(i, j - c0)];
+        } else {
+            t = tp[nd_pk<T, NB>(j, i - c0)];
+        }
+        A[(long)i * p.ld + j] = t;
+    }
+}
+
+// A_ij -= T_i O_j^T on 64 x 64 tiles: four waves of 32 x 32, operands in
+// fragment order straight from L2 (a wave needs 4 bytes per cycle of them
+// beside its MFMAs, so LDS staging would only add barriers).
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void k_nd_update(NdPhase<T> p, int kb)
+{
+    using V4 = typename Mfma<T>::v4;
+    constexpr int KG = sizeof(T) == 8 ? 4 : 8;  // k per 16-byte lane load
+    constexpr int KU = KG / 4;
+    struct alignas(16) Frag {
+        cx<T> e[KU];
+    };
+    const int nt = p.ld / 64, ntri = nt * (nt + 1) / 2;
+    const long flat = xcd_flat((long)p.items * ntri);
+    if (flat < 0) return;
+    const int item = (int)(flat / ntri);
+    int ti, tj;
+    tri_tile((int)(flat % ntri), ti, tj);
+    const int c0 = kb * NB, k0 = c0 / 64;
+    cx<T>* A = p.A + (long)item * p.sA;
+    const bool inrow = ti >= k0 && ti < k0 + NB / 64, incol = tj >= k0 && tj < k0 + NB / 64;
+    if (inrow || incol) {
+        nd_place<T, NB>(p, A, item, c0, ti, tj, inrow, incol);
+        return;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i0 = ti * 64 + (wave >> 1) * 32, j0 = tj * 64 + (wave & 1) * 32;
+    if (i0 >= p.dim || j0 >= p.dim || j0 > i0 + 31) return;
+    const int ng = (min(NB, p.dim - c0) + KG - 1) / KG;
+    constexpr long FS = (long)(NB / KG) * 64;  // fragments of one 16-row strip
+    const Frag* ta = (const Frag*)(p.tp + (long)item * p.sp) + (i0 / 16) * FS + lane;
+    const Frag* ob = (const Frag*)(p.op + (long)item * p.sp) + (j0 / 16) * FS + lane;
+    V4 re[2][2], im[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            re[i][j] = V4{0, 0, 0, 0};
+            im[i][j] = V4{0, 0, 0, 0};
+        }
+    Frag a[2], b[2], an[2], bn[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        a[i] = ta[i * FS];
+        b[i] = ob[i * FS];
+    }
+    for (int g = 0; g < ng; g++) {
+        const long o = (long)min(g + 1, ng - 1) * 64;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            an[i] = ta[i * FS + o];
+            bn[i] = ob[i * FS + o];
+        }
+#pragma unroll
+        for (int u = 0; u < KU; u++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const cx<T> x = a[i].e[u], y = b[j].e[u];
+                    re[i][j] = Mfma<T>::run(x.x, y.x, re[i][j]);
+                    im[i][j] = Mfma<T>::run(x.x, y.y, im[i][j]);
+                    re[i][j] = Mfma<T>::run(-x.y, y.y, re[i][j]);
+                    im[i][j] = Mfma<T>::run(x.y, y.x, im[i][j]);
+                }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            a[i] = an[i];
+            b[i] = bn[i];
+        }
+    }
+    // a strip past dim holds no operands
+    const bool j1 = j0 + 16 < p.dim;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        if (i0 + 16 * i >= p.dim) break;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            cx<T>* cr = A + (long)(i0 + 16 * i + Mfma<T>::row(lane, v)) * p.ld + j0 + (lane & 15);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                if (j && !j1) break;
+                const cx<T> o = cr[16 * j];
+                cr[16 * j] = cx<T>{o.x - re[i][j][v], o.y - im[i][j][v]};
+            }
+        }
+    }
+}
+
+// A_ij of the tiles above the diagonal from those below, 64 x 64 tiles through
+// LDS; the diagonal tiles' own upper halves too.
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_mirror(cx<T>* A, long sA, int ld, int items)
+{
+    const int nt = ld / 64, ntri = nt * (nt + 1) / 2;
+    const long flat = xcd_flat((long)items * ntri);
+    if (flat < 0) return;
+    A += (flat / ntri) * sA;
+    int ti, tj;
+    tri_tile((int)(flat % ntri), ti, tj);
+    __shared__ cx<T> t[64][33];
+    for (int half = 0; half < 2; half++) {
+        // columns 32 half .. + 31 of tile (ti, tj)
+        for (int e = threadIdx.x; e < 2048; e += 256) {
+            const int r = e >> 5, c = e & 31;
+            t[r][c] = A[(long)(ti * 64 + r) * ld + tj * 64 + 32 * half + c];
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < 2048; e += 256) {
+            const int c = e >> 6, r = e & 63;
+            if (ti != tj || r > 32 * half + c)
+                A[(long)(tj * 64 + 32 * half + c) * ld + ti * 64 + r] = t[r][c];
+        }
+        __syncthreads();
+    }
+}
+
+// F = Z in T (tiles on and below the diagonal, zero past m), item 2 q the Z_L
+// block of sample q, 2 q + 1 its Z_T block.
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_load(const c64* Z, long sZ, cx<T>* F, int ld, int m,
+                                                  int items)
+{
+    const int nt = ld / 64, ntri = nt * (nt + 1) / 2;
+    const long flat = xcd_flat((long)items * ntri);
+    if (flat < 0) return;
+    const long item = flat / ntri;
+    int ti, tj;
+    tri_tile((int)(flat % ntri), ti, tj);
+    const c64* src = Z + (item >> 1) * sZ + (item & 1) * ((long)m * m + m);
+    F += item * (long)ld * ld;
+    for (int e = threadIdx.x; e < 4096; e += 256) {
+        const int i = ti * 64 + (e >> 6), j = tj * 64 + (e & 63);
+        cx<T> o{0, 0};
+        if (i < m && j < m) {
+            const c64 s = src[(long)i * m + j];
+            o = cx<T>{(T)s.x, (T)s.y};
+        }
+        F[(long)i * ld + j] = o;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The node system
+// ---------------------------------------------------------------------------
+template <typename T>
+struct NdArgs {
+    int nb;
+    long m, n, mp, np, N;
+    const cx<T>* F;  // Y_L, Y_T (after the sweep)
+    cx<T>* S;
+    c64 *x, *r, *ysum, *dg, *cst;
+    cx<T>*v, *z, *f, *y, *h, *c;
+    const int *sn, *en, *node_ptr, *node_seg;
+    unsigned long long* norms;
+    long snorm;
+    const int* active;
+    long inj;
+};
+
+__device__ inline c64 wave_sum(c64 a)
+{
+    for (int o = 32; o > 0; o >>= 1) {
+        a.x += __shfl_xor(a.x, o);
+        a.y += __shfl_xor(a.y, o);
+    }
+    return a;
+}
+
+// ysum_i = (Y_T 1)_i and the diagonal's share dg_i = 2 Y_L,ii + Y_T,ii / 2; one
+// wave per row
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_rows(NdArgs<T> g)
+{
+    const long wg = (g.m + 3) / 4;
+    const long item = blockIdx.x / wg, i = (blockIdx.x % wg) * 4 + (threadIdx.x >> 6);
+    if (i >= g.m) return;
+    const int lane = threadIdx.x & 63;
+    const cx<T>* yl = g.F + 2 * item * g.mp * g.mp + i * g.mp;
+    const cx<T>* yt = yl + g.mp * g.mp;
+    c64 s{0, 0};
+    for (long c = lane; c < g.m; c += 64) {
+        s.x += yt[c].x;
+        s.y += yt[c].y;
+    }
+    s = wave_sum(s);
+    if (lane == 0) {
+        g.ysum[item * g.m + i] = s;
+        g.dg[item * g.m + i] = c64{2.0 * yl[i].x + 0.5 * yt[i].x, 2.0 * yl[i].y + 0.5 * yt[i].y};
+    }
+}
+
+__device__ inline c64 wg_sum(c64 a, c64* red)
+{
+    a = wave_sum(a);
+    const int nw = blockDim.x >> 6;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
+    __syncthreads();
+    c64 t{0, 0};
+    for (int i = 0; i < nw; i++) t = cadd(t, red[i]);
+    return t;
+}
+
+// tau, s and c of each item (one work-group)
+template <typename T>
+__global__ __launch_bounds__(1024) void k_nd_const(NdArgs<T> g)
+{
+    __shared__ c64 red[16];
+    const long item = blockIdx.x;
+    const c64 *ys = g.ysum + item * g.m, *dg = g.dg + item * g.m;
+    c64 a{0, 0}, d{0, 0};
+    for (long i = threadIdx.x; i < g.m; i += 1024) {
+        a = cadd(a, ys[i]);
+        d = cadd(d, dg[i]);
+    }
+    a = wg_sum(a, red);
+    d = wg_sum(d, red);
+    if (threadIdx.x == 0) {
+        const double s = 1.0 / ((double)g.n * (double)g.n);
+        g.cst[4 * item] = c64{d.x * s, d.y * s};
+        g.cst[4 * item + 1] = a;
+    }
+    for (long u = threadIdx.x; u < g.np; u += 1024) {
+        c64 t{0, 0};
+        if (u < g.n)
+            for (int p = g.node_ptr[u]; p < g.node_ptr[u + 1]; p++)
+                t = cadd(t, ys[g.node_seg[p] >> 1]);
+        g.c[item * g.np + u] = cx<T>{(T)(0.5 * t.x), (T)(0.5 * t.y)};
+    }
+}
+
+// -S_p on and below the diagonal (16 x 16 entries per work-group, zero past
+// n): four gathered entries of Y_L and Y_T per pair of segment ends.
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_schur(NdArgs<T> g)
+{
+    const int nt = (int)(g.np / 16), ntri = nt * (nt + 1) / 2;
+    const long flat = xcd_flat((long)g.nb * ntri);
+    if (flat < 0) return;
+    const long item = flat / ntri;
+    int ti, tj;
+    tri_tile((int)(flat % ntri), ti, tj);
+    const long u = ti * 16 + (threadIdx.x >> 4), w = tj * 16 + (threadIdx.x & 15);
+    const cx<T>* yl = g.F + 2 * item * g.mp * g.mp;
+    const cx<T>* yt = yl + g.mp * g.mp;
+    cx<T> o{0, 0};
+    if (u < g.n && w < g.n) {
+        const int p0 = g.node_ptr[u], p1 = g.node_ptr[u + 1];
+        const int q0 = g.node_ptr[w], q1 = g.node_ptr[w + 1];
+        c64 s = g.cst[4 * item];
+        for (int p = p0; p < p1; p++) {
+            const int a = g.node_seg[p];
+            const cx<T>* rl = yl + (a >> 1) * g.mp;
+            const cx<T>* rt = yt + (a >> 1) * g.mp;
+            for (int q = q0; q < q1; q++) {
+                const int b = g.node_seg[q];
+                const double sg = ((a ^ b) & 1) ? -1.0 : 1.0;
+                const cx<T> l = rl[b >> 1], t = rt[b >> 1];
+                s.x += sg * l.x + 0.25 * t.x;
+                s.y += sg * l.y + 0.25 * t.y;
+            }
+        }
+        o = cx<T>{(T)-s.x, (T)-s.y};
+    }
+    g.S[item * g.np * g.np + u * g.np + w] = o;
+}
+
+// out = M in for symmetric matrices, four rows per wave, 16 bytes per lane and
+// row: HBM-bound (one read of M). BLK 2: the Y blocks of each item, with in /
+// out of 2 mp values; BLK 1: the node inverse.
+template <typename T, int BLK>
+__device__ inline void nd_gemv_rows(const NdArgs<T>& g, const cx<T>* in, long item, int blk,
+                                    long row0, cx<T> (&acc)[4])
+{
+    const long ld = BLK == 2 ? g.mp : g.np;
+    const cx<T>* M = BLK == 2 ? g.F + (2 * item + blk) * ld * ld : g.S + item * ld * ld;
+    const cx<T>* xv = in + (BLK == 2 ? (2 * item + blk) * ld : item * ld);
+    constexpr int V = 16 / sizeof(cx<T>);
+    struct alignas(16) Vec {
+        cx<T> e[V];
+    };
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < 4; q++) acc[q] = cx<T>{0, 0};
+#pragma unroll 2
+    for (long c = (long)lane * V; c < ld; c += 64 * V) {
+        const Vec xx = *(const Vec*)(xv + c);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const Vec a = *(const Vec*)(M + (row0 + q) * ld + c);
+#pragma unroll
+            for (int e = 0; e < V; e++) {
+                const cx<T> s = a.e[e], t = xx.e[e];
+                acc[q].x = fma(s.x, t.x, fma(-s.y, t.y, acc[q].x));
+                acc[q].y = fma(s.x, t.y, fma(s.y, t.x, acc[q].y));
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        for (int o = 32; o > 0; o >>= 1) {
+            acc[q].x += __shfl_xor(acc[q].x, o);
+            acc[q].y += __shfl_xor(acc[q].y, o);
+        }
+}
+
+template <typename T, int BLK>
+__global__ __launch_bounds__(256) void k_nd_gemv(NdArgs<T> g, const cx<T>* in, cx<T>* out)
+{
+    const long ld = BLK == 2 ? g.mp : g.np, wg = ld / 16;
+    const long flat = xcd_flat((long)g.nb * BLK * wg);
+    if (flat < 0) return;
+    const long mat = flat / wg, item = mat / BLK;
+    if (g.active && !g.active[item]) return;
+    const long row0 = (flat % wg) * 16 + (threadIdx.x >> 6) * 4;
+    cx<T> acc[4];
+    nd_gemv_rows<T, BLK>(g, in, item, (int)(mat % BLK), row0, acc);
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[mat * ld + row0 + q] = acc[q];
+    }
+}
+
+// 1 / (s - c^T h) (one work-group per item)
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_den(NdArgs<T> g)
+{
+    __shared__ c64 red[4];
+    const long item = blockIdx.x;
+    c64 a{0, 0};
+    for (long u = threadIdx.x; u < g.n; u += 256) {
+        const cx<T> c = g.c[item * g.np + u], h = g.h[item * g.np + u];
+        a = cadd(a, cmul(c64{c.x, c.y}, c64{h.x, h.y}));
+    }
+    a = wg_sum(a, red);
+    if (threadIdx.x == 0) g.cst[4 * item + 2] = crecip(csub(g.cst[4 * item + 1], a));
+}
+
+__device__ inline double nd_scale(const unsigned long long* rn, bool single)
+{
+    if (!single) return 1.0;
+    const double s = __longlong_as_double((long long)*rn);
+    return s > 0.0 ? s : 1.0;
+}
+
+// v = r_L, r_T (complex64: over |r|, so that the correction stays in range)
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_in(NdArgs<T> g, int kprev)
+{
+    const long item = blockIdx.y;
+    if (g.active && !g.active[item]) return;
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= 2 * g.m) return;
+    const double s = 1.0 / nd_scale(g.norms + item * g.snorm + 4 * kprev, sizeof(T) == 4);
+    const c64 r = g.r[item * g.N + i];
+    const long o = i < g.m ? i : g.mp + i - g.m;
+    g.v[2 * item * g.mp + o] = cx<T>{(T)(r.x * s), (T)(r.y * s)};
+}
+
+// f = r_U + A^T z_L + B^T z_T
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_node(NdArgs<T> g, int kprev)
+{
+    const long item = blockIdx.y;
+    if (g.active && !g.active[item]) return;
+    const long u = (long)blockIdx.x * 256 + threadIdx.x;
+    if (u >= g.n) return;
+    const double s = 1.0 / nd_scale(g.norms + item * g.snorm + 4 * kprev, sizeof(T) == 4);
+    const c64 r = g.r[item * g.N + 2 * g.m + u];
+    c64 t{r.x * s, r.y * s};
+    const cx<T>* zl = g.z + 2 * item * g.mp;
+    const cx<T>* zt = zl + g.mp;
+    for (int p = g.node_ptr[u]; p < g.node_ptr[u + 1]; p++) {
+        const int a = g.node_seg[p];
+        const double sg = (a & 1) ? -1.0 : 1.0;
+        t.x += sg * zl[a >> 1].x + 0.5 * zt[a >> 1].x;
+        t.y += sg * zl[a >> 1].y + 0.5 * zt[a >> 1].y;
+    }
+    g.f[item * g.np + u] = cx<T>{(T)t.x, (T)t.y};
+}
+
+__device__ inline void dx_max(unsigned long long* p, double a)
+{
+    for (int o = 32; o > 0; o >>= 1) a = fmax(a, __shfl_xor(a, o));
+    if ((threadIdx.x & 63) == 0) atomicMax(p, (unsigned long long)__double_as_longlong(a));
+}
+
+// alpha and w (y is replaced by w), u += scale (w + alpha), and the segments'
+// A w - r_L, B u - r_T into v; one work-group per item. first: r is the unit
+// current at node inj, so f = e_inj, y is a row of the node inverse and r_L,
+// r_T are zero.
+template <typename T>
+__global__ __launch_bounds__(1024) void k_nd_alpha(NdArgs<T> g, int k, int first)
+{
+    __shared__ c64 red[16];
+    const long item = blockIdx.x;
+    if (g.active && !g.active[item]) return;
+    const unsigned long long* rn = g.norms + item * g.snorm + 4 * (k - 1);
+    const double scale = first ? 1.0 : nd_scale(rn, sizeof(T) == 4);
+    cx<T>* y = g.y + item * g.np;
+    const cx<T>*h = g.h + item * g.np, *c = g.c + item * g.np;
+    const cx<T>* yin = first ? g.S + item * g.np * g.np + g.inj * g.np : y;
+    const c64* r = g.r + item * g.N;
+    c64* x = g.x + item * g.N;
+    c64 a{0, 0};
+    for (long u = threadIdx.x; u < g.n; u += 1024) {
+        const cx<T> cu = c[u], yu = yin[u];
+        a = csub(a, cmul(c64{cu.x, cu.y}, c64{yu.x, yu.y}));
+        if (!first) a = cadd(a, c64{r[2 * g.m + u].x / scale, r[2 * g.m + u].y / scale});
+    }
+    if (!first) {
+        const cx<T>* zt = g.z + (2 * item + 1) * g.mp;
+        for (long i = threadIdx.x; i < g.m; i += 1024) a = cadd(a, c64{zt[i].x, zt[i].y});
+    }
+    a = wg_sum(a, red);
+    if (first) a.x += 1.0;
+    const c64 al = cmul(a, g.cst[4 * item + 2]);
+    double dm = 0.0;
+    for (long u = threadIdx.x; u < g.n; u += 1024) {
+        const cx<T> hu = h[u], yu = yin[u];
+        const c64 w = csub(c64{yu.x, yu.y}, cmul(al, c64{hu.x, hu.y}));
+        y[u] = cx<T>{(T)w.x, (T)w.y};
+        const c64 d = cscale(cadd(w, al), scale);
+        x[2 * g.m + u] = first ? d : cadd(x[2 * g.m + u], d);
+        dm = fmax(dm, sqrt(d.x * d.x + d.y * d.y));
+    }
+    dx_max(g.norms + item * g.snorm + 4 * k + 3, dm);
+    __syncthreads();
+    cx<T>* vl = g.v + 2 * item * g.mp;
+    cx<T>* vt = vl + g.mp;
+    const double inv = 1.0 / scale;
+    for (long i = threadIdx.x; i < g.m; i += 1024) {
+        const cx<T> ws = y[g.sn[i]], we = y[g.en[i]];
+        c64 l{(double)ws.x - we.x, (double)ws.y - we.y};
+        c64 t{0.5 * ((double)ws.x + we.x) + al.x, 0.5 * ((double)ws.y + we.y) + al.y};
+        if (!first) {
+            l = csub(l, cscale(r[i], inv));
+            t = csub(t, cscale(r[g.m + i], inv));
+        }
+        vl[i] = cx<T>{(T)l.x, (T)l.y};
+        vt[i] = cx<T>{(T)t.x, (T)t.y};
+    }
+}
+
+// i_L, i_T += scale Y v
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_currents(NdArgs<T> g, int k, int first)
+{
+    const long wg = g.mp / 16;
+    const long flat = xcd_flat((long)g.nb * 2 * wg);
+    if (flat < 0) return;
+    const long mat = flat / wg, item = mat >> 1;
+    if (g.active && !g.active[item]) return;
+    const long row0 = (flat % wg) * 16 + (threadIdx.x >> 6) * 4;
+    if (row0 >= g.m) return;
+    cx<T> acc[4];
+    nd_gemv_rows<T, 2>(g, g.v, item, (int)(mat & 1), row0, acc);
+    const int lane = threadIdx.x & 63;
+    double dm = 0.0;
+    if (lane < 4 && row0 + lane < g.m) {
+        const double s =
+            first ? 1.0 : nd_scale(g.norms + item * g.snorm + 4 * (k - 1), sizeof(T) == 4);
+        const cx<T> a = csel(lane < 2, csel(lane == 0, acc[0], acc[1]),
+                             csel(lane == 2, acc[2], acc[3]));
+        const c64 d{a.x * s, a.y * s};
+        c64* xi = g.x + item * g.N + (mat & 1) * g.m + row0 + lane;
+        *xi = first ? d : cadd(*xi, d);
+        dm = sqrt(d.x * d.x + d.y * d.y);
+    }
+    dx_max(g.norms + item * g.snorm + 4 * k + 3, dm);
+}
+
+// b = e_inj, zeroed norms, zero padding of the vectors
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_init(NdArgs<T> g, c64* b)
+{
+    const long item = blockIdx.y;
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i < g.N) b[item * g.N + i] = c64{i == 2 * g.m + g.inj ? 1.0 : 0.0, 0.0};
+    if (i < g.snorm) g.norms[item * g.snorm + i] = 0;
+    const cx<T> zero{0, 0};
+    if (i < 2 * g.mp) g.v[2 * item * g.mp + i] = zero;
+    if (i < g.np) g.f[item * g.np + i] = zero;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_nd_pick(NdArgs<T> g, c64* u)
+{
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    if (q < g.nb) u[q] = g.x[q * g.N + 2 * g.m + g.inj];
+}
+
+// ---------------------------------------------------------------------------
+// host
+// ---------------------------------------------------------------------------
+// Columns per sweep step: a step costs one diagonal-block sweep (latency) and
+// reads and writes every tile once, so wider steps pay once the tiles
+// outweigh the panel's work.
+constexpr int kWideDim = 600;
+static int nd_block(long dim) { return dim >= kWideDim ? 128 : 64; }
+static long up(long v, long a) { return (v + a - 1) / a * a; }
+
+template <typename T>
+size_t NodalSolver::partition(char* base, int batch)
+{
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        char* p = base + off;
+        off += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    const size_t B = (size_t)batch, e = sizeof(cx<T>);
+    const long bz = nd_block(m), bs = nd_block(n);
+    const size_t panel = std::max(2 * (size_t)mp * bz, (size_t)np * bs);
+    const size_t diag = (size_t)std::max(2 * bz * bz, bs * bs);
+    sZ = nodal_z_items(m);
+    Z = (c64*)take(sizeof(c64) * sZ * B);
+    F = take(e * 2 * mp * mp * B);
+    S = take(e * np * np * B);
+    tp = take(e * panel * B);
+    op_ = take(e * panel * B);
+    P = take(e * diag * B);
+    x = (c64*)take(sizeof(c64) * N * B);
+    r = (c64*)take(sizeof(c64) * N * B);
+    b = (c64*)take(sizeof(c64) * N * B);
+    ysum = (c64*)take(sizeof(c64) * m * B);
+    dg = (c64*)take(sizeof(c64) * m * B);
+    cst = (c64*)take(sizeof(c64) * 4 * B);
+    v = take(e * 2 * mp * B);
+    z = take(e * 2 * mp * B);
+    f = take(e * np * B);
+    y = take(e * np * B);
+    h = take(e * np * B);
+    c = take(e * np * B);
+    u = (c64*)take(sizeof(c64) * B);
+    norms = (unsigned long long*)take(sizeof(unsigned long long) * kNormStride * B);
+    active = (int*)take(sizeof(int) * B);
+    return off;
+}
+
+size_t NodalSolver::bytes(long m_, long n_, bool f64_, int batch)
+{
+    NodalSolver t;
+    t.m = m_;
+    t.n = n_;
+    t.N = n_ + 2 * m_;
+    t.mp = up(m_, 64);
+    t.np = up(n_, 64);
+    return f64_ ? t.partition<double>(nullptr, batch) : t.partition<float>(nullptr, batch);
+}
+
+int NodalSolver::ensure(const HemOp& hem, bool f64_, int batch)
+{
+    if (batch < 1 || hem.m < 1 || hem.n < 1) return TAGS_ERR_ARG;
+    op = hem;
+    op.zl_off = 0;
+    op.zt_off = hem.m;
+    op.node_off = 2 * hem.m;
+    m = hem.m;
+    n = hem.n;
+    N = n + 2 * m;
+    mp = up(m, 64);
+    np = up(n, 64);
+    f64 = f64_;
+    const size_t need = bytes(m, n, f64, batch);
+    if (need > arena_bytes) {
+        hipFree(arena);
+        arena = nullptr;
+        arena_bytes = 0;
+        TAGS_HIP(hipMalloc(&arena, need));
+        arena_bytes = need;
+    }
+    if (f64) partition<double>(arena, batch);
+    else partition<float>(arena, batch);
+    if (batch > host_cap) {
+        if (hnorms) hipHostFree(hnorms);
+        if (hu) hipHostFree(hu);
+        if (hactive) hipHostFree(hactive);
+        hnorms = nullptr;
+        hu = nullptr;
+        hactive = nullptr;
+        host_cap = 0;
+        TAGS_HIP(hipHostMalloc(&hnorms, sizeof(unsigned long long) * kNormStride * batch, 0));
+        TAGS_HIP(hipHostMalloc(&hu, sizeof(c64) * batch, 0));
+        TAGS_HIP(hipHostMalloc(&hactive, sizeof(int) * batch, 0));
+        host_cap = batch;
+    }
+    cap = batch;
+    return 0;
+}
+
+void NodalSolver::release()
+{
+    hipFree(arena);
+    if (hnorms) hipHostFree(hnorms);
+    if (hu) hipHostFree(hu);
+    if (hactive) hipHostFree(hactive);
+    arena = nullptr;
+    hnorms = nullptr;
+    hu = nullptr;
+    hactive = nullptr;
+    arena_bytes = 0;
+    host_cap = cap = 0;
+}
+
+template <typename T>
+static NdArgs<T> nd_args(NodalSolver& s, bool masked)
+{
+    NdArgs<T> g;
+    g.nb = s.nb;
+    g.m = s.m;
+    g.n = s.n;
+    g.mp = s.mp;
+    g.np = s.np;
+    g.N = s.N;
+    g.F = (const cx<T>*)s.F;
+    g.S = (cx<T>*)s.S;
+    g.x = s.x;
+    g.r = s.r;
+    g.ysum = s.ysum;
+    g.dg = s.dg;
+    g.cst = s.cst;
+    g.v = (cx<T>*)s.v;
+    g.z = (cx<T>*)s.z;
+    g.f = (cx<T>*)s.f;
+    g.y = (cx<T>*)s.y;
+    g.h = (cx<T>*)s.h;
+    g.c = (cx<T>*)s.c;
+    g.sn = s.op.sn;
+    g.en = s.op.en;
+    g.node_ptr = s.op.node_ptr;
+    g.node_seg = s.op.node_seg;
+    g.norms = s.norms;
+    g.snorm = NodalSolver::kNormStride;
+    g.active = masked ? s.active : nullptr;
+    g.inj = s.inj;
+    return g;
+}
+
+// A = -A^-1 for every item of the phase, then both triangles
+template <typename T, int NB>
+static int nd_sweep(const NdPhase<T>& p, hipStream_t st, Profiler* pr)
+{
+    const long nt = p.ld / 64, ntri = nt * (nt + 1) / 2;
+    for (int kb = 0; kb * NB < p.dim; kb++) {
+        {
+            Timed tm(pr, FAM_PANEL, st);
+            hipLaunchKernelGGL((k_nd_diag<T, NB>), dim3(p.items), dim3(1024), 0, st, p, kb);
+            hipLaunchKernelGGL((k_nd_panel<T, NB>), dim3(xcd_grid(p.items * nt * (NB / 64))),
+                               dim3(256), 0, st, p, kb);
+            tm.end();
+        }
+        Timed tm(pr, FAM_GEMM, st);
+        hipLaunchKernelGGL((k_nd_update<T, NB>), dim3(xcd_grid(p.items * ntri)), dim3(256), 0, st,
+                           p, kb);
+        const double d = p.dim, w = std::min(NB, p.dim - kb * NB);
+        tm.end(4.0 * d * d * w * p.items, true);
+    }
+    hipLaunchKernelGGL(k_nd_mirror<T>, dim3(xcd_grid(p.items * ntri)), dim3(256), 0, st, p.A, p.sA,
+                       p.ld, p.items);
+    TAGS_HIP(hipGetLastError());
+    return 0;
+}
+
+template <typename T>
+int NodalSolver::factor()
+{
+    const NdArgs<T> g = nd_args<T>(*this, false);
+    const long nt = mp / 64, ntri = nt * (nt + 1) / 2;
+    {
+        Timed tm(pr, FAM_OTHER, st);
+        hipLaunchKernelGGL(k_nd_load<T>, dim3(xcd_grid(2L * nb * ntri)), dim3(256), 0, st, Z, sZ,
+                           (cx<T>*)F, (int)mp, (int)m, 2 * nb);
+        tm.end();
+    }
+    int rc;
+    const int bz = nd_block(m), bs = nd_block(n);
+    const NdPhase<T> pz{(cx<T>*)F,  mp * mp,      (int)mp,  (int)m,  2 * nb,
+                        (cx<T>*)tp, (cx<T>*)op_, mp * bz, (cx<T>*)P};
+    if ((rc = bz == 128 ? nd_sweep<T, 128>(pz, st, pr) : nd_sweep<T, 64>(pz, st, pr))) return rc;
+    {
+        Timed tm(pr, FAM_OTHER, st);
+        hipLaunchKernelGGL(k_nd_rows<T>, dim3((unsigned)(nb * ((m + 3) / 4))), dim3(256), 0, st, g);
+        hipLaunchKernelGGL(k_nd_const<T>, dim3(nb), dim3(1024), 0, st, g);
+        const long n16 = np / 16;
+        hipLaunchKernelGGL(k_nd_schur<T>, dim3(xcd_grid((long)nb * (n16 * (n16 + 1) / 2))),
+                           dim3(256), 0, st, g);
+        tm.end();
+    }
+    const NdPhase<T> ps{(cx<T>*)S,  np * np,      (int)np,  (int)n,  nb,
+                        (cx<T>*)tp, (cx<T>*)op_, np * bs, (cx<T>*)P};
+    if ((rc = bs == 128 ? nd_sweep<T, 128>(ps, st, pr) : nd_sweep<T, 64>(ps, st, pr))) return rc;
+    hipLaunchKernelGGL((k_nd_gemv<T, 1>), dim3(xcd_grid(nb * (np / 16))), dim3(256), 0, st, g,
+                       (const cx<T>*)g.c, g.h);
+    hipLaunchKernelGGL(k_nd_den<T>, dim3(nb), dim3(256), 0, st, g);
+    TAGS_HIP(hipGetLastError());
+    return 0;
+}
+
+template <typename T>
+int NodalSolver::queue_step(int k, bool masked)
+{
+    const NdArgs<T> g = nd_args<T>(*this, masked);
+    const int first = k == 1;
+    const unsigned gm = (unsigned)((2 * m + 255) / 256), gn = (unsigned)((n + 255) / 256);
+    const unsigned gz = xcd_grid(2L * nb * (mp / 16));
+    {
+        Timed tm(pr, FAM_SOLVE, st);
+        if (!first) {
+            hipLaunchKernelGGL(k_nd_in<T>, dim3(gm, nb), dim3(256), 0, st, g, k - 1);
+            hipLaunchKernelGGL((k_nd_gemv<T, 2>), dim3(gz), dim3(256), 0, st, g,
+                               (const cx<T>*)g.v, g.z);
+            hipLaunchKernelGGL(k_nd_node<T>, dim3(gn, nb), dim3(256), 0, st, g, k - 1);
+            hipLaunchKernelGGL((k_nd_gemv<T, 1>), dim3(xcd_grid(nb * (np / 16))), dim3(256), 0, st,
+                               g, (const cx<T>*)g.f, g.y);
+        }
+        hipLaunchKernelGGL(k_nd_alpha<T>, dim3(nb), dim3(1024), 0, st, g, k, first);
+        hipLaunchKernelGGL(k_nd_currents<T>, dim3(gz), dim3(256), 0, st, g, k, first);
+        TAGS_HIP(hipGetLastError());
+        tm.end();
+    }
+    Timed tm(pr, FAM_RESID, st);
+    // |W| comes with the first residual
+    const int rc = hem_apply(Z, m, op, x, N, b, r, N, norms + 4 * k, kNormStride, first ? 2 : 1,
+                             nb, sZ, masked ? active : nullptr, st);
+    tm.end();
+    return rc;
+}
+
+int NodalSolver::issue(int nb_, long inj_)
+{
+    if (nb_ < 1 || nb_ > cap || inj_ < 0 || inj_ >= n) return TAGS_ERR_ARG;
+    nb = nb_;
+    inj = inj_;
+    const long w = std::max(std::max(N, 2 * mp), std::max(np, kNormStride));
+    const dim3 gi((unsigned)((w + 255) / 256), nb);
+    if (f64) hipLaunchKernelGGL(k_nd_init<double>, gi, dim3(256), 0, st, nd_args<double>(*this, false), b);
+    else hipLaunchKernelGGL(k_nd_init<float>, gi, dim3(256), 0, st, nd_args<float>(*this, false), b);
+    TAGS_HIP(hipGetLastError());
+    int rc = f64 ? factor<double>() : factor<float>();
+    if (rc) return rc;
+    step_ = f64 ? kSpec64 : kSpec32;
+    for (int k = 1; k <= step_; k++)
+        if ((rc = f64 ? queue_step<double>(k, false) : queue_step<float>(k, false))) return rc;
+    if (f64)
+        hipLaunchKernelGGL(k_nd_pick<double>, dim3((nb + 255) / 256), dim3(256), 0, st,
+                           nd_args<double>(*this, false), u);
+    else
+        hipLaunchKernelGGL(k_nd_pick<float>, dim3((nb + 255) / 256), dim3(256), 0, st,
+                           nd_args<float>(*this, false), u);
+    TAGS_HIP(hipGetLastError());
+    TAGS_HIP(hipMemcpyAsync(hnorms, norms, sizeof(unsigned long long) * kNormStride * nb,
+                            hipMemcpyDeviceToHost, st));
+    TAGS_HIP(hipMemcpyAsync(hu, u, sizeof(c64) * nb, hipMemcpyDeviceToHost, st));
+    first_ = true;
+    return 0;
+}
+
+double NodalSolver::norm_at(int q, int k, int i) const
+{
+    double d;
+    std::memcpy(&d, &hnorms[kNormStride * q + 4 * k + i], 8);
+    return d;
+}
+double NodalSolver::berr_at(int q, int k) const
+{
+    const double w = norm_at(q, 1, 2), rn = norm_at(q, k, 0), xn = norm_at(q, k, 1);
+    if (rn == 0.0 && xn > 0.0) return 0.0;
+    return w > 0 && xn > 0 ? rn / (w * xn) : NAN;
+}
+double NodalSolver::dx_at(int q, int k) const
+{
+    const double d = norm_at(q, k, 3), xn = norm_at(q, k, 1);
+    return xn > 0 ? d / xn : NAN;
+}
+// rho / (1 - rho) |dx| / |x| with rho the last step's contraction; |dx| / |x|
+// itself at the first step and where rho >= 1/2
+double NodalSolver::fwd_at(int q, int k) const
+{
+    const double d = dx_at(q, k);
+    if (k < 2 || d == 0.0) return d;
+    const double dp = dx_at(q, k - 1), rho = dp > 0.0 ? d / dp : 1.0;
+    return rho < 0.5 ? d * rho / (1.0 - rho) : d;
+}
+// Acceptance: backward error of a few ulps, and the error left in x below
+// 1e-10 (complex64 blocks: 100 x below the 1e-8 bar) or 1e-14 (complex128: the
+// level of a direct FP64 factorisation or better).
+bool NodalSolver::accept(int q) const
+{
+    return berr[q] <= 1e-15 && fwd[q] <= (f64 ? 1e-14 : 1e-10);
+}
+
+int NodalSolver::advance(bool* complete)
+{
+    *complete = false;
+    const int k = first_ ? step_ : ++step_;
+    if (first_) {
+        steps.assign(nb, k);
+        accepted.assign(nb, 0);
+        go.assign(nb, 1);
+        berr.assign(nb, 0.0);
+        fwd.assign(nb, 0.0);
+        hist.assign(8 * (size_t)nb, -1.0);
+        for (int q = 0; q < nb; q++)
+            for (int i = 1; i < k; i++) hist[8 * q + i - 1] = berr_at(q, i);
+    }
+    first_ = false;
+    int ngo = 0;
+    for (int q = 0; q < nb; q++) {
+        if (!go[q]) continue;
+        steps[q] = k;
+        berr[q] = berr_at(q, k);
+        fwd[q] = fwd_at(q, k);
+        if (k <= 8) hist[8 * q + k - 1] = berr[q];
+        accepted[q] = accept(q);
+        // on while a step still gains 20 % in either measure
+        go[q] = !accepted[q] && k < kMaxSteps && berr[q] == berr[q] && fwd[q] == fwd[q] &&
+                (k < 3 || berr[q] <= 0.8 * berr_at(q, k - 1) || dx_at(q, k) <= 0.8 * dx_at(q, k - 1));
+        ngo += go[q];
+    }
+    if (ngo == 0) {
+        *complete = true;
+        return 0;
+    }
+    for (int q = 0; q < nb; q++) hactive[q] = go[q];
+    TAGS_HIP(hipMemcpyAsync(active, hactive, sizeof(int) * nb, hipMemcpyHostToDevice, st));
+    int rc = f64 ? queue_step<double>(k + 1, true) : queue_step<float>(k + 1, true);
+    if (rc) return rc;
+    if (f64)
+        hipLaunchKernelGGL(k_nd_pick<double>, dim3((nb + 255) / 256), dim3(256), 0, st,
+                           nd_args<double>(*this, false), u);
+    else
+        hipLaunchKernelGGL(k_nd_pick<float>, dim3((nb + 255) / 256), dim3(256), 0, st,
+                           nd_args<float>(*this, false), u);
+    TAGS_HIP(hipGetLastError());
+    TAGS_HIP(hipMemcpyAsync(hnorms, norms, sizeof(unsigned long long) * kNormStride * nb,
+                            hipMemcpyDeviceToHost, st));
+    TAGS_HIP(hipMemcpyAsync(hu, u, sizeof(c64) * nb, hipMemcpyDeviceToHost, st));
+    return 0;
+}
+
+}  // namespace tags
