@@ -1,0 +1,77 @@
+"""GPU test of the sweep's impedance fill on both sides of each of its rules:
+the number of Chebyshev terms (12, 16, 24 or 32 by |gamma| times the longest
+segment) and the direct rule beyond them, on a geometry with touching
+segments (in line, at a right angle, at 10 degrees, of very different
+lengths), segments closer than two lengths down to a tenth of one, far ones,
+and images of shallow segments. Against the oracle's adaptive integrals
+(relative tolerance 1e-11): 1e-9 of each entry, the bar of the assembly
+tests; groups of several samples against single ones bit for bit in what they
+share (the terms of the group's largest |gamma| may differ): 1e-12."""
+import numpy as np
+import pytest
+
+import tags_pkg
+
+T = tags_pkg.load()
+O = tags_pkg.oracle()
+
+pytestmark = pytest.mark.gpu
+
+
+def _geometry():
+    d = -0.3
+    a = np.deg2rad(10.0)
+    chain = [(0, 0, d), (1, 0, d), (2, 0, d), (2, 1, d), (2 + np.cos(a), 1 + np.sin(a), d)]
+    segs = [(chain[i], chain[i + 1]) for i in range(4)]
+    segs += [((2, 1, d), (3, 1, d))]                       # 10 degrees beside the chain's last
+    segs += [((0, 0, d), (0, 0, d - 0.02))]                # fifty times shorter, touching
+    segs += [((0, 0.1, d), (1, 0.1, d)), ((0, 0.7, d), (1, 0.7, d)), ((0.2, 1.9, d), (1.1, 1.9, d))]
+    segs += [((40, 30, d), (41, 30, d)), ((7, -3, d - 2), (7.5, -3.5, d - 2.5))]
+    e = np.zeros(len(segs), T.ELECTRODE_DTYPE)
+    for i, (p, q) in enumerate(segs):
+        rc, one = T.populate_electrode(p, q, 5e-3)
+        e[i] = one[0]
+    ends = np.concatenate([e["start_point"], e["end_point"]])
+    nodes = np.unique(np.round(ends, 9), axis=0)
+    return e, nodes
+
+
+# |gamma| on either side of 0.38, 1.13, 3.7 and 7.3 over the longest segment (1 m)
+@pytest.mark.parametrize("glen", [0.02, 0.37, 0.39, 1.12, 1.14, 3.6, 3.8, 7.2, 7.4, 12.0])
+def test_fill_terms_vs_oracle(glen):
+    e, nodes = _geometry()
+    m, n = len(e), len(nodes)
+    # gamma^2 = s mu0 kappa with s = j w, kappa = sigma + s eps: equal conduction
+    # and displacement currents, so that both parts of gamma count
+    w = glen * np.sqrt(1.0 / (np.sqrt(2.0) * T.MU0 * 15.0 * T.EPS0))
+    f = w / (2 * np.pi)
+    sc = O.soil_scalars(f, w * 15.0 * T.EPS0, 15.0)
+    assert abs(abs(sc["gamma"]) - glen) < 1e-9 * glen
+    i, k = np.triu_indices(m)
+    pairs = np.column_stack([i, k])
+    zl, zt = O.z_entries(e, O.images_of(e), pairs, sc, rel_tol=1e-11, threads=8)
+    sw = T.Sweep(e, nodes)
+    got = [-sw.assemble_entries(sc["s"], sc["kappa"], o + i, o + k) for o in (n, n + m)]
+    low = [-sw.assemble_entries(sc["s"], sc["kappa"], o + k, o + i) for o in (n, n + m)]
+    sw.close()
+    for g, l, ref in zip(got, low, (zl, zt)):
+        err = np.abs(g - ref)
+        # entries e^{-|Re gamma| r} below the oracle's absolute floor are left out
+        assert np.all(err <= 1e-9 * np.abs(ref) + 1e-13 * np.abs(ref).max()), err.max()
+        assert np.array_equal(g, l)
+
+
+@pytest.mark.parametrize("m,nf", [(1, 3), (16, 5), (17, 1), (33, 70), (150, 9)])
+def test_group_fill_matches_single_samples(m, nf):
+    """Tiles and sample ranges of a group: U[inj] of a sweep solved in one group
+    and one sample at a time."""
+    rc, e, nodes = T.segment_electrode([0, 0, -0.5], [0.5 * m, 0, -0.5], m, 7e-3)
+    s = 2j * np.pi * 10.0 ** np.linspace(2, 7.5, nf)
+    kap = 5e-3 + s * 10.0 * T.EPS0
+    sw = T.Sweep(e, nodes)
+    res = []
+    for b in (0, 1):
+        sw.set_batch(b)
+        res.append(sw.solve(s, kap, 0, T.PREC_FP64)[0])
+    sw.close()
+    assert np.max(np.abs(res[0] - res[1]) / np.abs(res[1])) <= 1e-12

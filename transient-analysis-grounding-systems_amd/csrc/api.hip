@@ -1683,6 +1683,35 @@ struct OwnedStream {
     }
 };
 
+// The scalars of a group's samples: pinned staging, device copy, and the
+// moment fill's coefficients.
+struct ScalarBuf {
+    PairScalars* h = nullptr;
+    PairScalars* d = nullptr;
+    c64* cf = nullptr;
+    int cap = 0;
+    int ensure(int n)
+    {
+        if (n <= cap) return 0;
+        release();
+        TAGS_HIP(hipHostMalloc(&h, sizeof(PairScalars) * n, 0));
+        TAGS_HIP(hipMalloc(&d, sizeof(PairScalars) * n));
+        TAGS_HIP(hipMalloc(&cf, sizeof(c64) * kFillTermsMax * n));
+        cap = n;
+        return 0;
+    }
+    void release()
+    {
+        if (h) hipHostFree(h);
+        hipFree(d);
+        hipFree(cf);
+        h = d = nullptr;
+        cf = nullptr;
+        cap = 0;
+    }
+    ~ScalarBuf() { release(); }
+};
+
 // One frequency sample in flight: its own stream, W, right-hand side, solver
 // (factor work space, complex64 copy) and kernel timers. The sweep queues a
 // sample on every slot, then finishes them in turn from the calling thread,
@@ -1691,13 +1720,12 @@ struct OwnedStream {
 struct SweepSlot {
     OwnedStream stream;
     DevBuf<c64> W, rhs;        // cap items: W at stride N^2, rhs at stride N
-    DevBuf<PairScalars> dsc;   // the group's per-sample scalars
-    PairScalars* hsc = nullptr;  // pinned staging of dsc
+    ScalarBuf scal;            // the group's per-sample scalars
     Profiler prof;
     Solver sv;
     NodalSolver nd;         // the hybrid plan's solve (nodal_path)
     bool nodal_path = false;
-    int cap = 0, sc_cap = 0;
+    int cap = 0;
     const tags_sweep* bound = nullptr;  // the sweep whose plans the solver holds
     int bound_kind = -1;                // and its plan kind then
     long f = -1;            // first sample of the group in flight (-1: idle)
@@ -1719,17 +1747,7 @@ struct SweepSlot {
         if (!stream.s) TAGS_HIP(hipStreamCreate(&stream.s));
         nd.st = sv.st = stream.s;
         nd.pr = sv.pr = &prof;
-        if (batch <= sc_cap) return 0;
-        hipFree(dsc.p);
-        if (hsc) hipHostFree(hsc);
-        dsc.p = nullptr;
-        hsc = nullptr;
-        sc_cap = 0;
-        int rc = dsc.alloc((size_t)batch);
-        if (rc) return rc;
-        TAGS_HIP(hipHostMalloc(&hsc, sizeof(PairScalars) * batch, 0));
-        sc_cap = batch;
-        return 0;
+        return scal.ensure(batch);
     }
     int init(long N, int batch)
     {
@@ -1757,7 +1775,6 @@ struct SweepSlot {
     ~SweepSlot()
     {
         if (stream.s) hipStreamSynchronize(stream.s);
-        if (hsc) hipHostFree(hsc);
     }
 };
 
@@ -1841,6 +1858,8 @@ struct tags_sweep {
     tags::BlockLayout layout{};
     hipStream_t st = nullptr;  // set-up and assembly stream
     tags::DevSegs e, img;
+    double dmax = 0.0;  // the longest segment, by its end points
+    ScalarBuf scal;     // of single assemblies on st
     int* sn = nullptr;
     int* en = nullptr;
     // each node's segment ends (node_ptr: n + 1, node_seg: 2 m at most) and the
@@ -2047,10 +2066,9 @@ static PairScalars sample_scalars(TAGS_COMPLEX s_, TAGS_COMPLEX kappa_, double m
 }
 
 // Assembly of nb samples' W (item z at W + z N^2) in the sweep's block layout:
-// one sample from `sc`, several from their scalars `dsc` in device memory.
+// their scalars in sb.h (uploaded here).
 static int sweep_fill_items(tags_sweep* sw, c64* W, hipStream_t st, Profiler* prof, int nb,
-                            const PairScalars& sc, const PairScalars* dsc,
-                            bool fill_static = true, long ld = 0, long sW = 0)
+                            ScalarBuf& sb, bool fill_static = true, long ld = 0, long sW = 0)
 {
     // a compact store of the impedance blocks (ld > 0: see nodal_z_items) is
     // addressed as a matrix of that pitch with the blocks in its first rows
@@ -2060,30 +2078,40 @@ static int sweep_fill_items(tags_sweep* sw, c64* W, hipStream_t st, Profiler* pr
     else sW = N * N;
     Timed tm(prof, FAM_FILL, st);
     int rc;
-    const PairScalars* scs = nb > 1 ? dsc : nullptr;
+    TAGS_HIP(hipMemcpyAsync(sb.d, sb.h, sizeof(PairScalars) * nb, hipMemcpyHostToDevice, st));
+    double gabs = 0.0;
+    for (int z = 0; z < nb; z++) {
+        const double g = std::hypot(sb.h[z].gamma.x, sb.h[z].gamma.y);
+        gabs = g > gabs || g != g ? g : gabs;
+    }
     if (fill_static && (rc = launch_fill_static(W, N, sw->layout, sw->sn, sw->en, st, nb, sW)))
         return rc;
     if (sw->formulation == TAGS_FORM_MHEM) {
         if (!sw->pot) return TAGS_ERR_ARG;
         const size_t mm = (size_t)sw->m * sw->m;
         if ((rc = launch_fill_mhem(W, N, L, sw->e.soa(), sw->img.soa(), sw->pot,
-                                   sw->pot + mm, sw->pot + 2 * mm, sw->pot + 3 * mm, sc, st, nb,
-                                   sW, scs)))
+                                   sw->pot + mm, sw->pot + 2 * mm, sw->pot + 3 * mm, sb.d, st, nb,
+                                   sW)))
             return rc;
-    } else if ((rc = launch_fill_zblocks(W, N, L, sw->e.soa(), sw->img.soa(), sc, st, nb, sW,
-                                         scs))) {
+    } else if (sw->dmax > 0.0 && fill_terms(gabs * sw->dmax) > 0) {
+        if ((rc = launch_fill_moments(W, N, L, sw->e.soa(), sw->img.soa(), sb.d, sb.cf, nb, sW,
+                                      sw->dmax, gabs, st)))
+            return rc;
+    } else if ((rc = launch_fill_zblocks(W, N, L, sw->e.soa(), sw->img.soa(), sb.d, st, nb, sW))) {
         return rc;
     }
     tm.end();
     return 0;
 }
 
-static int sweep_fill(tags_sweep* sw, c64* W, hipStream_t st, Profiler* prof, TAGS_COMPLEX s_,
+static int sweep_fill(tags_sweep* sw, c64* W, hipStream_t st, ScalarBuf& sb, TAGS_COMPLEX s_,
                       TAGS_COMPLEX kappa_, double mur, const TAGS_COMPLEX* gamma_,
                       const TAGS_COMPLEX* ref_l_, const TAGS_COMPLEX* ref_t_)
 {
-    const PairScalars sc = sample_scalars(s_, kappa_, mur, gamma_, ref_l_, ref_t_);
-    return sweep_fill_items(sw, W, st, prof, 1, sc, nullptr);
+    const int rc = sb.ensure(1);
+    if (rc) return rc;
+    sb.h[0] = sample_scalars(s_, kappa_, mur, gamma_, ref_l_, ref_t_);
+    return sweep_fill_items(sw, W, st, nullptr, 1, sb);
 }
 
 // The mHEM potentials, once per geometry (on the set-up stream, finished
@@ -2126,6 +2154,11 @@ int tags_sweep_create(tags_sweep** out, const Electrode* electrodes, const Elect
     }
     if ((rc = sw->e.upload(electrodes, sw->m, sw->st))) return rc;
     if ((rc = sw->img.upload(images, sw->m, sw->st))) return rc;
+    for (const Electrode* q : {electrodes, images})
+        for (long i = 0; i < sw->m; i++) {
+            const double d = vlen(q[i].start_point, q[i].end_point);
+            sw->dmax = d > sw->dmax || d != d ? d : sw->dmax;
+        }
     const long m = sw->m, n = sw->n;
     std::vector<double> sp = seg_points(electrodes, m);
     DevBuf<double> dsp, dnodes;
@@ -2202,7 +2235,7 @@ int tags_sweep_assemble(tags_sweep* sw, TAGS_COMPLEX s, TAGS_COMPLEX kappa, doub
     DevBuf<c64> W;
     int rc = sweep_potentials(sw);
     if (rc || (rc = W.alloc((size_t)N * N))) return rc;
-    if ((rc = sweep_fill(sw, W.p, sw->st, nullptr, s, kappa, mur, nullptr, nullptr, nullptr)))
+    if ((rc = sweep_fill(sw, W.p, sw->st, sw->scal, s, kappa, mur, nullptr, nullptr, nullptr)))
         return rc;
     std::vector<c64> h((size_t)N * N);
     TAGS_HIP(hipMemcpyAsync(h.data(), W.p, sizeof(c64) * N * N, hipMemcpyDeviceToHost, sw->st));
@@ -2258,7 +2291,7 @@ int tags_sweep_assemble_entries(tags_sweep* sw, TAGS_COMPLEX s, TAGS_COMPLEX kap
     if (rc || (rc = W.alloc((size_t)N * N)) || (rc = dout.alloc(count)) ||
         (rc = didx.alloc(count)))
         return rc;
-    if ((rc = sweep_fill(sw, W.p, sw->st, nullptr, s, kappa, mur, nullptr, nullptr, nullptr)))
+    if ((rc = sweep_fill(sw, W.p, sw->st, sw->scal, s, kappa, mur, nullptr, nullptr, nullptr)))
         return rc;
     if (count) {
         TAGS_HIP(hipMemcpyAsync(didx.p, idx.data(), sizeof(long) * count, hipMemcpyHostToDevice,
@@ -2429,21 +2462,14 @@ static int sweep_issue(tags_sweep* sw, SweepSlot& sl, size_t f, const SweepCall&
         for (int i = 0; i < 8; i++) q.refine_hist[i] = -1.0;
     sl.info.assign(cnt, 0);
     hipStream_t st = sl.stream.s;
-    PairScalars sc0{};
     for (int z = 0; z < cnt; z++) {
         const size_t q = f + z;
-        const PairScalars sc = sample_scalars(c.s[q], c.kappa[q], c.mur,
-                                              c.gamma ? &c.gamma[q] : nullptr,
-                                              c.ref_l ? &c.ref_l[q] : nullptr,
-                                              c.ref_t ? &c.ref_t[q] : nullptr);
-        if (z == 0) sc0 = sc;
-        sl.hsc[z] = sc;
+        sl.scal.h[z] = sample_scalars(c.s[q], c.kappa[q], c.mur, c.gamma ? &c.gamma[q] : nullptr,
+                                      c.ref_l ? &c.ref_l[q] : nullptr,
+                                      c.ref_t ? &c.ref_t[q] : nullptr);
     }
-    if (cnt > 1)
-        TAGS_HIP(hipMemcpyAsync(sl.dsc.p, sl.hsc, sizeof(PairScalars) * cnt,
-                                hipMemcpyHostToDevice, st));
     if (sl.nodal_path) {
-        if ((rc = sweep_fill_items(sw, sl.nd.Z, st, &sl.prof, cnt, sc0, sl.dsc.p, false, sw->m,
+        if ((rc = sweep_fill_items(sw, sl.nd.Z, st, &sl.prof, cnt, sl.scal, false, sw->m,
                                    sl.nd.sZ)))
             return rc;
         rc = sl.nd.issue(cnt, (long)c.inj_node);
@@ -2453,7 +2479,7 @@ static int sweep_issue(tags_sweep* sw, SweepSlot& sl, size_t f, const SweepCall&
     // sweep on this slot unless a factor in FP64 replaced W since
     const bool keep = c.mixed && sl.static_sw == sw && sl.static_kind == sw->layout_kind &&
                       sl.static_items >= cnt;
-    if ((rc = sweep_fill_items(sw, sl.W.p, st, &sl.prof, cnt, sc0, sl.dsc.p, !keep))) return rc;
+    if ((rc = sweep_fill_items(sw, sl.W.p, st, &sl.prof, cnt, sl.scal, !keep))) return rc;
     if (!c.mixed) {
         sl.static_items = 0;  // the FP64 factor replaces W
     } else if (!keep) {
@@ -2479,7 +2505,7 @@ static int sweep_verify64(tags_sweep* sw, SweepSlot& sl, c64* Wz, const c64* xz,
     hipStream_t st = sl.stream.s;
     Solver& sv = sl.sv;
     int rc;
-    if ((rc = sweep_fill(sw, Wz, st, nullptr, c.s[f], c.kappa[f], c.mur,
+    if ((rc = sweep_fill(sw, Wz, st, sl.scal, c.s[f], c.kappa[f], c.mur,
                          c.gamma ? &c.gamma[f] : nullptr, c.ref_l ? &c.ref_l[f] : nullptr,
                          c.ref_t ? &c.ref_t[f] : nullptr)))
         return rc;
@@ -2508,7 +2534,7 @@ static int sweep_nodal_retry(tags_sweep* sw, SweepSlot& sl, int q, size_t f, con
     slot_bind(sw, sl);
     sl.static_items = 0;
     hipStream_t st = sl.stream.s;
-    if ((rc = sweep_fill(sw, sl.W.p, st, nullptr, c.s[f], c.kappa[f], c.mur,
+    if ((rc = sweep_fill(sw, sl.W.p, st, sl.scal, c.s[f], c.kappa[f], c.mur,
                          c.gamma ? &c.gamma[f] : nullptr, c.ref_l ? &c.ref_l[f] : nullptr,
                          c.ref_t ? &c.ref_t[f] : nullptr)))
         return rc;

@@ -17,6 +17,7 @@
 //
 // The diagonal of the direct part is the reference's gamma-independent closed
 // form (src/electrode.c:238-245, used at :346-348).
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <vector>
@@ -478,14 +479,12 @@ constexpr int kFT = 32;  // tile edge of the mHEM fill
 // 32 x 32 tile, three 16 x 16 ones).
 template <int FT>
 __global__ __launch_bounds__(256) void k_fill_zblocks(c64* W, long ldw, long zl_off, long zt_off,
-                                                       long m, SegSoA e, SegSoA img, PairScalars sc,
-                                                       long sw, const PairScalars* scs)
+                                                       long m, SegSoA e, SegSoA img, long sw,
+                                                       const PairScalars* scs)
 {
     // item blockIdx.z of a batch: its own W and frequency-sample scalars
-    if (scs) {
-        sc = scs[blockIdx.z];
-        W += (long)blockIdx.z * sw;
-    }
+    const PairScalars sc = scs[blockIdx.z];
+    W += (long)blockIdx.z * sw;
     // triangular tile index -> (ti >= tk)
     const long b = blockIdx.x;
     long ti = (long)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
@@ -577,25 +576,379 @@ __global__ __launch_bounds__(256) void k_fill_zblocks(c64* W, long ldw, long zl_
 }
 
 int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
-                        const PairScalars& sc, hipStream_t st, int nb, long sw,
-                        const PairScalars* scs)
+                        const PairScalars* scs, hipStream_t st, int nb, long sw)
 {
     const long m = L.m;
     if (m <= 0 || nb <= 0) return 0;
-    if (nb > 1 && !scs) return TAGS_ERR_ARG;
+    if (!scs) return TAGS_ERR_ARG;
     int rc = gl_tables_init();
     if (rc) return rc;
     const long T32 = (m + 31) / 32;
     if (T32 * (T32 + 1) / 2 * nb >= 512) {
         hipLaunchKernelGGL(k_fill_zblocks<32>, dim3((unsigned)(T32 * (T32 + 1) / 2), 1,
                                                     (unsigned)nb),
-                           dim3(256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, sc, sw, scs);
+                           dim3(256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, sw, scs);
     } else {
         const long T16 = (m + 15) / 16;
         hipLaunchKernelGGL(k_fill_zblocks<16>, dim3((unsigned)(T16 * (T16 + 1) / 2), 1,
                                                     (unsigned)nb),
-                           dim3(256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, sc, sw, scs);
+                           dim3(256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, sw, scs);
     }
+    TAGS_HIP(hipGetLastError());
+    return 0;
+}
+
+// ---------------------------------------------------------------------------
+// Assembly of a group's samples from frequency-independent moments. With
+// R the middle-point distance of a pair and |r - R| <= D for every two of its
+// points (D: the longest segment; the triangle inequality gives the mean of
+// the two lengths),
+//   e^{-gamma r} = e^{-gamma R} sum_k c_k(gamma) T_k((r - R) / D),
+// so that the pair integral of every sample is
+//   J(gamma) = e^{-gamma R} sum_{k < K} c_k(gamma) M_k,
+//   M_k = int int T_k((r - R) / D) / r over the unit square:
+// K real moments per pair and group of samples, on the quadrature points the
+// direct rule would take, then one complex exponential and 2 K multiply-adds
+// per sample, where the direct rule takes a square root, an exponential and a
+// sine and cosine at every point of every sample. The Chebyshev tail beyond K
+// terms is below 1e-17 for |gamma| D <= 7.3 (K = 32, see fill_terms); larger
+// ones keep the direct rule (k_fill_zblocks).
+//
+// One thread per pair of a 16 x 16 tile on or below the diagonal, work-groups
+// of one tile and a range of the samples (so that few segments still fill the
+// device). Pairs that touch or are closer than two lengths, which need the
+// Duffy rule or 144 points and more, are listed in LDS and taken by whole
+// waves, the lanes sharing the points; moments pass through LDS, so that few
+// of them are live in registers at a time. Bound: the samples' exponentials and
+// sines (FP64 VALU, about 300 instructions per pair and sample), then the
+// writes of both triangles.
+// ---------------------------------------------------------------------------
+template <int K>
+struct Moments {
+    double m[K];
+    double rc, invd;
+    __device__ void zero()
+    {
+#pragma unroll
+        for (int k = 0; k < K; k++) m[k] = 0.0;
+    }
+    // a point at distance r with weight w (1 / r included)
+    __device__ inline void add(double r, double w)
+    {
+        const double t = (r - rc) * invd, t2 = t + t;
+        double a = w, b = w * t;
+        m[0] += a;
+        if constexpr (K > 1) m[1] += b;
+#pragma unroll
+        for (int k = 2; k < K; k++) {
+            const double c = fma(t2, b, -a);
+            m[k] += c;
+            a = b;
+            b = c;
+        }
+    }
+};
+
+__device__ inline V3 vmid(const DSeg& s) { return vmul(vadd(s.a, s.b), 0.5); }
+
+// tensor Gauss-Legendre rule of order index oi; points p0, p0 + step, ...
+template <int K>
+__device__ inline void mom_gl(Moments<K>& M, const DSeg& S, const DSeg& R, int oi, int p0,
+                              int step, double scale)
+{
+    const int q = dev_order(oi), off = g_gloff[oi];
+    const V3 ds = vsub(S.b, S.a), dr = vsub(R.b, R.a);
+    for (int i = p0; i < q * q; i += step) {
+        const int a = i / q, b = i - a * q;
+        const V3 d = vsub(vadd(R.a, vmul(dr, g_glx[off + a])), vadd(S.a, vmul(ds, g_glx[off + b])));
+        const double r = vnorm(d);
+        M.add(r, scale * g_glw[off + a] * g_glw[off + b] / r);
+    }
+}
+
+// One Duffy triangle (see duffy_line), the radial integral of the moments'
+// polynomials by a Gauss-Legendre rule of order `nr` (exact to degree 2 nr - 1)
+template <int K>
+__device__ inline void mom_duffy(Moments<K>& M, V3 p, V3 q, bool w_on_p, int lane)
+{
+    constexpr int RI = K <= 16 ? 3 : K <= 24 ? 4 : 5;  // radial order 8, 12 or 16
+    const int nr = dev_order(RI), roff = g_gloff[RI];
+    const double pp = vdot(p, p), qq = vdot(q, q), pq = vdot(p, q);
+    const double den = w_on_p ? pp : qq;
+    const double re = pq / den, im = sqrt(fmax(pp * qq - pq * pq, 0.0)) / den;
+    const double wc = fmin(fmax(re, 0.0), 1.0);
+    const double dist = sqrt((re - wc) * (re - wc) + im * im);
+    const bool graded = dist < 0.5;
+    const double h0 = fmax(dist, 1e-6);
+    const int nq = 20, off = g_gloff[6];
+    for (int side = 0; side < (graded ? 2 : 1); side++) {
+        const double span = graded ? (side ? 1.0 - wc : wc) : 1.0;
+        double lo = 0.0, hi = graded ? h0 : 1.0;
+        while (lo < span) {
+            const double h = fmin(hi, span) - lo;
+            for (int i = lane; i < nq * nr; i += 64) {
+                const int a = i / nr, b = i - a * nr;
+                const double u = lo + h * g_glx[off + a];
+                const double w = graded ? (side ? wc + u : wc - u) : u;
+                const V3 d = w_on_p ? vsub(vmul(p, w), q) : vsub(p, vmul(q, w));
+                const double R = vnorm(d);
+                M.add(g_glx[roff + b] * R, h * g_glw[off + a] * g_glw[roff + b] / R);
+            }
+            lo = hi;
+            hi += hi;
+        }
+    }
+}
+
+// Moments of a pair by one wave (touching, or closer than two lengths)
+template <int K>
+__device__ inline void mom_wave(Moments<K>& M, const DSeg& S, const DSeg& R, double gabs, int lane)
+{
+    const double lmax = fmax(S.len, R.len), tol = 1e-9 * lmax;
+    // end points i of S and k of R that coincide, in the order of pair_integral_unit
+    auto meet = [&](V3 p, V3 q) {
+        const V3 d = vsub(p, q);
+        return vdot(d, d) <= tol * tol;
+    };
+    const bool aa = meet(S.a, R.a), ab = meet(S.a, R.b), ba = meet(S.b, R.a), bb = meet(S.b, R.b);
+    if (aa || ab || ba || bb) {
+        const bool sb = !(aa || ab), rb = sb ? !ba : !aa;
+        const V3 C = sb ? S.b : S.a;
+        const V3 ds = vsub(sb ? S.a : S.b, C), dr = vsub(rb ? R.a : R.b, C);
+        mom_duffy(M, dr, ds, false, lane);
+        mom_duffy(M, dr, ds, true, lane);
+        return;
+    }
+    const double rho = seg_seg_distance(S, R) / lmax;
+    if (rho >= 0.25) {
+        mom_gl(M, S, R, geometric_order(rho, gabs * lmax), lane, 64, 1.0);
+        return;
+    }
+    int ns = (int)ceil(1.0 / fmax(rho, 1.0 / 64.0));
+    ns = ns > 64 ? 64 : ns;
+    const V3 ds = vmul(vsub(S.b, S.a), 1.0 / ns), dr = vmul(vsub(R.b, R.a), 1.0 / ns);
+    const double sc = 1.0 / ((double)ns * ns);
+    for (int i = 0; i < ns; i++)
+        for (int k = 0; k < ns; k++) {
+            const DSeg Ss{vadd(S.a, vmul(ds, i)), vadd(S.a, vmul(ds, i + 1)), S.len / ns};
+            const DSeg Rs{vadd(R.a, vmul(dr, k)), vadd(R.a, vmul(dr, k + 1)), R.len / ns};
+            const double l = fmax(Ss.len, Rs.len), rs = seg_seg_distance(Ss, Rs) / l;
+            mom_gl(M, Ss, Rs, geometric_order(rs < 0.25 ? 0.25 : rs, gabs * l), lane, 64, sc);
+        }
+}
+
+// Whether a pair goes to the waves: shared end points, or closer than two lengths
+__device__ inline bool pair_near(const DSeg& S, const DSeg& R, double* rho)
+{
+    const double lmax = fmax(S.len, R.len);
+    *rho = seg_seg_distance(S, R) / lmax;
+    return !(*rho >= 2.0);
+}
+
+template <int K>
+__global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, long ldw,
+                                                       long zl_off, long zt_off, long m, SegSoA e,
+                                                       SegSoA img,
+                                                       const PairScalars* __restrict__ scs, long sw,
+                                                       const c64* __restrict__ cf, int nf, int per, double D,
+                                                       double gabs)
+{
+    const long b = blockIdx.x;
+    long ti = (long)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
+    while ((ti + 1) * (ti + 2) / 2 <= b) ti++;
+    while (ti * (ti + 1) / 2 > b) ti--;
+    const long tk = b - ti * (ti + 1) / 2;
+    const int t = threadIdx.x, a = t >> 4, c = t & 15;
+    const long i0 = ti * 16, k0 = tk * 16, i = i0 + a, k = k0 + c;
+    const bool in = i < m && k < m && k <= i;
+
+    __shared__ double geo[3][8][16];  // columns, rows, the rows' images
+    // every pair's moments of one kind while they are formed; then the tiles
+    // being transposed
+    union Stage {
+        double mom[K][256];
+        c64 tile[2][2][16][17];
+    };
+    __shared__ Stage stage;
+    __shared__ int near_n[2], near_at[2][256];
+    if (t < 2) near_n[t] = 0;
+    if (t < 48) {
+        const int side = t >> 4, s = t & 15;
+        const long idx = (side == 0 ? k0 : i0) + s;
+        const SegSoA& g = side == 2 ? img : e;
+        if (idx < m) {
+            geo[side][0][s] = g.ax[idx];
+            geo[side][1][s] = g.ay[idx];
+            geo[side][2][s] = g.az[idx];
+            geo[side][3][s] = g.bx[idx];
+            geo[side][4][s] = g.by[idx];
+            geo[side][5][s] = g.bz[idx];
+            geo[side][6][s] = g.len[idx];
+            geo[side][7][s] = g.rad[idx];
+        }
+    }
+    __syncthreads();
+    auto seg = [&](int side, int s) {
+        return DSeg{V3{geo[side][0][s], geo[side][1][s], geo[side][2][s]},
+                    V3{geo[side][3][s], geo[side][4][s], geo[side][5][s]}, geo[side][6][s]};
+    };
+    double md[K], mi[K];  // direct, image
+    double rd = 0.0, ri = 0.0, cost = 0.0, cosi = 0.0, ll = 1.0;
+    const int wave = t >> 6, lane = t & 63;
+#pragma unroll
+    for (int kind = 0; kind < 2; kind++) {
+        {
+            Moments<K> M;
+            M.zero();
+            if (in) {
+                const DSeg S = seg(0, c), R = seg(1 + kind, a);
+                M.rc = vnorm(vsub(vmid(S), vmid(R)));
+                M.invd = 1.0 / D;
+                (kind ? ri : rd) = M.rc;
+                (kind ? cosi : cost) = abs_dot(S, R);
+                if (!kind) ll = S.len * R.len;
+                double rho;
+                if (kind || k != i) {
+                    if (pair_near(S, R, &rho))
+                        near_at[kind][atomicAdd(&near_n[kind], 1)] = t;
+                    else
+                        mom_gl(M, S, R, geometric_order(rho, gabs * fmax(S.len, R.len)), 0, 1, 1.0);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < K; j++) stage.mom[j][t] = M.m[j];
+        }
+        __syncthreads();
+        const int nn = near_n[kind];
+        for (int q = wave; q < nn; q += 4) {
+            const int w = near_at[kind][q];
+            const DSeg S = seg(0, w & 15), R = seg(1 + kind, w >> 4);
+            Moments<K> M;
+            M.zero();
+            M.invd = 1.0 / D;
+            M.rc = vnorm(vsub(vmid(S), vmid(R)));
+            mom_wave(M, S, R, gabs, lane);
+#pragma unroll
+            for (int j = 0; j < K; j++) {
+                double v = M.m[j];
+                for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+                if (lane == 0) stage.mom[j][w] = v;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < K; j++) (kind ? mi[j] : md[j]) = stage.mom[j][t];
+        __syncthreads();
+    }
+    const double self = in && k == i ? self_integral_dev(geo[1][6][a], geo[1][7][a]) : 0.0;
+    const int f0 = blockIdx.y * per, f1 = min(nf, f0 + per);
+    for (int f = f0; f < f1; f++) {
+        const PairScalars& sc = scs[f];
+        const c64* cq = cf + (long)f * K;
+        c64 vl{0, 0}, vt{0, 0};
+        if (in) {
+            double dx = 0, dy = 0, ix = 0, iy = 0;
+#pragma unroll
+            for (int j = 0; j < K; j++) {
+                const c64 q = cq[j];
+                dx = fma(q.x, md[j], dx);
+                dy = fma(q.y, md[j], dy);
+                ix = fma(q.x, mi[j], ix);
+                iy = fma(q.y, mi[j], iy);
+            }
+            double sn, cs;
+            sincos(-sc.gamma.y * rd, &sn, &cs);
+            double mag = exp(-sc.gamma.x * rd);
+            const c64 jd = cmul(c64{mag * cs, mag * sn}, c64{dx, dy});
+            sincos(-sc.gamma.y * ri, &sn, &cs);
+            mag = exp(-sc.gamma.x * ri);
+            const c64 ji = cmul(c64{mag * cs, mag * sn}, c64{ix, iy});
+            // the formulas of k_fill_zblocks, J the integral over L_r L_s
+            if (k == i) {
+                vl = cscale(sc.zl_dir, self);
+                vt = cscale(sc.zt_dir, self / ll);
+            } else {
+                vt = cmul(sc.zt_dir, jd);
+                if (!(cost < 2.220446049250313e-16)) vl = cscale(cmul(sc.zl_dir, jd), cost);
+            }
+            vt = cadd(vt, cmul(sc.zt_img, ji));
+            if (cosi > 2.220446049250313e-16)
+                vl = cadd(vl, cscale(cmul(sc.zl_img, ji), cosi));
+            vl = c64{-vl.x, -vl.y};
+            vt = c64{-vt.x, -vt.y};
+            c64* Wf = W + (long)f * sw;
+            Wf[(zl_off + i) * ldw + zl_off + k] = vl;
+            Wf[(zt_off + i) * ldw + zt_off + k] = vt;
+        }
+        const int h = f & 1;
+        stage.tile[h][0][a][c] = vl;
+        stage.tile[h][1][a][c] = vt;
+        __syncthreads();
+        const long ko = k0 + a, io = i0 + c;  // entry (ko, io) of the other triangle
+        if (io < m && ko < io) {
+            c64* Wf = W + (long)f * sw;
+            Wf[(zl_off + ko) * ldw + zl_off + io] = stage.tile[h][0][c][a];
+            Wf[(zt_off + ko) * ldw + zt_off + io] = stage.tile[h][1][c][a];
+        }
+    }
+}
+
+// c_k(gamma_f) = (2 - [k = 0]) / P sum_p cos(k theta_p) e^{-gamma D cos theta_p},
+// theta_p = pi (p + 1/2) / P, P = 64; one wave per sample
+__global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, double D, int K,
+                                                    c64* cf)
+{
+    __shared__ c64 ex[64];
+    const int p = threadIdx.x;
+    const c64 g = scs[blockIdx.x].gamma;
+    const double x = D * cospi((p + 0.5) / 64.0);
+    double sn, cs;
+    sincos(-g.y * x, &sn, &cs);
+    const double mag = exp(-g.x * x);
+    ex[p] = c64{mag * cs, mag * sn};
+    __syncthreads();
+    if (p >= K) return;
+    c64 s{0, 0};
+    for (int q = 0; q < 64; q++) {
+        const double w = cospi(p * (q + 0.5) / 64.0);
+        s.x = fma(w, ex[q].x, s.x);
+        s.y = fma(w, ex[q].y, s.y);
+    }
+    cf[(long)blockIdx.x * K + p] = cscale(s, (p == 0 ? 1.0 : 2.0) / 64.0);
+}
+
+// Chebyshev terms for |gamma| D = z: 2 (z / 2)^K / K! <= 1e-17, the size of the
+// first coefficient left out; 0 beyond the largest table entry
+int fill_terms(double z)
+{
+    return z <= 0.38 ? 12 : z <= 1.13 ? 16 : z <= 3.7 ? 24 : z <= 7.3 ? kFillTermsMax : 0;
+}
+
+int launch_fill_moments(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
+                        const PairScalars* scs, c64* cf, int nb, long sw, double D, double gabs,
+                        hipStream_t st)
+{
+    const long m = L.m;
+    if (m <= 0 || nb <= 0) return 0;
+    const int K = fill_terms(gabs * D);
+    if (K == 0 || !(D > 0.0) || !scs || !cf) return TAGS_ERR_ARG;
+    int rc = gl_tables_init();
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_fill_coefs, dim3(nb), dim3(64), 0, st, scs, D, K, cf);
+    const long T = (m + 15) / 16, tiles = T * (T + 1) / 2;
+    // samples per work-group: all of them once the tiles alone give every CU
+    // four work-groups, else fewer (the moments are then formed more often)
+    const long chunks = std::max(1L, std::min((long)nb, 1024 / tiles));
+    const int per = (int)((nb + chunks - 1) / chunks);
+    const dim3 g((unsigned)tiles, (unsigned)((nb + per - 1) / per));
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, g, dim3(256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, scs,
+                           sw, (const c64*)cf, nb, per, D, gabs);
+    };
+    if (K == 12) go(k_fill_moments<12>);
+    else if (K == 16) go(k_fill_moments<16>);
+    else if (K == 24) go(k_fill_moments<24>);
+    else go(k_fill_moments<kFillTermsMax>);
     TAGS_HIP(hipGetLastError());
     return 0;
 }
@@ -663,13 +1016,10 @@ __global__ __launch_bounds__(256) void k_fill_mhem(c64* W, long ldw, long zl_off
                                                     const double* __restrict__ pt,
                                                     const double* __restrict__ pli,
                                                     const double* __restrict__ pti,
-                                                    PairScalars sc, long sw,
-                                                    const PairScalars* scs)
+                                                    long sw, const PairScalars* scs)
 {
-    if (scs) {
-        sc = scs[blockIdx.z];
-        W += (long)blockIdx.z * sw;
-    }
+    const PairScalars sc = scs[blockIdx.z];
+    W += (long)blockIdx.z * sw;
     const long b = blockIdx.x;
     long ti = (long)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
     while ((ti + 1) * (ti + 2) / 2 <= b) ti++;
@@ -735,16 +1085,15 @@ __global__ __launch_bounds__(256) void k_fill_mhem(c64* W, long ldw, long zl_off
 
 int launch_fill_mhem(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
                      const double* pl, const double* pt, const double* pli, const double* pti,
-                     const PairScalars& sc, hipStream_t st, int nb, long sw,
-                     const PairScalars* scs)
+                     const PairScalars* scs, hipStream_t st, int nb, long sw)
 {
     const long m = L.m;
     if (m <= 0 || nb <= 0) return 0;
-    if (nb > 1 && !scs) return TAGS_ERR_ARG;
+    if (!scs) return TAGS_ERR_ARG;
     const long T = (m + kFT - 1) / kFT;
     const long nt = T * (T + 1) / 2;
     hipLaunchKernelGGL(k_fill_mhem, dim3((unsigned)nt, 1, (unsigned)nb), dim3(256), 0, st, W, ldw,
-                       L.zl_off, L.zt_off, m, e, img, pl, pt, pli, pti, sc, sw, scs);
+                       L.zl_off, L.zt_off, m, e, img, pl, pt, pli, pti, sw, scs);
     TAGS_HIP(hipGetLastError());
     return 0;
 }
