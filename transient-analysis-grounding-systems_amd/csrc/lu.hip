@@ -1305,14 +1305,19 @@ __global__ __launch_bounds__(256) void k_residual(const c64* W, long ld, int n, 
     }
 }
 
-// Products with a W of HEM structure (HemOp). Work-groups [0, 2m) take one
-// impedance row each (the Z_L block's rows, then Z_T's): the row's m entries
-// of the block from W, strided over the threads and summed in the order of
-// k_residual, then its one or two incidence entries. The remaining
-// work-groups take 256 node rows each, one thread per row, summing over the
-// node's segment ends in list order. mode 0: r = W x; 1: r = b - W x with
-// |r| and |x| max-reductions into norms[0], norms[1]; 2: also |W| (row sums
-// of |W_ij|) into norms[2]. The residual modes sum in double-double.
+// Products with a W of HEM structure (HemOp). The first work-groups take 16
+// impedance rows each (the Z_L block's rows, then Z_T's), a wave four of them,
+// so that x is read once per four rows and the reduction over the lanes, which
+// outweighs a row of a few hundred entries, is shared: eight sums (four rows,
+// real and imaginary) are folded over the lanes so that each halving of the
+// lanes halves the sums a lane holds, 10 exchanges instead of 48 (20 x 20 m
+// grid, 50 samples: 226 us at one row per work-group). Then each row's one or
+// two incidence entries. The remaining work-groups take 256 node rows each, one
+// thread per row, summing over the node's segment ends in list order. mode 0:
+// r = W x; 1: r = b - W x with |r| and |x| max-reductions into norms[0],
+// norms[1]; 2: also |W| (row sums of |W_ij|) into norms[2]. The residual modes
+// (RES) sum in double-double.
+template <bool RES>
 __global__ __launch_bounds__(256) void k_hem_apply(const c64* W, long ld, HemOp op, const c64* x,
                                                     long sx, const c64* b, c64* r, long sr,
                                                     unsigned long long* norms, long sn, int mode,
@@ -1326,74 +1331,81 @@ __global__ __launch_bounds__(256) void k_hem_apply(const c64* W, long ld, HemOp 
     r += z_ * sr;
     if (norms) norms += z_ * sn;
     const bool want_w = mode == 2;
-    // residuals (modes 1 and 2) in double-double; plain products (mode 0) in FP64
-    const bool comp = mode != 0;
-    const long m = op.m;
-    if ((long)blockIdx.x < 2 * m) {
-        const bool tblk = (long)blockIdx.x >= m;
-        const long i = tblk ? (long)blockIdx.x - m : (long)blockIdx.x;
+    const long m = op.m, wg = (m + 15) / 16;
+    if ((long)blockIdx.x < 2 * wg) {
+        const bool tblk = (long)blockIdx.x >= wg;
+        const int lane = threadIdx.x & 63;
+        const long i0 = ((long)blockIdx.x - (tblk ? wg : 0)) * 16 + (threadIdx.x >> 6) * 4;
+        if (i0 >= m) return;
         const long off = tblk ? op.zt_off : op.zl_off;
-        const long row = off + i;
-        const c64* Wr = W + row * ld + off;
+        const c64* Wr = W + off * ld + off;
         const c64* xz = x + off;
-        DD sx_{0, 0}, sy_{0, 0};
-        double an = 0;
-        // unrolled so that several loads per lane are in flight
-        if (comp) {
-#pragma unroll 4
-            for (long c = threadIdx.x; c < m; c += 256) {
-                const c64 a = Wr[c], v = xz[c];
-                dd_mac(sx_, a.x, v.x);
-                dd_mac(sx_, -a.y, v.y);
-                dd_mac(sy_, a.x, v.y);
-                dd_mac(sy_, a.y, v.x);
-                if (want_w) an += sqrt(a.x * a.x + a.y * a.y);
+        DD s[8];
+        double an[4];
+#pragma unroll
+        for (int q = 0; q < 8; q++) s[q] = DD{0, 0};
+#pragma unroll
+        for (int q = 0; q < 4; q++) an[q] = 0;
+#pragma unroll 2
+        for (long c = lane; c < m; c += 64) {
+            const c64 v = xz[c];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const c64 a = Wr[min(i0 + q, m - 1) * ld + c];
+                if (RES) {
+                    dd_mac(s[2 * q], a.x, v.x);
+                    dd_mac(s[2 * q], -a.y, v.y);
+                    dd_mac(s[2 * q + 1], a.x, v.y);
+                    dd_mac(s[2 * q + 1], a.y, v.x);
+                    if (want_w) an[q] += sqrt(a.x * a.x + a.y * a.y);
+                } else {
+                    s[2 * q].hi += a.x * v.x - a.y * v.y;
+                    s[2 * q + 1].hi += a.x * v.y + a.y * v.x;
+                }
             }
-        } else {
-#pragma unroll 4
-            for (long c = threadIdx.x; c < m; c += 256) {
-                const c64 a = Wr[c], v = xz[c];
-                sx_.hi += a.x * v.x - a.y * v.y;
-                sy_.hi += a.x * v.y + a.y * v.x;
-            }
         }
-        __shared__ DD red[2][4];
-        __shared__ double reda[4];
-        for (int o = 32; o > 0; o >>= 1) {
-            sx_ = dd_plus(sx_, dd_shfl_xor(sx_, o));
-            sy_ = dd_plus(sy_, dd_shfl_xor(sy_, o));
-            an += __shfl_xor(an, o);
-        }
-        const int wv = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0) {
-            red[0][wv] = sx_;
-            red[1][wv] = sy_;
-            reda[wv] = an;
-        }
-        __syncthreads();
-        if (threadIdx.x != 0) return;
-        DD tx{0, 0}, ty{0, 0};
+        // lane bit 5 keeps sums 4 .. 7, bit 4 the odd row of two, bit 3 the
+        // imaginary part
+        const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
+        auto fold = [&](DD lo, DD hi, bool up, int o) {
+            const DD mine = up ? hi : lo, other = up ? lo : hi;
+            return dd_plus(mine, dd_shfl_xor(other, o));
+        };
+        DD f4[4], f2[2];
+#pragma unroll
+        for (int q = 0; q < 4; q++) f4[q] = fold(s[q], s[q + 4], b5, 32);
+#pragma unroll
+        for (int q = 0; q < 2; q++) f2[q] = fold(f4[q], f4[q + 2], b4, 16);
+        DD t = fold(f2[0], f2[1], b3, 8);
+        for (int o = 4; o > 0; o >>= 1) t = dd_plus(t, dd_shfl_xor(t, o));
+        DD tx = t, ty = dd_shfl_xor(t, 8);  // lanes with bit 3 clear: real, imaginary
         double ta = 0;
-        for (int q = 0; q < 4; q++) {
-            tx = dd_plus(tx, red[0][q]);
-            ty = dd_plus(ty, red[1][q]);
-            ta += reda[q];
+        if (want_w) {
+            double a2[2];
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+                a2[q] = (b5 ? an[q + 2] : an[q]) + __shfl_xor(b5 ? an[q] : an[q + 2], 32);
+            ta = (b4 ? a2[1] : a2[0]) + __shfl_xor(b4 ? a2[0] : a2[1], 16);
+            for (int o = 8; o > 0; o >>= 1) ta += __shfl_xor(ta, o);
         }
+        const long i = i0 + (b5 ? 2 : 0) + (b4 ? 1 : 0);
+        if ((lane & 15) || i >= m) return;
+        const long row = off + i;
         // incidence: A (+1 start, -1 end) on Z_L rows, B (1/2, 1/2) on Z_T rows
         // (products by +-1 and 1/2 are exact)
-        const int s = op.sn[i], e = op.en[i];
+        const int sg = op.sn[i], e = op.en[i];
         const double cs = tblk ? 0.5 : 1.0, ce = tblk ? 0.5 : -1.0;
-        const c64 xs = x[op.node_off + s];
+        const c64 xs = x[op.node_off + sg];
         dd_add(tx, cs * xs.x);
         dd_add(ty, cs * xs.y);
         ta += fabs(cs);
-        if (e != s) {
+        if (e != sg) {
             const c64 xe = x[op.node_off + e];
             dd_add(tx, ce * xe.x);
             dd_add(ty, ce * xe.y);
             ta += fabs(ce);
         }
-        if (mode == 0) {
+        if (!RES) {
             r[row] = c64{tx.hi + tx.lo, ty.hi + ty.lo};
             return;
         }
@@ -1407,7 +1419,7 @@ __global__ __launch_bounds__(256) void k_hem_apply(const c64* W, long ld, HemOp 
         return;
     }
     // node rows: sum over the node's segment ends of A^T (x_L) and B^T (x_T)
-    const long u = ((long)blockIdx.x - 2 * m) * 256 + threadIdx.x;
+    const long u = ((long)blockIdx.x - 2 * wg) * 256 + threadIdx.x;
     double ra = 0, xa = 0, ta = 0;
     if (u < op.n) {
         DD tx{0, 0}, ty{0, 0};
@@ -2699,9 +2711,13 @@ int hem_apply(const c64* W, long ld, const HemOp& op, const c64* x, long sx, con
     if (op.m < 1 || op.n < 1 || nb < 1 || !op.sn || !op.en || !op.node_ptr || !op.node_seg)
         return TAGS_ERR_ARG;
     if (mode != 0 && (!b || !norms)) return TAGS_ERR_ARG;
-    const long g = 2 * op.m + (op.n + 255) / 256;
-    hipLaunchKernelGGL(k_hem_apply, dim3((unsigned)g, 1, (unsigned)nb), dim3(256), 0, st, W, ld, op,
-                       x, sx, b, r, sr, norms, sn, mode, sw, active);
+    const dim3 g((unsigned)(2 * ((op.m + 15) / 16) + (op.n + 255) / 256), 1, (unsigned)nb);
+    if (mode != 0)
+        hipLaunchKernelGGL(k_hem_apply<true>, g, dim3(256), 0, st, W, ld, op, x, sx, b, r, sr,
+                           norms, sn, mode, sw, active);
+    else
+        hipLaunchKernelGGL(k_hem_apply<false>, g, dim3(256), 0, st, W, ld, op, x, sx, b, r, sr,
+                           norms, sn, mode, sw, active);
     TAGS_HIP(hipGetLastError());
     return 0;
 }

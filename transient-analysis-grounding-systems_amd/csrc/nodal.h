@@ -43,7 +43,7 @@ struct NodalSolver {
     c64* Z = nullptr;   // impedance blocks, item stride sZ
     long sZ = 0;
     void *F = nullptr, *S = nullptr;    // factored blocks (2 per item), node systems
-    void *tp = nullptr, *op_ = nullptr, *tt = nullptr, *P = nullptr;
+    void *tp = nullptr, *op_ = nullptr, *P = nullptr, *xt = nullptr, *xo = nullptr;
     c64 *x = nullptr, *r = nullptr, *b = nullptr, *ysum = nullptr, *dg = nullptr, *cst = nullptr;
     void *v = nullptr, *z = nullptr, *f = nullptr, *y = nullptr, *h = nullptr, *c = nullptr;
     c64* u = nullptr;
@@ -59,6 +59,8 @@ struct NodalSolver {
     // Queues the solve of nb samples whose Z is filled (or queued on st): unit
     // current at node inj. No host wait.
     int issue(int nb, long inj);
+    // The same for one sample with the right-hand side in b (complex128 only).
+    int issue_rhs();
     // Called when st is idle. While samples still refine: queues one more step
     // for them, *complete false. Then per item: done steps, backward error,
     // forward estimate and whether it was accepted; u in hu, x in x.
@@ -70,6 +72,9 @@ struct NodalSolver {
 private:
     int step_ = 0;
     bool first_ = true;
+    bool unit_ = true;  // the right-hand side is a unit current at inj
+    int queue_spec();
+    int queue_results();
     double norm_at(int q, int k, int i) const;
     double berr_at(int q, int k) const;
     double dx_at(int q, int k) const;
@@ -82,5 +87,28 @@ private:
     template <typename T>
     size_t partition(char* base, int batch);
 };
+
+// Explicit inverses of complex symmetric matrices without row exchanges, `items`
+// of order dim: src row-major with pitch lds (the upper triangle is read, item
+// stride ssrc), X with pitch ld = dim rounded up to 64 (both triangles, zero
+// beyond dim, item stride ld ld). work: sym_inverse_bytes.
+size_t sym_inverse_bytes(long dim, int items);
+int sym_inverse(const c64* src, long lds, long ssrc, c64* X, long dim, int items, char* work,
+                hipStream_t st);
+// x += X r (n of them), the largest |X r| into *dmax (a max-reduction)
+int sym_apply(const c64* X, long ld, long n, const c64* r, c64* x, unsigned long long* dmax,
+              hipStream_t st);
+// R -= I for `items` m x m matrices, the largest |entry| into *dmax
+int sub_identity(c64* R, long m, int items, unsigned long long* dmax, hipStream_t st);
+// upper triangles of X by rows (see copy_out_rows), items one after the other
+int sym_pack(const c64* X, long ld, long m, int items, c64* out, hipStream_t st);
+
+// Whether W (N x N, N = n + 2 m; lower triangle column-major) is an immittance
+// matrix of the HEM in the reference order: out = start nodes (m), end nodes
+// (m), the number of start and of end entries found per segment (2 m), and the
+// count of entries that do not fit.
+int imm_structure(const c64* W, long N, long m, long n, int* out, hipStream_t st);
+// its impedance blocks in NodalSolver's storage
+int imm_blocks(const c64* W, long N, long m, long n, c64* Z, hipStream_t st);
 
 }  // namespace tags

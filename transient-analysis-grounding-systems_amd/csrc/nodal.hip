@@ -39,8 +39,16 @@
 
 #include "mfma.h"
 #include "nodal.h"
+#include "x6.h"
 
 namespace tags {
+
+// Order from which complex64 inversions take 256-column steps and the bf16 MFMA
+// cores. With 128 columns the split operands (12 bytes per value) and the
+// tile's start and end outweigh the faster products: 48 samples of the 30 x 30
+// m grid (order 1320), per step 615 us on the fp32 cores with 128 columns, 861
+// us on the bf16 cores, 951 us per 256 columns there.
+constexpr long kX6Dim = 4096;
 
 // Work-group index over `total` pieces of work such that each XCD (blockIdx.x
 // mod 8) takes a contiguous range, so that the pieces of one item meet in one
@@ -63,7 +71,9 @@ struct NdPhase {
     int ld, dim, items;
     cx<T>*tp, *op;  // T and O of the current step in MFMA fragment order
     long sp;
-    cx<T>* P;       // inverse of the current diagonal block
+    cx<T>* P;       // inverses of the step's diagonal blocks
+    u32x4 *xt, *xo;  // the same for the split-bf16 update (complex64; null: not used)
+    long sx;
 };
 
 // Fragment order of a ld x NB panel: a wave's MFMA operand (16 rows, 4 k) is
@@ -79,123 +89,281 @@ __device__ inline long nd_pk(int i, int k)
                ((k >> 2) & 1);
 }
 
+// re, im (tiles of a wave) += T_i O_j^T over the k groups [g0, g1) of 16-row
+// strips: operands in fragment order straight from memory, the next group's
+// loads in flight during the current one's MFMAs.
+template <typename T, int NB, int TI, int TJ>
+__device__ __forceinline__ void nd_mma(const cx<T>* tp, const cx<T>* op, int i0, int j0, int g0,
+                                       int g1, typename Mfma<T>::v4 (&re)[TI][TJ],
+                                       typename Mfma<T>::v4 (&im)[TI][TJ])
+{
+    constexpr int KG = sizeof(T) == 8 ? 4 : 8;  // k per 16-byte lane load
+    constexpr int KU = KG / 4;
+    constexpr long FS = (long)(NB / KG) * 64;  // loads of one 16-row strip
+    struct alignas(16) Frag {
+        cx<T> e[KU];
+    };
+    const int lane = threadIdx.x & 63;
+    const Frag* ta = (const Frag*)tp + (i0 / 16) * FS + lane;
+    const Frag* ob = (const Frag*)op + (j0 / 16) * FS + lane;
+    if (g0 >= g1) return;
+    Frag a[TI], b[TJ], an[TI], bn[TJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++) a[i] = ta[i * FS + (long)g0 * 64];
+#pragma unroll
+    for (int j = 0; j < TJ; j++) b[j] = ob[j * FS + (long)g0 * 64];
+    for (int g = g0; g < g1; g++) {
+        const long o = (long)min(g + 1, g1 - 1) * 64;
+#pragma unroll
+        for (int i = 0; i < TI; i++) an[i] = ta[i * FS + o];
+#pragma unroll
+        for (int j = 0; j < TJ; j++) bn[j] = ob[j * FS + o];
+#pragma unroll
+        for (int u = 0; u < KU; u++)
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int j = 0; j < TJ; j++) {
+                    const cx<T> x = a[i].e[u], y = b[j].e[u];
+                    re[i][j] = Mfma<T>::run(x.x, y.x, re[i][j]);
+                    im[i][j] = Mfma<T>::run(x.x, y.y, im[i][j]);
+                    re[i][j] = Mfma<T>::run(-x.y, y.y, re[i][j]);
+                    im[i][j] = Mfma<T>::run(x.y, y.x, im[i][j]);
+                }
+#pragma unroll
+        for (int i = 0; i < TI; i++) a[i] = an[i];
+#pragma unroll
+        for (int j = 0; j < TJ; j++) b[j] = bn[j];
+    }
+}
+template <typename T>
+constexpr int nd_groups(int k)  // k groups of nd_mma in k columns
+{
+    return sizeof(T) == 8 ? k / 4 : k / 8;
+}
+
 // ---------------------------------------------------------------------------
-// One step of the symmetric sweep for the block K = [c0, c0 + NB):
+// The symmetric sweep of a block K of columns:
 //   P = A_KK^-1, T = A_*K P, A_ij -= T_i A_jK^T, A_*K = T, A_KK = -P;
-// after all steps A holds -A^-1. Every matrix in between is symmetric, rows
+// after all blocks A holds -A^-1. Every matrix in between is symmetric, rows
 // before and after K are treated alike, and only tiles on and below the
 // diagonal are touched.
+//
+// A step takes NB / 64 blocks K_0, K_1, .. of 64 columns from c0 on. Per block
+// t, k_nd_diag forms P_t and k_nd_panel O_t = A_*K_t as the earlier blocks of
+// the step leave it and T_t = O_t P_t, both without touching A:
+//   O_t(i) = A_iK_t - sum_{s < t} T_s(i) O_s(K_t)^T,
+// and for a row block K_s of the step itself, s < t (already swept),
+//   O_t(K_s) = T_s(K_t)^T - sum_{s < u < t} T_u(K_s) O_u(K_t)^T.
+// Then one k_nd_update reads and writes every tile once with all NB columns:
+//   A_ij -= sum_u T_u(i) O_u(j)^T,
+// and a tile of row block K_s and / or column block K_r, q = max(s, r), gets
+//   (-P_q if s = r, else T_q of the other side) - sum_{u > q} T_u(i) O_u(j)^T.
 // ---------------------------------------------------------------------------
 
-// P by an unblocked sweep, one work-group of 1024 threads per item: thread t
-// holds NB^2 / 1024 entries of one row in registers; per step the pivot row
-// goes through LDS (it is the pivot column too), one barrier. Latency-bound:
-// NB steps of a broadcast, a reciprocal and NB^2 / 1024 multiply-adds.
+// P_t by an unblocked sweep, one work-group per item: a thread holds 4 x 4
+// entries in registers; per pivot the pivot row goes through LDS (it is the
+// pivot column too), one barrier. Latency-bound: 64 steps of a broadcast, a
+// reciprocal and 16 complex multiply-adds.
 template <typename T, int NB>
-__global__ __launch_bounds__(1024) void k_nd_diag(NdPhase<T> p, int kb)
-{
-    constexpr int TPR = 1024 / NB, E = NB / TPR;
-    const cx<T>* A = p.A + (long)blockIdx.x * p.sA;
-    cx<T>* P = p.P + (long)blockIdx.x * NB * NB;
-    const int c0 = kb * NB, kv = min(NB, p.dim - c0);
-    const int r = threadIdx.x / TPR, q = threadIdx.x % TPR;
-    __shared__ cx<T> row[2][NB];
-    cx<T> a[E];
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        const int c = q + TPR * e;
-        a[e] = cx<T>{0, 0};
-        if (r < kv && c < kv) a[e] = A[(long)(c0 + max(r, c)) * p.ld + c0 + min(r, c)];
-    }
-    for (int j = 0; j < kv; j++) {
-        cx<T>* rj = row[j & 1];
-        if (r == j) {
-#pragma unroll
-            for (int e = 0; e < E; e++) rj[q + TPR * e] = a[e];
-        }
-        __syncthreads();
-        const cx<T> d = crecip_fast(rj[j]);
-        const cx<T> l = cmul(rj[r], d);
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            const int c = q + TPR * e;
-            const cx<T> o = rj[c];
-            const cx<T> upd = cfnma(a[e], l, o);
-            const cx<T> own = cmul(o, d);
-            cx<T> nv = csel(r == j, own, csel(c == j, l, upd));
-            if (r == j && c == j) nv = cx<T>{-d.x, -d.y};
-            a[e] = nv;
-        }
-    }
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        const int c = q + TPR * e;
-        const bool in = r < kv && c < kv;
-        P[r * NB + c] = in ? cx<T>{-a[e].x, -a[e].y} : cx<T>{0, 0};
-    }
-}
-
-// O(i, k) of the current panel: A_iK from the stored tiles (rows before K from
-// the row block, transposed).
-template <typename T>
-__device__ inline cx<T> nd_panel_at(const cx<T>* A, long ld, int i, int c, bool before)
-{
-    return before ? A[(long)c * ld + i] : A[(long)i * ld + c];
-}
-
-// T = O P for 64 rows and 64 columns of the panel, with T and O written in
-// fragment order for the update. Four waves of 16 rows; operands straight from
-// memory (O is read once per 64 columns, P stays in L2).
-template <typename T, int NB>
-__global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int kb)
+__global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t)
 {
     using V4 = typename Mfma<T>::v4;
-    constexpr int YC = NB / 64;
-    const int nt = p.ld / 64;
-    const long flat = xcd_flat((long)p.items * nt * YC);
-    if (flat < 0) return;
-    const int item = (int)(flat / (nt * YC)), rem = (int)(flat % (nt * YC));
-    const int rb = rem / YC, yc = rem % YC;
-    const int c0 = kb * NB;
-    if (rb * 64 >= c0 && rb * 64 < c0 + NB) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int i0 = rb * 64 + wave * 16;
-    if (i0 >= p.dim) return;
-    const bool before = rb * 64 < c0;
-    const int kv = min(NB, p.dim - c0);
-    const cx<T>* A = p.A + (long)item * p.sA;
-    const cx<T>* P = p.P + (long)item * NB * NB + yc * 64;
-    cx<T>* tp = p.tp + (long)item * p.sp;
-    cx<T>* op = p.op + (long)item * p.sp;
-    const int lr = lane & 15, lk = lane >> 4;
-    V4 re[4], im[4];
+    const long item = blockIdx.x;
+    const cx<T>* A = p.A + item * p.sA;
+    cx<T>* P = p.P + (item * (NB / 64) + t) * 4096;
+    const int cK = c0 + 64 * t, kv = min(64, p.dim - cK);
+    const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
+    __shared__ cx<T> row[2][64];
+    cx<T> a[4][4];
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-        re[t] = V4{0, 0, 0, 0};
-        im[t] = V4{0, 0, 0, 0};
-    }
-#pragma unroll 4
-    for (int g = 0; g < NB / 4; g++) {
-        const int k = 4 * g + lk;
-        cx<T> a{0, 0};
-        if (k < kv) a = nd_panel_at(A, p.ld, i0 + lr, c0 + k, before);
-        if (yc == 0) op[nd_pk<T, NB>(i0 + lr, k)] = a;
-        const T na = -a.y;
+    for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const cx<T> b = P[k * NB + t * 16 + lr];
-            re[t] = Mfma<T>::run(a.x, b.x, re[t]);
-            im[t] = Mfma<T>::run(a.x, b.y, im[t]);
-            re[t] = Mfma<T>::run(na, b.y, re[t]);
-            im[t] = Mfma<T>::run(a.y, b.x, im[t]);
+        for (int j = 0; j < 4; j++) {
+            const int r = ty + 16 * i, c = tx + 16 * j;
+            a[i][j] = cx<T>{0, 0};
+            if (r < kv && c < kv) a[i][j] = A[(long)(cK + max(r, c)) * p.ld + cK + min(r, c)];
+        }
+    if constexpr (NB > 64) {
+        if (t > 0) {
+            // less the step's earlier blocks, four waves of 32 x 32
+            __shared__ cx<T> up[64][65];
+            const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+            const int i0 = (wave >> 1) * 32, j0 = (wave & 1) * 32;
+            V4 re[2][2], im[2][2];
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    re[i][j] = V4{0, 0, 0, 0};
+                    im[i][j] = V4{0, 0, 0, 0};
+                }
+            nd_mma<T, NB, 2, 2>(p.tp + item * p.sp, p.op + item * p.sp, cK + i0, cK + j0, 0,
+                                nd_groups<T>(64 * t), re, im);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        up[i0 + 16 * i + Mfma<T>::row(lane, v)][j0 + 16 * j + (lane & 15)] =
+                            cx<T>{re[i][j][v], im[i][j][v]};
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int r = ty + 16 * i, c = tx + 16 * j;
+                    if (r < kv && c < kv) a[i][j] = csub(a[i][j], up[max(r, c)][min(r, c)]);
+                }
         }
     }
+    for (int k = 0; k < kv; k++) {
+        cx<T>* rk = row[k & 1];
+        if (ty == (k & 15)) {
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+            for (int j = 0; j < 4; j++) {
+                // row k = ty + 16 (k >> 4)
+                const cx<T> lo = csel((k >> 4) & 1, a[1][j], a[0][j]);
+                const cx<T> hi = csel((k >> 4) & 1, a[3][j], a[2][j]);
+                rk[tx + 16 * j] = csel(k >> 5, hi, lo);
+            }
+        }
+        __syncthreads();
+        const cx<T> d = crecip_fast(rk[k]);
+        cx<T> o[4], l[4];
 #pragma unroll
-        for (int v = 0; v < 4; v++)
-            tp[nd_pk<T, NB>(i0 + Mfma<T>::row(lane, v), yc * 64 + t * 16 + lr)] =
-                cx<T>{re[t][v], im[t][v]};
+        for (int j = 0; j < 4; j++) o[j] = rk[tx + 16 * j];
+#pragma unroll
+        for (int i = 0; i < 4; i++) l[i] = cmul(rk[ty + 16 * i], d);
+        const bool mr = ty == (k & 15), mc = tx == (k & 15);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const bool pr = mr && i == (k >> 4), pc = mc && j == (k >> 4);
+                cx<T> n = cfnma(a[i][j], l[i], o[j]);
+                n = csel(pr, cmul(o[j], d), csel(pc, l[i], n));
+                n = csel(pr && pc, cx<T>{-d.x, -d.y}, n);
+                a[i][j] = n;
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int r = ty + 16 * i, c = tx + 16 * j;
+            const bool in = r < kv && c < kv;
+            P[r * 64 + c] = in ? cx<T>{-a[i][j].x, -a[i][j].y} : cx<T>{0, 0};
+        }
+}
+
+// O_t and T_t of 64 rows: four waves of 16 rows and 64 columns. O_t passes
+// through LDS from the MFMA result layout to the operand layout (each wave its
+// own rows).
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int c0, int t)
+{
+    using V4 = typename Mfma<T>::v4;
+    const int nt = p.ld / 64;
+    const long flat = xcd_flat((long)p.items * nt);
+    if (flat < 0) return;
+    const int item = (int)(flat / nt), rb = (int)(flat % nt);
+    const int s = rb * 64 - c0, cK = c0 + 64 * t;
+    const int own = s >= 0 && s < NB ? s / 64 : -1;  // block of the step these rows are in
+    if (own == t) return;
+    const bool swept = own >= 0 && own < t;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int i0 = rb * 64 + wave * 16;
+    const bool before = s < 0;
+    const int kv = min(64, p.dim - cK);
+    const cx<T>* A = p.A + (long)item * p.sA;
+    const cx<T>* P = p.P + ((long)item * (NB / 64) + t) * 4096;
+    cx<T>* tp = p.tp + (long)item * p.sp;
+    cx<T>* op = p.op + (long)item * p.sp;
+    __shared__ cx<T> tile[64][65];
+    const bool live = i0 < p.dim;
+    V4 re[1][4], im[1][4];
+    if (live) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            re[0][c] = V4{0, 0, 0, 0};
+            im[0][c] = V4{0, 0, 0, 0};
+        }
+        if (NB > 64 && t > 0)
+            nd_mma<T, NB, 1, 4>(tp, op, i0, cK, nd_groups<T>(swept ? 64 * (own + 1) : 0),
+                                nd_groups<T>(64 * t), re, im);
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = i0 + Mfma<T>::row(lane, v), k = 16 * c + lr;
+                cx<T> o{0, 0};
+                if (k < kv) {
+                    o = swept ? tp[nd_pk<T, NB>(cK + k, i - c0)]
+                              : A[before ? (long)(cK + k) * p.ld + i : (long)i * p.ld + cK + k];
+                    o = cx<T>{o.x - re[0][c][v], o.y - im[0][c][v]};
+                }
+                tile[wave * 16 + Mfma<T>::row(lane, v)][k] = o;
+            }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            re[0][c] = V4{0, 0, 0, 0};
+            im[0][c] = V4{0, 0, 0, 0};
+        }
+    }
+    __syncthreads();
+    if (live) {
+#pragma unroll 4
+        for (int g = 0; g < 16; g++) {
+            const int k = 4 * g + lk;
+            const cx<T> a = tile[wave * 16 + lr][k];
+            op[nd_pk<T, NB>(i0 + lr, 64 * t + k)] = a;
+            const T na = -a.y;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const cx<T> b = P[k * 64 + 16 * c + lr];
+                re[0][c] = Mfma<T>::run(a.x, b.x, re[0][c]);
+                im[0][c] = Mfma<T>::run(a.x, b.y, im[0][c]);
+                re[0][c] = Mfma<T>::run(na, b.y, re[0][c]);
+                im[0][c] = Mfma<T>::run(a.y, b.x, im[0][c]);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                tp[nd_pk<T, NB>(i0 + Mfma<T>::row(lane, v), 64 * t + 16 * c + lr)] =
+                    cx<T>{re[0][c][v], im[0][c][v]};
+    }
+    if constexpr (sizeof(T) == 4) {
+        if (!p.xt) return;
+        // the same, split into bf16 parts (rows past dim: zero)
+        auto pack = [&](u32x4* out) {
+            for (int e = threadIdx.x; e < 512; e += 256) {
+                const int r = e & 63, k8 = e >> 6;  // 8 columns from 8 k8
+                c32 x[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++)
+                    x[q] = rb * 64 + r < p.dim ? tile[r][8 * k8 + q] : c32{0, 0};
+                x6_pack8(x, out + (long)item * p.sx +
+                                x6_word(rb * 64 + r, 64 * t + 8 * k8, NB / 16));
+            }
+        };
+        pack(p.xo);
+        __syncthreads();
+        if (live) {
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    tile[wave * 16 + Mfma<T>::row(lane, v)][16 * c + lr] =
+                        cx<T>{re[0][c][v], im[0][c][v]};
+        }
+        __syncthreads();
+        pack(p.xt);
+    }
 }
 
 // row and column tile of index t of a triangle's tiles (row >= column)
@@ -207,61 +375,42 @@ __device__ inline void tri_tile(int t, int& ti, int& tj)
     tj = t - ti * (ti + 1) / 2;
 }
 
-// Tiles of block K after the update: A_*K = T, A_KK = -P. ti, tj: 64 x 64 tile.
+// 64 x 64 tiles of the update: four waves of 32 x 32, operands in fragment
+// order straight from L2 (a wave needs 4 bytes per cycle of them beside its
+// MFMAs, so LDS staging would only add barriers). placed: only the tiles of the
+// step's own blocks (the others are k_nd_update_x6's).
 template <typename T, int NB>
-__device__ inline void nd_place(const NdPhase<T>& p, cx<T>* A, int item, int c0, int ti, int tj,
-                                bool inrow, bool incol)
-{
-    const cx<T>* tp = p.tp + (long)item * p.sp;
-    const cx<T>* P = p.P + (long)item * NB * NB;
-    for (int e = threadIdx.x; e < 4096; e += 256) {
-        const int i = ti * 64 + (e >> 6), j = tj * 64 + (e & 63);
-        if (i >= p.dim || j >= p.dim) continue;
-        cx<T> t;
-        if (inrow && incol) {
-            t = P[(i - c0) * NB + j - c0];
-            t = cx<T>{-t.x, -t.y};
-        } else if (incol) {
-            t = tp[nd_pk<T, NB>(i, j - c0)];
-        } else {
-            t = tp[nd_pk<T, NB>(j, i - c0)];
-        }
-        A[(long)i * p.ld + j] = t;
-    }
-}
-
-// A_ij -= T_i O_j^T on 64 x 64 tiles: four waves of 32 x 32, operands in
-// fragment order straight from L2 (a wave needs 4 bytes per cycle of them
-// beside its MFMAs, so LDS staging would only add barriers).
-template <typename T, int NB>
-__global__ __launch_bounds__(256) void k_nd_update(NdPhase<T> p, int kb)
+__global__ __launch_bounds__(256) void k_nd_update(NdPhase<T> p, int c0, int placed)
 {
     using V4 = typename Mfma<T>::v4;
-    constexpr int KG = sizeof(T) == 8 ? 4 : 8;  // k per 16-byte lane load
-    constexpr int KU = KG / 4;
-    struct alignas(16) Frag {
-        cx<T> e[KU];
-    };
-    const int nt = p.ld / 64, ntri = nt * (nt + 1) / 2;
-    const long flat = xcd_flat((long)p.items * ntri);
-    if (flat < 0) return;
-    const int item = (int)(flat / ntri);
-    int ti, tj;
-    tri_tile((int)(flat % ntri), ti, tj);
-    const int c0 = kb * NB, k0 = c0 / 64;
-    cx<T>* A = p.A + (long)item * p.sA;
-    const bool inrow = ti >= k0 && ti < k0 + NB / 64, incol = tj >= k0 && tj < k0 + NB / 64;
-    if (inrow || incol) {
-        nd_place<T, NB>(p, A, item, c0, ti, tj, inrow, incol);
-        return;
+    const int nt = p.ld / 64, k0 = c0 / 64, nq = min(NB / 64, nt - k0);
+    int item, ti, tj;
+    if (placed) {
+        // nt tiles per block: row block K_s (columns up to it), then the rows below
+        const long flat = xcd_flat((long)p.items * nq * nt);
+        if (flat < 0) return;
+        item = (int)(flat / (nq * nt));
+        const int r = (int)(flat % (nq * nt)), s = k0 + r / nt, o = r % nt;
+        ti = max(s, o);
+        tj = min(s, o);
+        // a tile of two of the step's blocks is its row block's
+        if (o > s && o < k0 + nq) return;
+    } else {
+        const int ntri = nt * (nt + 1) / 2;
+        const long flat = xcd_flat((long)p.items * ntri);
+        if (flat < 0) return;
+        item = (int)(flat / ntri);
+        tri_tile((int)(flat % ntri), ti, tj);
     }
+    const int si = ti >= k0 && ti < k0 + nq ? ti - k0 : -1;
+    const int sj = tj >= k0 && tj < k0 + nq ? tj - k0 : -1;
+    const int q = max(si, sj);
+    cx<T>* A = p.A + (long)item * p.sA;
+    const cx<T>* tp = p.tp + (long)item * p.sp;
+    const cx<T>* op = p.op + (long)item * p.sp;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i0 = ti * 64 + (wave >> 1) * 32, j0 = tj * 64 + (wave & 1) * 32;
     if (i0 >= p.dim || j0 >= p.dim || j0 > i0 + 31) return;
-    const int ng = (min(NB, p.dim - c0) + KG - 1) / KG;
-    constexpr long FS = (long)(NB / KG) * 64;  // fragments of one 16-row strip
-    const Frag* ta = (const Frag*)(p.tp + (long)item * p.sp) + (i0 / 16) * FS + lane;
-    const Frag* ob = (const Frag*)(p.op + (long)item * p.sp) + (j0 / 16) * FS + lane;
     V4 re[2][2], im[2][2];
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -270,53 +419,63 @@ __global__ __launch_bounds__(256) void k_nd_update(NdPhase<T> p, int kb)
             re[i][j] = V4{0, 0, 0, 0};
             im[i][j] = V4{0, 0, 0, 0};
         }
-    Frag a[2], b[2], an[2], bn[2];
+    const int kt = (min(NB, p.dim - c0) + 7) & ~7;
+    nd_mma<T, NB, 2, 2>(tp, op, i0, j0, nd_groups<T>(64 * (q + 1)), nd_groups<T>(kt), re, im);
+    const cx<T>* P = q < 0 ? nullptr : p.P + ((long)item * (NB / 64) + q) * 4096;
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        a[i] = ta[i * FS];
-        b[i] = ob[i * FS];
-    }
-    for (int g = 0; g < ng; g++) {
-        const long o = (long)min(g + 1, ng - 1) * 64;
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            an[i] = ta[i * FS + o];
-            bn[i] = ob[i * FS + o];
-        }
-#pragma unroll
-        for (int u = 0; u < KU; u++)
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const cx<T> x = a[i].e[u], y = b[j].e[u];
-                    re[i][j] = Mfma<T>::run(x.x, y.x, re[i][j]);
-                    im[i][j] = Mfma<T>::run(x.x, y.y, im[i][j]);
-                    re[i][j] = Mfma<T>::run(-x.y, y.y, re[i][j]);
-                    im[i][j] = Mfma<T>::run(x.y, y.x, im[i][j]);
-                }
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            a[i] = an[i];
-            b[i] = bn[i];
-        }
-    }
-    // a strip past dim holds no operands
-    const bool j1 = j0 + 16 < p.dim;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        if (i0 + 16 * i >= p.dim) break;
+    for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            cx<T>* cr = A + (long)(i0 + 16 * i + Mfma<T>::row(lane, v)) * p.ld + j0 + (lane & 15);
+            const int r = i0 + 16 * i + Mfma<T>::row(lane, v);
+            if (r >= p.dim) continue;
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                if (j && !j1) break;
-                const cx<T> o = cr[16 * j];
-                cr[16 * j] = cx<T>{o.x - re[i][j][v], o.y - im[i][j][v]};
+                const int c = j0 + 16 * j + (lane & 15);
+                if (c >= p.dim) continue;
+                cx<T>* a = A + (long)r * p.ld + c;
+                cx<T> o;
+                if (q < 0) {
+                    o = *a;
+                } else if (si == sj) {
+                    o = P[(r - ti * 64) * 64 + c - tj * 64];
+                    o = cx<T>{-o.x, -o.y};
+                } else {
+                    o = si > sj ? tp[nd_pk<T, NB>(c, r - c0)] : tp[nd_pk<T, NB>(r, c - c0)];
+                }
+                *a = cx<T>{o.x - re[i][j][v], o.y - im[i][j][v]};
             }
         }
-    }
+}
+
+// The update's other tiles in complex64 on the bf16 MFMA cores (see x6.h):
+// 128 x 64 tiles of four waves. dim > NB.
+template <int NB>
+__global__ __launch_bounds__(256, 1) void k_nd_update_x6(NdPhase<float> p, int c0)
+{
+    // tiles on and below the diagonal: row tile I has 2 I + 2 column tiles
+    const int nm = (p.ld + 127) / 128, nn = p.ld / 64;
+    const int per = nm * (nm + 1);
+    const long flat = xcd_flat((long)p.items * per);
+    if (flat < 0) return;
+    const int item = (int)(flat / per);
+    int I, J;
+    tri_tile((int)(flat % per) / 2, I, J);
+    J = 2 * J + ((int)(flat % per) & 1);
+    if (J >= nn) return;
+    const int r0 = I * 128, q0 = J * 64;
+    if ((r0 >= c0 && r0 < c0 + NB) || (q0 >= c0 && q0 < c0 + NB)) return;
+    if (r0 >= p.dim || q0 >= p.dim) return;
+    X6Args g;
+    g.M = g.N = p.dim;
+    g.K = min(NB, p.dim - c0);
+    g.ks = NB / 16;
+    g.pa = p.xt + (long)item * p.sx;
+    g.pb = p.xo + (long)item * p.sx;
+    g.C = p.A + (long)item * p.sA;
+    g.ldc = p.ld;
+    g.crow = nullptr;
+    g.mode = 1;
+    x6l_tile<4, 1, 1, 2, false, 2>(g, I, J);
 }
 
 // A_ij of the tiles above the diagonal from those below, 64 x 64 tiles through
@@ -703,13 +862,13 @@ __global__ __launch_bounds__(256) void k_nd_currents(NdArgs<T> g, int k, int fir
     dx_max(g.norms + item * g.snorm + 4 * k + 3, dm);
 }
 
-// b = e_inj, zeroed norms, zero padding of the vectors
+// b = e_inj (unless null), zeroed norms, zero padding of the vectors
 template <typename T>
 __global__ __launch_bounds__(256) void k_nd_init(NdArgs<T> g, c64* b)
 {
     const long item = blockIdx.y;
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i < g.N) b[item * g.N + i] = c64{i == 2 * g.m + g.inj ? 1.0 : 0.0, 0.0};
+    if (b && i < g.N) b[item * g.N + i] = c64{i == 2 * g.m + g.inj ? 1.0 : 0.0, 0.0};
     if (i < g.snorm) g.norms[item * g.snorm + i] = 0;
     const cx<T> zero{0, 0};
     if (i < 2 * g.mp) g.v[2 * item * g.mp + i] = zero;
@@ -726,12 +885,18 @@ __global__ __launch_bounds__(256) void k_nd_pick(NdArgs<T> g, c64* u)
 // ---------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------
-// Columns per sweep step: a step costs one diagonal-block sweep (latency) and
-// reads and writes every tile once, so wider steps pay once the tiles
-// outweigh the panel's work.
-constexpr int kWideDim = 600;
-static int nd_block(long dim) { return dim >= kWideDim ? 128 : 64; }
+// Columns per sweep step. A step reads and writes every tile once, which at 64
+// columns takes as long as its MFMAs; more blocks per step cost the panels'
+// products with the step's earlier blocks.
+static int nd_block(long dim, bool f64)
+{
+    if (dim <= 128) return 64;
+    return !f64 && dim >= kX6Dim ? 256 : 128;
+}
+static bool nd_x6(long dim, bool f64) { return !f64 && dim >= kX6Dim; }
 static long up(long v, long a) { return (v + a - 1) / a * a; }
+// 16-byte words of one matrix's split-bf16 panel
+static long nd_x6_words(long ld, int nb) { return ld / 32 * (nb / 16) * X6_PARTS * X6_FRAG; }
 
 template <typename T>
 size_t NodalSolver::partition(char* base, int batch)
@@ -743,9 +908,12 @@ size_t NodalSolver::partition(char* base, int batch)
         return p;
     };
     const size_t B = (size_t)batch, e = sizeof(cx<T>);
-    const long bz = nd_block(m), bs = nd_block(n);
+    const bool d = sizeof(T) == 8;
+    const long bz = nd_block(m, d), bs = nd_block(n, d);
     const size_t panel = std::max(2 * (size_t)mp * bz, (size_t)np * bs);
-    const size_t diag = (size_t)std::max(2 * bz * bz, bs * bs);
+    const size_t diag = 64 * (size_t)std::max(2 * bz, bs);
+    const size_t words = std::max(nd_x6(m, d) ? 2 * (size_t)nd_x6_words(mp, bz) : 0,
+                                  nd_x6(n, d) ? (size_t)nd_x6_words(np, bs) : 0);
     sZ = nodal_z_items(m);
     Z = (c64*)take(sizeof(c64) * sZ * B);
     F = take(e * 2 * mp * mp * B);
@@ -753,6 +921,8 @@ size_t NodalSolver::partition(char* base, int batch)
     tp = take(e * panel * B);
     op_ = take(e * panel * B);
     P = take(e * diag * B);
+    xt = take(16 * words * B);
+    xo = take(16 * words * B);
     x = (c64*)take(sizeof(c64) * N * B);
     r = (c64*)take(sizeof(c64) * N * B);
     b = (c64*)take(sizeof(c64) * N * B);
@@ -875,24 +1045,50 @@ template <typename T, int NB>
 static int nd_sweep(const NdPhase<T>& p, hipStream_t st, Profiler* pr)
 {
     const long nt = p.ld / 64, ntri = nt * (nt + 1) / 2;
-    for (int kb = 0; kb * NB < p.dim; kb++) {
+    for (int c0 = 0; c0 < p.dim; c0 += NB) {
+        const int nq = (int)std::min<long>(NB / 64, nt - c0 / 64);
         {
             Timed tm(pr, FAM_PANEL, st);
-            hipLaunchKernelGGL((k_nd_diag<T, NB>), dim3(p.items), dim3(1024), 0, st, p, kb);
-            hipLaunchKernelGGL((k_nd_panel<T, NB>), dim3(xcd_grid(p.items * nt * (NB / 64))),
-                               dim3(256), 0, st, p, kb);
+            for (int t = 0; t < nq; t++) {
+                hipLaunchKernelGGL((k_nd_diag<T, NB>), dim3(p.items), dim3(256), 0, st, p, c0, t);
+                if (nt > 1)
+                    hipLaunchKernelGGL((k_nd_panel<T, NB>), dim3(xcd_grid(p.items * nt)), dim3(256),
+                                       0, st, p, c0, t);
+            }
             tm.end();
         }
         Timed tm(pr, FAM_GEMM, st);
+        const double d = p.dim, w = std::min(NB, p.dim - c0);
+        if constexpr (sizeof(T) == 4 && NB > 64) {
+            if (p.xt && nt > NB / 64) {
+                hipLaunchKernelGGL((k_nd_update<T, NB>), dim3(xcd_grid(p.items * nq * nt)),
+                                   dim3(256), 0, st, p, c0, 1);
+                const long nm = (p.ld + 127) / 128;
+                hipLaunchKernelGGL((k_nd_update_x6<NB>), dim3(xcd_grid(p.items * nm * (nm + 1))),
+                                   dim3(256), 0, st, p, c0);
+                tm.end(4.0 * d * d * w * p.items, true);
+                continue;
+            }
+        }
         hipLaunchKernelGGL((k_nd_update<T, NB>), dim3(xcd_grid(p.items * ntri)), dim3(256), 0, st,
-                           p, kb);
-        const double d = p.dim, w = std::min(NB, p.dim - kb * NB);
+                           p, c0, 0);
         tm.end(4.0 * d * d * w * p.items, true);
     }
     hipLaunchKernelGGL(k_nd_mirror<T>, dim3(xcd_grid(p.items * ntri)), dim3(256), 0, st, p.A, p.sA,
                        p.ld, p.items);
     TAGS_HIP(hipGetLastError());
     return 0;
+}
+
+template <typename T>
+static int nd_invert(NdPhase<T> p, int nb, bool x6, hipStream_t st, Profiler* pr)
+{
+    p.sx = nd_x6_words(p.ld, nb);
+    if (!x6) p.xt = p.xo = nullptr;
+    if constexpr (sizeof(T) == 4) {
+        if (nb == 256) return nd_sweep<T, 256>(p, st, pr);
+    }
+    return nb == 128 ? nd_sweep<T, 128>(p, st, pr) : nd_sweep<T, 64>(p, st, pr);
 }
 
 template <typename T>
@@ -907,10 +1103,10 @@ int NodalSolver::factor()
         tm.end();
     }
     int rc;
-    const int bz = nd_block(m), bs = nd_block(n);
-    const NdPhase<T> pz{(cx<T>*)F,  mp * mp,      (int)mp,  (int)m,  2 * nb,
-                        (cx<T>*)tp, (cx<T>*)op_, mp * bz, (cx<T>*)P};
-    if ((rc = bz == 128 ? nd_sweep<T, 128>(pz, st, pr) : nd_sweep<T, 64>(pz, st, pr))) return rc;
+    const int bz = nd_block(m, f64), bs = nd_block(n, f64);
+    const NdPhase<T> pz{(cx<T>*)F,   mp * mp, (int)mp,   (int)m,     2 * nb,     (cx<T>*)tp,
+                        (cx<T>*)op_, mp * bz, (cx<T>*)P, (u32x4*)xt, (u32x4*)xo, 0};
+    if ((rc = nd_invert<T>(pz, bz, nd_x6(m, f64), st, pr))) return rc;
     {
         Timed tm(pr, FAM_OTHER, st);
         hipLaunchKernelGGL(k_nd_rows<T>, dim3((unsigned)(nb * ((m + 3) / 4))), dim3(256), 0, st, g);
@@ -920,9 +1116,9 @@ int NodalSolver::factor()
                            dim3(256), 0, st, g);
         tm.end();
     }
-    const NdPhase<T> ps{(cx<T>*)S,  np * np,      (int)np,  (int)n,  nb,
-                        (cx<T>*)tp, (cx<T>*)op_, np * bs, (cx<T>*)P};
-    if ((rc = bs == 128 ? nd_sweep<T, 128>(ps, st, pr) : nd_sweep<T, 64>(ps, st, pr))) return rc;
+    const NdPhase<T> ps{(cx<T>*)S,   np * np, (int)np,   (int)n,     nb,         (cx<T>*)tp,
+                        (cx<T>*)op_, np * bs, (cx<T>*)P, (u32x4*)xt, (u32x4*)xo, 0};
+    if ((rc = nd_invert<T>(ps, bs, nd_x6(n, f64), st, pr))) return rc;
     hipLaunchKernelGGL((k_nd_gemv<T, 1>), dim3(xcd_grid(nb * (np / 16))), dim3(256), 0, st, g,
                        (const cx<T>*)g.c, g.h);
     hipLaunchKernelGGL(k_nd_den<T>, dim3(nb), dim3(256), 0, st, g);
@@ -934,7 +1130,7 @@ template <typename T>
 int NodalSolver::queue_step(int k, bool masked)
 {
     const NdArgs<T> g = nd_args<T>(*this, masked);
-    const int first = k == 1;
+    const int first = k == 1 && unit_;
     const unsigned gm = (unsigned)((2 * m + 255) / 256), gn = (unsigned)((n + 255) / 256);
     const unsigned gz = xcd_grid(2L * nb * (mp / 16));
     {
@@ -954,7 +1150,7 @@ int NodalSolver::queue_step(int k, bool masked)
     }
     Timed tm(pr, FAM_RESID, st);
     // |W| comes with the first residual
-    const int rc = hem_apply(Z, m, op, x, N, b, r, N, norms + 4 * k, kNormStride, first ? 2 : 1,
+    const int rc = hem_apply(Z, m, op, x, N, b, r, N, norms + 4 * k, kNormStride, k == 1 ? 2 : 1,
                              nb, sZ, masked ? active : nullptr, st);
     tm.end();
     return rc;
@@ -970,22 +1166,47 @@ int NodalSolver::issue(int nb_, long inj_)
     if (f64) hipLaunchKernelGGL(k_nd_init<double>, gi, dim3(256), 0, st, nd_args<double>(*this, false), b);
     else hipLaunchKernelGGL(k_nd_init<float>, gi, dim3(256), 0, st, nd_args<float>(*this, false), b);
     TAGS_HIP(hipGetLastError());
+    unit_ = true;
+    return queue_spec();
+}
+
+int NodalSolver::issue_rhs()
+{
+    if (!f64 || cap < 1) return TAGS_ERR_ARG;
+    nb = 1;
+    inj = 0;
+    const long w = std::max(std::max(N, 2 * mp), std::max(np, kNormStride));
+    hipLaunchKernelGGL(k_nd_init<double>, dim3((unsigned)((w + 255) / 256)), dim3(256), 0, st,
+                       nd_args<double>(*this, false), (c64*)nullptr);
+    TAGS_HIP(hipGetLastError());
+    TAGS_HIP(hipMemcpyAsync(r, b, sizeof(c64) * N, hipMemcpyDeviceToDevice, st));
+    int rc = fill_c64(x, N, c64{0.0, 0.0}, st);
+    if (rc) return rc;
+    unit_ = false;
+    return queue_spec();
+}
+
+// the factors, the first steps and their results
+int NodalSolver::queue_spec()
+{
     int rc = f64 ? factor<double>() : factor<float>();
     if (rc) return rc;
     step_ = f64 ? kSpec64 : kSpec32;
     for (int k = 1; k <= step_; k++)
         if ((rc = f64 ? queue_step<double>(k, false) : queue_step<float>(k, false))) return rc;
-    if (f64)
-        hipLaunchKernelGGL(k_nd_pick<double>, dim3((nb + 255) / 256), dim3(256), 0, st,
-                           nd_args<double>(*this, false), u);
-    else
-        hipLaunchKernelGGL(k_nd_pick<float>, dim3((nb + 255) / 256), dim3(256), 0, st,
-                           nd_args<float>(*this, false), u);
+    first_ = true;
+    return queue_results();
+}
+
+int NodalSolver::queue_results()
+{
+    const dim3 g((nb + 255) / 256);
+    if (f64) hipLaunchKernelGGL(k_nd_pick<double>, g, dim3(256), 0, st, nd_args<double>(*this, false), u);
+    else hipLaunchKernelGGL(k_nd_pick<float>, g, dim3(256), 0, st, nd_args<float>(*this, false), u);
     TAGS_HIP(hipGetLastError());
     TAGS_HIP(hipMemcpyAsync(hnorms, norms, sizeof(unsigned long long) * kNormStride * nb,
                             hipMemcpyDeviceToHost, st));
     TAGS_HIP(hipMemcpyAsync(hu, u, sizeof(c64) * nb, hipMemcpyDeviceToHost, st));
-    first_ = true;
     return 0;
 }
 
@@ -1058,17 +1279,203 @@ int NodalSolver::advance(bool* complete)
     for (int q = 0; q < nb; q++) hactive[q] = go[q];
     TAGS_HIP(hipMemcpyAsync(active, hactive, sizeof(int) * nb, hipMemcpyHostToDevice, st));
     int rc = f64 ? queue_step<double>(k + 1, true) : queue_step<float>(k + 1, true);
-    if (rc) return rc;
-    if (f64)
-        hipLaunchKernelGGL(k_nd_pick<double>, dim3((nb + 255) / 256), dim3(256), 0, st,
-                           nd_args<double>(*this, false), u);
-    else
-        hipLaunchKernelGGL(k_nd_pick<float>, dim3((nb + 255) / 256), dim3(256), 0, st,
-                           nd_args<float>(*this, false), u);
+    return rc ? rc : queue_results();
+}
+
+// ---------------------------------------------------------------------------
+// Dense symmetric inverses and the structure of a host immittance matrix
+// ---------------------------------------------------------------------------
+// A = -src (upper triangle, row-major) on 64 x 64 tiles on and below the
+// diagonal, transposed through LDS, zero beyond dim
+__global__ __launch_bounds__(256) void k_sym_load(const c64* src, long lds, long ssrc, c64* A,
+                                                   int ld, int dim, int items)
+{
+    const int nt = ld / 64, ntri = nt * (nt + 1) / 2;
+    const long flat = xcd_flat((long)items * ntri);
+    if (flat < 0) return;
+    const long item = flat / ntri;
+    int ti, tj;
+    tri_tile((int)(flat % ntri), ti, tj);
+    src += item * ssrc;
+    A += item * (long)ld * ld;
+    __shared__ c64 t[32][65];
+    for (int half = 0; half < 2; half++) {
+        for (int e = threadIdx.x; e < 2048; e += 256) {
+            const int c = e >> 6, r = e & 63;
+            const int i = ti * 64 + r, j = tj * 64 + 32 * half + c;
+            c64 v{0, 0};
+            if (i < dim && j < dim) v = src[(long)min(i, j) * lds + max(i, j)];
+            t[c][r] = c64{-v.x, -v.y};
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < 2048; e += 256) {
+            const int r = e >> 5, c = e & 31;
+            A[(long)(ti * 64 + r) * ld + tj * 64 + 32 * half + c] = t[c][r];
+        }
+        __syncthreads();
+    }
+}
+
+size_t sym_inverse_bytes(long dim, int items)
+{
+    const size_t ld = (size_t)up(dim, 64), nb = (size_t)nd_block(dim, true);
+    return sizeof(c64) * (size_t)items * (2 * ld * nb + 64 * nb) + 1024;
+}
+
+int sym_inverse(const c64* src, long lds, long ssrc, c64* X, long dim, int items, char* work,
+                hipStream_t st)
+{
+    if (dim < 1 || dim >= 65536 || items < 1) return TAGS_ERR_ARG;
+    const long ld = up(dim, 64), nt = ld / 64;
+    const int nb = nd_block(dim, true);
+    hipLaunchKernelGGL(k_sym_load, dim3(xcd_grid(items * (nt * (nt + 1) / 2))), dim3(256), 0, st,
+                       src, lds, ssrc, X, (int)ld, (int)dim, items);
     TAGS_HIP(hipGetLastError());
-    TAGS_HIP(hipMemcpyAsync(hnorms, norms, sizeof(unsigned long long) * kNormStride * nb,
-                            hipMemcpyDeviceToHost, st));
-    TAGS_HIP(hipMemcpyAsync(hu, u, sizeof(c64) * nb, hipMemcpyDeviceToHost, st));
+    c64* tp = (c64*)work;
+    c64* op = tp + (size_t)items * ld * nb;
+    c64* P = op + (size_t)items * ld * nb;
+    const NdPhase<double> p{X, ld * ld, (int)ld, (int)dim, items, tp, op, ld * nb, P, nullptr, nullptr, 0};
+    return nd_invert<double>(p, nb, false, st, nullptr);
+}
+
+__global__ __launch_bounds__(256) void k_sym_apply(const c64* X, long ld, long n, const c64* r,
+                                                    c64* x, unsigned long long* dmax)
+{
+    const long i = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (i >= n) return;
+    const int lane = threadIdx.x & 63;
+    c64 s{0, 0};
+    for (long c = lane; c < n; c += 64) s = cadd(s, cmul(X[i * ld + c], r[c]));
+    s = wave_sum(s);
+    if (lane) return;
+    x[i] = cadd(x[i], s);
+    atomicMax(dmax, (unsigned long long)__double_as_longlong(sqrt(s.x * s.x + s.y * s.y)));
+}
+int sym_apply(const c64* X, long ld, long n, const c64* r, c64* x, unsigned long long* dmax,
+              hipStream_t st)
+{
+    hipLaunchKernelGGL(k_sym_apply, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, X, ld, n, r, x,
+                       dmax);
+    TAGS_HIP(hipGetLastError());
+    return 0;
+}
+
+__global__ __launch_bounds__(256) void k_sub_identity(c64* R, long m, long total,
+                                                       unsigned long long* dmax)
+{
+    unsigned long long a = 0;
+    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < total; e += (long)gridDim.x * 256) {
+        const long q = e % (m * m);
+        c64 v = R[e];
+        if (q % (m + 1) == 0) {
+            v.x -= 1.0;
+            R[e] = v;
+        }
+        // as bit patterns: a NaN counts as larger than any number
+        const unsigned long long b =
+            (unsigned long long)__double_as_longlong(fabs(v.x) + fabs(v.y));
+        a = b > a ? b : a;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long b = __shfl_xor(a, o);
+        a = b > a ? b : a;
+    }
+    if ((threadIdx.x & 63) == 0) atomicMax(dmax, a);
+}
+int sub_identity(c64* R, long m, int items, unsigned long long* dmax, hipStream_t st)
+{
+    const long total = m * m * items;
+    hipLaunchKernelGGL(k_sub_identity, dim3((unsigned)std::min((total + 255) / 256, 1024L)),
+                       dim3(256), 0, st, R, m, total, dmax);
+    TAGS_HIP(hipGetLastError());
+    return 0;
+}
+
+__global__ __launch_bounds__(256) void k_sym_pack(const c64* X, long ld, long m, c64* out)
+{
+    X += blockIdx.z * ld * ld;
+    out += blockIdx.z * (m * (m + 1) / 2);
+    for (long i = blockIdx.y; i < m; i += gridDim.y) {
+        const long o = i * m - i * (i - 1) / 2 - i;
+        for (long k = i + (long)blockIdx.x * 256 + threadIdx.x; k < m; k += (long)gridDim.x * 256)
+            out[o + k] = X[i * ld + k];
+    }
+}
+int sym_pack(const c64* X, long ld, long m, int items, c64* out, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_sym_pack, dim3((unsigned)std::min((m + 255) / 256, 16L),
+                                        (unsigned)std::min(m, 16384L), (unsigned)items),
+                       dim3(256), 0, st, X, ld, m, out);
+    TAGS_HIP(hipGetLastError());
+    return 0;
+}
+
+// row (column of the caller's array) c of W, entries r >= c
+__global__ __launch_bounds__(256) void k_imm_structure(const c64* W, long N, long m, long n,
+                                                        int* out)
+{
+    int *sn = out, *en = out + m, *cnt = out + 2 * m, *bad = out + 4 * m;
+    int wrong = 0;
+    for (long c = blockIdx.y; c < n + m; c += gridDim.y)
+        for (long r = c + (long)blockIdx.x * 256 + threadIdx.x; r < N; r += (long)gridDim.x * 256) {
+            if (c >= n && r < n + m) continue;  // Z_L
+            const c64 v = W[c * N + r];
+            if (r < n || c >= n || r >= n + m) {
+                if (c < n && r >= n + m) {
+                    // B: 1/2 exactly where A is not zero
+                    const c64 a = W[c * N + r - m];
+                    wrong += v.y != 0.0 || v.x != (a.x != 0.0 ? 0.5 : 0.0);
+                } else {
+                    wrong += v.x != 0.0 || v.y != 0.0;
+                }
+            } else if (v.x != 0.0 || v.y != 0.0) {
+                // A: +1 at the start node, -1 at the end node
+                const long s = r - n;
+                if (v.y == 0.0 && v.x == 1.0) {
+                    sn[s] = (int)c;
+                    atomicAdd(&cnt[s], 1);
+                } else if (v.y == 0.0 && v.x == -1.0) {
+                    en[s] = (int)c;
+                    atomicAdd(&cnt[m + s], 1);
+                } else {
+                    wrong++;
+                }
+            }
+        }
+    // (NaN entries compare unequal to everything and count as wrong)
+    if (wrong) atomicAdd(bad, wrong);
+}
+__global__ void k_int_zero(int* p, long n)
+{
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = 0;
+}
+int imm_structure(const c64* W, long N, long m, long n, int* out, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_int_zero, dim3((unsigned)((4 * m + 256) / 256)), dim3(256), 0, st, out,
+                       4 * m + 1);
+    hipLaunchKernelGGL(k_imm_structure, dim3((unsigned)std::min((N + 255) / 256, 16L),
+                                             (unsigned)std::min(n + m, 8192L)),
+                       dim3(256), 0, st, W, N, m, n, out);
+    TAGS_HIP(hipGetLastError());
+    return 0;
+}
+
+__global__ __launch_bounds__(256) void k_imm_blocks(const c64* W, long N, long m, long n, c64* Z)
+{
+    const long blk = blockIdx.z;
+    const c64* src = W + (n + blk * m) * N + n + blk * m;
+    c64* dst = Z + blk * (m * m + m);
+    for (long i = blockIdx.y; i < m; i += gridDim.y)
+        for (long k = (long)blockIdx.x * 256 + threadIdx.x; k < m; k += (long)gridDim.x * 256)
+            dst[i * m + k] = src[min(i, k) * N + max(i, k)];
+}
+int imm_blocks(const c64* W, long N, long m, long n, c64* Z, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_imm_blocks, dim3((unsigned)std::min((m + 255) / 256, 16L),
+                                          (unsigned)std::min(m, 16384L), 2),
+                       dim3(256), 0, st, W, N, m, n, Z);
+    TAGS_HIP(hipGetLastError());
     return 0;
 }
 
