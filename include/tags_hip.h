@@ -691,6 +691,10 @@ const char *tags_version(void);
 /* Waits for all work on the current device (hipDeviceSynchronize). */
 int tags_device_synchronize(void);
 
+/* Frees the idle pinned staging buffers (at most 4 of 8 MiB) that the host-pointer
+ * calls keep between calls. Safe at any time, from any thread. */
+void tags_release_staging(void);
+
 /* GEMM tuning. The trailing update C -= A B of the LU has several MFMA tile
  * variants per precision (precision: tags_precision). Complex64 variants
  * 0-21 and 33 run on the fp32 MFMA cores; 22-32 run on the bf16 MFMA cores,

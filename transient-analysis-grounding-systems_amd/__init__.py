@@ -27,8 +27,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB_PATH = os.path.join(HERE, "libtags_hip.so")
 CSRC = os.path.join(HERE, "csrc")
-SOURCES = ["fill.hip", "gemm.hip", "lu.hip", "tslu.hip", "gmres.hip", "nodal.hip", "api.hip",
-           "nlt.hip", "io.hip", "field.hip"]
+SOURCES = ["fill.hip", "gemm.hip", "lu.hip", "tslu.hip", "gmres.hip", "nodal.hip",
+           "hostcopy.hip", "api.hip", "nlt.hip", "io.hip", "field.hip"]
 
 ELECTRODE_DTYPE = np.dtype(
     [("start_point", "<f8", 3), ("end_point", "<f8", 3), ("middle_point", "<f8", 3),
@@ -174,7 +174,7 @@ EXPORTED = ["populate_electrode", "segment_electrode", "number_segments", "numbe
             "tags_cases_set_profiling", "tags_cases_get_timers", "tags_cases_destroy",
             "tags_sweep_autotune", "tags_sweep_set_tuning", "tags_sweep_get_tuning",
             "tags_cases_autotune",
-            "tags_sweep_set_gmres"]
+            "tags_sweep_set_gmres", "tags_release_staging"]
 
 _lib = None
 
@@ -234,6 +234,7 @@ def lib():
         "tags_dense_solve": ([P, P, S, I, P], I),
         "tags_version": ([], ctypes.c_char_p),
         "tags_device_synchronize": ([], I),
+        "tags_release_staging": ([], None),
         "tags_gemm_bench": ([I, I, I, I, I, I, ctypes.POINTER(D)], I),
         "tags_gemm_variants": ([I], I),
         "tags_gemm_select": ([I, I, I], I),
@@ -621,6 +622,8 @@ def _close_live():
             obj.close()
         except Exception:
             pass
+    if _lib is not None:
+        _lib.tags_release_staging()
 
 
 class Sweep:
