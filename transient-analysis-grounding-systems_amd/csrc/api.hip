@@ -13,6 +13,7 @@
 #include <string>
 #include <vector>
 
+#include "hostcopy.h"
 #include "lu.h"
 #include "nodal.h"
 
@@ -64,9 +65,7 @@ struct DevSegs {
             h[7 * m + i] = e[i].radius;
         }
         TAGS_HIP(hipMalloc(&buf, sizeof(double) * 8 * (size_t)(m > 0 ? m : 1)));
-        TAGS_HIP(hipMemcpyAsync(buf, h.data(), sizeof(double) * 8 * m, hipMemcpyHostToDevice, st));
-        TAGS_HIP(hipStreamSynchronize(st));
-        return 0;
+        return copy_in(buf, h.data(), sizeof(double) * 8 * m, st);
     }
     SegSoA soa() const
     {
@@ -1058,26 +1057,40 @@ static int pairs_dropin(TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const Electrode* e,
     Stream S;
     DevSegs de, di;
     int rc;
-    if ((rc = de.upload(e, (long)m, S.s))) return rc;
-    if ((rc = di.upload(img ? img : e, (long)m, S.s))) return rc;
-    const bool alias = (void*)zl == (void*)zt;
-    const size_t bytes = sizeof(c64) * m * m;
+    const long M = (long)m;
+    if ((rc = de.upload(e, M, S.s))) return rc;
+    if (images && (rc = di.upload(img, M, S.s))) return rc;
+    const size_t np = m * (m + 1) / 2;
     DevBuf<c64> dl, dt;
-    if ((rc = dl.alloc(m * m))) return rc;
-    TAGS_HIP(hipMemcpyAsync(dl.p, zl, bytes, hipMemcpyHostToDevice, S.s));
-    c64* dtp = dl.p;
-    if (!alias) {
-        if ((rc = dt.alloc(m * m))) return rc;
-        TAGS_HIP(hipMemcpyAsync(dt.p, zt, bytes, hipMemcpyHostToDevice, S.s));
-        dtp = dt.p;
-    }
-    if ((rc = launch_pairs_dropin((double*)dl.p, (double*)dtp, alias, de.soa(), di.soa(),
-                                  (long)m, sc, images, S.s)))
+    if ((rc = dl.alloc(np)) || (rc = dt.alloc(np))) return rc;
+    if ((rc = launch_pairs_packed(dl.p, dt.p, de.soa(), images ? di.soa() : de.soa(), M, sc,
+                                  images, S.s)))
         return rc;
-    TAGS_HIP(hipMemcpyAsync(zl, dl.p, bytes, hipMemcpyDeviceToHost, S.s));
-    if (!alias) TAGS_HIP(hipMemcpyAsync(zt, dtp, bytes, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipStreamSynchronize(S.s));
-    return 0;
+    // only the entries (i, k >= i) are written (images: added to), the device
+    // never sees the caller's arrays. With zl == zt the last writer of the
+    // reference wins (Z_T on the diagonal, Z_L off it); both image parts add up.
+    c64 *L = (c64*)zl, *T = (c64*)zt;
+    const bool alias = (void*)zl == (void*)zt;
+    auto put = [M](c64* dst, long i, long k, const c64* v, long n) {
+        std::memcpy(dst + i * M + k, v, sizeof(c64) * (size_t)n);
+    };
+    auto add = [M](c64* dst, long i, long k, const c64* v, long n) {
+        c64* d = dst + i * M + k;
+        for (long q = 0; q < n; q++) d[q] = cadd(d[q], v[q]);
+    };
+    if (images) {
+        rc = copy_out_rows(dt.p, M, S.s, [&](long i, long k, const c64* v, long n) { add(T, i, k, v, n); });
+        if (!rc)
+            rc = copy_out_rows(dl.p, M, S.s, [&](long i, long k, const c64* v, long n) { add(L, i, k, v, n); });
+        return rc;
+    }
+    rc = copy_out_rows(dt.p, M, S.s, [&](long i, long k, const c64* v, long n) { put(T, i, k, v, n); });
+    if (!rc)
+        rc = copy_out_rows(dl.p, M, S.s, [&](long i, long k, const c64* v, long n) {
+            if (alias && k == i) put(L, i, k + 1, v + 1, n - 1);
+            else put(L, i, k, v, n);
+        });
+    return rc;
 }
 
 int calculate_impedances(TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const Electrode* electrodes,
@@ -1123,46 +1136,6 @@ int impedances_images(TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const Electrode* elect
 // ---------------------------------------------------------------------------
 }  // extern "C"
 
-namespace tags {
-// blk1: rows n..N of columns 0..nw (column-major, ld 2m): A (rows s) then B
-// (rows m+s); blk2: rows 0..nw of columns n..N (column-major, ld nw).
-// counts[0] = #start matches, counts[1] = #end matches (over nodes < nw).
-__global__ __launch_bounds__(256) void k_incidence_blocks(const double* __restrict__ sp, long m,
-                                                          const double* __restrict__ nodes,
-                                                          long nw, c64* blk1, c64* blk2,
-                                                          unsigned long long* counts)
-{
-    const double tol = 1e-5;
-    unsigned long long cs = 0, ce = 0;
-    for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < nw * m;
-         idx += (long)gridDim.x * 256) {
-        const long nd = idx / m, s = idx % m;
-        const double x = nodes[3 * nd], y = nodes[3 * nd + 1], z = nodes[3 * nd + 2];
-        const bool st = fabs(sp[6 * s] - x) <= tol && fabs(sp[6 * s + 1] - y) <= tol &&
-                        fabs(sp[6 * s + 2] - z) <= tol;
-        const bool ed = !st && fabs(sp[6 * s + 3] - x) <= tol && fabs(sp[6 * s + 4] - y) <= tol &&
-                        fabs(sp[6 * s + 5] - z) <= tol;
-        const double a = st ? 1.0 : (ed ? -1.0 : 0.0);
-        const double b = (st || ed) ? 0.5 : 0.0;
-        blk1[s + 2 * m * nd] = c64{a, 0.0};
-        blk1[m + s + 2 * m * nd] = c64{b, 0.0};
-        blk2[nd + nw * s] = c64{a, 0.0};
-        blk2[nd + nw * (m + s)] = c64{b, 0.0};
-        cs += st;
-        ce += ed;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        cs += __shfl_xor(cs, off);
-        ce += __shfl_xor(ce, off);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&counts[0], cs);
-        atomicAdd(&counts[1], ce);
-    }
-}
-}  // namespace tags
-
-extern "C" {
 
 static std::vector<double> seg_points(const Electrode* e, size_t m)
 {
@@ -1175,33 +1148,44 @@ static std::vector<double> seg_points(const Electrode* e, size_t m)
     return sp;
 }
 
-// Node/segment incidence on the GPU, in the reference's node order: nodes up to
-// and including the first one no segment touches (nw of them; bad = its index
-// or -1), as blk1 (2m x nw column-major: A in rows s, B in rows m + s) and blk2
-// (nw x 2m column-major: the transposes); counts = start and end matches.
+// Node/segment incidence from the GPU, in the reference's node order: nodes up
+// to and including the first one no segment touches (nw of them; bad = its
+// index or -1), each segment's start and end node (-1: none), the count of start
+// and end matches among the nw nodes, and, where a segment end matches several
+// nodes (nodes within 1e-5 of each other), the further matches (segment, node,
+// end).
 struct Incidence {
-    DevBuf<c64> b1, b2;
+    std::vector<int> sn, en;
+    struct More {
+        long s, nd;
+        bool end;
+    };
+    std::vector<More> more;
     long nw = 0, bad = -1;
     unsigned long long c[2] = {0, 0};
 };
 
-static int incidence_blocks(Incidence& inc, const Electrode* electrodes, long m,
-                            const double* nodes, long n, hipStream_t st)
+static int incidence(Incidence& inc, const Electrode* electrodes, long m, const double* nodes,
+                     long n, hipStream_t st)
 {
     int rc;
     std::vector<double> sp = seg_points(electrodes, m);
     DevBuf<double> dsp, dnodes;
-    DevBuf<int> dsn, den, dhits;
-    if ((rc = dsp.alloc(6 * m)) || (rc = dnodes.alloc(3 * n)) || (rc = dsn.alloc(m)) ||
-        (rc = den.alloc(m)) || (rc = dhits.alloc(n + 2 * m)))
+    DevBuf<int> dse, dhits;
+    const size_t nh = (size_t)n + 2 * m;
+    if ((rc = dsp.alloc(6 * m)) || (rc = dnodes.alloc(3 * n)) || (rc = dse.alloc(2 * m)) ||
+        (rc = dhits.alloc(nh)))
         return rc;
-    TAGS_HIP(hipMemcpyAsync(dsp.p, sp.data(), sizeof(double) * 6 * m, hipMemcpyHostToDevice, st));
-    TAGS_HIP(hipMemcpyAsync(dnodes.p, nodes, sizeof(double) * 3 * n, hipMemcpyHostToDevice, st));
-    TAGS_HIP(hipMemsetAsync(dhits.p, 0, sizeof(int) * (n + 2 * m), st));
-    if ((rc = launch_incidence(dsp.p, m, dnodes.p, n, dsn.p, den.p, dhits.p, st))) return rc;
-    std::vector<int> hits(n + 2 * m);
-    TAGS_HIP(hipMemcpyAsync(hits.data(), dhits.p, sizeof(int) * n, hipMemcpyDeviceToHost, st));
-    TAGS_HIP(hipStreamSynchronize(st));
+    if ((rc = copy_in(dsp.p, sp.data(), sizeof(double) * 6 * m, st)) ||
+        (rc = copy_in(dnodes.p, nodes, sizeof(double) * 3 * n, st)))
+        return rc;
+    TAGS_HIP(hipMemsetAsync(dhits.p, 0, sizeof(int) * nh, st));
+    TAGS_HIP(hipMemsetAsync(dse.p, 0xff, sizeof(int) * 2 * m, st));
+    if ((rc = launch_incidence(dsp.p, m, dnodes.p, n, dse.p, dse.p + m, dhits.p, st))) return rc;
+    std::vector<int> hits(nh), se(2 * (size_t)m);
+    if ((rc = copy_out(hits.data(), dhits.p, sizeof(int) * nh, st)) ||
+        (rc = copy_out(se.data(), dse.p, sizeof(int) * 2 * m, st)))
+        return rc;
     // the reference stops after the first node without a segment (src/linalg.c:72-75)
     inc.nw = n;
     inc.bad = -1;
@@ -1211,21 +1195,65 @@ static int incidence_blocks(Incidence& inc, const Electrode* electrodes, long m,
             inc.nw = i + 1;
             break;
         }
-    DevBuf<unsigned long long> cnt;
-    if ((rc = inc.b1.alloc((size_t)2 * m * inc.nw)) || (rc = inc.b2.alloc((size_t)2 * m * inc.nw)) ||
-        (rc = cnt.alloc(2)))
-        return rc;
-    TAGS_HIP(hipMemsetAsync(cnt.p, 0, sizeof(unsigned long long) * 2, st));
-    {
-        long tot = inc.nw * m;
-        unsigned g = (unsigned)std::min<long>((tot + 255) / 256, 4096);
-        hipLaunchKernelGGL(k_incidence_blocks, dim3(g), dim3(256), 0, st, dsp.p, m, dnodes.p,
-                           inc.nw, inc.b1.p, inc.b2.p, cnt.p);
-        TAGS_HIP(hipGetLastError());
+    inc.sn.assign(se.begin(), se.begin() + m);
+    inc.en.assign(se.begin() + m, se.end());
+    auto near = [&](const double* p, long nd) {
+        return std::fabs(p[0] - nodes[3 * nd]) <= 1e-5 &&
+               std::fabs(p[1] - nodes[3 * nd + 1]) <= 1e-5 &&
+               std::fabs(p[2] - nodes[3 * nd + 2]) <= 1e-5;
+    };
+    for (long s = 0; s < m; s++) {
+        if (hits[n + 2 * s] > 1 || hits[n + 2 * s + 1] > 1) {
+            // several nodes: every match, start before end as the kernel decides
+            inc.sn[s] = inc.en[s] = -1;
+            for (long nd = 0; nd < inc.nw; nd++) {
+                if (near(&sp[6 * s], nd)) inc.more.push_back({s, nd, false});
+                else if (near(&sp[6 * s + 3], nd)) inc.more.push_back({s, nd, true});
+            }
+        }
+        if (inc.sn[s] >= inc.nw) inc.sn[s] = -1;
+        if (inc.en[s] >= inc.nw) inc.en[s] = -1;
+        inc.c[0] += inc.sn[s] >= 0;
+        inc.c[1] += inc.en[s] >= 0;
     }
-    TAGS_HIP(hipMemcpyAsync(inc.c, cnt.p, sizeof(inc.c), hipMemcpyDeviceToHost, st));
-    TAGS_HIP(hipStreamSynchronize(st));
+    for (const Incidence::More& q : inc.more) inc.c[q.end ? 1 : 0]++;
     return 0;
+}
+
+// Each node's segment ends in segment order (2 s: start of segment s, 2 s + 1:
+// its end; a segment whose two ends share a node has its start entry only, as W
+// has one entry there, and clears *distinct). false: a node out of range.
+static bool node_lists(const std::vector<int>& sn, const std::vector<int>& en, long n,
+                       std::vector<int>& ptr, std::vector<int>& seg, bool* distinct)
+{
+    const long m = (long)sn.size();
+    *distinct = true;
+    ptr.assign(n + 1, 0);
+    for (long s = 0; s < m; s++) {
+        if (sn[s] < 0 || sn[s] >= n || en[s] < 0 || en[s] >= n) return false;
+        ptr[sn[s] + 1]++;
+        if (en[s] != sn[s]) ptr[en[s] + 1]++;
+        else *distinct = false;
+    }
+    for (long u = 0; u < n; u++) ptr[u + 1] += ptr[u];
+    seg.assign(ptr[n], 0);
+    std::vector<int> at(ptr.begin(), ptr.end() - 1);
+    for (long s = 0; s < m; s++) {
+        seg[at[sn[s]]++] = (int)(2 * s);
+        if (en[s] != sn[s]) seg[at[en[s]]++] = (int)(2 * s + 1);
+    }
+    return true;
+}
+
+// Calls put(segment, node, end) for every match.
+template <typename F>
+static void incidence_each(const Incidence& inc, F put)
+{
+    for (long s = 0; s < (long)inc.sn.size(); s++) {
+        if (inc.sn[s] >= 0) put(s, (long)inc.sn[s], false);
+        if (inc.en[s] >= 0) put(s, (long)inc.en[s], true);
+    }
+    for (const Incidence::More& q : inc.more) put(q.s, q.nd, q.end);
 }
 
 // the reference's return codes and messages (src/linalg.c:72-84, :186-198)
@@ -1246,6 +1274,8 @@ static int incidence_verdict(long bad, long suma, double sumb, long m)
     return 0;
 }
 
+extern "C" {
+
 int fill_incidence_imm(TAGS_COMPLEX* wg, const Electrode* electrodes, size_t num_electrodes,
                        const double* nodes, size_t num_nodes)
 {
@@ -1256,16 +1286,21 @@ int fill_incidence_imm(TAGS_COMPLEX* wg, const Electrode* electrodes, size_t num
     if (m == 0) return incidence_verdict(0, 0, 0.0, 0);
     Stream S;
     Incidence inc;
-    int rc = incidence_blocks(inc, electrodes, m, nodes, n, S.s);
+    int rc = incidence(inc, electrodes, m, nodes, n, S.s);
     if (rc) return rc;
+    // rows n..N of columns 0..nw and rows 0..nw of columns n..N, zero but for A
+    // (+1 at a start node, -1 at an end node), B (1/2) and their transposes:
+    // written here, where strided copies of dense blocks from the device ran at
+    // 1 GB/s
     const long nw = inc.nw;
-    // blk1 -> W rows n..N, columns 0..nw ; blk2 -> W rows 0..nw, columns n..N
     c64* W = (c64*)wg;
-    TAGS_HIP(hipMemcpy2DAsync(W + n, sizeof(c64) * N, inc.b1.p, sizeof(c64) * 2 * m,
-                              sizeof(c64) * 2 * m, nw, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipMemcpy2DAsync(W + N * n, sizeof(c64) * N, inc.b2.p, sizeof(c64) * nw,
-                              sizeof(c64) * nw, 2 * m, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipStreamSynchronize(S.s));
+    for (long c = 0; c < nw; c++) std::memset(W + c * N + n, 0, sizeof(c64) * 2 * m);
+    for (long c = n; c < N; c++) std::memset(W + c * N, 0, sizeof(c64) * nw);
+    incidence_each(inc, [&](long s, long u, bool end) {
+        const c64 va{end ? -1.0 : 1.0, 0.0}, vb{0.5, 0.0};
+        W[u * N + n + s] = W[(n + s) * N + u] = va;
+        W[u * N + n + m + s] = W[(n + m + s) * N + u] = vb;
+    });
     return incidence_verdict(inc.bad, (long)inc.c[0] - (long)inc.c[1],
                              0.5 * (double)(inc.c[0] + inc.c[1]), m);
 }
@@ -1282,14 +1317,14 @@ int fill_incidence_adm(TAGS_COMPLEX* a, TAGS_COMPLEX* b, const Electrode* electr
     if (m == 0) return incidence_verdict(0, 0, 0.0, 0);
     Stream S;
     Incidence inc;
-    int rc = incidence_blocks(inc, electrodes, m, nodes, n, S.s);
+    int rc = incidence(inc, electrodes, m, nodes, n, S.s);
     if (rc) return rc;
-    const long nw = inc.nw;
-    TAGS_HIP(hipMemcpy2DAsync(b, sizeof(c64) * m, inc.b1.p + m, sizeof(c64) * 2 * m,
-                              sizeof(c64) * m, nw, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipMemcpy2DAsync(a, sizeof(c64) * m, inc.b1.p, sizeof(c64) * 2 * m,
-                              sizeof(c64) * m, nw, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipStreamSynchronize(S.s));
+    c64 *A = (c64*)a, *B = (c64*)b;
+    const size_t cols = sizeof(c64) * (size_t)(m * inc.nw);
+    std::memset(B, 0, cols);
+    incidence_each(inc, [&](long s, long u, bool) { B[u * m + s] = c64{0.5, 0.0}; });
+    std::memset(A, 0, cols);
+    incidence_each(inc, [&](long s, long u, bool end) { A[u * m + s] = c64{end ? -1.0 : 1.0, 0.0}; });
     const long suma = (long)inc.c[0] - (long)inc.c[1];
     const double sumb = a == b ? (double)suma : 0.5 * (double)(inc.c[0] + inc.c[1]);
     return incidence_verdict(inc.bad, suma, sumb, m);
@@ -1297,49 +1332,22 @@ int fill_incidence_adm(TAGS_COMPLEX* a, TAGS_COMPLEX* b, const Electrode* electr
 
 }  // extern "C"
 
-namespace tags {
-// Z-region of W (rows/cols n..N), column-major with ld 2m:
-// [[-zl, 0], [0, -zt]] with zl[i + m k] at (i, k) (src/linalg.c:96-103).
-__global__ void k_zregion(const c64* zl, const c64* zt, long m, c64* blk)
-{
-    const long M2 = 2 * m;
-    for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < M2 * M2;
-         idx += (long)gridDim.x * 256) {
-        const long col = idx / M2, row = idx % M2;
-        c64 v = c64{0.0, 0.0};
-        if (row < m && col < m) {
-            const c64 z = zl[row + m * col];
-            v = c64{-z.x, -z.y};
-        } else if (row >= m && col >= m) {
-            const c64 z = zt[(row - m) + m * (col - m)];
-            v = c64{-z.x, -z.y};
-        }
-        blk[idx] = v;
-    }
-}
-}  // namespace tags
-
 extern "C" {
 
 int fill_impedance_imm(TAGS_COMPLEX* wg, const TAGS_COMPLEX* zl, const TAGS_COMPLEX* zt,
                        size_t num_electrodes, size_t num_nodes)
 {
     const long m = (long)num_electrodes, n = (long)num_nodes, N = n + 2 * m;
-    Stream S;
-    int rc;
+    // columns n..N: [[-zl, 0], [0, -zt]] below row n (src/linalg.c:96-103), a
+    // move of the caller's arrays to the caller's array
     c64* W = (c64*)wg;
-    if (m > 0) {
-        DevBuf<c64> dl, dt, blk;
-        if ((rc = dl.alloc(m * m)) || (rc = dt.alloc(m * m)) || (rc = blk.alloc(4 * m * m)))
-            return rc;
-        TAGS_HIP(hipMemcpyAsync(dl.p, zl, sizeof(c64) * m * m, hipMemcpyHostToDevice, S.s));
-        TAGS_HIP(hipMemcpyAsync(dt.p, zt, sizeof(c64) * m * m, hipMemcpyHostToDevice, S.s));
-        unsigned g = (unsigned)std::min<long>((4 * m * m + 255) / 256, 8192);
-        hipLaunchKernelGGL(k_zregion, dim3(g), dim3(256), 0, S.s, dl.p, dt.p, m, blk.p);
-        TAGS_HIP(hipGetLastError());
-        TAGS_HIP(hipMemcpy2DAsync(W + n + N * n, sizeof(c64) * N, blk.p, sizeof(c64) * 2 * m,
-                                  sizeof(c64) * 2 * m, 2 * m, hipMemcpyDeviceToHost, S.s));
-        TAGS_HIP(hipStreamSynchronize(S.s));
+    for (long c = 0; c < 2 * m; c++) {
+        const bool t = c >= m;
+        c64* col = W + (n + c) * N + n;
+        const c64* z = (const c64*)(t ? zt : zl) + (t ? c - m : c) * m;
+        c64* out = col + (t ? m : 0);
+        for (long r = 0; r < m; r++) out[r] = c64{-z[r].x, -z[r].y};
+        std::memset(col + (t ? 0 : m), 0, sizeof(c64) * (size_t)m);
     }
     for (long k = 0; k < n; k++) std::memset(W + N * k, 0, sizeof(c64) * n);
     return 0;
@@ -1348,37 +1356,154 @@ int fill_impedance_imm(TAGS_COMPLEX* wg, const TAGS_COMPLEX* zl, const TAGS_COMP
 // ---------------------------------------------------------------------------
 // solve_immittance (src/linalg.c:113-139)
 // ---------------------------------------------------------------------------
+// The immittance system of a host W (N x N, lower triangle column-major) by the
+// nodal solve: W is on the device in Wd; where it has the structure of the HEM
+// (fill_incidence_imm and fill_impedance_imm's) and the refinement is accepted,
+// x replaces bx and *done is set. (20 x 20 m grid, N = 1185: 8.7 ms by the
+// pivoted factor of W.)
+static int immittance_nodal(const c64* Wd, c64* bx, long m, long n, hipStream_t st, bool* done)
+{
+    *done = false;
+    const long N = n + 2 * m;
+    int rc;
+    DevBuf<int> d;
+    const size_t ni = 4 * (size_t)m + 1;  // sn, en, their counts, entries out of place
+    if ((rc = d.alloc(ni))) return rc;
+    if ((rc = imm_structure(Wd, N, m, n, d.p, st))) return rc;
+    std::vector<int> h(ni);
+    if ((rc = copy_out(h.data(), d.p, sizeof(int) * ni, st))) return rc;
+    if (h[4 * m] != 0) return 0;
+    for (long s = 0; s < 2 * m; s++)
+        if (h[2 * m + s] != 1) return 0;
+    const std::vector<int> sn(h.begin(), h.begin() + m), en(h.begin() + m, h.begin() + 2 * m);
+    std::vector<int> ptr, seg;
+    bool distinct;
+    if (!node_lists(sn, en, n, ptr, seg, &distinct) || !distinct) return 0;
+    DevBuf<int> dp, ds;
+    if ((rc = dp.alloc(n + 1)) || (rc = ds.alloc(seg.size()))) return rc;
+    if ((rc = copy_in(dp.p, ptr.data(), sizeof(int) * (n + 1), st)) ||
+        (rc = copy_in(ds.p, seg.data(), sizeof(int) * seg.size(), st)))
+        return rc;
+    HemOp op;
+    op.m = m;
+    op.n = n;
+    op.sn = d.p;
+    op.en = d.p + m;
+    op.node_ptr = dp.p;
+    op.node_seg = ds.p;
+    NodalSolver nd;
+    nd.st = st;
+    if ((rc = nd.ensure(op, true, 1))) return rc;
+    if ((rc = imm_blocks(Wd, N, m, n, nd.Z, st))) return rc;
+    // the nodal order is [I_L; I_T; U]
+    std::vector<c64> b(N);
+    std::copy(bx + n, bx + N, b.begin());
+    std::copy(bx, bx + n, b.begin() + 2 * m);
+    if ((rc = copy_in(nd.b, b.data(), sizeof(c64) * N, st))) return rc;
+    if ((rc = nd.issue_rhs())) return rc;
+    bool complete = false;
+    while (!complete) {
+        TAGS_HIP(hipStreamSynchronize(st));
+        if ((rc = nd.advance(&complete))) return rc;
+    }
+    if (!nd.accepted[0]) return 0;
+    if ((rc = copy_out(b.data(), nd.x, sizeof(c64) * N, st))) return rc;
+    std::copy(b.begin(), b.begin() + 2 * m, bx + n);
+    std::copy(b.begin() + 2 * m, b.end(), bx);
+    *done = true;
+    return 0;
+}
+
+// A dense symmetric system (Wd: n x n with both triangles, on the device; b in
+// bd, replaced by x) by its explicit inverse with refinement; *done unless the
+// refinement does not meet its acceptance rule (a zero pivot or growth without
+// row exchanges among them). (n = 559: 4.4 ms by the pivoted factor.)
+static int symmetric_solve(const c64* Wd, c64* bd, long n, hipStream_t st, bool* done)
+{
+    *done = false;
+    const long ld = (n + 63) / 64 * 64;
+    int rc;
+    DevBuf<c64> X, v;
+    DevBuf<char> work;
+    DevBuf<unsigned long long> norms;
+    constexpr int kSteps = 6;
+    if ((rc = X.alloc((size_t)ld * ld)) || (rc = v.alloc(2 * n)) ||
+        (rc = work.alloc(sym_inverse_bytes(n, 1))) || (rc = norms.alloc(4 * (kSteps + 1))))
+        return rc;
+    c64 *x = v.p, *r = v.p + n;
+    if ((rc = sym_inverse(Wd, n, 0, X.p, n, 1, work.p, st))) return rc;
+    if ((rc = fill_c64(x, n, c64{0.0, 0.0}, st)) ||
+        (rc = fill_c64((c64*)norms.p, 2 * (kSteps + 1), c64{0.0, 0.0}, st)))
+        return rc;
+    TAGS_HIP(hipMemcpyAsync(r, bd, sizeof(c64) * n, hipMemcpyDeviceToDevice, st));
+    double h[4 * (kSteps + 1)];
+    for (int k = 1; k <= kSteps; k++) {
+        if ((rc = sym_apply(X.p, ld, n, r, x, norms.p + 4 * k + 3, st)) ||
+            (rc = residual64(Wd, n, (int)n, x, bd, r, norms.p + 4 * k, k == 1, st, nullptr, false)))
+            return rc;
+        if (k < 2) continue;
+        if ((rc = copy_out(h, norms.p, sizeof(h), st))) return rc;
+        const double xn = h[4 * k + 1], be = h[4 * k] / (h[6] * xn);
+        const double dx = h[4 * k + 3] / xn, dp = h[4 * k - 1] / h[4 * k - 3];
+        if (!(xn > 0.0) || !(be == be) || !(dx == dx)) return 0;
+        const double rho = dp > 0.0 ? dx / dp : 1.0;
+        const double fe = dx == 0.0 ? 0.0 : rho < 0.5 ? dx * rho / (1.0 - rho) : dx;
+        if (be <= 1e-15 && fe <= 1e-14) {
+            *done = true;
+            TAGS_HIP(hipMemcpyAsync(bd, x, sizeof(c64) * n, hipMemcpyDeviceToDevice, st));
+            return 0;
+        }
+        if (rho > 0.8) return 0;
+    }
+    return 0;
+}
+
+// imm_m >= 0: an immittance system of imm_m segments
 static int dense_solve_host(const c64* a, c64* bx, long n, int precision, bool sym_lower_cm,
                             tags_item_stats* stt, const LUPlan* plan = nullptr,
-                            const LUPlan* plan32 = nullptr, Grounding ground = Grounding{})
+                            const LUPlan* plan32 = nullptr, Grounding ground = Grounding{},
+                            long imm_m = -1)
 {
     if (n <= 0) return 0;
     if (n >= 65536) return TAGS_ERR_TOO_LARGE;
     Stream S;
-    Solver sv;
-    sv.st = S.s;
     int rc;
     const bool mixed = precision == TAGS_PREC_MIXED;
-    if ((rc = sv.ensure((int)n, mixed))) return rc;
     DevBuf<c64> W, bv;
     if ((rc = W.alloc((size_t)n * n)) || (rc = bv.alloc(n))) return rc;
-    TAGS_HIP(hipMemcpyAsync(W.p, a, sizeof(c64) * n * n, hipMemcpyHostToDevice, S.s));
-    TAGS_HIP(hipMemcpyAsync(bv.p, bx, sizeof(c64) * n, hipMemcpyHostToDevice, S.s));
-    if (sym_lower_cm && (rc = sym_from_upper(W.p, n, (int)n, S.s))) return rc;
+    if ((rc = copy_in(W.p, a, sizeof(c64) * n * n, S.s))) return rc;
+    if (sym_lower_cm) {
+        bool done = false;
+        if (imm_m > 0 && n > 2 * imm_m) {
+            if ((rc = immittance_nodal(W.p, bx, imm_m, n - 2 * imm_m, S.s, &done))) return rc;
+            if (done) return 0;
+        }
+        if ((rc = copy_in(bv.p, bx, sizeof(c64) * n, S.s)) ||
+            (rc = sym_from_upper(W.p, n, (int)n, S.s)))
+            return rc;
+        if (imm_m < 0) {
+            if ((rc = symmetric_solve(W.p, bv.p, n, S.s, &done))) return rc;
+            if (done) return copy_out(bx, bv.p, sizeof(c64) * n, S.s);
+        }
+    } else if ((rc = copy_in(bv.p, bx, sizeof(c64) * n, S.s))) {
+        return rc;
+    }
+    Solver sv;
+    sv.st = S.s;
+    if ((rc = sv.ensure((int)n, mixed))) return rc;
     sv.plan = plan;
     sv.plan32 = plan32;
     sv.ground = ground;
     rc = mixed ? sv.solve_mixed(W.p, bv.p, stt) : sv.solve64(W.p, bv.p, stt);
     if (rc) return rc;
-    TAGS_HIP(hipMemcpyAsync(bx, bv.p, sizeof(c64) * n, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipStreamSynchronize(S.s));
-    return 0;
+    return copy_out(bx, bv.p, sizeof(c64) * n, S.s);
 }
 
 int solve_immittance(TAGS_COMPLEX* wg, TAGS_COMPLEX* ie, size_t num_electrodes, size_t num_nodes)
 {
     const long N = (long)(2 * num_electrodes + num_nodes);
-    int rc = dense_solve_host((const c64*)wg, (c64*)ie, N, TAGS_PREC_FP64, true, nullptr);
+    int rc = dense_solve_host((const c64*)wg, (c64*)ie, N, TAGS_PREC_FP64, true, nullptr, nullptr,
+                              nullptr, Grounding{}, (long)num_electrodes);
     if (rc > 0) {
         std::printf("The diagonal element of the triangular factor of YN,\n");
         std::printf("U(%i,%i) is zero, so that YN is singular;\n", rc, rc);
@@ -1538,7 +1663,84 @@ extern "C" {
 // Device copies of the host arrays of one admittance call.
 struct AdmArrays {
     DevBuf<c64> zl, zt, arm, brm, yla, ytb, yn;
+    DevBuf<c64> z2;  // zl then zt, as uploaded
 };
+
+// Largest entry of Z X - I for which one Newton step leaves the inverse at
+// working accuracy (its square times m stays far below an ulp).
+constexpr double kInvGate = 1e-10;
+
+// Both inverses without row exchanges, as explicit symmetric inverses X of z2's
+// blocks with a Newton step X + X (I - Z X); *done unless a product Z X is
+// further from I than kInvGate (then nothing of the caller's is touched and the
+// pivoted factorisation follows). Then yla^T = A^T X_L and ytb^T = B^T X_T
+// (row-major n x m: the column-major m x n the caller takes) from a and b as
+// uploaded in arm and brm, and the lower triangles to zl and zt.
+// (m = 606, n = 559: 10.6 ms for the whole call by the pivoted factors.)
+static int adm_symmetric(AdmArrays& d, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const c64* av,
+                         const c64* bv, long m, long n, hipStream_t st, bool* done)
+{
+    *done = false;
+    const long ld = (m + 63) / 64 * 64;
+    int rc;
+    DevBuf<c64> X, X2, Z, R;
+    DevBuf<char> work;
+    DevBuf<unsigned long long> dev;
+    if ((rc = X.alloc((size_t)2 * ld * ld)) || (rc = X2.alloc((size_t)2 * ld * ld)) ||
+        (rc = Z.alloc((size_t)2 * m * m)) || (rc = R.alloc((size_t)2 * m * m)) ||
+        (rc = work.alloc(sym_inverse_bytes(m, 2))) || (rc = dev.alloc(2)))
+        return rc;
+    TAGS_HIP(hipMemcpyAsync(Z.p, d.z2.p, sizeof(c64) * 2 * m * m, hipMemcpyDeviceToDevice, st));
+    for (int i = 0; i < 2; i++)
+        if ((rc = sym_from_upper(Z.p + i * m * m, m, (int)m, st))) return rc;
+    if ((rc = sym_inverse(Z.p, m, m * m, X.p, m, 2, work.p, st))) return rc;
+    // R = Z X - I
+    GemmArgs<double> g{(int)m, (int)m, (int)m, Z.p, m, nullptr, X.p, ld, nullptr, R.p, m, nullptr, 0};
+    g.nb = 2;
+    g.sa = m * m;
+    g.sb = ld * ld;
+    g.sc = m * m;
+    if ((rc = launch_gemm<double>(g, st))) return rc;
+    if ((rc = fill_c64((c64*)dev.p, 1, c64{0.0, 0.0}, st))) return rc;
+    if ((rc = sub_identity(R.p, m, 2, dev.p, st))) return rc;
+    double h[2];
+    if ((rc = copy_out(h, dev.p, sizeof(h), st))) return rc;
+    if (!(h[0] <= kInvGate)) return 0;
+    // X2 = X - X R
+    TAGS_HIP(hipMemcpyAsync(X2.p, X.p, sizeof(c64) * 2 * ld * ld, hipMemcpyDeviceToDevice, st));
+    g.A = X.p;
+    g.lda = ld;
+    g.sa = ld * ld;
+    g.B = R.p;
+    g.ldb = m;
+    g.sb = m * m;
+    g.C = X2.p;
+    g.ldc = ld;
+    g.sc = ld * ld;
+    g.mode = 1;
+    if ((rc = launch_gemm<double>(g, st))) return rc;
+    if (n > 0) {
+        GemmArgs<double> p{(int)n, (int)m, (int)m, av, m, nullptr, X2.p, ld, nullptr, d.yla.p, m, nullptr, 0};
+        if ((rc = launch_gemm<double>(p, st))) return rc;
+        p.A = bv;
+        p.B = X2.p + ld * ld;
+        p.C = d.ytb.p;
+        if ((rc = launch_gemm<double>(p, st))) return rc;
+    }
+    // the lower triangles (entry (k, i), k >= i, at i m + k of the caller's arrays)
+    c64* packed = Z.p;
+    const long np = m * (m + 1) / 2;
+    if ((rc = sym_pack(X2.p, ld, m, 2, packed, st))) return rc;
+    for (int i = 0; i < 2; i++) {
+        c64* dst = (c64*)(i ? zt : zl);
+        rc = copy_out_rows(packed + i * np, m, st, [&](long q, long k, const c64* v, long cnt) {
+            std::memcpy(dst + q * m + k, v, sizeof(c64) * (size_t)cnt);
+        });
+        if (rc) return rc;
+    }
+    *done = true;
+    return 0;
+}
 
 // Z^-1 (lower triangles, into zl and zt on the host), yla = Z_L^-1 A and
 // ytb = Z_T^-1 B (on the device, column-major m x n) and the row-major A and
@@ -1552,26 +1754,31 @@ static int adm_inverses(AdmArrays& d, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const 
         (rc = d.arm.alloc((size_t)m * n)) || (rc = d.brm.alloc((size_t)m * n)) ||
         (rc = d.yla.alloc((size_t)m * n)) || (rc = d.ytb.alloc((size_t)m * n)))
         return rc;
-    {
-        // a, b (column-major m x n) staged in yla / ytb, transposed to row-major
-        TAGS_HIP(hipMemcpyAsync(d.yla.p, a, sizeof(c64) * m * n, hipMemcpyHostToDevice, st));
-        TAGS_HIP(hipMemcpyAsync(d.ytb.p, b, sizeof(c64) * m * n, hipMemcpyHostToDevice, st));
-        if ((rc = transpose(d.yla.p, m, nullptr, d.arm.p, n, n, m, 1.0, false, st)) ||
-            (rc = transpose(d.ytb.p, m, nullptr, d.brm.p, n, n, m, -1.0, false, st)))
-            return rc;
+    const size_t mm = (size_t)m * m, mn = (size_t)m * n;
+    // a, b (column-major m x n) staged in X order, transposed to row-major
+    DevBuf<c64> ab;
+    if ((rc = ab.alloc(2 * mn)) || (rc = d.z2.alloc(2 * mm))) return rc;
+    if ((rc = copy_in(ab.p, a, sizeof(c64) * mn, st)) ||
+        (rc = copy_in(ab.p + mn, b, sizeof(c64) * mn, st)) ||
+        (rc = copy_in(d.z2.p, zl, sizeof(c64) * mm, st)) ||
+        (rc = copy_in(d.z2.p + mm, zt, sizeof(c64) * mm, st)))
+        return rc;
+    if ((rc = transpose(ab.p, m, nullptr, d.arm.p, n, n, m, 1.0, false, st)) ||
+        (rc = transpose(ab.p + mn, m, nullptr, d.brm.p, n, n, m, -1.0, false, st)))
+        return rc;
+    if (zl != zt) {  // one array for both takes the reference's order of writes
+        bool done = false;
+        if ((rc = adm_symmetric(d, zl, zt, ab.p, ab.p + mn, m, n, st, &done)) || done) return rc;
     }
-    TAGS_HIP(hipMemcpyAsync(d.zl.p, zl, sizeof(c64) * m * m, hipMemcpyHostToDevice, st));
-    TAGS_HIP(hipMemcpyAsync(d.zt.p, zt, sizeof(c64) * m * m, hipMemcpyHostToDevice, st));
+    TAGS_HIP(hipMemcpyAsync(d.zl.p, d.z2.p, sizeof(c64) * mm, hipMemcpyDeviceToDevice, st));
+    TAGS_HIP(hipMemcpyAsync(d.zt.p, d.z2.p + mm, sizeof(c64) * mm, hipMemcpyDeviceToDevice, st));
     LUWork<double> w;
     // Z_L first, written back before Z_T is factored: as with zsytrf/zsytri in
     // the reference, a singular Z_T leaves zl already inverted
     if ((rc = adm_block(w, d.zl.p, d.arm.p, 1.0, m, n, d.yla.p, st))) return rc;
-    TAGS_HIP(hipMemcpyAsync(zl, d.zl.p, sizeof(c64) * m * m, hipMemcpyDeviceToHost, st));
-    TAGS_HIP(hipStreamSynchronize(st));
+    if ((rc = copy_out(zl, d.zl.p, sizeof(c64) * mm, st))) return rc;
     if ((rc = adm_block(w, d.zt.p, d.brm.p, -1.0, m, n, d.ytb.p, st))) return rc;
-    TAGS_HIP(hipMemcpyAsync(zt, d.zt.p, sizeof(c64) * m * m, hipMemcpyDeviceToHost, st));
-    TAGS_HIP(hipStreamSynchronize(st));
-    return 0;
+    return copy_out(zt, d.zt.p, sizeof(c64) * mm, st);
 }
 
 // yn (n x n column-major) = A^T yla + B^T ytb: as row-major products,
@@ -1603,9 +1810,7 @@ int fill_impedance_adm(TAGS_COMPLEX* yn, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, TAG
     int rc = adm_inverses(d, zl, zt, a, b, m, n, S.s);
     if (rc) return rc;
     if ((rc = adm_products(d, m, n, S.s))) return rc;
-    TAGS_HIP(hipMemcpyAsync(yn, d.yn.p, sizeof(c64) * n * n, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipStreamSynchronize(S.s));
-    return 0;
+    return copy_out(yn, d.yn.p, sizeof(c64) * n * n, S.s);
 }
 
 int calculate_yla_ytb(TAGS_COMPLEX* yla, TAGS_COMPLEX* ytb, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt,
@@ -1617,10 +1822,8 @@ int calculate_yla_ytb(TAGS_COMPLEX* yla, TAGS_COMPLEX* ytb, TAGS_COMPLEX* zl, TA
     AdmArrays d;
     int rc = adm_inverses(d, zl, zt, a, b, m, n, S.s);
     if (rc) return rc;
-    TAGS_HIP(hipMemcpyAsync(yla, d.yla.p, sizeof(c64) * m * n, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipMemcpyAsync(ytb, d.ytb.p, sizeof(c64) * m * n, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipStreamSynchronize(S.s));
-    return 0;
+    if ((rc = copy_out(yla, d.yla.p, sizeof(c64) * m * n, S.s))) return rc;
+    return copy_out(ytb, d.ytb.p, sizeof(c64) * m * n, S.s);
 }
 
 int fill_impedance_adm2(TAGS_COMPLEX* yn, TAGS_COMPLEX* yla, TAGS_COMPLEX* ytb, TAGS_COMPLEX* a,
@@ -1638,19 +1841,16 @@ int fill_impedance_adm2(TAGS_COMPLEX* yn, TAGS_COMPLEX* yla, TAGS_COMPLEX* ytb, 
         // a and b pass through one staging buffer to their row-major copies
         DevBuf<c64> stage;
         if ((rc = stage.alloc((size_t)m * n))) return rc;
-        TAGS_HIP(hipMemcpyAsync(stage.p, a, sizeof(c64) * m * n, hipMemcpyHostToDevice, S.s));
+        if ((rc = copy_in(stage.p, a, sizeof(c64) * m * n, S.s))) return rc;
         if ((rc = transpose(stage.p, m, nullptr, d.arm.p, n, n, m, 1.0, false, S.s))) return rc;
-        TAGS_HIP(hipStreamSynchronize(S.s));
-        TAGS_HIP(hipMemcpyAsync(stage.p, b, sizeof(c64) * m * n, hipMemcpyHostToDevice, S.s));
+        if ((rc = copy_in(stage.p, b, sizeof(c64) * m * n, S.s))) return rc;
         if ((rc = transpose(stage.p, m, nullptr, d.brm.p, n, n, m, -1.0, false, S.s))) return rc;
-        TAGS_HIP(hipMemcpyAsync(d.yla.p, yla, sizeof(c64) * m * n, hipMemcpyHostToDevice, S.s));
-        TAGS_HIP(hipMemcpyAsync(d.ytb.p, ytb, sizeof(c64) * m * n, hipMemcpyHostToDevice, S.s));
-        TAGS_HIP(hipStreamSynchronize(S.s));
+        if ((rc = copy_in(d.yla.p, yla, sizeof(c64) * m * n, S.s)) ||
+            (rc = copy_in(d.ytb.p, ytb, sizeof(c64) * m * n, S.s)))
+            return rc;
     }
     if ((rc = adm_products(d, m, n, S.s))) return rc;
-    TAGS_HIP(hipMemcpyAsync(yn, d.yn.p, sizeof(c64) * n * n, hipMemcpyDeviceToHost, S.s));
-    TAGS_HIP(hipStreamSynchronize(S.s));
-    return 0;
+    return copy_out(yn, d.yn.p, sizeof(c64) * n * n, S.s);
 }
 
 int solve_admittance(TAGS_COMPLEX* yn, TAGS_COMPLEX* ic, size_t num_nodes)
@@ -1924,16 +2124,20 @@ static int sweep_batch(const tags_sweep* sw, bool mixed)
     return (int)std::max(1.0, std::min((double)kBatchMax, b));
 }
 
-// Samples per group of the nodal solve, by the same rule on its own bytes.
+// Samples per group of the nodal solve, by the same rule on its own bytes and
+// limits: its steps are a chain of short launches, which more samples share
+// (200 samples of the 20 x 20 m grid, mixed: 7.3 ms in groups of 50, 6.3 of
+// 100; four of the 60 x 60 m grid: 213 ms in groups of one, 198 of two).
+constexpr int kNdBatchMax = 128, kNdBatchLarge = 2;
 // A call's nfreq samples are shared out evenly among the groups it takes.
 static int sweep_nd_batch(const tags_sweep* sw, bool mixed, size_t nfreq)
 {
-    size_t lim = 1;
+    size_t lim = kNdBatchLarge;
     if (sw->batch_req > 0) {
         lim = (size_t)sw->batch_req;
     } else if (sw->N < kBatchOneAbove) {
         const double per = (double)NodalSolver::bytes(sw->m, sw->n, !mixed, 1);
-        lim = (size_t)std::max(1.0, std::min((double)kBatchMax, std::floor(kBatchBytes / per)));
+        lim = (size_t)std::max(1.0, std::min((double)kNdBatchMax, std::floor(kBatchBytes / per)));
     }
     const size_t groups = std::max<size_t>(1, (nfreq + lim - 1) / lim);
     return (int)std::max<size_t>(1, sw->batch_req > 0 ? std::min(lim, nfreq)
@@ -2194,27 +2398,11 @@ int tags_sweep_create(tags_sweep** out, const Electrode* electrodes, const Elect
             return TAGS_ERR_ARG;
         }
     }
-    // each node's segment ends in segment order (a segment whose two ends
-    // share a node has its start entry only, as W has one entry there)
     std::vector<int> hsn(m), hen(m);
     TAGS_HIP(hipMemcpy(hsn.data(), sw->sn, sizeof(int) * m, hipMemcpyDeviceToHost));
     TAGS_HIP(hipMemcpy(hen.data(), sw->en, sizeof(int) * m, hipMemcpyDeviceToHost));
-    std::vector<int> ptr(n + 1, 0), seg;
-    for (long s = 0; s < m; s++) {
-        if (hsn[s] < 0 || hsn[s] >= n || hen[s] < 0 || hen[s] >= n) return TAGS_ERR_ARG;
-        ptr[hsn[s] + 1]++;
-        if (hen[s] != hsn[s]) ptr[hen[s] + 1]++;
-        else sw->nodal_ok = false;  // A 1 = 0 and B 1 = 1 need two nodes per segment
-    }
-    for (long u = 0; u < n; u++) ptr[u + 1] += ptr[u];
-    seg.assign(ptr[n], 0);
-    {
-        std::vector<int> fill(ptr.begin(), ptr.end() - 1);
-        for (long s = 0; s < m; s++) {
-            seg[fill[hsn[s]]++] = (int)(2 * s);
-            if (hen[s] != hsn[s]) seg[fill[hen[s]]++] = (int)(2 * s + 1);
-        }
-    }
+    std::vector<int> ptr, seg;
+    if (!node_lists(hsn, hen, n, ptr, seg, &sw->nodal_ok)) return TAGS_ERR_ARG;
     TAGS_HIP(hipMalloc(&sw->node_ptr, sizeof(int) * (n + 1)));
     TAGS_HIP(hipMalloc(&sw->node_seg, sizeof(int) * std::max<size_t>(1, seg.size())));
     TAGS_HIP(hipMemcpy(sw->node_ptr, ptr.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice));
@@ -3547,8 +3735,7 @@ int calculate_impedances_noalloc(TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const Elect
                    soa + 7 * m};
     const PairScalars sc = make_scalars(from_c(gamma), from_c(s), mur, from_c(kappa), c64{1, 0},
                                         c64{1, 0}, integration_type);
-    return launch_pairs_dropin((double*)zl, (double*)zt, (void*)zl == (void*)zt, g, g, m, sc,
-                               false, st);
+    return launch_pairs_dropin((double*)zl, (double*)zt, (void*)zl == (void*)zt, g, m, sc, st);
 }
 
 }  // extern "C"

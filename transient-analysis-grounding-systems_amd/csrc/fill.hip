@@ -351,7 +351,7 @@ __device__ c64 single_unit(const DSeg& S, V3 M, c64 g)
         const double span = side ? 1.0 - t0 : t0;
         double u0 = 0.0;
         while (u0 < span) {
-            const double u1 = fmin(u0 + (u0 == 0.0 ? wmin : fmin(u0, wmax)), span);
+            const double u1 = fmin(u0 + fmin(u0 == 0.0 ? wmin : u0, wmax), span);
             const double h = u1 - u0;
             for (int q = 0; q < 16; q++) {
                 const double u = u0 + h * g_glx[off + q];
@@ -400,66 +400,92 @@ __device__ inline double abs_dot(const DSeg& a, const DSeg& b)
 }
 
 // ---------------------------------------------------------------------------
-// Drop-in calculate_impedances / impedances_images on a device copy of the
-// caller's m*m arrays (lower-half convention, entry (i, k >= i) at i*m + k).
+// Drop-in calculate_impedances (device arrays, lower-half convention, entry (i,
+// k >= i) at i*m + k) and, packed for the host arrays, calculate_impedances and
+// impedances_images.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_pairs_dropin(c64* zl, c64* zt, int alias, SegSoA e,
-                                                       SegSoA img, long m, PairScalars sc,
-                                                       int images)
+struct PairZ {
+    c64 l, t;  // Z_L, Z_T entries
+    bool has_l;  // image part: whether Z_L receives one
+};
+__device__ inline PairZ pair_entry(const DSeg& Si, double rad, const DSeg& Rk, bool self,
+                                   const PairScalars& sc, bool images)
 {
-    long k = blockIdx.x * 16 + threadIdx.x % 16;
-    long i = blockIdx.y * 16 + threadIdx.x / 16;
-    if (i >= m || k >= m || k < i) return;
-    DSeg Si = load_seg(e, i);
-    long idx = i * m + k;
+    PairZ z;
+    z.l = c64{0.0, 0.0};
+    z.has_l = true;
     const double ls = Si.len;
-    if (!images) {
-        if (k == i) {
-            // src/electrode.c:346-348
-            double intg = self_integral_dev(ls, e.rad[i]);
-            c64 vl = cscale(sc.zl_dir, intg);
-            c64 vt = cscale(cscale(sc.zt_dir, 1.0 / (ls * ls)), intg);
-            zl[idx] = vl;
-            zt[idx] = vt;  // zt written last: wins when zl == zt
-            return;
-        }
-        DSeg Rk = load_seg(e, k);
-        const double lr = Rk.len;
-        double cost = abs_dot(Si, Rk);
-        c64 intg = pair_result(Si, Rk, sc.gamma, sc.intg_type);
-        c64 vt = cmul(cscale(sc.zt_dir, 1.0 / (ls * lr)), intg);
-        c64 vl = c64{0.0, 0.0};
-        if (!(cost < 2.220446049250313e-16)) vl = cscale(cmul(sc.zl_dir, intg), cost / (ls * lr));
-        if (alias) {
-            zl[idx] = vl;  // zt then zl: zl wins off the diagonal
-        } else {
-            zt[idx] = vt;
-            zl[idx] = vl;
-        }
-        return;
+    if (self) {
+        // src/electrode.c:346-348
+        const double intg = self_integral_dev(ls, rad);
+        z.l = cscale(sc.zl_dir, intg);
+        z.t = cscale(cscale(sc.zt_dir, 1.0 / (ls * ls)), intg);
+        return z;
     }
-    // images (src/electrode.c:403-429)
-    DSeg Rk = load_seg(img, k);
-    const double lr = Rk.len;
-    double cost = abs_dot(Si, Rk);
-    c64 intg = pair_result(Si, Rk, sc.gamma, sc.intg_type);
-    c64 vt = cmul(cscale(sc.zt_img, 1.0 / (ls * lr)), intg);
-    zt[idx] = cadd(zt[idx], vt);
-    if (cost > 2.220446049250313e-16) {
-        c64 vl = cscale(cmul(sc.zl_img, intg), cost / (ls * lr));
-        zl[idx] = cadd(zl[idx], vl);  // same buffer twice when zl == zt
+    const double lr = Rk.len, cost = abs_dot(Si, Rk);
+    const c64 intg = pair_result(Si, Rk, sc.gamma, sc.intg_type);
+    z.t = cmul(cscale(images ? sc.zt_img : sc.zt_dir, 1.0 / (ls * lr)), intg);
+    // src/electrode.c:349-372 and, for images, :403-429
+    z.has_l = images ? cost > 2.220446049250313e-16 : !(cost < 2.220446049250313e-16);
+    if (z.has_l) z.l = cscale(cmul(images ? sc.zl_img : sc.zl_dir, intg), cost / (ls * lr));
+    return z;
+}
+
+__global__ __launch_bounds__(256) void k_pairs_dropin(c64* zl, c64* zt, int alias, SegSoA e,
+                                                       long m, PairScalars sc)
+{
+    const long k = blockIdx.x * 16 + threadIdx.x % 16;
+    const long i = blockIdx.y * 16 + threadIdx.x / 16;
+    if (i >= m || k >= m || k < i) return;
+    const PairZ z = pair_entry(load_seg(e, i), e.rad[i], load_seg(e, k), k == i, sc, false);
+    const long idx = i * m + k;
+    if (alias) {
+        // the reference writes zl then zt on the diagonal, zt then zl off it
+        zl[idx] = k == i ? z.t : z.l;
+    } else {
+        zt[idx] = z.t;
+        zl[idx] = z.l;
     }
 }
 
-int launch_pairs_dropin(double* zl, double* zt, bool alias, SegSoA e, SegSoA img, long m,
-                        const PairScalars& sc, bool images, hipStream_t st)
+// The same entries (images: of e against img), packed by rows: entry (i, k >= i)
+// at i m - i (i - 1) / 2 + k - i; an image part that Z_L does not receive is zero.
+__global__ __launch_bounds__(256) void k_pairs_packed(c64* zl, c64* zt, SegSoA e, SegSoA img,
+                                                       long m, PairScalars sc, int images)
+{
+    const long k = blockIdx.x * 16 + threadIdx.x % 16;
+    const long i = blockIdx.y * 16 + threadIdx.x / 16;
+    if (i >= m || k >= m || k < i) return;
+    const PairZ z = pair_entry(load_seg(e, i), e.rad[i], load_seg(images ? img : e, k),
+                               !images && k == i, sc, images != 0);
+    const long o = i * m - i * (i - 1) / 2 + k - i;
+    zl[o] = z.l;
+    zt[o] = z.t;
+}
+
+int launch_pairs_packed(c64* zl, c64* zt, SegSoA e, SegSoA img, long m, const PairScalars& sc,
+                        bool images, hipStream_t st)
+{
+    if (m <= 0) return 0;
+    if ((m + 15) / 16 > 65535) return TAGS_ERR_TOO_LARGE;
+    int rc = gl_tables_init();
+    if (rc) return rc;
+    const dim3 grid((unsigned)((m + 15) / 16), (unsigned)((m + 15) / 16));
+    hipLaunchKernelGGL(k_pairs_packed, grid, dim3(256), 0, st, zl, zt, e, img, m, sc,
+                       images ? 1 : 0);
+    TAGS_HIP(hipGetLastError());
+    return 0;
+}
+
+int launch_pairs_dropin(double* zl, double* zt, bool alias, SegSoA e, long m,
+                        const PairScalars& sc, hipStream_t st)
 {
     if (m <= 0) return 0;
     int rc = gl_tables_init();
     if (rc) return rc;
     dim3 grid((unsigned)((m + 15) / 16), (unsigned)((m + 15) / 16));
     hipLaunchKernelGGL(k_pairs_dropin, grid, dim3(256), 0, st, (c64*)zl, (c64*)zt,
-                       alias ? 1 : 0, e, img, m, sc, images ? 1 : 0);
+                       alias ? 1 : 0, e, m, sc);
     TAGS_HIP(hipGetLastError());
     return 0;
 }

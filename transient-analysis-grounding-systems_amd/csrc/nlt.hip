@@ -6,8 +6,8 @@
 // batch of signals (the examples transform one signal per node or right-hand
 // side, src/auxiliary.c's layout: signal i at f[i nt ..], g[i ns ..]):
 //  * nt a power of two: radix-2 Stockham passes (autosort, no bit reversal),
-//    one launch per pass, ping-pong buffers, twiddles from a table computed on
-//    the host (exp(-2 pi i t / nt), t < nt);
+//    one launch per pass, ping-pong buffers, twiddles from a table
+//    (exp(-2 pi i t / nt), t < nt);
 //  * any other nt: the direct sum with the exact table index (j k mod nt).
 // The weights that the reference computes per sample (exp(-c k dt) dt, the
 // data windows) are computed on the host with the same formulas, so that only
@@ -16,7 +16,7 @@
 #include <complex>
 #include <vector>
 
-#include "tags_common.h"
+#include "hostcopy.h"
 
 namespace tags {
 
@@ -137,17 +137,33 @@ static int dft_batch(c64* buf, c64* tmp, const c64* w, long n, long batch, bool 
     return 0;
 }
 
-// exp(-2 pi i t / n) for t < n, evaluated in extended precision and rounded
-// once, so that every entry is within half an ulp or so
-static std::vector<c64> twiddles(long n)
+// w[t] = exp(-2 pi i t / n), t < n. The angle 2 t / n (in units of pi) is
+// reduced to at most 1/4 by symmetries of the integers, exactly; what rounding
+// leaves of the division is put back to first order, so that the values are
+// within an ulp. (In extended precision on the host the table took 3 ms at
+// n = 16,384, more than the transforms.)
+__global__ __launch_bounds__(256) void k_twiddles(c64* w, long n)
 {
-    std::vector<c64> w(n);
-    for (long t = 0; t < n; t++) {
-        const long double a = 2.0L * 3.14159265358979323846264338327950288L * (long double)t /
-                              (long double)n;
-        w[t] = c64{(double)std::cos(a), (double)-std::sin(a)};
+    const long t = (long)blockIdx.x * 256 + threadIdx.x;
+    if (t >= n) return;
+    // the nearest multiple q of a quarter turn, and what is left of the angle:
+    // pi num / (4 n), |num| <= n
+    const long q = (8 * t / n + 1) / 2;
+    const long num = 8 * t - 2 * q * n;
+    const double d = 4.0 * (double)n, x = (double)num / d;
+    const double lo = fma(-x, d, (double)num) / d * 3.14159265358979323846;
+    double s, c;
+    sincospi(x, &s, &c);
+    const double s1 = fma(c, lo, s), c1 = fma(-s, lo, c);
+    // rotate by q quarter turns: exp(-i (angle + q pi / 2))
+    double re = c1, im = -s1;
+    switch (q & 3) {
+    case 1: re = -s1; im = -c1; break;
+    case 2: re = -c1; im = s1; break;
+    case 3: re = s1; im = c1; break;
+    default: break;
     }
-    return w;
+    w[t] = c64{re, im};
 }
 
 struct NltBuffers {
@@ -172,8 +188,8 @@ struct NltBuffers {
         TAGS_HIP(hipMalloc(&a, sizeof(c64) * n * batch));
         TAGS_HIP(hipMalloc(&b, sizeof(c64) * n * batch));
         TAGS_HIP(hipMalloc(&v, sizeof(double) * n));
-        std::vector<c64> tw = twiddles(n);
-        TAGS_HIP(hipMemcpyAsync(w, tw.data(), sizeof(c64) * n, hipMemcpyHostToDevice, st));
+        hipLaunchKernelGGL(k_twiddles, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w, n);
+        TAGS_HIP(hipGetLastError());
         return 0;
     }
 };
@@ -240,16 +256,17 @@ int tags_laplace_batch(const double* f, TAGS_COMPLEX* g, TAGS_COMPLEX* s, double
     if (rc) return rc;
     // the real samples travel as doubles (staged in the second buffer)
     double* fd = (double*)nb.b;
-    TAGS_HIP(hipMemcpyAsync(fd, f, sizeof(double) * n * B, hipMemcpyHostToDevice, nb.st));
-    TAGS_HIP(hipMemcpyAsync(nb.v, wk.data(), sizeof(double) * n, hipMemcpyHostToDevice, nb.st));
+    if ((rc = copy_in(fd, f, sizeof(double) * n * B, nb.st)) ||
+        (rc = copy_in(nb.v, wk.data(), sizeof(double) * n, nb.st)))
+        return rc;
     hipLaunchKernelGGL(k_weight_real, dim3(grid_for(n * B)), dim3(256), 0, nb.st, fd, nb.v, nb.a,
                        n, B);
     TAGS_HIP(hipGetLastError());
     if ((rc = dft_batch(nb.a, nb.b, nb.w, n, B, false, nb.st))) return rc;
-    TAGS_HIP(hipMemcpy2DAsync(g, sizeof(c64) * ns, nb.a, sizeof(c64) * n, sizeof(c64) * ns, B,
-                              hipMemcpyDeviceToHost, nb.st));
-    TAGS_HIP(hipStreamSynchronize(nb.st));
-    return 0;
+    // the half spectra, packed (in the second buffer) and copied out
+    TAGS_HIP(hipMemcpy2DAsync(nb.b, sizeof(c64) * ns, nb.a, sizeof(c64) * n, sizeof(c64) * ns, B,
+                              hipMemcpyDeviceToDevice, nb.st));
+    return copy_out(g, nb.b, sizeof(c64) * ns * B, nb.st);
 }
 
 // Data windows of src/auxiliary.c:271-305 (the Lanczos window is 0/0 at
@@ -295,9 +312,10 @@ int tags_inv_laplace_batch(double* f, const TAGS_COMPLEX* g, const TAGS_COMPLEX*
     nb.v = nullptr;
     TAGS_HIP(hipMalloc(&nb.v, sizeof(double) * (n + ns)));
     double* dw = nb.v + n;
-    TAGS_HIP(hipMemcpyAsync(nb.b, gg, sizeof(c64) * ns * B, hipMemcpyHostToDevice, nb.st));
-    TAGS_HIP(hipMemcpyAsync(dw, win.data(), sizeof(double) * ns, hipMemcpyHostToDevice, nb.st));
-    TAGS_HIP(hipMemcpyAsync(nb.v, sc.data(), sizeof(double) * n, hipMemcpyHostToDevice, nb.st));
+    if ((rc = copy_in(nb.b, gg, sizeof(c64) * ns * B, nb.st)) ||
+        (rc = copy_in(dw, win.data(), sizeof(double) * ns, nb.st)) ||
+        (rc = copy_in(nb.v, sc.data(), sizeof(double) * n, nb.st)))
+        return rc;
     hipLaunchKernelGGL(k_hermitian, dim3(grid_for(n * B)), dim3(256), 0, nb.st, nb.b, dw, nb.a, n,
                        ns, B);
     TAGS_HIP(hipGetLastError());
@@ -306,9 +324,7 @@ int tags_inv_laplace_batch(double* f, const TAGS_COMPLEX* g, const TAGS_COMPLEX*
     hipLaunchKernelGGL(k_real_scale, dim3(grid_for(n * B)), dim3(256), 0, nb.st, nb.a, nb.v, fd,
                        n, B);
     TAGS_HIP(hipGetLastError());
-    TAGS_HIP(hipMemcpyAsync(f, fd, sizeof(double) * n * B, hipMemcpyDeviceToHost, nb.st));
-    TAGS_HIP(hipStreamSynchronize(nb.st));
-    return 0;
+    return copy_out(f, fd, sizeof(double) * n * B, nb.st);
 }
 
 int laplace_trans(double* f, TAGS_COMPLEX* g, TAGS_COMPLEX* s, double tmax, size_t nt)
