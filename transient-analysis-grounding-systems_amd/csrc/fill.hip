@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "tags_common.h"
@@ -640,14 +641,15 @@ int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
 // terms is below 1e-17 for |gamma| D <= 7.3 (K = 32, see fill_terms); larger
 // ones keep the direct rule (k_fill_zblocks).
 //
-// One thread per pair of a 16 x 16 tile on or below the diagonal, work-groups
+// One thread per pair of a TS x TS tile on or below the diagonal, work-groups
 // of one tile and a range of the samples (so that few segments still fill the
 // device). Pairs that touch or are closer than two lengths, which need the
 // Duffy rule or 144 points and more, are listed in LDS and taken by whole
 // waves, the lanes sharing the points; moments pass through LDS, so that few
-// of them are live in registers at a time. Bound: the samples' exponentials and
-// sines (FP64 VALU, about 300 instructions per pair and sample), then the
-// writes of both triangles.
+// of them are live in registers at a time. TS is 16, or 8 for few segments (a
+// fourth of the listed pairs per work-group, whose four waves then take a
+// sample each). Bound: the samples' exponentials and sines (FP64 VALU, about
+// 300 instructions per pair and sample), then the writes of both triangles.
 // ---------------------------------------------------------------------------
 template <int K>
 struct Moments {
@@ -771,35 +773,39 @@ __device__ inline bool pair_near(const DSeg& S, const DSeg& R, double* rho)
     return !(*rho >= 2.0);
 }
 
-template <int K>
+template <int K, int TS>
 __global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, long ldw,
                                                        long zl_off, long zt_off, long m, SegSoA e,
                                                        SegSoA img,
                                                        const PairScalars* __restrict__ scs, long sw,
-                                                       const c64* __restrict__ cf, int nf, int per, double D,
-                                                       double gabs)
+                                                       const c64* __restrict__ cf, int nf, int per,
+                                                       double D, double gabs)
 {
     const long b = blockIdx.x;
     long ti = (long)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
     while ((ti + 1) * (ti + 2) / 2 <= b) ti++;
     while (ti * (ti + 1) / 2 > b) ti--;
     const long tk = b - ti * (ti + 1) / 2;
-    const int t = threadIdx.x, a = t >> 4, c = t & 15;
-    const long i0 = ti * 16, k0 = tk * 16, i = i0 + a, k = k0 + c;
+    constexpr int NP = TS * TS;  // pairs
+    // (the wave index is uniform: a sample's scalars and coefficients stay scalar)
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+    // with 8 x 8 tiles every wave holds all pairs (and forms them once, in wave 0)
+    const int pr = TS == 8 ? lane : t, a = pr / TS, c = pr % TS;
+    const long i0 = ti * TS, k0 = tk * TS, i = i0 + a, k = k0 + c;
     const bool in = i < m && k < m && k <= i;
 
-    __shared__ double geo[3][8][16];  // columns, rows, the rows' images
+    __shared__ double geo[3][8][TS];  // columns, rows, the rows' images
     // every pair's moments of one kind while they are formed; then the tiles
     // being transposed
     union Stage {
-        double mom[K][256];
-        c64 tile[2][2][16][17];
+        double mom[K][NP];
+        c64 tile[2][2][TS][TS + 1];
     };
     __shared__ Stage stage;
-    __shared__ int near_n[2], near_at[2][256];
+    __shared__ int near_n[2], near_at[2][NP];
     if (t < 2) near_n[t] = 0;
-    if (t < 48) {
-        const int side = t >> 4, s = t & 15;
+    if (t < 3 * TS) {
+        const int side = t / TS, s = t % TS;
         const long idx = (side == 0 ? k0 : i0) + s;
         const SegSoA& g = side == 2 ? img : e;
         if (idx < m) {
@@ -820,7 +826,6 @@ __global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, lo
     };
     double md[K], mi[K];  // direct, image
     double rd = 0.0, ri = 0.0, cost = 0.0, cosi = 0.0, ll = 1.0;
-    const int wave = t >> 6, lane = t & 63;
 #pragma unroll
     for (int kind = 0; kind < 2; kind++) {
         {
@@ -834,21 +839,22 @@ __global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, lo
                 (kind ? cosi : cost) = abs_dot(S, R);
                 if (!kind) ll = S.len * R.len;
                 double rho;
-                if (kind || k != i) {
+                if ((TS == 16 || wave == 0) && (kind || k != i)) {
                     if (pair_near(S, R, &rho))
-                        near_at[kind][atomicAdd(&near_n[kind], 1)] = t;
+                        near_at[kind][atomicAdd(&near_n[kind], 1)] = pr;
                     else
                         mom_gl(M, S, R, geometric_order(rho, gabs * fmax(S.len, R.len)), 0, 1, 1.0);
                 }
             }
 #pragma unroll
-            for (int j = 0; j < K; j++) stage.mom[j][t] = M.m[j];
+            for (int j = 0; j < K; j++)
+                if (TS == 16 || wave == 0) stage.mom[j][pr] = M.m[j];
         }
         __syncthreads();
         const int nn = near_n[kind];
         for (int q = wave; q < nn; q += 4) {
             const int w = near_at[kind][q];
-            const DSeg S = seg(0, w & 15), R = seg(1 + kind, w >> 4);
+            const DSeg S = seg(0, w % TS), R = seg(1 + kind, w / TS);
             Moments<K> M;
             M.zero();
             M.invd = 1.0 / D;
@@ -863,12 +869,12 @@ __global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, lo
         }
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < K; j++) (kind ? mi[j] : md[j]) = stage.mom[j][t];
+        for (int j = 0; j < K; j++) (kind ? mi[j] : md[j]) = stage.mom[j][pr];
         __syncthreads();
     }
     const double self = in && k == i ? self_integral_dev(geo[1][6][a], geo[1][7][a]) : 0.0;
     const int f0 = blockIdx.y * per, f1 = min(nf, f0 + per);
-    for (int f = f0; f < f1; f++) {
+    for (int f = f0 + (TS == 8 ? wave : 0); f < f1; f += TS == 8 ? 4 : 1) {
         const PairScalars& sc = scs[f];
         const c64* cq = cf + (long)f * K;
         c64 vl{0, 0}, vt{0, 0};
@@ -906,15 +912,28 @@ __global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, lo
             Wf[(zl_off + i) * ldw + zl_off + k] = vl;
             Wf[(zt_off + i) * ldw + zt_off + k] = vt;
         }
-        const int h = f & 1;
-        stage.tile[h][0][a][c] = vl;
-        stage.tile[h][1][a][c] = vt;
-        __syncthreads();
-        const long ko = k0 + a, io = i0 + c;  // entry (ko, io) of the other triangle
-        if (io < m && ko < io) {
-            c64* Wf = W + (long)f * sw;
-            Wf[(zl_off + ko) * ldw + zl_off + io] = stage.tile[h][0][c][a];
-            Wf[(zt_off + ko) * ldw + zt_off + io] = stage.tile[h][1][c][a];
+        if constexpr (TS == 8) {
+            // the other triangle's entry (k0 + a, i0 + c) is lane (c, a)'s
+            const int from = c * 8 + a;
+            const c64 ol{__shfl(vl.x, from), __shfl(vl.y, from)};
+            const c64 ot{__shfl(vt.x, from), __shfl(vt.y, from)};
+            const long ko = k0 + a, io = i0 + c;
+            if (io < m && ko < io) {
+                c64* Wf = W + (long)f * sw;
+                Wf[(zl_off + ko) * ldw + zl_off + io] = ol;
+                Wf[(zt_off + ko) * ldw + zt_off + io] = ot;
+            }
+        } else {
+            const int h = f & 1;
+            stage.tile[h][0][a][c] = vl;
+            stage.tile[h][1][a][c] = vt;
+            __syncthreads();
+            const long ko = k0 + a, io = i0 + c;  // entry (ko, io) of the other triangle
+            if (io < m && ko < io) {
+                c64* Wf = W + (long)f * sw;
+                Wf[(zl_off + ko) * ldw + zl_off + io] = stage.tile[h][0][c][a];
+                Wf[(zt_off + ko) * ldw + zt_off + io] = stage.tile[h][1][c][a];
+            }
         }
     }
 }
@@ -961,20 +980,28 @@ int launch_fill_moments(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
     int rc = gl_tables_init();
     if (rc) return rc;
     hipLaunchKernelGGL(k_fill_coefs, dim3(nb), dim3(64), 0, st, scs, D, K, cf);
-    const long T = (m + 15) / 16, tiles = T * (T + 1) / 2;
+    const bool small = m <= 256;
+    const long T = small ? (m + 7) / 8 : (m + 15) / 16, tiles = T * (T + 1) / 2;
     // samples per work-group: all of them once the tiles alone give every CU
-    // four work-groups, else fewer (the moments are then formed more often)
-    const long chunks = std::max(1L, std::min((long)nb, 1024 / tiles));
+    // four work-groups (8 x 8 tiles: two, of four samples at least), else fewer
+    // (the moments are then formed more often)
+    const long chunks = std::max(1L, std::min(small ? (nb + 3L) / 4 : (long)nb,
+                                              (small ? 512 : 1024) / tiles));
     const int per = (int)((nb + chunks - 1) / chunks);
     const dim3 g((unsigned)tiles, (unsigned)((nb + per - 1) / per));
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, g, dim3(256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, scs,
                            sw, (const c64*)cf, nb, per, D, gabs);
     };
-    if (K == 12) go(k_fill_moments<12>);
-    else if (K == 16) go(k_fill_moments<16>);
-    else if (K == 24) go(k_fill_moments<24>);
-    else go(k_fill_moments<kFillTermsMax>);
+    auto terms = [&](auto kt) {
+        constexpr int k = decltype(kt)::value;
+        if (small) go(k_fill_moments<k, 8>);
+        else go(k_fill_moments<k, 16>);
+    };
+    if (K == 12) terms(std::integral_constant<int, 12>());
+    else if (K == 16) terms(std::integral_constant<int, 16>());
+    else if (K == 24) terms(std::integral_constant<int, 24>());
+    else terms(std::integral_constant<int, kFillTermsMax>());
     TAGS_HIP(hipGetLastError());
     return 0;
 }

@@ -37,6 +37,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "dd.h"
 #include "mfma.h"
 #include "nodal.h"
 #include "x6.h"
@@ -161,12 +162,66 @@ constexpr int nd_groups(int k)  // k groups of nd_mma in k columns
 //   (-P_q if s = r, else T_q of the other side) - sum_{u > q} T_u(i) O_u(j)^T.
 // ---------------------------------------------------------------------------
 
-// P_t by an unblocked sweep, one work-group per item: a thread holds 4 x 4
-// entries in registers; per pivot the pivot row goes through LDS (it is the
-// pivot column too), one barrier. Latency-bound: 64 steps of a broadcast, a
-// reciprocal and 16 complex multiply-adds.
+// The unblocked sweep of a 64 x 64 matrix in the registers of 256 threads (ty,
+// tx: rows ty + 16 i, columns tx + 16 j): a = -a^-1 over its first kv rows and
+// columns. Per pivot k the pivot row goes through LDS (it is the pivot column
+// too); with the pivot row's and column's own entries cleared, the multiplier
+// of row k set to -1/p and the entry of column k to -1, one multiply-add serves
+// every entry. Row k + 1 is formed and stored before the barrier, so that the
+// rest of step k runs beside the next pivot's read and reciprocal: latency per
+// pivot, not the 16 multiply-adds per thread, bounds it (64 pivots in complex128:
+// 50 us with the update before the next row).
+template <typename T>
+__device__ __forceinline__ void nd_sweep64(cx<T> (&a)[4][4], cx<T> (*row)[64], int kv, int ty,
+                                           int tx)
+{
+    if (ty == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) row[0][tx + 16 * j] = a[0][j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+        for (int kl = 0; kl < 16; kl++) {
+            const int k = 16 * kb + kl;
+            if (k >= kv) return;
+            const cx<T>* rk = row[k & 1];
+            const cx<T> d = crecip_fast(rk[k]);
+            cx<T> o[4], l[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = rk[tx + 16 * j];
+#pragma unroll
+            for (int i = 0; i < 4; i++) l[i] = cmul(rk[ty + 16 * i], d);
+            const bool pr = ty == kl, pc = tx == kl;
+            const cx<T> zero{0, 0};
+            l[kb] = csel(pr, cx<T>{-d.x, -d.y}, l[kb]);
+            o[kb] = csel(pc, cx<T>{-1, 0}, o[kb]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                a[kb][j] = csel(pr, zero, a[kb][j]);
+                a[j][kb] = csel(pc, zero, a[j][kb]);
+            }
+            if (k + 1 < kv && ty == ((kl + 1) & 15)) {
+                const int nx = kb < 3 ? kb + 1 : kb;
+                const cx<T> ln = csel(kl < 15, l[kb], l[nx]);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    row[(k + 1) & 1][tx + 16 * j] =
+                        cfnma(csel(kl < 15, a[kb][j], a[nx][j]), ln, o[j]);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) a[i][j] = cfnma(a[i][j], l[i], o[j]);
+        }
+}
+
+// P_t, one work-group per item. A matrix of one block (whole) is finished here:
+// both triangles of A get -P.
 template <typename T, int NB>
-__global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t)
+__global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t,
+                                                  int whole)
 {
     using V4 = typename Mfma<T>::v4;
     const long item = blockIdx.x;
@@ -218,43 +273,19 @@ __global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t)
                 }
         }
     }
-    for (int k = 0; k < kv; k++) {
-        cx<T>* rk = row[k & 1];
-        if (ty == (k & 15)) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                // row k = ty + 16 (k >> 4)
-                const cx<T> lo = csel((k >> 4) & 1, a[1][j], a[0][j]);
-                const cx<T> hi = csel((k >> 4) & 1, a[3][j], a[2][j]);
-                rk[tx + 16 * j] = csel(k >> 5, hi, lo);
-            }
-        }
-        __syncthreads();
-        const cx<T> d = crecip_fast(rk[k]);
-        cx<T> o[4], l[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = rk[tx + 16 * j];
-#pragma unroll
-        for (int i = 0; i < 4; i++) l[i] = cmul(rk[ty + 16 * i], d);
-        const bool mr = ty == (k & 15), mc = tx == (k & 15);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const bool pr = mr && i == (k >> 4), pc = mc && j == (k >> 4);
-                cx<T> n = cfnma(a[i][j], l[i], o[j]);
-                n = csel(pr, cmul(o[j], d), csel(pc, l[i], n));
-                n = csel(pr && pc, cx<T>{-d.x, -d.y}, n);
-                a[i][j] = n;
-            }
-    }
+    nd_sweep64(a, row, kv, ty, tx);
+    cx<T>* own = p.A + item * p.sA;
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int r = ty + 16 * i, c = tx + 16 * j;
             const bool in = r < kv && c < kv;
-            P[r * 64 + c] = in ? cx<T>{-a[i][j].x, -a[i][j].y} : cx<T>{0, 0};
+            if (whole) {
+                own[(long)r * p.ld + c] = in ? a[i][j] : cx<T>{0, 0};
+            } else {
+                P[r * 64 + c] = in ? cx<T>{-a[i][j].x, -a[i][j].y} : cx<T>{0, 0};
+            }
         }
 }
 
@@ -883,6 +914,290 @@ __global__ __launch_bounds__(256) void k_nd_pick(NdArgs<T> g, c64* u)
 }
 
 // ---------------------------------------------------------------------------
+// Small systems (at most 64 segments and 64 nodes) in one launch
+// ---------------------------------------------------------------------------
+__device__ inline void lds_max(unsigned long long* p, double a)
+{
+    atomicMax(p, (unsigned long long)__double_as_longlong(a));
+}
+
+// Everything of a sample after the fill: both inverses (256 threads each), the
+// node system, its inverse, and `spec` refinement steps, by one work-group, with
+// the operations of the kernels above and the vectors in LDS. The blocks, S^-1
+// and the vectors are left where those kernels take further steps from. As
+// separate launches the same work is 25 of 4 to 6 us each beside two sweeps.
+template <typename T>
+__global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, long sZ, c64* ball,
+                                                   int spec)
+{
+    const long item = blockIdx.x;
+    const int t = threadIdx.x, grp = t >> 8, ty = (t & 255) >> 4, tx = t & 15;
+    const int m = (int)g.m, n = (int)g.n, N = (int)g.N;
+    const c64* Z = Zall + item * sZ;
+    const c64* Zg = Z + grp * (m * m + m);
+    cx<T>* F = const_cast<cx<T>*>(g.F) + 2 * item * 4096;
+    cx<T>* Fg = F + grp * 4096;
+    cx<T>* S = g.S + item * 4096;
+    c64 *xo = g.x + item * N, *ro = g.r + item * N;
+    __shared__ cx<T> row[2][2][64];
+    __shared__ cx<T> v[2][64], z[2][64], f[64], y[64], h[64], c[64];
+    __shared__ c64 ys[64], dg[64], x[192], r[192], cst[3];
+    __shared__ unsigned long long nrm[4 * 4];
+    if (t < 16) nrm[t] = 0;
+    if (t < 128) v[t >> 6][t & 63] = z[t >> 6][t & 63] = cx<T>{0, 0};
+    if (t < 64) f[t] = y[t] = h[t] = c[t] = cx<T>{0, 0};
+    cx<T> a[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int p = ty + 16 * i, q = tx + 16 * j;
+            a[i][j] = cx<T>{0, 0};
+            if (p < m && q < m) {
+                const c64 s = Zg[max(p, q) * m + min(p, q)];
+                a[i][j] = cx<T>{(T)s.x, (T)s.y};
+            }
+        }
+    nd_sweep64(a, row[grp], m, ty, tx);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int p = ty + 16 * i, q = tx + 16 * j;
+            Fg[p * 64 + q] = p < m && q < m ? a[i][j] : cx<T>{0, 0};
+        }
+    __syncthreads();
+    // four lanes per row of the own block from here on
+    const int rw = (t & 255) >> 2, q4 = t & 3;
+    if (grp == 1) {
+        c64 s{0, 0};
+        for (int k = q4; k < m; k += 4) s = cadd(s, c64{Fg[rw * 64 + k].x, Fg[rw * 64 + k].y});
+        for (int o = 2; o > 0; o >>= 1) s = cadd(s, c64{__shfl_xor(s.x, o), __shfl_xor(s.y, o)});
+        if (q4 == 0) {
+            const cx<T> l = F[rw * 65], u = Fg[rw * 65];
+            ys[rw] = s;
+            dg[rw] = c64{2.0 * l.x + 0.5 * u.x, 2.0 * l.y + 0.5 * u.y};
+        }
+    }
+    __syncthreads();
+    if (t < 64) {
+        const c64 sa = wave_sum(t < m ? ys[t] : c64{0, 0}), sd = wave_sum(t < m ? dg[t] : c64{0, 0});
+        if (t == 0) {
+            const double w = 1.0 / ((double)n * (double)n);
+            cst[0] = c64{sd.x * w, sd.y * w};
+            cst[1] = sa;
+        }
+        if (t < n) {
+            c64 s{0, 0};
+            for (int p = g.node_ptr[t]; p < g.node_ptr[t + 1]; p++) s = cadd(s, ys[g.node_seg[p] >> 1]);
+            c[t] = cx<T>{(T)(0.5 * s.x), (T)(0.5 * s.y)};
+        }
+    }
+    __syncthreads();
+    // -S_p (both halves of the work-group alike)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int u = max(ty + 16 * i, tx + 16 * j), w = min(ty + 16 * i, tx + 16 * j);
+            a[i][j] = cx<T>{0, 0};
+            if (u < n) {
+                c64 s = cst[0];
+                for (int p = g.node_ptr[u]; p < g.node_ptr[u + 1]; p++) {
+                    const int sa = g.node_seg[p];
+                    for (int q = g.node_ptr[w]; q < g.node_ptr[w + 1]; q++) {
+                        const int sb = g.node_seg[q];
+                        const double sg = ((sa ^ sb) & 1) ? -1.0 : 1.0;
+                        const cx<T> l = F[(sa >> 1) * 64 + (sb >> 1)];
+                        const cx<T> d = F[4096 + (sa >> 1) * 64 + (sb >> 1)];
+                        s.x += sg * l.x + 0.25 * d.x;
+                        s.y += sg * l.y + 0.25 * d.y;
+                    }
+                }
+                a[i][j] = cx<T>{(T)-s.x, (T)-s.y};
+            }
+        }
+    nd_sweep64(a, row[grp], n, ty, tx);
+    if (grp == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int p = ty + 16 * i, q = tx + 16 * j;
+                S[p * 64 + q] = p < n && q < n ? a[i][j] : cx<T>{0, 0};
+            }
+    }
+    __syncthreads();
+    // out_row = M in (row rw of a 64 x 64 matrix, four lanes)
+    auto gemv = [&](const cx<T>* M, const cx<T>* in) {
+        cx<T> s{0, 0};
+#pragma unroll 4
+        for (int k = 0; k < 16; k++) {
+            const cx<T> p = M[rw * 64 + 4 * k + q4], q = in[4 * k + q4];
+            s.x = fma(p.x, q.x, fma(-p.y, q.y, s.x));
+            s.y = fma(p.x, q.y, fma(p.y, q.x, s.y));
+        }
+        for (int o = 2; o > 0; o >>= 1) {
+            s.x += __shfl_xor(s.x, o);
+            s.y += __shfl_xor(s.y, o);
+        }
+        return s;
+    };
+    {
+        const cx<T> s = gemv(S, c);
+        if (grp == 0 && q4 == 0) h[rw] = s;
+    }
+    __syncthreads();
+    if (t < 64) {
+        c64 s{0, 0};
+        if (t < n) s = cmul(c64{c[t].x, c[t].y}, c64{h[t].x, h[t].y});
+        s = wave_sum(s);
+        if (t == 0) cst[2] = crecip(csub(cst[1], s));
+    }
+    __syncthreads();
+    for (int k = 1; k <= spec; k++) {
+        const bool first = k == 1;
+        const double scale = first ? 1.0 : nd_scale(&nrm[4 * (k - 1)], sizeof(T) == 4);
+        const double inv = 1.0 / scale;
+        if (first) {
+            if (t < 64) y[t] = S[g.inj * 64 + t];
+        } else {
+            if ((t & 255) < m) {
+                const c64 q = r[grp * m + (t & 255)];
+                v[grp][t & 255] = cx<T>{(T)(q.x * inv), (T)(q.y * inv)};
+            }
+            __syncthreads();
+            const cx<T> s = gemv(Fg, v[grp]);
+            if (q4 == 0) z[grp][rw] = s;
+            __syncthreads();
+            if (t < n) {
+                c64 s{r[2 * m + t].x * inv, r[2 * m + t].y * inv};
+                for (int p = g.node_ptr[t]; p < g.node_ptr[t + 1]; p++) {
+                    const int sa = g.node_seg[p];
+                    const double sg = (sa & 1) ? -1.0 : 1.0;
+                    s.x += sg * z[0][sa >> 1].x + 0.5 * z[1][sa >> 1].x;
+                    s.y += sg * z[0][sa >> 1].y + 0.5 * z[1][sa >> 1].y;
+                }
+                f[t] = cx<T>{(T)s.x, (T)s.y};
+            }
+            __syncthreads();
+            const cx<T> w = gemv(S, f);
+            if (grp == 0 && q4 == 0) y[rw] = w;
+        }
+        __syncthreads();
+        // alpha (every wave alike), w and u
+        c64 al{0, 0};
+        {
+            const int u = t & 63;
+            if (u < n) {
+                al = csub(al, cmul(c64{c[u].x, c[u].y}, c64{y[u].x, y[u].y}));
+                if (!first) al = cadd(al, c64{r[2 * m + u].x / scale, r[2 * m + u].y / scale});
+            }
+            if (!first && u < m) al = cadd(al, c64{z[1][u].x, z[1][u].y});
+            al = wave_sum(al);
+            if (first) al.x += 1.0;
+            al = cmul(al, cst[2]);
+        }
+        __syncthreads();
+        if (t < n) {
+            const c64 w = csub(c64{y[t].x, y[t].y}, cmul(al, c64{h[t].x, h[t].y}));
+            y[t] = cx<T>{(T)w.x, (T)w.y};
+            const c64 d = cscale(cadd(w, al), scale);
+            x[2 * m + t] = first ? d : cadd(x[2 * m + t], d);
+            lds_max(&nrm[4 * k + 3], sqrt(d.x * d.x + d.y * d.y));
+        }
+        __syncthreads();
+        if ((t & 255) < m) {
+            const int i = t & 255;
+            const cx<T> ws = y[g.sn[i]], we = y[g.en[i]];
+            c64 l = grp ? c64{0.5 * ((double)ws.x + we.x) + al.x, 0.5 * ((double)ws.y + we.y) + al.y}
+                        : c64{(double)ws.x - we.x, (double)ws.y - we.y};
+            if (!first) l = csub(l, cscale(r[grp * m + i], inv));
+            v[grp][i] = cx<T>{(T)l.x, (T)l.y};
+        }
+        __syncthreads();
+        {
+            const cx<T> s = gemv(Fg, v[grp]);
+            if (q4 == 0 && rw < m) {
+                const c64 d{s.x * scale, s.y * scale};
+                c64* xi = &x[grp * m + rw];
+                *xi = first ? d : cadd(*xi, d);
+                lds_max(&nrm[4 * k + 3], sqrt(d.x * d.x + d.y * d.y));
+            }
+        }
+        __syncthreads();
+        // r = b - W x, in double-double as k_hem_apply
+        if (rw < m) {
+            DD sx{0, 0}, sy{0, 0};
+            double ta = 0;
+            for (int k4 = q4; k4 < m; k4 += 4) {
+                const c64 p = Zg[rw * m + k4], q = x[grp * m + k4];
+                dd_mac(sx, p.x, q.x);
+                dd_mac(sx, -p.y, q.y);
+                dd_mac(sy, p.x, q.y);
+                dd_mac(sy, p.y, q.x);
+                if (first) ta += sqrt(p.x * p.x + p.y * p.y);
+            }
+            for (int o = 2; o > 0; o >>= 1) {
+                sx = dd_plus(sx, dd_shfl_xor(sx, o));
+                sy = dd_plus(sy, dd_shfl_xor(sy, o));
+                ta += __shfl_xor(ta, o);
+            }
+            if (q4 == 0) {
+                const c64 xs = x[2 * m + g.sn[rw]], xe = x[2 * m + g.en[rw]];
+                const double cs = grp ? 0.5 : 1.0, ce = grp ? 0.5 : -1.0;
+                dd_add(sx, cs * xs.x);
+                dd_add(sy, cs * xs.y);
+                dd_add(sx, ce * xe.x);
+                dd_add(sy, ce * xe.y);
+                const int i = grp * m + rw;
+                const c64 rr{dd_sub_from(0.0, sx), dd_sub_from(0.0, sy)};
+                r[i] = rr;
+                lds_max(&nrm[4 * k], sqrt(rr.x * rr.x + rr.y * rr.y));
+                lds_max(&nrm[4 * k + 1], sqrt(x[i].x * x[i].x + x[i].y * x[i].y));
+                if (first) lds_max(&nrm[4 * k + 2], ta + 2.0 * cs);
+            }
+        }
+        if (t < n) {
+            DD sx{0, 0}, sy{0, 0};
+            double ta = 0;
+            for (int p = g.node_ptr[t]; p < g.node_ptr[t + 1]; p++) {
+                const int sa = g.node_seg[p];
+                const double cl = (sa & 1) ? -1.0 : 1.0;
+                const c64 xl = x[sa >> 1], xt = x[m + (sa >> 1)];
+                dd_add(sx, cl * xl.x);
+                dd_add(sx, 0.5 * xt.x);
+                dd_add(sy, cl * xl.y);
+                dd_add(sy, 0.5 * xt.y);
+                ta += 1.5;
+            }
+            const int i = 2 * m + t;
+            const c64 rr{dd_sub_from(t == g.inj ? 1.0 : 0.0, sx), dd_sub_from(0.0, sy)};
+            r[i] = rr;
+            lds_max(&nrm[4 * k], sqrt(rr.x * rr.x + rr.y * rr.y));
+            lds_max(&nrm[4 * k + 1], sqrt(x[i].x * x[i].x + x[i].y * x[i].y));
+            if (first) lds_max(&nrm[4 * k + 2], ta);
+        }
+        __syncthreads();
+    }
+    // what further steps start from
+    for (int i = t; i < N; i += 512) {
+        xo[i] = x[i];
+        ro[i] = r[i];
+        ball[item * N + i] = c64{i == 2 * m + g.inj ? 1.0 : 0.0, 0.0};
+    }
+    for (int i = t; i < g.snorm; i += 512)
+        g.norms[item * g.snorm + i] = i < 4 * (spec + 1) ? nrm[i] : 0;
+    if (t < 128) g.v[128 * item + t] = v[t >> 6][t & 63];
+    if (t < 64) {
+        g.f[64 * item + t] = f[t];
+        g.h[64 * item + t] = h[t];
+        g.c[64 * item + t] = c[t];
+    }
+    if (t < 3) g.cst[4 * item + t] = cst[t];
+}
+
+// ---------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------
 // Columns per sweep step. A step reads and writes every tile once, which at 64
@@ -1045,15 +1360,22 @@ template <typename T, int NB>
 static int nd_sweep(const NdPhase<T>& p, hipStream_t st, Profiler* pr)
 {
     const long nt = p.ld / 64, ntri = nt * (nt + 1) / 2;
+    if (nt == 1) {
+        Timed tm(pr, FAM_PANEL, st);
+        hipLaunchKernelGGL((k_nd_diag<T, NB>), dim3(p.items), dim3(256), 0, st, p, 0, 0, 1);
+        tm.end();
+        TAGS_HIP(hipGetLastError());
+        return 0;
+    }
     for (int c0 = 0; c0 < p.dim; c0 += NB) {
         const int nq = (int)std::min<long>(NB / 64, nt - c0 / 64);
         {
             Timed tm(pr, FAM_PANEL, st);
             for (int t = 0; t < nq; t++) {
-                hipLaunchKernelGGL((k_nd_diag<T, NB>), dim3(p.items), dim3(256), 0, st, p, c0, t);
-                if (nt > 1)
-                    hipLaunchKernelGGL((k_nd_panel<T, NB>), dim3(xcd_grid(p.items * nt)), dim3(256),
-                                       0, st, p, c0, t);
+                hipLaunchKernelGGL((k_nd_diag<T, NB>), dim3(p.items), dim3(256), 0, st, p, c0, t,
+                                   0);
+                hipLaunchKernelGGL((k_nd_panel<T, NB>), dim3(xcd_grid(p.items * nt)), dim3(256), 0,
+                                   st, p, c0, t);
             }
             tm.end();
         }
@@ -1161,12 +1483,26 @@ int NodalSolver::issue(int nb_, long inj_)
     if (nb_ < 1 || nb_ > cap || inj_ < 0 || inj_ >= n) return TAGS_ERR_ARG;
     nb = nb_;
     inj = inj_;
+    unit_ = true;
+    if (m <= 64 && n <= 64) {
+        step_ = f64 ? kSpec64 : kSpec32;
+        Timed tm(pr, FAM_SOLVE, st);
+        if (f64)
+            hipLaunchKernelGGL(k_nd_small<double>, dim3(nb), dim3(512), 0, st,
+                               nd_args<double>(*this, false), (const c64*)Z, sZ, b, step_);
+        else
+            hipLaunchKernelGGL(k_nd_small<float>, dim3(nb), dim3(512), 0, st,
+                               nd_args<float>(*this, false), (const c64*)Z, sZ, b, step_);
+        TAGS_HIP(hipGetLastError());
+        tm.end();
+        first_ = true;
+        return queue_results();
+    }
     const long w = std::max(std::max(N, 2 * mp), std::max(np, kNormStride));
     const dim3 gi((unsigned)((w + 255) / 256), nb);
     if (f64) hipLaunchKernelGGL(k_nd_init<double>, gi, dim3(256), 0, st, nd_args<double>(*this, false), b);
     else hipLaunchKernelGGL(k_nd_init<float>, gi, dim3(256), 0, st, nd_args<float>(*this, false), b);
     TAGS_HIP(hipGetLastError());
-    unit_ = true;
     return queue_spec();
 }
 
