@@ -43,7 +43,7 @@ struct NodalSolver {
     c64* Z = nullptr;   // impedance blocks, item stride sZ
     long sZ = 0;
     void *F = nullptr, *S = nullptr;    // factored blocks (2 per item), node systems
-    void *tp = nullptr, *op_ = nullptr, *P = nullptr, *xt = nullptr, *xo = nullptr;
+    void *tp = nullptr, *op_ = nullptr, *P = nullptr;
     c64 *x = nullptr, *r = nullptr, *b = nullptr, *ysum = nullptr, *dg = nullptr, *cst = nullptr;
     void *v = nullptr, *z = nullptr, *f = nullptr, *y = nullptr, *h = nullptr, *c = nullptr;
     c64* u = nullptr;

@@ -40,16 +40,8 @@
 #include "dd.h"
 #include "mfma.h"
 #include "nodal.h"
-#include "x6.h"
 
 namespace tags {
-
-// Order from which complex64 inversions take 256-column steps and the bf16 MFMA
-// cores. With 128 columns the split operands (12 bytes per value) and the
-// tile's start and end outweigh the faster products: 48 samples of the 30 x 30
-// m grid (order 1320), per step 615 us on the fp32 cores with 128 columns, 861
-// us on the bf16 cores, 951 us per 256 columns there.
-constexpr long kX6Dim = 4096;
 
 // Work-group index over `total` pieces of work such that each XCD (blockIdx.x
 // mod 8) takes a contiguous range, so that the pieces of one item meet in one
@@ -72,9 +64,7 @@ struct NdPhase {
     int ld, dim, items;
     cx<T>*tp, *op;  // T and O of the current step in MFMA fragment order
     long sp;
-    cx<T>* P;       // inverses of the step's diagonal blocks
-    u32x4 *xt, *xo;  // the same for the split-bf16 update (complex64; null: not used)
-    long sx;
+    cx<T>* P;       // inverses of the step's diagonal blocks, in fragment order
 };
 
 // Fragment order of a ld x NB panel: a wave's MFMA operand (16 rows, 4 k) is
@@ -90,13 +80,54 @@ __device__ inline long nd_pk(int i, int k)
                ((k >> 2) & 1);
 }
 
-// re, im (tiles of a wave) += T_i O_j^T over the k groups [g0, g1) of 16-row
-// strips: operands in fragment order straight from memory, the next group's
-// loads in flight during the current one's MFMAs.
-template <typename T, int NB, int TI, int TJ>
+// Complex MFMA accumulators: complex128 by four real products (re, im),
+// complex64 by three (re re, im im, (re + im)(re + im); Gauss), as the LU's
+// products of each type.
+template <typename T>
+struct NdAcc;
+template <>
+struct NdAcc<double> {
+    typename Mfma<double>::v4 re, im;
+    __device__ void zero() { re = im = typename Mfma<double>::v4{0, 0, 0, 0}; }
+    __device__ void mac(c64 x, c64 y)
+    {
+        re = Mfma<double>::run(x.x, y.x, re);
+        im = Mfma<double>::run(x.x, y.y, im);
+        re = Mfma<double>::run(-x.y, y.y, re);
+        im = Mfma<double>::run(x.y, y.x, im);
+    }
+    __device__ c64 get(int v) const { return c64{re[v], im[v]}; }
+};
+template <>
+struct NdAcc<float> {
+    typename Mfma<float>::v4 rr, ii, ss;
+    __device__ void zero() { rr = ii = ss = typename Mfma<float>::v4{0, 0, 0, 0}; }
+    __device__ void mac(c32 x, c32 y)
+    {
+        rr = Mfma<float>::run(x.x, y.x, rr);
+        ii = Mfma<float>::run(x.y, y.y, ii);
+        ss = Mfma<float>::run(x.x + x.y, y.x + y.y, ss);
+    }
+    __device__ c32 get(int v) const { return c32{rr[v] - ii[v], ss[v] - rr[v] - ii[v]}; }
+};
+
+// The value is needed here: keeps the loads of the next k group ahead of this
+// one's products (the compiler otherwise moves them to their use, one iteration
+// later, and every wave waits out each load).
+template <typename T, int N>
+__device__ __forceinline__ void nd_pin(cx<T> (&e)[N])
+{
+#pragma unroll
+    for (int i = 0; i < N; i++) asm volatile("" : "+v"(e[i].x), "+v"(e[i].y));
+}
+
+// acc (tiles of a wave) += T_i O_j^T over the k groups [g0, g1) of 16-row
+// strips: operands in fragment order straight from memory, the loads of the next
+// D - 1 groups in flight during one group's MFMAs. Two hide the latency where
+// several waves share a SIMD; the diagonal block's product has one wave on each.
+template <typename T, int NB, int TI, int TJ, int D = 2>
 __device__ __forceinline__ void nd_mma(const cx<T>* tp, const cx<T>* op, int i0, int j0, int g0,
-                                       int g1, typename Mfma<T>::v4 (&re)[TI][TJ],
-                                       typename Mfma<T>::v4 (&im)[TI][TJ])
+                                       int g1, NdAcc<T> (&acc)[TI][TJ])
 {
     constexpr int KG = sizeof(T) == 8 ? 4 : 8;  // k per 16-byte lane load
     constexpr int KU = KG / 4;
@@ -108,34 +139,38 @@ __device__ __forceinline__ void nd_mma(const cx<T>* tp, const cx<T>* op, int i0,
     const Frag* ta = (const Frag*)tp + (i0 / 16) * FS + lane;
     const Frag* ob = (const Frag*)op + (j0 / 16) * FS + lane;
     if (g0 >= g1) return;
-    Frag a[TI], b[TJ], an[TI], bn[TJ];
+    Frag a[D][TI], b[D][TJ];
+    auto load = [&](int d, int g) {
+        const long o = (long)min(g, g1 - 1) * 64;
 #pragma unroll
-    for (int i = 0; i < TI; i++) a[i] = ta[i * FS + (long)g0 * 64];
+        for (int i = 0; i < TI; i++) a[d][i] = ta[i * FS + o];
 #pragma unroll
-    for (int j = 0; j < TJ; j++) b[j] = ob[j * FS + (long)g0 * 64];
-    for (int g = g0; g < g1; g++) {
-        const long o = (long)min(g + 1, g1 - 1) * 64;
+        for (int j = 0; j < TJ; j++) b[d][j] = ob[j * FS + o];
+        // otherwise the compiler moves the loads to their use, past the products
+        // they are to run beside
+        __builtin_amdgcn_sched_barrier(0);
+    };
 #pragma unroll
-        for (int i = 0; i < TI; i++) an[i] = ta[i * FS + o];
-#pragma unroll
-        for (int j = 0; j < TJ; j++) bn[j] = ob[j * FS + o];
+    for (int d = 0; d < D; d++) load(d, g0 + d);
+    auto mac = [&](int d) {
 #pragma unroll
         for (int u = 0; u < KU; u++)
 #pragma unroll
             for (int i = 0; i < TI; i++)
 #pragma unroll
-                for (int j = 0; j < TJ; j++) {
-                    const cx<T> x = a[i].e[u], y = b[j].e[u];
-                    re[i][j] = Mfma<T>::run(x.x, y.x, re[i][j]);
-                    im[i][j] = Mfma<T>::run(x.x, y.y, im[i][j]);
-                    re[i][j] = Mfma<T>::run(-x.y, y.y, re[i][j]);
-                    im[i][j] = Mfma<T>::run(x.y, y.x, im[i][j]);
-                }
+                for (int j = 0; j < TJ; j++) acc[i][j].mac(a[d][i].e[u], b[d][j].e[u]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int g = g0;
+    for (; g + D <= g1; g += D)
 #pragma unroll
-        for (int i = 0; i < TI; i++) a[i] = an[i];
+        for (int d = 0; d < D; d++) {
+            mac(d);
+            load(d, g + d + D);
+        }
 #pragma unroll
-        for (int j = 0; j < TJ; j++) b[j] = bn[j];
-    }
+    for (int d = 0; d + 1 < D; d++)
+        if (g + d < g1) mac(d);
 }
 template <typename T>
 constexpr int nd_groups(int k)  // k groups of nd_mma in k columns
@@ -162,59 +197,117 @@ constexpr int nd_groups(int k)  // k groups of nd_mma in k columns
 //   (-P_q if s = r, else T_q of the other side) - sum_{u > q} T_u(i) O_u(j)^T.
 // ---------------------------------------------------------------------------
 
+// LDS of nd_sweep64
+template <typename T>
+struct NdSweep {
+    cx<T> row[2][2][64];  // two pivot rows, of this step and of the next
+    cx<T> piv[2][3];      // their 2 x 2 block
+};
+
 // The unblocked sweep of a 64 x 64 matrix in the registers of 256 threads (ty,
 // tx: rows ty + 16 i, columns tx + 16 j): a = -a^-1 over its first kv rows and
-// columns. Per pivot k the pivot row goes through LDS (it is the pivot column
-// too); with the pivot row's and column's own entries cleared, the multiplier
-// of row k set to -1/p and the entry of column k to -1, one multiply-add serves
-// every entry. Row k + 1 is formed and stored before the barrier, so that the
-// rest of step k runs beside the next pivot's read and reciprocal: latency per
-// pivot, not the 16 multiply-adds per thread, bounds it (64 pivots in complex128:
-// 50 us with the update before the next row).
+// columns, two pivots at a time (the inverse I of the symmetric 2 x 2 block in
+// closed form; past kv the matrix is taken as the identity). The pivot rows go
+// through LDS (they are the pivot columns too) with minus the identity in place
+// of the block, which is kept apart: then a -= (o I) o^T over both rows serves
+// every entry, once the pivot rows and columns themselves are cleared. The next
+// two rows are formed and stored before the barrier, so that the rest of a step
+// runs beside the next one's reads and reciprocal. Bound by the issue of one
+// wave per SIMD (about 300 instructions a step, 128 of them the update's
+// multiply-adds), so nothing is selected per entry that a branch or the stored
+// row can settle. 64 pivots in complex128: see k_nd_diag. All threads of the
+// work-group have to call this; those of `idle` only meet the barriers.
 template <typename T>
-__device__ __forceinline__ void nd_sweep64(cx<T> (&a)[4][4], cx<T> (*row)[64], int kv, int ty,
-                                           int tx)
+__device__ __forceinline__ void nd_sweep64(cx<T> (&a)[4][4], NdSweep<T>& sh, int kv, int ty, int tx,
+                                           bool idle = false)
 {
-    if (ty == 0) {
+    const cx<T> zero{0, 0};
+    // pivot rows n0, n0 + 1 (of 16 from 16 nb on), given as w[]
+    auto store = [&](int buf, int n0, int nb, const cx<T>(&w)[4]) {
+        const int h = ty - n0;
 #pragma unroll
-        for (int j = 0; j < 4; j++) row[0][tx + 16 * j] = a[0][j];
+        for (int j = 0; j < 4; j++) {
+            cx<T> x = w[j];
+            if (j == nb && (tx == n0 || tx == n0 + 1)) {
+                if (tx - n0 >= h) sh.piv[buf][h + tx - n0] = x;
+                x = cx<T>{tx == ty ? (T)-1 : (T)0, 0};
+            }
+            sh.row[buf][h][tx + 16 * j] = x;
+        }
+    };
+    if (!idle) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (ty == tx && ty + 16 * i >= kv) a[i][i] = cx<T>{1, 0};
+        if (ty < 2) {
+            store(0, 0, 0, a[0]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) a[0][j] = zero;
+        }
+        if (tx < 2) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) a[i][0] = zero;
+        }
     }
     __syncthreads();
-#pragma unroll
-    for (int kb = 0; kb < 4; kb++)
-        for (int kl = 0; kl < 16; kl++) {
-            const int k = 16 * kb + kl;
-            if (k >= kv) return;
-            const cx<T>* rk = row[k & 1];
-            const cx<T> d = crecip_fast(rk[k]);
-            cx<T> o[4], l[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) o[j] = rk[tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; i++) l[i] = cmul(rk[ty + 16 * i], d);
-            const bool pr = ty == kl, pc = tx == kl;
-            const cx<T> zero{0, 0};
-            l[kb] = csel(pr, cx<T>{-d.x, -d.y}, l[kb]);
-            o[kb] = csel(pc, cx<T>{-1, 0}, o[kb]);
+    // pivots k, k + 1; the next ones are rows n0, n0 + 1 of 16 from 16 nb on
+    auto step = [&](int k, int n0, auto nbc) {
+        constexpr int nb = decltype(nbc)::value;
+        const int buf = (k >> 1) & 1;
+        cx<T> o0[4], o1[4], l0[4], l1[4];
+        if (!idle) {
+            const cx<T> p = sh.piv[buf][0], q = sh.piv[buf][1], s = sh.piv[buf][2];
+            const cx<T> d = crecip_fast(cfnma(cmul(p, s), q, q));
+            const cx<T> i00 = cmul(s, d), i11 = cmul(p, d), t = cmul(q, d);
+            const cx<T>(*r)[64] = sh.row[buf];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                a[kb][j] = csel(pr, zero, a[kb][j]);
-                a[j][kb] = csel(pc, zero, a[j][kb]);
+                o0[j] = r[0][tx + 16 * j];
+                o1[j] = r[1][tx + 16 * j];
             }
-            if (k + 1 < kv && ty == ((kl + 1) & 15)) {
-                const int nx = kb < 3 ? kb + 1 : kb;
-                const cx<T> ln = csel(kl < 15, l[kb], l[nx]);
 #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    row[(k + 1) & 1][tx + 16 * j] =
-                        cfnma(csel(kl < 15, a[kb][j], a[nx][j]), ln, o[j]);
+            for (int i = 0; i < 4; i++) {
+                const cx<T> u = r[0][ty + 16 * i], v = r[1][ty + 16 * i];
+                l0[i] = cfnma(cmul(u, i00), v, t);
+                l1[i] = cfnma(cmul(v, i11), u, t);
             }
-            __syncthreads();
+            if (k + 2 < kv) {
+                if (ty == n0 || ty == n0 + 1) {
+                    cx<T> w[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+                    for (int j = 0; j < 4; j++) {
+                        w[j] = cfnma(cfnma(a[nb][j], l0[nb], o0[j]), l1[nb], o1[j]);
+                        a[nb][j] = zero;
+                    }
+                    store(buf ^ 1, n0, nb, w);
+                    l0[nb] = l1[nb] = zero;
+                }
+                if (tx == n0 || tx == n0 + 1) {
 #pragma unroll
-                for (int j = 0; j < 4; j++) a[i][j] = cfnma(a[i][j], l[i], o[j]);
+                    for (int i = 0; i < 4; i++) a[i][nb] = zero;
+                    o0[nb] = o1[nb] = zero;
+                }
+            }
         }
+        __syncthreads();
+        if (idle) return;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                a[i][j] = cfnma(cfnma(a[i][j], l0[i], o0[j]), l1[i], o1[j]);
+    };
+    auto block = [&](auto kbc) {
+        constexpr int kb = decltype(kbc)::value, nx = kb < 3 ? kb + 1 : kb;
+        const int end = min(kv - 16 * kb, 14);
+        for (int kl = 0; kl < end; kl += 2)
+            step(16 * kb + kl, kl + 2, std::integral_constant<int, kb>{});
+        if (16 * kb + 14 < kv) step(16 * kb + 14, 0, std::integral_constant<int, nx>{});
+    };
+    block(std::integral_constant<int, 0>{});
+    block(std::integral_constant<int, 1>{});
+    block(std::integral_constant<int, 2>{});
+    block(std::integral_constant<int, 3>{});
 }
 
 // P_t, one work-group per item. A matrix of one block (whole) is finished here:
@@ -223,13 +316,12 @@ template <typename T, int NB>
 __global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t,
                                                   int whole)
 {
-    using V4 = typename Mfma<T>::v4;
     const long item = blockIdx.x;
     const cx<T>* A = p.A + item * p.sA;
     cx<T>* P = p.P + (item * (NB / 64) + t) * 4096;
     const int cK = c0 + 64 * t, kv = min(64, p.dim - cK);
     const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-    __shared__ cx<T> row[2][64];
+    __shared__ NdSweep<T> sh;
     cx<T> a[4][4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
@@ -245,16 +337,13 @@ __global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t,
             __shared__ cx<T> up[64][65];
             const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
             const int i0 = (wave >> 1) * 32, j0 = (wave & 1) * 32;
-            V4 re[2][2], im[2][2];
+            NdAcc<T> acc[2][2];
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    re[i][j] = V4{0, 0, 0, 0};
-                    im[i][j] = V4{0, 0, 0, 0};
-                }
-            nd_mma<T, NB, 2, 2>(p.tp + item * p.sp, p.op + item * p.sp, cK + i0, cK + j0, 0,
-                                nd_groups<T>(64 * t), re, im);
+                for (int j = 0; j < 2; j++) acc[i][j].zero();
+            nd_mma<T, NB, 2, 2, 4>(p.tp + item * p.sp, p.op + item * p.sp, cK + i0, cK + j0, 0,
+                                nd_groups<T>(64 * t), acc);
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -262,7 +351,7 @@ __global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t,
 #pragma unroll
                     for (int v = 0; v < 4; v++)
                         up[i0 + 16 * i + Mfma<T>::row(lane, v)][j0 + 16 * j + (lane & 15)] =
-                            cx<T>{re[i][j][v], im[i][j][v]};
+                            acc[i][j].get(v);
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -273,7 +362,7 @@ __global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t,
                 }
         }
     }
-    nd_sweep64(a, row, kv, ty, tx);
+    nd_sweep64(a, sh, kv, ty, tx);
     cx<T>* own = p.A + item * p.sA;
 #pragma unroll
     for (int i = 0; i < 4; i++)
@@ -284,7 +373,7 @@ __global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t,
             if (whole) {
                 own[(long)r * p.ld + c] = in ? a[i][j] : cx<T>{0, 0};
             } else {
-                P[r * 64 + c] = in ? cx<T>{-a[i][j].x, -a[i][j].y} : cx<T>{0, 0};
+                P[nd_pk<T, 64>(c, r)] = in ? cx<T>{-a[i][j].x, -a[i][j].y} : cx<T>{0, 0};
             }
         }
 }
@@ -295,7 +384,12 @@ __global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t,
 template <typename T, int NB>
 __global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int c0, int t)
 {
-    using V4 = typename Mfma<T>::v4;
+    constexpr int KG = sizeof(T) == 8 ? 4 : 8, KU = KG / 4;  // as in nd_mma
+    constexpr long FS = (long)(NB / KG) * 64;
+    constexpr int GP = 64 / KG;  // k groups of one block
+    struct alignas(16) Frag {
+        cx<T> e[KU];
+    };
     const int nt = p.ld / 64;
     const long flat = xcd_flat((long)p.items * nt);
     if (flat < 0) return;
@@ -307,93 +401,105 @@ __global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int c0, int t)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane & 15, lk = lane >> 4;
     const int i0 = rb * 64 + wave * 16;
-    const bool before = s < 0;
+    if (i0 >= p.dim) return;
     const int kv = min(64, p.dim - cK);
     const cx<T>* A = p.A + (long)item * p.sA;
-    const cx<T>* P = p.P + ((long)item * (NB / 64) + t) * 4096;
     cx<T>* tp = p.tp + (long)item * p.sp;
     cx<T>* op = p.op + (long)item * p.sp;
-    __shared__ cx<T> tile[64][65];
-    const bool live = i0 < p.dim;
-    V4 re[1][4], im[1][4];
-    if (live) {
+    const Frag* P = (const Frag*)(p.P + ((long)item * (NB / 64) + t) * 4096) + lane;
+    __shared__ cx<T> tile[4][16][65];  // each wave's own
+    cx<T>(*my)[65] = tile[wave];
+    cx<T> o[4][4];
+    // O_t(i): rows before the step are read from the transposed tiles, with the
+    // product transposed alike, so that the lanes of a load are neighbours
+    auto block = [&](auto& acc, auto at, bool tr) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            re[0][c] = V4{0, 0, 0, 0};
-            im[0][c] = V4{0, 0, 0, 0};
-        }
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = Mfma<T>::row(lane, v);
+                const int i = tr ? lr : r, k = 16 * c + (tr ? r : lr);
+                my[i][k] = k < kv ? csub(o[c][v], at(acc, c).get(v)) : cx<T>{0, 0};
+            }
+    };
+    if (s < 0) {
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int k = 16 * c + Mfma<T>::row(lane, v);
+                o[c][v] = k < kv ? A[(long)(cK + k) * p.ld + i0 + lr] : cx<T>{0, 0};
+            }
+        NdAcc<T> acc[4][1];
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[c][0].zero();
         if (NB > 64 && t > 0)
-            nd_mma<T, NB, 1, 4>(tp, op, i0, cK, nd_groups<T>(swept ? 64 * (own + 1) : 0),
-                                nd_groups<T>(64 * t), re, im);
+            nd_mma<T, NB, 4, 1>(op, tp, cK, i0, 0, nd_groups<T>(64 * t), acc);
+        block(acc, [](auto& a, int c) { return a[c][0]; }, true);
+    } else {
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int i = i0 + Mfma<T>::row(lane, v), k = 16 * c + lr;
-                cx<T> o{0, 0};
-                if (k < kv) {
-                    o = swept ? tp[nd_pk<T, NB>(cK + k, i - c0)]
-                              : A[before ? (long)(cK + k) * p.ld + i : (long)i * p.ld + cK + k];
-                    o = cx<T>{o.x - re[0][c][v], o.y - im[0][c][v]};
-                }
-                tile[wave * 16 + Mfma<T>::row(lane, v)][k] = o;
+                o[c][v] = k >= kv ? cx<T>{0, 0}
+                          : swept ? tp[nd_pk<T, NB>(cK + k, i - c0)]
+                                  : A[(long)i * p.ld + cK + k];
             }
+        NdAcc<T> acc[1][4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[0][c].zero();
+        if (NB > 64 && t > 0)
+            nd_mma<T, NB, 1, 4>(tp, op, i0, cK, nd_groups<T>(swept ? 64 * (own + 1) : 0),
+                                nd_groups<T>(64 * t), acc);
+        block(acc, [](auto& a, int c) { return a[0][c]; }, false);
+    }
+    // T_t(i) = O_t(i) P_t; both stored a fragment at a time
+    auto sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    Frag* oo = (Frag*)op + (i0 / 16) * FS + (long)t * GP * 64 + lane;
+    Frag* to = (Frag*)tp + (i0 / 16) * FS + (long)t * GP * 64 + lane;
+    Frag b[4], bn[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) b[c] = P[c * GP * 64];
+    NdAcc<T> acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c].zero();
+    sync();
+    for (int g = 0; g < GP; g++) {
+        const int gn = min(g + 1, GP - 1);
+#pragma unroll
+        for (int c = 0; c < 4; c++) bn[c] = P[(c * GP + gn) * 64];
+        Frag a;
+#pragma unroll
+        for (int u = 0; u < KU; u++) a.e[u] = my[lr][KG * g + 4 * u + lk];
+        oo[g * 64] = a;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < KU; u++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc[c].mac(a.e[u], b[c].e[u]);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            re[0][c] = V4{0, 0, 0, 0};
-            im[0][c] = V4{0, 0, 0, 0};
+            nd_pin(bn[c].e);
+            b[c] = bn[c];
         }
     }
-    __syncthreads();
-    if (live) {
-#pragma unroll 4
-        for (int g = 0; g < 16; g++) {
-            const int k = 4 * g + lk;
-            const cx<T> a = tile[wave * 16 + lr][k];
-            op[nd_pk<T, NB>(i0 + lr, 64 * t + k)] = a;
-            const T na = -a.y;
+    sync();
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const cx<T> b = P[k * 64 + 16 * c + lr];
-                re[0][c] = Mfma<T>::run(a.x, b.x, re[0][c]);
-                im[0][c] = Mfma<T>::run(a.x, b.y, im[0][c]);
-                re[0][c] = Mfma<T>::run(na, b.y, re[0][c]);
-                im[0][c] = Mfma<T>::run(a.y, b.x, im[0][c]);
-            }
-        }
+    for (int c = 0; c < 4; c++)
 #pragma unroll
-        for (int c = 0; c < 4; c++)
+        for (int v = 0; v < 4; v++) my[Mfma<T>::row(lane, v)][16 * c + lr] = acc[c].get(v);
+    sync();
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                tp[nd_pk<T, NB>(i0 + Mfma<T>::row(lane, v), 64 * t + 16 * c + lr)] =
-                    cx<T>{re[0][c][v], im[0][c][v]};
-    }
-    if constexpr (sizeof(T) == 4) {
-        if (!p.xt) return;
-        // the same, split into bf16 parts (rows past dim: zero)
-        auto pack = [&](u32x4* out) {
-            for (int e = threadIdx.x; e < 512; e += 256) {
-                const int r = e & 63, k8 = e >> 6;  // 8 columns from 8 k8
-                c32 x[8];
+    for (int g = 0; g < GP; g++) {
+        Frag a;
 #pragma unroll
-                for (int q = 0; q < 8; q++)
-                    x[q] = rb * 64 + r < p.dim ? tile[r][8 * k8 + q] : c32{0, 0};
-                x6_pack8(x, out + (long)item * p.sx +
-                                x6_word(rb * 64 + r, 64 * t + 8 * k8, NB / 16));
-            }
-        };
-        pack(p.xo);
-        __syncthreads();
-        if (live) {
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    tile[wave * 16 + Mfma<T>::row(lane, v)][16 * c + lr] =
-                        cx<T>{re[0][c][v], im[0][c][v]};
-        }
-        __syncthreads();
-        pack(p.xt);
+        for (int u = 0; u < KU; u++) a.e[u] = my[lr][KG * g + 4 * u + lk];
+        to[g * 64] = a;
     }
 }
 
@@ -408,31 +514,21 @@ __device__ inline void tri_tile(int t, int& ti, int& tj)
 
 // 64 x 64 tiles of the update: four waves of 32 x 32, operands in fragment
 // order straight from L2 (a wave needs 4 bytes per cycle of them beside its
-// MFMAs, so LDS staging would only add barriers). placed: only the tiles of the
-// step's own blocks (the others are k_nd_update_x6's).
+// MFMAs, so LDS staging would only add barriers). At order 7440 and 256 columns
+// 114 TFLOP/s of fp32 products (154 reached by large matrix products); waves of
+// 32 x 64 and 64 x 64, of which fewer fit, take 1.3 and 1.9 times as long, tiles
+// in 8 x 8 groups for L2 as long, and the bf16 cores (six products of split
+// parts for each of four real ones) twice as long.
 template <typename T, int NB>
-__global__ __launch_bounds__(256) void k_nd_update(NdPhase<T> p, int c0, int placed)
+__global__ __launch_bounds__(256) void k_nd_update(NdPhase<T> p, int c0)
 {
-    using V4 = typename Mfma<T>::v4;
     const int nt = p.ld / 64, k0 = c0 / 64, nq = min(NB / 64, nt - k0);
-    int item, ti, tj;
-    if (placed) {
-        // nt tiles per block: row block K_s (columns up to it), then the rows below
-        const long flat = xcd_flat((long)p.items * nq * nt);
-        if (flat < 0) return;
-        item = (int)(flat / (nq * nt));
-        const int r = (int)(flat % (nq * nt)), s = k0 + r / nt, o = r % nt;
-        ti = max(s, o);
-        tj = min(s, o);
-        // a tile of two of the step's blocks is its row block's
-        if (o > s && o < k0 + nq) return;
-    } else {
-        const int ntri = nt * (nt + 1) / 2;
-        const long flat = xcd_flat((long)p.items * ntri);
-        if (flat < 0) return;
-        item = (int)(flat / ntri);
-        tri_tile((int)(flat % ntri), ti, tj);
-    }
+    const int ntri = nt * (nt + 1) / 2;
+    const long flat = xcd_flat((long)p.items * ntri);
+    if (flat < 0) return;
+    const int item = (int)(flat / ntri);
+    int ti, tj;
+    tri_tile((int)(flat % ntri), ti, tj);
     const int si = ti >= k0 && ti < k0 + nq ? ti - k0 : -1;
     const int sj = tj >= k0 && tj < k0 + nq ? tj - k0 : -1;
     const int q = max(si, sj);
@@ -442,16 +538,13 @@ __global__ __launch_bounds__(256) void k_nd_update(NdPhase<T> p, int c0, int pla
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i0 = ti * 64 + (wave >> 1) * 32, j0 = tj * 64 + (wave & 1) * 32;
     if (i0 >= p.dim || j0 >= p.dim || j0 > i0 + 31) return;
-    V4 re[2][2], im[2][2];
+    NdAcc<T> acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            re[i][j] = V4{0, 0, 0, 0};
-            im[i][j] = V4{0, 0, 0, 0};
-        }
+        for (int j = 0; j < 2; j++) acc[i][j].zero();
     const int kt = (min(NB, p.dim - c0) + 7) & ~7;
-    nd_mma<T, NB, 2, 2>(tp, op, i0, j0, nd_groups<T>(64 * (q + 1)), nd_groups<T>(kt), re, im);
+    nd_mma<T, NB, 2, 2>(tp, op, i0, j0, nd_groups<T>(64 * (q + 1)), nd_groups<T>(kt), acc);
     const cx<T>* P = q < 0 ? nullptr : p.P + ((long)item * (NB / 64) + q) * 4096;
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -468,45 +561,14 @@ __global__ __launch_bounds__(256) void k_nd_update(NdPhase<T> p, int c0, int pla
                 if (q < 0) {
                     o = *a;
                 } else if (si == sj) {
-                    o = P[(r - ti * 64) * 64 + c - tj * 64];
+                    o = P[nd_pk<T, 64>(c - tj * 64, r - ti * 64)];
                     o = cx<T>{-o.x, -o.y};
                 } else {
                     o = si > sj ? tp[nd_pk<T, NB>(c, r - c0)] : tp[nd_pk<T, NB>(r, c - c0)];
                 }
-                *a = cx<T>{o.x - re[i][j][v], o.y - im[i][j][v]};
+                *a = csub(o, acc[i][j].get(v));
             }
         }
-}
-
-// The update's other tiles in complex64 on the bf16 MFMA cores (see x6.h):
-// 128 x 64 tiles of four waves. dim > NB.
-template <int NB>
-__global__ __launch_bounds__(256, 1) void k_nd_update_x6(NdPhase<float> p, int c0)
-{
-    // tiles on and below the diagonal: row tile I has 2 I + 2 column tiles
-    const int nm = (p.ld + 127) / 128, nn = p.ld / 64;
-    const int per = nm * (nm + 1);
-    const long flat = xcd_flat((long)p.items * per);
-    if (flat < 0) return;
-    const int item = (int)(flat / per);
-    int I, J;
-    tri_tile((int)(flat % per) / 2, I, J);
-    J = 2 * J + ((int)(flat % per) & 1);
-    if (J >= nn) return;
-    const int r0 = I * 128, q0 = J * 64;
-    if ((r0 >= c0 && r0 < c0 + NB) || (q0 >= c0 && q0 < c0 + NB)) return;
-    if (r0 >= p.dim || q0 >= p.dim) return;
-    X6Args g;
-    g.M = g.N = p.dim;
-    g.K = min(NB, p.dim - c0);
-    g.ks = NB / 16;
-    g.pa = p.xt + (long)item * p.sx;
-    g.pb = p.xo + (long)item * p.sx;
-    g.C = p.A + (long)item * p.sA;
-    g.ldc = p.ld;
-    g.crow = nullptr;
-    g.mode = 1;
-    x6l_tile<4, 1, 1, 2, false, 2>(g, I, J);
 }
 
 // A_ij of the tiles above the diagonal from those below, 64 x 64 tiles through
@@ -916,9 +978,10 @@ __global__ __launch_bounds__(256) void k_nd_pick(NdArgs<T> g, c64* u)
 // ---------------------------------------------------------------------------
 // Small systems (at most 64 segments and 64 nodes) in one launch
 // ---------------------------------------------------------------------------
-__device__ inline void lds_max(unsigned long long* p, double a)
+// the larger of two values >= 0 as bits (a NaN is larger than all)
+__device__ inline void bits_max(unsigned long long& m, double a)
 {
-    atomicMax(p, (unsigned long long)__double_as_longlong(a));
+    m = max(m, (unsigned long long)__double_as_longlong(a));
 }
 
 // Everything of a sample after the fill: both inverses (256 threads each), the
@@ -939,11 +1002,20 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
     cx<T>* Fg = F + grp * 4096;
     cx<T>* S = g.S + item * 4096;
     c64 *xo = g.x + item * N, *ro = g.r + item * N;
-    __shared__ cx<T> row[2][2][64];
+    __shared__ NdSweep<T> sh[2];
     __shared__ cx<T> v[2][64], z[2][64], f[64], y[64], h[64], c[64];
     __shared__ c64 ys[64], dg[64], x[192], r[192], cst[3];
     __shared__ unsigned long long nrm[4 * 4];
+    // the incidence lists, read many times by one lane after another
+    __shared__ int nptr[65], nseg[128], end0[64], end1[64];
+    if (t <= n) nptr[t] = g.node_ptr[t];
+    if (t < 2 * m) nseg[t] = g.node_seg[t];
+    if (t < m) {
+        end0[t] = g.sn[t];
+        end1[t] = g.en[t];
+    }
     if (t < 16) nrm[t] = 0;
+    if (t < 192) x[t] = c64{0, 0};
     if (t < 128) v[t >> 6][t & 63] = z[t >> 6][t & 63] = cx<T>{0, 0};
     if (t < 64) f[t] = y[t] = h[t] = c[t] = cx<T>{0, 0};
     cx<T> a[4][4];
@@ -958,7 +1030,7 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
                 a[i][j] = cx<T>{(T)s.x, (T)s.y};
             }
         }
-    nd_sweep64(a, row[grp], m, ty, tx);
+    nd_sweep64(a, sh[grp], m, ty, tx);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -971,7 +1043,8 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
     const int rw = (t & 255) >> 2, q4 = t & 3;
     if (grp == 1) {
         c64 s{0, 0};
-        for (int k = q4; k < m; k += 4) s = cadd(s, c64{Fg[rw * 64 + k].x, Fg[rw * 64 + k].y});
+#pragma unroll 4
+        for (int k = q4; k < 64; k += 4) s = cadd(s, c64{Fg[rw * 64 + k].x, Fg[rw * 64 + k].y});
         for (int o = 2; o > 0; o >>= 1) s = cadd(s, c64{__shfl_xor(s.x, o), __shfl_xor(s.y, o)});
         if (q4 == 0) {
             const cx<T> l = F[rw * 65], u = Fg[rw * 65];
@@ -989,24 +1062,24 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
         }
         if (t < n) {
             c64 s{0, 0};
-            for (int p = g.node_ptr[t]; p < g.node_ptr[t + 1]; p++) s = cadd(s, ys[g.node_seg[p] >> 1]);
+            for (int p = nptr[t]; p < nptr[t + 1]; p++) s = cadd(s, ys[nseg[p] >> 1]);
             c[t] = cx<T>{(T)(0.5 * s.x), (T)(0.5 * s.y)};
         }
     }
     __syncthreads();
-    // -S_p (both halves of the work-group alike)
+    // -S_p
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int u = max(ty + 16 * i, tx + 16 * j), w = min(ty + 16 * i, tx + 16 * j);
             a[i][j] = cx<T>{0, 0};
-            if (u < n) {
+            if (grp == 0 && u < n) {
                 c64 s = cst[0];
-                for (int p = g.node_ptr[u]; p < g.node_ptr[u + 1]; p++) {
-                    const int sa = g.node_seg[p];
-                    for (int q = g.node_ptr[w]; q < g.node_ptr[w + 1]; q++) {
-                        const int sb = g.node_seg[q];
+                for (int p = nptr[u]; p < nptr[u + 1]; p++) {
+                    const int sa = nseg[p];
+                    for (int q = nptr[w]; q < nptr[w + 1]; q++) {
+                        const int sb = nseg[q];
                         const double sg = ((sa ^ sb) & 1) ? -1.0 : 1.0;
                         const cx<T> l = F[(sa >> 1) * 64 + (sb >> 1)];
                         const cx<T> d = F[4096 + (sa >> 1) * 64 + (sb >> 1)];
@@ -1017,7 +1090,7 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
                 a[i][j] = cx<T>{(T)-s.x, (T)-s.y};
             }
         }
-    nd_sweep64(a, row[grp], n, ty, tx);
+    nd_sweep64(a, sh[grp], n, ty, tx, grp == 1);
     if (grp == 0) {
 #pragma unroll
         for (int i = 0; i < 4; i++)
@@ -1028,12 +1101,21 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
             }
     }
     __syncthreads();
-    // out_row = M in (row rw of a 64 x 64 matrix, four lanes)
-    auto gemv = [&](const cx<T>* M, const cx<T>* in) {
+    // the four lanes' parts of row rw of the inverse and of the matrix (zero beyond
+    // m; x is finite there)
+    cx<T> fr[16];
+    c64 zr[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        const int c = 4 * k + q4;
+        fr[k] = Fg[rw * 64 + c];
+        zr[k] = rw < m && c < m ? Zg[rw * m + c] : c64{0, 0};
+    }
+    auto gemv = [&](auto row, const cx<T>* in) {
         cx<T> s{0, 0};
-#pragma unroll 4
+#pragma unroll
         for (int k = 0; k < 16; k++) {
-            const cx<T> p = M[rw * 64 + 4 * k + q4], q = in[4 * k + q4];
+            const cx<T> p = row(k), q = in[4 * k + q4];
             s.x = fma(p.x, q.x, fma(-p.y, q.y, s.x));
             s.y = fma(p.x, q.y, fma(p.y, q.x, s.y));
         }
@@ -1043,8 +1125,10 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
         }
         return s;
     };
+    auto frow = [&](int k) { return fr[k]; };
+    auto srow = [&](int k) { return S[rw * 64 + 4 * k + q4]; };
     {
-        const cx<T> s = gemv(S, c);
+        const cx<T> s = gemv(srow, c);
         if (grp == 0 && q4 == 0) h[rw] = s;
     }
     __syncthreads();
@@ -1059,6 +1143,7 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
         const bool first = k == 1;
         const double scale = first ? 1.0 : nd_scale(&nrm[4 * (k - 1)], sizeof(T) == 4);
         const double inv = 1.0 / scale;
+        unsigned long long nr = 0, nx = 0, na = 0, nd = 0;  // maxima of this thread
         if (first) {
             if (t < 64) y[t] = S[g.inj * 64 + t];
         } else {
@@ -1067,13 +1152,13 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
                 v[grp][t & 255] = cx<T>{(T)(q.x * inv), (T)(q.y * inv)};
             }
             __syncthreads();
-            const cx<T> s = gemv(Fg, v[grp]);
+            const cx<T> s = gemv(frow, v[grp]);
             if (q4 == 0) z[grp][rw] = s;
             __syncthreads();
             if (t < n) {
                 c64 s{r[2 * m + t].x * inv, r[2 * m + t].y * inv};
-                for (int p = g.node_ptr[t]; p < g.node_ptr[t + 1]; p++) {
-                    const int sa = g.node_seg[p];
+                for (int p = nptr[t]; p < nptr[t + 1]; p++) {
+                    const int sa = nseg[p];
                     const double sg = (sa & 1) ? -1.0 : 1.0;
                     s.x += sg * z[0][sa >> 1].x + 0.5 * z[1][sa >> 1].x;
                     s.y += sg * z[0][sa >> 1].y + 0.5 * z[1][sa >> 1].y;
@@ -1081,7 +1166,7 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
                 f[t] = cx<T>{(T)s.x, (T)s.y};
             }
             __syncthreads();
-            const cx<T> w = gemv(S, f);
+            const cx<T> w = gemv(srow, f);
             if (grp == 0 && q4 == 0) y[rw] = w;
         }
         __syncthreads();
@@ -1104,12 +1189,12 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
             y[t] = cx<T>{(T)w.x, (T)w.y};
             const c64 d = cscale(cadd(w, al), scale);
             x[2 * m + t] = first ? d : cadd(x[2 * m + t], d);
-            lds_max(&nrm[4 * k + 3], sqrt(d.x * d.x + d.y * d.y));
+            bits_max(nd, sqrt(d.x * d.x + d.y * d.y));
         }
         __syncthreads();
         if ((t & 255) < m) {
             const int i = t & 255;
-            const cx<T> ws = y[g.sn[i]], we = y[g.en[i]];
+            const cx<T> ws = y[end0[i]], we = y[end1[i]];
             c64 l = grp ? c64{0.5 * ((double)ws.x + we.x) + al.x, 0.5 * ((double)ws.y + we.y) + al.y}
                         : c64{(double)ws.x - we.x, (double)ws.y - we.y};
             if (!first) l = csub(l, cscale(r[grp * m + i], inv));
@@ -1117,12 +1202,12 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
         }
         __syncthreads();
         {
-            const cx<T> s = gemv(Fg, v[grp]);
+            const cx<T> s = gemv(frow, v[grp]);
             if (q4 == 0 && rw < m) {
                 const c64 d{s.x * scale, s.y * scale};
                 c64* xi = &x[grp * m + rw];
                 *xi = first ? d : cadd(*xi, d);
-                lds_max(&nrm[4 * k + 3], sqrt(d.x * d.x + d.y * d.y));
+                bits_max(nd, sqrt(d.x * d.x + d.y * d.y));
             }
         }
         __syncthreads();
@@ -1130,8 +1215,9 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
         if (rw < m) {
             DD sx{0, 0}, sy{0, 0};
             double ta = 0;
-            for (int k4 = q4; k4 < m; k4 += 4) {
-                const c64 p = Zg[rw * m + k4], q = x[grp * m + k4];
+#pragma unroll
+            for (int k4 = 0; k4 < 16; k4++) {
+                const c64 p = zr[k4], q = x[grp * m + 4 * k4 + q4];
                 dd_mac(sx, p.x, q.x);
                 dd_mac(sx, -p.y, q.y);
                 dd_mac(sy, p.x, q.y);
@@ -1144,7 +1230,7 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
                 ta += __shfl_xor(ta, o);
             }
             if (q4 == 0) {
-                const c64 xs = x[2 * m + g.sn[rw]], xe = x[2 * m + g.en[rw]];
+                const c64 xs = x[2 * m + end0[rw]], xe = x[2 * m + end1[rw]];
                 const double cs = grp ? 0.5 : 1.0, ce = grp ? 0.5 : -1.0;
                 dd_add(sx, cs * xs.x);
                 dd_add(sy, cs * xs.y);
@@ -1153,16 +1239,16 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
                 const int i = grp * m + rw;
                 const c64 rr{dd_sub_from(0.0, sx), dd_sub_from(0.0, sy)};
                 r[i] = rr;
-                lds_max(&nrm[4 * k], sqrt(rr.x * rr.x + rr.y * rr.y));
-                lds_max(&nrm[4 * k + 1], sqrt(x[i].x * x[i].x + x[i].y * x[i].y));
-                if (first) lds_max(&nrm[4 * k + 2], ta + 2.0 * cs);
+                bits_max(nr, sqrt(rr.x * rr.x + rr.y * rr.y));
+                bits_max(nx, sqrt(x[i].x * x[i].x + x[i].y * x[i].y));
+                if (first) bits_max(na, ta + 2.0 * cs);
             }
         }
         if (t < n) {
             DD sx{0, 0}, sy{0, 0};
             double ta = 0;
-            for (int p = g.node_ptr[t]; p < g.node_ptr[t + 1]; p++) {
-                const int sa = g.node_seg[p];
+            for (int p = nptr[t]; p < nptr[t + 1]; p++) {
+                const int sa = nseg[p];
                 const double cl = (sa & 1) ? -1.0 : 1.0;
                 const c64 xl = x[sa >> 1], xt = x[m + (sa >> 1)];
                 dd_add(sx, cl * xl.x);
@@ -1174,9 +1260,21 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
             const int i = 2 * m + t;
             const c64 rr{dd_sub_from(t == g.inj ? 1.0 : 0.0, sx), dd_sub_from(0.0, sy)};
             r[i] = rr;
-            lds_max(&nrm[4 * k], sqrt(rr.x * rr.x + rr.y * rr.y));
-            lds_max(&nrm[4 * k + 1], sqrt(x[i].x * x[i].x + x[i].y * x[i].y));
-            if (first) lds_max(&nrm[4 * k + 2], ta);
+            bits_max(nr, sqrt(rr.x * rr.x + rr.y * rr.y));
+            bits_max(nx, sqrt(x[i].x * x[i].x + x[i].y * x[i].y));
+            if (first) bits_max(na, ta);
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            nr = max(nr, __shfl_xor(nr, o));
+            nx = max(nx, __shfl_xor(nx, o));
+            nd = max(nd, __shfl_xor(nd, o));
+            if (first) na = max(na, __shfl_xor(na, o));
+        }
+        if ((t & 63) == 0) {
+            atomicMax(&nrm[4 * k], nr);
+            atomicMax(&nrm[4 * k + 1], nx);
+            atomicMax(&nrm[4 * k + 2], na);
+            atomicMax(&nrm[4 * k + 3], nd);
         }
         __syncthreads();
     }
@@ -1203,15 +1301,13 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
 // Columns per sweep step. A step reads and writes every tile once, which at 64
 // columns takes as long as its MFMAs; more blocks per step cost the panels'
 // products with the step's earlier blocks.
+constexpr long kWide = 300;
 static int nd_block(long dim, bool f64)
 {
     if (dim <= 128) return 64;
-    return !f64 && dim >= kX6Dim ? 256 : 128;
+    return !f64 && dim >= kWide ? 256 : 128;
 }
-static bool nd_x6(long dim, bool f64) { return !f64 && dim >= kX6Dim; }
 static long up(long v, long a) { return (v + a - 1) / a * a; }
-// 16-byte words of one matrix's split-bf16 panel
-static long nd_x6_words(long ld, int nb) { return ld / 32 * (nb / 16) * X6_PARTS * X6_FRAG; }
 
 template <typename T>
 size_t NodalSolver::partition(char* base, int batch)
@@ -1227,8 +1323,6 @@ size_t NodalSolver::partition(char* base, int batch)
     const long bz = nd_block(m, d), bs = nd_block(n, d);
     const size_t panel = std::max(2 * (size_t)mp * bz, (size_t)np * bs);
     const size_t diag = 64 * (size_t)std::max(2 * bz, bs);
-    const size_t words = std::max(nd_x6(m, d) ? 2 * (size_t)nd_x6_words(mp, bz) : 0,
-                                  nd_x6(n, d) ? (size_t)nd_x6_words(np, bs) : 0);
     sZ = nodal_z_items(m);
     Z = (c64*)take(sizeof(c64) * sZ * B);
     F = take(e * 2 * mp * mp * B);
@@ -1236,8 +1330,6 @@ size_t NodalSolver::partition(char* base, int batch)
     tp = take(e * panel * B);
     op_ = take(e * panel * B);
     P = take(e * diag * B);
-    xt = take(16 * words * B);
-    xo = take(16 * words * B);
     x = (c64*)take(sizeof(c64) * N * B);
     r = (c64*)take(sizeof(c64) * N * B);
     b = (c64*)take(sizeof(c64) * N * B);
@@ -1381,19 +1473,8 @@ static int nd_sweep(const NdPhase<T>& p, hipStream_t st, Profiler* pr)
         }
         Timed tm(pr, FAM_GEMM, st);
         const double d = p.dim, w = std::min(NB, p.dim - c0);
-        if constexpr (sizeof(T) == 4 && NB > 64) {
-            if (p.xt && nt > NB / 64) {
-                hipLaunchKernelGGL((k_nd_update<T, NB>), dim3(xcd_grid(p.items * nq * nt)),
-                                   dim3(256), 0, st, p, c0, 1);
-                const long nm = (p.ld + 127) / 128;
-                hipLaunchKernelGGL((k_nd_update_x6<NB>), dim3(xcd_grid(p.items * nm * (nm + 1))),
-                                   dim3(256), 0, st, p, c0);
-                tm.end(4.0 * d * d * w * p.items, true);
-                continue;
-            }
-        }
         hipLaunchKernelGGL((k_nd_update<T, NB>), dim3(xcd_grid(p.items * ntri)), dim3(256), 0, st,
-                           p, c0, 0);
+                           p, c0);
         tm.end(4.0 * d * d * w * p.items, true);
     }
     hipLaunchKernelGGL(k_nd_mirror<T>, dim3(xcd_grid(p.items * ntri)), dim3(256), 0, st, p.A, p.sA,
@@ -1403,10 +1484,8 @@ static int nd_sweep(const NdPhase<T>& p, hipStream_t st, Profiler* pr)
 }
 
 template <typename T>
-static int nd_invert(NdPhase<T> p, int nb, bool x6, hipStream_t st, Profiler* pr)
+static int nd_invert(const NdPhase<T>& p, int nb, hipStream_t st, Profiler* pr)
 {
-    p.sx = nd_x6_words(p.ld, nb);
-    if (!x6) p.xt = p.xo = nullptr;
     if constexpr (sizeof(T) == 4) {
         if (nb == 256) return nd_sweep<T, 256>(p, st, pr);
     }
@@ -1427,8 +1506,8 @@ int NodalSolver::factor()
     int rc;
     const int bz = nd_block(m, f64), bs = nd_block(n, f64);
     const NdPhase<T> pz{(cx<T>*)F,   mp * mp, (int)mp,   (int)m,     2 * nb,     (cx<T>*)tp,
-                        (cx<T>*)op_, mp * bz, (cx<T>*)P, (u32x4*)xt, (u32x4*)xo, 0};
-    if ((rc = nd_invert<T>(pz, bz, nd_x6(m, f64), st, pr))) return rc;
+                        (cx<T>*)op_, mp * bz, (cx<T>*)P};
+    if ((rc = nd_invert<T>(pz, bz, st, pr))) return rc;
     {
         Timed tm(pr, FAM_OTHER, st);
         hipLaunchKernelGGL(k_nd_rows<T>, dim3((unsigned)(nb * ((m + 3) / 4))), dim3(256), 0, st, g);
@@ -1439,8 +1518,8 @@ int NodalSolver::factor()
         tm.end();
     }
     const NdPhase<T> ps{(cx<T>*)S,   np * np, (int)np,   (int)n,     nb,         (cx<T>*)tp,
-                        (cx<T>*)op_, np * bs, (cx<T>*)P, (u32x4*)xt, (u32x4*)xo, 0};
-    if ((rc = nd_invert<T>(ps, bs, nd_x6(n, f64), st, pr))) return rc;
+                        (cx<T>*)op_, np * bs, (cx<T>*)P};
+    if ((rc = nd_invert<T>(ps, bs, st, pr))) return rc;
     hipLaunchKernelGGL((k_nd_gemv<T, 1>), dim3(xcd_grid(nb * (np / 16))), dim3(256), 0, st, g,
                        (const cx<T>*)g.c, g.h);
     hipLaunchKernelGGL(k_nd_den<T>, dim3(nb), dim3(256), 0, st, g);
@@ -1670,8 +1749,8 @@ int sym_inverse(const c64* src, long lds, long ssrc, c64* X, long dim, int items
     c64* tp = (c64*)work;
     c64* op = tp + (size_t)items * ld * nb;
     c64* P = op + (size_t)items * ld * nb;
-    const NdPhase<double> p{X, ld * ld, (int)ld, (int)dim, items, tp, op, ld * nb, P, nullptr, nullptr, 0};
-    return nd_invert<double>(p, nb, false, st, nullptr);
+    const NdPhase<double> p{X, ld * ld, (int)ld, (int)dim, items, tp, op, ld * nb, P};
+    return nd_invert<double>(p, nb, st, nullptr);
 }
 
 __global__ __launch_bounds__(256) void k_sym_apply(const c64* X, long ld, long n, const c64* r,
