@@ -773,8 +773,9 @@ __device__ inline bool pair_near(const DSeg& S, const DSeg& R, double* rho)
     return !(*rho >= 2.0);
 }
 
+constexpr int fill_waves(int ts) { return ts == 8 ? 8 : 4; }
 template <int K, int TS>
-__global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, long ldw,
+__global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __restrict__ W, long ldw,
                                                        long zl_off, long zt_off, long m, SegSoA e,
                                                        SegSoA img,
                                                        const PairScalars* __restrict__ scs, long sw,
@@ -787,18 +788,20 @@ __global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, lo
     while (ti * (ti + 1) / 2 > b) ti--;
     const long tk = b - ti * (ti + 1) / 2;
     constexpr int NP = TS * TS;  // pairs
+    constexpr int NW = fill_waves(TS);
+    constexpr int KINDS = TS == 8 ? 2 : 1;  // kinds of moments formed at a time
     // (the wave index is uniform: a sample's scalars and coefficients stay scalar)
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
-    // with 8 x 8 tiles every wave holds all pairs (and forms them once, in wave 0)
+    // with 8 x 8 tiles every wave holds all pairs
     const int pr = TS == 8 ? lane : t, a = pr / TS, c = pr % TS;
     const long i0 = ti * TS, k0 = tk * TS, i = i0 + a, k = k0 + c;
     const bool in = i < m && k < m && k <= i;
 
     __shared__ double geo[3][8][TS];  // columns, rows, the rows' images
-    // every pair's moments of one kind while they are formed; then the tiles
-    // being transposed
+    // every pair's moments of one kind or both while they are formed; then the
+    // tiles being transposed
     union Stage {
-        double mom[K][NP];
+        double mom[KINDS][K][NP];
         c64 tile[2][2][TS][TS + 1];
     };
     __shared__ Stage stage;
@@ -826,55 +829,74 @@ __global__ __launch_bounds__(256, 2) void k_fill_moments(c64* __restrict__ W, lo
     };
     double md[K], mi[K];  // direct, image
     double rd = 0.0, ri = 0.0, cost = 0.0, cosi = 0.0, ll = 1.0;
-#pragma unroll
-    for (int kind = 0; kind < 2; kind++) {
-        {
-            Moments<K> M;
-            M.zero();
-            if (in) {
-                const DSeg S = seg(0, c), R = seg(1 + kind, a);
+    // far pairs by a lane each (with 8 x 8 tiles a wave to each kind) ..
+    auto far = [&](int kind) {
+        Moments<K> M;
+        M.zero();
+        double rho;
+        if (in && (kind || k != i)) {
+            const DSeg S = seg(0, c), R = seg(1 + kind, a);
+            if (pair_near(S, R, &rho)) {
+                near_at[kind][atomicAdd(&near_n[kind], 1)] = pr;
+            } else {
                 M.rc = vnorm(vsub(vmid(S), vmid(R)));
                 M.invd = 1.0 / D;
-                (kind ? ri : rd) = M.rc;
-                (kind ? cosi : cost) = abs_dot(S, R);
-                if (!kind) ll = S.len * R.len;
-                double rho;
-                if ((TS == 16 || wave == 0) && (kind || k != i)) {
-                    if (pair_near(S, R, &rho))
-                        near_at[kind][atomicAdd(&near_n[kind], 1)] = pr;
-                    else
-                        mom_gl(M, S, R, geometric_order(rho, gabs * fmax(S.len, R.len)), 0, 1, 1.0);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < K; j++)
-                if (TS == 16 || wave == 0) stage.mom[j][pr] = M.m[j];
-        }
-        __syncthreads();
-        const int nn = near_n[kind];
-        for (int q = wave; q < nn; q += 4) {
-            const int w = near_at[kind][q];
-            const DSeg S = seg(0, w % TS), R = seg(1 + kind, w / TS);
-            Moments<K> M;
-            M.zero();
-            M.invd = 1.0 / D;
-            M.rc = vnorm(vsub(vmid(S), vmid(R)));
-            mom_wave(M, S, R, gabs, lane);
-#pragma unroll
-            for (int j = 0; j < K; j++) {
-                double v = M.m[j];
-                for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-                if (lane == 0) stage.mom[j][w] = v;
+                mom_gl(M, S, R, geometric_order(rho, gabs * fmax(S.len, R.len)), 0, 1, 1.0);
             }
         }
+#pragma unroll
+        for (int j = 0; j < K; j++) stage.mom[KINDS == 2 ? kind : 0][j][pr] = M.m[j];
+    };
+    // .. and near ones by a wave each
+    auto near = [&](int kind, int w) {
+        const DSeg S = seg(0, w % TS), R = seg(1 + kind, w / TS);
+        Moments<K> M;
+        M.zero();
+        M.invd = 1.0 / D;
+        M.rc = vnorm(vsub(vmid(S), vmid(R)));
+        mom_wave(M, S, R, gabs, lane);
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            double v = M.m[j];
+            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+            if (lane == 0) stage.mom[KINDS == 2 ? kind : 0][j][w] = v;
+        }
+    };
+    if constexpr (KINDS == 2) {
+        if (wave < 2) far(wave);
+        __syncthreads();
+        const int n0 = near_n[0], nn = n0 + near_n[1];
+        for (int q = wave; q < nn; q += NW) near(q >= n0, near_at[q >= n0][q >= n0 ? q - n0 : q]);
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < K; j++) (kind ? mi[j] : md[j]) = stage.mom[j][pr];
-        __syncthreads();
+        for (int j = 0; j < K; j++) {
+            md[j] = stage.mom[0][j][pr];
+            mi[j] = stage.mom[KINDS - 1][j][pr];
+        }
+    } else {
+#pragma unroll
+        for (int kind = 0; kind < 2; kind++) {
+            far(kind);
+            __syncthreads();
+            const int nn = near_n[kind];
+            for (int q = wave; q < nn; q += NW) near(kind, near_at[kind][q]);
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < K; j++) (kind ? mi[j] : md[j]) = stage.mom[0][j][pr];
+            __syncthreads();
+        }
+    }
+    if (in) {
+        const DSeg S = seg(0, c), R = seg(1, a), Ri = seg(2, a);
+        rd = vnorm(vsub(vmid(S), vmid(R)));
+        ri = vnorm(vsub(vmid(S), vmid(Ri)));
+        cost = abs_dot(S, R);
+        cosi = abs_dot(S, Ri);
+        ll = S.len * R.len;
     }
     const double self = in && k == i ? self_integral_dev(geo[1][6][a], geo[1][7][a]) : 0.0;
     const int f0 = blockIdx.y * per, f1 = min(nf, f0 + per);
-    for (int f = f0 + (TS == 8 ? wave : 0); f < f1; f += TS == 8 ? 4 : 1) {
+    for (int f = f0 + (TS == 8 ? wave : 0); f < f1; f += TS == 8 ? NW : 1) {
         const PairScalars& sc = scs[f];
         const c64* cq = cf + (long)f * K;
         c64 vl{0, 0}, vt{0, 0};
@@ -983,14 +1005,14 @@ int launch_fill_moments(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
     const bool small = m <= 256;
     const long T = small ? (m + 7) / 8 : (m + 15) / 16, tiles = T * (T + 1) / 2;
     // samples per work-group: all of them once the tiles alone give every CU
-    // four work-groups (8 x 8 tiles: two, of four samples at least), else fewer
+    // four work-groups (8 x 8 tiles: two, of eight samples at least), else fewer
     // (the moments are then formed more often)
-    const long chunks = std::max(1L, std::min(small ? (nb + 3L) / 4 : (long)nb,
+    const long chunks = std::max(1L, std::min(small ? (nb + 7L) / 8 : (long)nb,
                                               (small ? 512 : 1024) / tiles));
     const int per = (int)((nb + chunks - 1) / chunks);
     const dim3 g((unsigned)tiles, (unsigned)((nb + per - 1) / per));
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, g, dim3(256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, scs,
+        hipLaunchKernelGGL(kern, g, dim3(small ? 512 : 256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, scs,
                            sw, (const c64*)cf, nb, per, D, gabs);
     };
     auto terms = [&](auto kt) {
