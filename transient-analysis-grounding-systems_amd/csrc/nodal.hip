@@ -200,182 +200,207 @@ constexpr int nd_groups(int k)  // k groups of nd_mma in k columns
 // LDS of nd_sweep64
 template <typename T>
 struct NdSweep {
-    cx<T> row[2][2][64];  // two pivot rows, of this step and of the next
-    cx<T> piv[2][3];      // their 2 x 2 block
+    cx<T> O[2][64][17];  // block column of 16, of this step and of the next
+    cx<T> W[64][17];     // each wave's rows of it times the inverse
+    cx<T> P[2][16][17];  // minus the inverse of its diagonal block
+    cx<T> row[2][16];    // two pivot rows of the diagonal block ..
+    cx<T> piv[3];        // .. and their 2 x 2 block
 };
 
-// The unblocked sweep of a 64 x 64 matrix in the registers of 256 threads (ty,
-// tx: rows ty + 16 i, columns tx + 16 j): a = -a^-1 over its first kv rows and
-// columns, two pivots at a time (the inverse I of the symmetric 2 x 2 block in
-// closed form; past kv the matrix is taken as the identity). The pivot rows go
-// through LDS (they are the pivot columns too) with minus the identity in place
-// of the block, which is kept apart: then a -= (o I) o^T over both rows serves
-// every entry, once the pivot rows and columns themselves are cleared. The next
-// two rows are formed and stored before the barrier, so that the rest of a step
-// runs beside the next one's reads and reciprocal. Bound by the issue of one
-// wave per SIMD (about 300 instructions a step, 128 of them the update's
-// multiply-adds), so nothing is selected per entry that a branch or the stored
-// row can settle. 64 pivots in complex128: see k_nd_diag. All threads of the
-// work-group have to call this; those of `idle` only meet the barriers.
-template <typename T>
-__device__ __forceinline__ void nd_sweep64(cx<T> (&a)[4][4], NdSweep<T>& sh, int kv, int ty, int tx,
-                                           bool idle = false)
+// orders LDS accesses of a wave's lanes
+__device__ __forceinline__ void nd_wave_sync()
 {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// out = -M^-1 over the first kv rows and columns of a symmetric 16 x 16 matrix
+// (which is taken as the identity past kv), by one wave: lanes hold four columns
+// of a row. Two pivots at a time, with the inverse I of their 2 x 2 block in
+// closed form: the pivot rows (they are the pivot columns too) go through LDS
+// with minus the identity in place of the block, which is kept apart; then
+// a -= (o I) o^T over both rows serves every entry, once the pivot rows and
+// columns themselves are cleared.
+template <typename T>
+__device__ __forceinline__ void nd_sweep16(const cx<T> (*M)[17], cx<T> (*out)[17], NdSweep<T>& sh,
+                                           int kv, int lane)
+{
+    const int r = lane >> 2, c0 = 4 * (lane & 3);
     const cx<T> zero{0, 0};
-    // pivot rows n0, n0 + 1 (of 16 from 16 nb on), given as w[]
-    auto store = [&](int buf, int n0, int nb, const cx<T>(&w)[4]) {
-        const int h = ty - n0;
+    cx<T> a[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            cx<T> x = w[j];
-            if (j == nb && (tx == n0 || tx == n0 + 1)) {
-                if (tx - n0 >= h) sh.piv[buf][h + tx - n0] = x;
-                x = cx<T>{tx == ty ? (T)-1 : (T)0, 0};
-            }
-            sh.row[buf][h][tx + 16 * j] = x;
-        }
-    };
-    if (!idle) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (ty == tx && ty + 16 * i >= kv) a[i][i] = cx<T>{1, 0};
-        if (ty < 2) {
-            store(0, 0, 0, a[0]);
-#pragma unroll
-            for (int j = 0; j < 4; j++) a[0][j] = zero;
-        }
-        if (tx < 2) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) a[i][0] = zero;
-        }
-    }
-    __syncthreads();
-    // pivots k, k + 1; the next ones are rows n0, n0 + 1 of 16 from 16 nb on
-    auto step = [&](int k, int n0, auto nbc) {
-        constexpr int nb = decltype(nbc)::value;
-        const int buf = (k >> 1) & 1;
-        cx<T> o0[4], o1[4], l0[4], l1[4];
-        if (!idle) {
-            const cx<T> p = sh.piv[buf][0], q = sh.piv[buf][1], s = sh.piv[buf][2];
-            const cx<T> d = crecip_fast(cfnma(cmul(p, s), q, q));
-            const cx<T> i00 = cmul(s, d), i11 = cmul(p, d), t = cmul(q, d);
-            const cx<T>(*r)[64] = sh.row[buf];
+    for (int j = 0; j < 4; j++) a[j] = r == c0 + j && r >= kv ? cx<T>{1, 0} : M[r][c0 + j];
+    auto put = [&](int n) {
+        if (r == n || r == n + 1) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                o0[j] = r[0][tx + 16 * j];
-                o1[j] = r[1][tx + 16 * j];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const cx<T> u = r[0][ty + 16 * i], v = r[1][ty + 16 * i];
-                l0[i] = cfnma(cmul(u, i00), v, t);
-                l1[i] = cfnma(cmul(v, i11), u, t);
-            }
-            if (k + 2 < kv) {
-                if (ty == n0 || ty == n0 + 1) {
-                    cx<T> w[4];
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        w[j] = cfnma(cfnma(a[nb][j], l0[nb], o0[j]), l1[nb], o1[j]);
-                        a[nb][j] = zero;
-                    }
-                    store(buf ^ 1, n0, nb, w);
-                    l0[nb] = l1[nb] = zero;
+                const int c = c0 + j;
+                cx<T> x = a[j];
+                if (c == n || c == n + 1) {
+                    if (c >= r) sh.piv[r - n + c - n] = x;
+                    x = cx<T>{c == r ? (T)-1 : (T)0, 0};
                 }
-                if (tx == n0 || tx == n0 + 1) {
-#pragma unroll
-                    for (int i = 0; i < 4; i++) a[i][nb] = zero;
-                    o0[nb] = o1[nb] = zero;
-                }
+                sh.row[r - n][c] = x;
+                a[j] = zero;
             }
         }
-        __syncthreads();
-        if (idle) return;
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int j = 0; j < 4; j++) a[j] = csel(c0 + j == n || c0 + j == n + 1, zero, a[j]);
+        nd_wave_sync();
+    };
+    put(0);
+    for (int k = 0; k < kv; k += 2) {
+        const cx<T> p = sh.piv[0], q = sh.piv[1], s = sh.piv[2];
+        const cx<T> u = sh.row[0][r], v = sh.row[1][r];
+        cx<T> o0[4], o1[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            o0[j] = sh.row[0][c0 + j];
+            o1[j] = sh.row[1][c0 + j];
+        }
+        const cx<T> d = crecip_fast(cfnma(cmul(p, s), q, q));
+        const cx<T> i00 = cmul(s, d), i11 = cmul(p, d), t = cmul(q, d);
+        const cx<T> l0 = cfnma(cmul(u, i00), v, t), l1 = cfnma(cmul(v, i11), u, t);
+#pragma unroll
+        for (int j = 0; j < 4; j++) a[j] = cfnma(cfnma(a[j], l0, o0[j]), l1, o1[j]);
+        nd_wave_sync();
+        if (k + 2 < kv) put(k + 2);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) out[r][c0 + j] = a[j];
+    nd_wave_sync();
+}
+
+// The sweep of a 64 x 64 matrix by four waves, which hold 16 rows each in the
+// layout of MFMA results (a[j][v]: column 16 j + lane % 16): a = -a^-1 over its
+// first kv rows and columns, 16 at a time. One wave inverts the diagonal block;
+// then with O the block column as it was and P that inverse, wave w forms
+// W = O_w P and its tiles A_wj -= W O_j^T (in the block's own rows, from zero
+// and with W = -P), and the block column becomes W (-P). The tiles of the next
+// block column come first, so that its inverse runs beside the other waves'
+// remaining products. Per 16 columns one barrier, eight dependent steps of two
+// pivots and 16 MFMA products a wave: 64 columns take 25 us in complex128 and 19
+// us in complex64, against 28 and 26 us with every entry swept by two pivots at a
+// time on the vector units (about 380 instructions per step and thread) and 40 us
+// by one. The dependent steps bound it. All threads of the work-group call this;
+// those of `idle` only meet the barriers.
+template <typename T>
+__device__ __forceinline__ void nd_sweep64(cx<T> (&a)[4][4], NdSweep<T>& sh, int kv, int w,
+                                           int lane, bool idle = false)
+{
+    const int lr = lane & 15, lk = lane >> 4, nb = (kv + 15) / 16;
+    if (!idle) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) sh.O[0][16 * w + Mfma<T>::row(lane, v)][lr] = a[0][v];
+        nd_wave_sync();
+        if (w == 0) nd_sweep16(&sh.O[0][0], sh.P[0], sh, min(16, kv), lane);
+    }
+    __syncthreads();
+    auto step = [&](auto bc) {
+        constexpr int b = decltype(bc)::value, h = b & 1;
+        if (b >= nb) return;
+        if (!idle) {
+            cx<T> l[4];
+            if (w != b) {
+                NdAcc<T> acc;
+                acc.zero();
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    acc.mac(sh.O[h][16 * w + lr][4 * g + lk], sh.P[h][4 * g + lk][lr]);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const cx<T> x = acc.get(v);
+                    a[b][v] = cx<T>{-x.x, -x.y};
+                    sh.W[16 * w + Mfma<T>::row(lane, v)][lr] = a[b][v];
+                }
+                nd_wave_sync();
+#pragma unroll
+                for (int g = 0; g < 4; g++) l[g] = sh.W[16 * w + lr][4 * g + lk];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        a[j][v] = j == b ? sh.P[h][Mfma<T>::row(lane, v)][lr] : cx<T>{0, 0};
+#pragma unroll
+                for (int g = 0; g < 4; g++) l[g] = sh.P[h][lr][4 * g + lk];
+            }
+            auto tile = [&](int j) {
+                NdAcc<T> acc;
+                acc.zero();
+#pragma unroll
+                for (int g = 0; g < 4; g++) acc.mac(l[g], sh.O[h][16 * j + lr][4 * g + lk]);
+#pragma unroll
+                for (int v = 0; v < 4; v++) a[j][v] = csub(a[j][v], acc.get(v));
+            };
+            if (b < 3 && b + 1 < nb) {
+                constexpr int x = b < 3 ? b + 1 : b;
+                tile(x);
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    sh.O[h ^ 1][16 * w + Mfma<T>::row(lane, v)][lr] = a[x][v];
+                nd_wave_sync();
+                if (w == x)
+                    nd_sweep16(&sh.O[h ^ 1][16 * x], sh.P[h ^ 1], sh, min(16, kv - 16 * x), lane);
+            }
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                a[i][j] = cfnma(cfnma(a[i][j], l0[i], o0[j]), l1[i], o1[j]);
+                if (j != b && j != b + 1 && j < nb) tile(j);
+        }
+        __syncthreads();
     };
-    auto block = [&](auto kbc) {
-        constexpr int kb = decltype(kbc)::value, nx = kb < 3 ? kb + 1 : kb;
-        const int end = min(kv - 16 * kb, 14);
-        for (int kl = 0; kl < end; kl += 2)
-            step(16 * kb + kl, kl + 2, std::integral_constant<int, kb>{});
-        if (16 * kb + 14 < kv) step(16 * kb + 14, 0, std::integral_constant<int, nx>{});
-    };
-    block(std::integral_constant<int, 0>{});
-    block(std::integral_constant<int, 1>{});
-    block(std::integral_constant<int, 2>{});
-    block(std::integral_constant<int, 3>{});
+    step(std::integral_constant<int, 0>{});
+    step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 3>{});
 }
 
 // P_t, one work-group per item. A matrix of one block (whole) is finished here:
 // both triangles of A get -P.
 template <typename T, int NB>
-__global__ __launch_bounds__(256) void k_nd_diag(NdPhase<T> p, int c0, int t,
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 1) void k_nd_diag(NdPhase<T> p, int c0, int t,
                                                   int whole)
 {
     const long item = blockIdx.x;
     const cx<T>* A = p.A + item * p.sA;
     cx<T>* P = p.P + (item * (NB / 64) + t) * 4096;
     const int cK = c0 + 64 * t, kv = min(64, p.dim - cK);
-    const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15;
     __shared__ NdSweep<T> sh;
     cx<T> a[4][4];
+    // (entry r, c of the tile: row 16 wave + .., column 16 j + ..)
+    auto each = [&](auto&& f) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+        for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int r = ty + 16 * i, c = tx + 16 * j;
-            a[i][j] = cx<T>{0, 0};
-            if (r < kv && c < kv) a[i][j] = A[(long)(cK + max(r, c)) * p.ld + cK + min(r, c)];
-        }
+            for (int v = 0; v < 4; v++)
+                f(16 * wave + Mfma<T>::row(lane, v), 16 * j + lr, a[j][v], j, v);
+    };
+    each([&](int r, int c, cx<T>& x, int, int) {
+        x = r < kv && c < kv ? A[(long)(cK + max(r, c)) * p.ld + cK + min(r, c)] : cx<T>{0, 0};
+    });
     if constexpr (NB > 64) {
         if (t > 0) {
-            // less the step's earlier blocks, four waves of 32 x 32
-            __shared__ cx<T> up[64][65];
-            const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-            const int i0 = (wave >> 1) * 32, j0 = (wave & 1) * 32;
-            NdAcc<T> acc[2][2];
+            // less the step's earlier blocks
+            NdAcc<T> acc[1][4];
 #pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j].zero();
-            nd_mma<T, NB, 2, 2, 4>(p.tp + item * p.sp, p.op + item * p.sp, cK + i0, cK + j0, 0,
-                                nd_groups<T>(64 * t), acc);
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        up[i0 + 16 * i + Mfma<T>::row(lane, v)][j0 + 16 * j + (lane & 15)] =
-                            acc[i][j].get(v);
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int r = ty + 16 * i, c = tx + 16 * j;
-                    if (r < kv && c < kv) a[i][j] = csub(a[i][j], up[max(r, c)][min(r, c)]);
-                }
+            for (int j = 0; j < 4; j++) acc[0][j].zero();
+            nd_mma<T, NB, 1, 4, sizeof(T) == 4 ? 3 : 4>(p.tp + item * p.sp, p.op + item * p.sp, cK + 16 * wave, cK, 0,
+                                   nd_groups<T>(64 * t), acc);
+            each([&](int r, int c, cx<T>& x, int j, int v) {
+                if (r < kv && c < kv) x = csub(x, acc[0][j].get(v));
+            });
         }
     }
-    nd_sweep64(a, sh, kv, ty, tx);
+    nd_sweep64(a, sh, kv, wave, lane);
     cx<T>* own = p.A + item * p.sA;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int r = ty + 16 * i, c = tx + 16 * j;
-            const bool in = r < kv && c < kv;
-            if (whole) {
-                own[(long)r * p.ld + c] = in ? a[i][j] : cx<T>{0, 0};
-            } else {
-                P[nd_pk<T, 64>(c, r)] = in ? cx<T>{-a[i][j].x, -a[i][j].y} : cx<T>{0, 0};
-            }
-        }
+    each([&](int r, int c, cx<T>& x, int, int) {
+        const bool in = r < kv && c < kv;
+        if (whole)
+            own[(long)r * p.ld + c] = in ? x : cx<T>{0, 0};
+        else
+            P[nd_pk<T, 64>(c, r)] = in ? cx<T>{-x.x, -x.y} : cx<T>{0, 0};
+    });
 }
 
 // O_t and T_t of 64 rows: four waves of 16 rows and 64 columns. O_t passes
@@ -455,10 +480,6 @@ __global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int c0, int t)
         block(acc, [](auto& a, int c) { return a[0][c]; }, false);
     }
     // T_t(i) = O_t(i) P_t; both stored a fragment at a time
-    auto sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    };
     Frag* oo = (Frag*)op + (i0 / 16) * FS + (long)t * GP * 64 + lane;
     Frag* to = (Frag*)tp + (i0 / 16) * FS + (long)t * GP * 64 + lane;
     Frag b[4], bn[4];
@@ -467,7 +488,7 @@ __global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int c0, int t)
     NdAcc<T> acc[4];
 #pragma unroll
     for (int c = 0; c < 4; c++) acc[c].zero();
-    sync();
+    nd_wave_sync();
     for (int g = 0; g < GP; g++) {
         const int gn = min(g + 1, GP - 1);
 #pragma unroll
@@ -488,12 +509,12 @@ __global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int c0, int t)
             b[c] = bn[c];
         }
     }
-    sync();
+    nd_wave_sync();
 #pragma unroll
     for (int c = 0; c < 4; c++)
 #pragma unroll
         for (int v = 0; v < 4; v++) my[Mfma<T>::row(lane, v)][16 * c + lr] = acc[c].get(v);
-    sync();
+    nd_wave_sync();
 #pragma unroll
     for (int g = 0; g < GP; g++) {
         Frag a;
@@ -994,7 +1015,8 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
                                                    int spec)
 {
     const long item = blockIdx.x;
-    const int t = threadIdx.x, grp = t >> 8, ty = (t & 255) >> 4, tx = t & 15;
+    const int t = threadIdx.x, grp = t >> 8;
+    const int lane = t & 63, wave = (t & 255) >> 6, lr = lane & 15;
     const int m = (int)g.m, n = (int)g.n, N = (int)g.N;
     const c64* Z = Zall + item * sZ;
     const c64* Zg = Z + grp * (m * m + m);
@@ -1018,26 +1040,24 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
     if (t < 192) x[t] = c64{0, 0};
     if (t < 128) v[t >> 6][t & 63] = z[t >> 6][t & 63] = cx<T>{0, 0};
     if (t < 64) f[t] = y[t] = h[t] = c[t] = cx<T>{0, 0};
+    // the matrix being inverted, 16 rows a wave in the layout of nd_sweep64
     cx<T> a[4][4];
+    auto each = [&](auto&& f) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+        for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int p = ty + 16 * i, q = tx + 16 * j;
-            a[i][j] = cx<T>{0, 0};
-            if (p < m && q < m) {
-                const c64 s = Zg[max(p, q) * m + min(p, q)];
-                a[i][j] = cx<T>{(T)s.x, (T)s.y};
-            }
+            for (int v = 0; v < 4; v++)
+                f(16 * wave + Mfma<T>::row(lane, v), 16 * j + lr, a[j][v]);
+    };
+    each([&](int p, int q, cx<T>& x) {
+        x = cx<T>{0, 0};
+        if (p < m && q < m) {
+            const c64 s = Zg[max(p, q) * m + min(p, q)];
+            x = cx<T>{(T)s.x, (T)s.y};
         }
-    nd_sweep64(a, sh[grp], m, ty, tx);
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int p = ty + 16 * i, q = tx + 16 * j;
-            Fg[p * 64 + q] = p < m && q < m ? a[i][j] : cx<T>{0, 0};
-        }
+    });
+    nd_sweep64(a, sh[grp], m, wave, lane);
+    each([&](int p, int q, cx<T>& x) { Fg[p * 64 + q] = p < m && q < m ? x : cx<T>{0, 0}; });
     __syncthreads();
     // four lanes per row of the own block from here on
     const int rw = (t & 255) >> 2, q4 = t & 3;
@@ -1068,38 +1088,27 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
     }
     __syncthreads();
     // -S_p
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int u = max(ty + 16 * i, tx + 16 * j), w = min(ty + 16 * i, tx + 16 * j);
-            a[i][j] = cx<T>{0, 0};
-            if (grp == 0 && u < n) {
-                c64 s = cst[0];
-                for (int p = nptr[u]; p < nptr[u + 1]; p++) {
-                    const int sa = nseg[p];
-                    for (int q = nptr[w]; q < nptr[w + 1]; q++) {
-                        const int sb = nseg[q];
-                        const double sg = ((sa ^ sb) & 1) ? -1.0 : 1.0;
-                        const cx<T> l = F[(sa >> 1) * 64 + (sb >> 1)];
-                        const cx<T> d = F[4096 + (sa >> 1) * 64 + (sb >> 1)];
-                        s.x += sg * l.x + 0.25 * d.x;
-                        s.y += sg * l.y + 0.25 * d.y;
-                    }
-                }
-                a[i][j] = cx<T>{(T)-s.x, (T)-s.y};
+    each([&](int p, int q, cx<T>& x) {
+        const int u = max(p, q), w = min(p, q);
+        x = cx<T>{0, 0};
+        if (grp == 1 || u >= n) return;
+        c64 s = cst[0];
+        for (int i = nptr[u]; i < nptr[u + 1]; i++) {
+            const int sa = nseg[i];
+            for (int k = nptr[w]; k < nptr[w + 1]; k++) {
+                const int sb = nseg[k];
+                const double sg = ((sa ^ sb) & 1) ? -1.0 : 1.0;
+                const cx<T> l = F[(sa >> 1) * 64 + (sb >> 1)];
+                const cx<T> d = F[4096 + (sa >> 1) * 64 + (sb >> 1)];
+                s.x += sg * l.x + 0.25 * d.x;
+                s.y += sg * l.y + 0.25 * d.y;
             }
         }
-    nd_sweep64(a, sh[grp], n, ty, tx, grp == 1);
-    if (grp == 0) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int p = ty + 16 * i, q = tx + 16 * j;
-                S[p * 64 + q] = p < n && q < n ? a[i][j] : cx<T>{0, 0};
-            }
-    }
+        x = cx<T>{(T)-s.x, (T)-s.y};
+    });
+    nd_sweep64(a, sh[0], n, wave, lane, grp == 1);
+    if (grp == 0)
+        each([&](int p, int q, cx<T>& x) { S[p * 64 + q] = p < n && q < n ? x : cx<T>{0, 0}; });
     __syncthreads();
     // the four lanes' parts of row rw of the inverse and of the matrix (zero beyond
     // m; x is finite there)
