@@ -61,7 +61,7 @@ def test_fill_terms_vs_oracle(glen):
         assert np.array_equal(g, l)
 
 
-@pytest.mark.parametrize("m,nf", [(1, 3), (16, 5), (17, 1), (33, 70), (150, 9)])
+@pytest.mark.parametrize("m,nf", [(1, 3), (16, 5), (17, 1), (33, 70), (150, 9), (256, 9), (257, 9)])
 def test_group_fill_matches_single_samples(m, nf):
     """Tiles and sample ranges of a group: U[inj] of a sweep solved in one group
     and one sample at a time."""

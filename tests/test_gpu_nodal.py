@@ -1,7 +1,7 @@
 """GPU test of the hybrid plan's nodal solve (explicit symmetric inverses with
 refinement) against the pivoted Z_L-first FP64 factor of the assembled W, at
 the sizes where its kernels change shape: segment and node counts around the
-16-row strips, the 64-row tiles and the 64- / 128-column steps (600 rows), one
+16-row strips, the 64-row tiles and the 64-, 128- and 256-column steps, one
 segment, and the route out of it (a zero frequency makes Z_L vanish, so the
 nodal solve cannot accept and the pivoted factor answers).
 
@@ -62,6 +62,12 @@ def test_conductors_at_tile_edges(m):
 @pytest.mark.parametrize("shape", [(2, 2, 3, 2), (7, 5, 5, 4), (9, 8, 5, 5), (11, 8, 4, 5)])
 def test_grids_across_the_step_widths(shape):
     _compare(*_grid(*shape), f=[100.0, 2e5])
+
+
+# around the order from which complex64 takes 256-column steps, and its second step
+@pytest.mark.parametrize("m", [299, 300, 321, 511, 513])
+def test_conductors_across_wide_steps(m):
+    _compare(*_rod(m), f=[1e4, 3e6])
 
 
 def test_mhem_blocks():

@@ -403,9 +403,11 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 1) void k_nd_diag(NdPhase
     });
 }
 
-// O_t and T_t of 64 rows: four waves of 16 rows and 64 columns. O_t passes
-// through LDS from the MFMA result layout to the operand layout (each wave its
-// own rows).
+// O_t and T_t of 64 rows: four waves of 16 rows and 64 columns, which need no
+// barrier: O_t and T_t pass through LDS from the MFMA result layout to the
+// operand layout within a wave, so that both are stored a 16-byte fragment per
+// lane. Bound by the MFMAs (200 matrices of order 400: 36 us a panel, 55 with
+// 8-byte stores and the rows before the step read across the tiles' rows).
 template <typename T, int NB>
 __global__ __launch_bounds__(256) void k_nd_panel(NdPhase<T> p, int c0, int t)
 {
@@ -735,40 +737,64 @@ __global__ __launch_bounds__(1024) void k_nd_const(NdArgs<T> g)
     }
 }
 
-// -S_p on and below the diagonal (16 x 16 entries per work-group, zero past
-// n): four gathered entries of Y_L and Y_T per pair of segment ends.
+// -S_p on and below the diagonal (zero past n): an entry of Y_L and of Y_T per
+// pair of segment ends. 16 x 64 entries per work-group, a wave four rows: the
+// rows' lists are scalar loads, a lane keeps the first two segments of its column
+// (inside a conductor a node has two), and their four entries are loaded at once;
+// a chain of list and entry loads per entry took 1.58 ms for 96 systems of 1221
+// nodes, latency-bound.
 template <typename T>
 __global__ __launch_bounds__(256) void k_nd_schur(NdArgs<T> g)
 {
-    const int nt = (int)(g.np / 16), ntri = nt * (nt + 1) / 2;
-    const long flat = xcd_flat((long)g.nb * ntri);
+    const int nt = (int)(g.np / 64), per = nt * (nt + 1) / 2 * 4;
+    const long flat = xcd_flat((long)g.nb * per);
     if (flat < 0) return;
-    const long item = flat / ntri;
+    const long item = flat / per;
+    const int e = (int)(flat % per);
     int ti, tj;
-    tri_tile((int)(flat % ntri), ti, tj);
-    const long u = ti * 16 + (threadIdx.x >> 4), w = tj * 16 + (threadIdx.x & 15);
+    tri_tile(e >> 2, ti, tj);
+    const int n = (int)g.n, w = tj * 64 + (threadIdx.x & 63);
+    // (the wave's rows are uniform, so their lists are read by scalar loads)
+    const int u0 = ti * 64 + (e & 3) * 16 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 4;
     const cx<T>* yl = g.F + 2 * item * g.mp * g.mp;
     const cx<T>* yt = yl + g.mp * g.mp;
-    cx<T> o{0, 0};
-    if (u < g.n && w < g.n) {
-        const int p0 = g.node_ptr[u], p1 = g.node_ptr[u + 1];
-        const int q0 = g.node_ptr[w], q1 = g.node_ptr[w + 1];
-        c64 s = g.cst[4 * item];
-        for (int p = p0; p < p1; p++) {
-            const int a = g.node_seg[p];
-            const cx<T>* rl = yl + (a >> 1) * g.mp;
-            const cx<T>* rt = yt + (a >> 1) * g.mp;
-            for (int q = q0; q < q1; q++) {
-                const int b = g.node_seg[q];
-                const double sg = ((a ^ b) & 1) ? -1.0 : 1.0;
-                const cx<T> l = rl[b >> 1], t = rt[b >> 1];
-                s.x += sg * l.x + 0.25 * t.x;
-                s.y += sg * l.y + 0.25 * t.y;
-            }
-        }
-        o = cx<T>{(T)-s.x, (T)-s.y};
+    const c64 s0 = g.cst[4 * item];
+    int q0 = 0, q1 = 0, b0 = 0, b1 = 0;
+    if (w < n) {
+        q0 = g.node_ptr[w];
+        q1 = g.node_ptr[w + 1];
+        if (q1 > q0) b0 = g.node_seg[q0];
+        b1 = q1 > q0 + 1 ? g.node_seg[q0 + 1] : b0;
     }
-    g.S[item * g.np * g.np + u * g.np + w] = o;
+    const bool has0 = q1 > q0, has1 = q1 > q0 + 1;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int u = u0 + r;
+        cx<T> o{0, 0};
+        if (u < n) {
+            c64 s = s0;
+            const int p1 = g.node_ptr[u + 1];
+            for (int p = g.node_ptr[u]; p < p1; p++) {
+                const int a = g.node_seg[p];
+                const cx<T>* rl = yl + (a >> 1) * g.mp;
+                const cx<T>* rt = yt + (a >> 1) * g.mp;
+                auto add = [&](bool on, int b, cx<T> l, cx<T> t) {
+                    const double sg = ((a ^ b) & 1) ? -1.0 : 1.0;
+                    const c64 x{s.x + (sg * l.x + 0.25 * t.x), s.y + (sg * l.y + 0.25 * t.y)};
+                    s = csel(on, x, s);
+                };
+                const cx<T> l0 = rl[b0 >> 1], t0 = rt[b0 >> 1], l1 = rl[b1 >> 1], t1 = rt[b1 >> 1];
+                add(has0, b0, l0, t0);
+                add(has1, b1, l1, t1);
+                for (int q = q0 + 2; q < q1; q++) {
+                    const int b = g.node_seg[q];
+                    add(true, b, rl[b >> 1], rt[b >> 1]);
+                }
+            }
+            if (w < n) o = cx<T>{(T)-s.x, (T)-s.y};
+        }
+        g.S[item * g.np * g.np + (long)u * g.np + w] = o;
+    }
 }
 
 // out = M in for symmetric matrices, four rows per wave, 16 bytes per lane and
@@ -1309,7 +1335,10 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
 // ---------------------------------------------------------------------------
 // Columns per sweep step. A step reads and writes every tile once, which at 64
 // columns takes as long as its MFMAs; more blocks per step cost the panels'
-// products with the step's earlier blocks.
+// products with the step's earlier blocks. In complex64 256 columns win from
+// order 300 on (200 samples of order 400: 5.39 against 5.71 ms with 128; 96 of
+// order 1320: 38.1 against 40.6 ms); complex128, whose products take four times
+// as long per byte, gains nothing past 128.
 constexpr long kWide = 300;
 static int nd_block(long dim, bool f64)
 {
@@ -1521,8 +1550,8 @@ int NodalSolver::factor()
         Timed tm(pr, FAM_OTHER, st);
         hipLaunchKernelGGL(k_nd_rows<T>, dim3((unsigned)(nb * ((m + 3) / 4))), dim3(256), 0, st, g);
         hipLaunchKernelGGL(k_nd_const<T>, dim3(nb), dim3(1024), 0, st, g);
-        const long n16 = np / 16;
-        hipLaunchKernelGGL(k_nd_schur<T>, dim3(xcd_grid((long)nb * (n16 * (n16 + 1) / 2))),
+        const long n64 = np / 64;
+        hipLaunchKernelGGL(k_nd_schur<T>, dim3(xcd_grid((long)nb * (n64 * (n64 + 1) / 2 * 4))),
                            dim3(256), 0, st, g);
         tm.end();
     }
