@@ -433,10 +433,10 @@ enum tags_formulation { TAGS_FORM_HEM = 0, TAGS_FORM_MHEM = 1 };
 int tags_sweep_set_formulation(tags_sweep *sw, int formulation);
 
 /* Refinement of nodal complex64 factors (TAGS_PLAN_NODAL, mixed form; the
- * hybrid plan's nodal solve refines classically at every frequency): a sample at |s| / 2 pi < below_hz (default 2e4 Hz) refines by
- * FGMRES in FP64 right-preconditioned by the complex64 factor, `steps`
- * (1 .. 32, default 6) Arnoldi steps per refinement step (GMRES-based
- * refinement), where the classic correction from the factor alone converges
+ * hybrid plan's nodal solve refines classically at every frequency): a
+ * sample at |s| / 2 pi < below_hz (default 2e4 Hz) refines by FGMRES in FP64
+ * right-preconditioned by the complex64 factor, `steps` (1 .. 32, default 6)
+ * Arnoldi steps per refinement step (GMRES-based refinement), where the classic correction from the factor alone converges
  * slowly or not at all (the node block's Schur complement is dominated by
  * A^T Z_L^-1 A, whose complex64 rounding swamps the grounding terms at low
  * frequency); a higher one refines classically. No counterpart in the
@@ -452,8 +452,10 @@ int tags_sweep_set_gmres(tags_sweep *sw, double below_hz, int steps);
  * or TAGS_ERR_ARG for hz < 0. */
 int tags_sweep_set_nodal_above(tags_sweep *sw, double hz);
 
-/* Frequency samples per group (0 .. 4096; 0, the default, chooses from N: one
- * sample from N = 8192 up, else as many as keep a group's matrices within
+/* Frequency samples per group (0 .. 4096; 0, the default, chooses from N. The
+ * hybrid plan's nodal solve: two samples from N = 8192 up, else as many as keep
+ * a group's buffers within 16 GiB, at most 128, shared evenly. The other plans:
+ * one sample from N = 8192 up, else as many as keep a group's matrices within
  * 16 GiB, at most 64). A group's samples are assembled, factored, solved and
  * refined together: every kernel launch covers all of them (one work-group
  * grid per sample, side by side), so that mid-size systems fill the device.

@@ -283,9 +283,6 @@ struct Solver {
 
     const LUPlan* plan = nullptr;  // nullptr: dense partial pivoting
     const LUPlan* plan32 = nullptr;  // plan of the mixed form's factor (nullptr: `plan`)
-    // a second complex64 plan tried, on the intact W, when the refinement with
-    // plan32 fails, before the FP64 factor (nullptr: none)
-    const LUPlan* plan32_retry = nullptr;
     bool equilibrate = false;      // symmetric row-max scaling before the FP32 factor
                                    // (not applied with grounding)
 
@@ -449,9 +446,8 @@ struct Solver {
     // them (masked to those items) and returns with *complete false; then it
     // accepts an item's last iterate at a backward error <= kAccept and
     // |dx| / |x| <= kFwdAccept. An item that fails, or whose complex64 factor
-    // broke down, starts again alone with plan32_retry's complex64 factor if
-    // one is set, else the FP64 factor of its intact W gives its answer (these
-    // wait). Solutions in `bvec`; stt (nullable) and info (nullable) receive
+    // broke down, gets its answer from the FP64 factor of its intact W, alone
+    // (these wait). Solutions in `bvec`; stt (nullable) and info (nullable) receive
     // each item's. Returns 0, an error, or for one item its info.
     std::vector<int> m_info32, m_done, m_go;
     std::vector<double> m_berr, m_fwd;
@@ -581,8 +577,6 @@ struct Solver {
         }
         int first = 0;
         // items that failed, one at a time on the intact W of each
-        const LUPlan* retry = plan32_retry;
-        const LUPlan* p32 = plan32;
         for (int z : failed) {
             c64* Wz = W + (long)z * sWi;
             c64* bz = bvec + (long)z * n;
@@ -592,26 +586,10 @@ struct Solver {
             // b_z again (bvec holds the failed iterate)
             TAGS_HIP(hipMemcpyAsync(bz, b + (long)z * n, sizeof(c64) * n, hipMemcpyDeviceToDevice,
                                     st));
-            if (retry) {
-                // the second complex64 plan, with classic refinement; its steps
-                // add to this one's
-                const int gk = gmres_k;
-                plan32 = retry;
-                plan32_retry = nullptr;
-                gmres_k = 0;
-                rc = issue_mixed(Wz, bz);
-                if (!rc) rc = finish_mixed(Wz, bz, sz);
-                plan32 = p32;
-                plan32_retry = retry;
-                gmres_k = gk;
-                if (rc >= 0) sz->refine_iters += done[z];
-            } else {
-                // FP64 fallback on the intact W
-                rc = issue64(Wz, bz);
-                if (!rc) rc = finish64(sz);
-                if (rc >= 0) sz->refine_iters = done[z];
-            }
+            rc = issue64(Wz, bz);
+            if (!rc) rc = finish64(sz);
             if (rc < 0) return rc;
+            sz->refine_iters = done[z];
             if (info) info[z] = rc;
             if (!first) first = rc;
             TAGS_HIP(hipStreamSynchronize(st));
@@ -2099,7 +2077,6 @@ static void slot_bind(tags_sweep* sw, SweepSlot& sl)
     sl.bound_kind = sw->layout_kind;
     sl.sv.plan = sw->bind64;
     sl.sv.plan32 = sw->bind32;
-    sl.sv.plan32_retry = nullptr;
     sl.sv.ground = sw->bindgr;
     sl.sv.gmres_k = 0;
     sl.sv.hem = &sw->hem;
