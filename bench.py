@@ -294,9 +294,15 @@ def _timed_solve(T, obj, prec, *args):
     return r, time.perf_counter() - t0
 
 
-def gemm_basis(mixed, tuning):
+def gemm_basis(mixed, tuning, plan=7):
     """(kernel label, peak TFLOP/s, what the peak is) of the trailing update's
-    large products under a tuning (a dict with gemm_big, or the defaults)."""
+    large products under a tuning (a dict with gemm_big, or the defaults). The
+    hybrid plan inverts symmetric blocks, whose update has one shape."""
+    if plan == 7:
+        if mixed:
+            return ("k_nd_update<float> (symmetric, three real products per complex one)",
+                    PEAK["fp32"], "fp32 dense MFMA peak")
+        return "k_nd_update<double> (symmetric)", PEAK["fp64"], "fp64 dense MFMA peak"
     big = tuning.get("gemm_big", -1) if isinstance(tuning, dict) else -1
     if big < 0:
         big = DEFAULT_BIG["mixed" if mixed else "fp64"]
@@ -356,7 +362,7 @@ def sweep_config(T, e, nodes, inj, s, kap, plan=7, tuning=("table", TUNING_TABLE
         sw.set_profiling(False)
         us[name] = u
         r = {"samples_per_s": len(s) / dt, "s": dt,
-             "roofline": _roofline(tm, gemm_basis(prec == T.PREC_MIXED, tu)),
+             "roofline": _roofline(tm, gemm_basis(prec == T.PREC_MIXED, tu, plan)),
              "executed_gemm_flops_per_sample": tm["gemm_flops"] / len(s),
              "tuning": tu}
         if prec == T.PREC_MIXED:
@@ -541,11 +547,11 @@ def main():
     ap.add_argument("--plan-mixed", type=int, default=7,
                     help="LU plan of the mixed form: 0 dense, 1 structured, 2 Z_L first, "
                          "3 Z_L-block pivoting, 4 grounded without row exchanges, 5 "
-                         "grounded with pivoting, 6 nodal, 7 hybrid (default: nodal "
-                         "complex64 factor from --nodal-above, Z_L first below)")
+                         "grounded with pivoting, 6 nodal, 7 hybrid (default: the nodal "
+                         "solve from --nodal-above, Z_L first below)")
     ap.add_argument("--nodal-above", type=float, default=0.0,
                     help="switch frequency of the hybrid plan (Hz, default 0: the nodal "
-                         "complex64 factor at every frequency)")
+                         "solve at every frequency)")
     ap.add_argument("--gmres-below", type=float, default=2e4,
                     help="nodal factors below this frequency refine by FGMRES (Hz, "
                          "default 2e4)")
@@ -769,13 +775,15 @@ def main():
         out["rel_err_zh_vs_fp64_per_sample"] = [float(v) for v in
                                                 np.abs(u_mx - u64) / np.abs(u64)]
     ach = tm_mx["trailing_flops"] / tm_mx["trailing_ms"] / 1e9 if tm_mx["trailing_ms"] > 0 else 0.0
-    kernel, peak, what = gemm_basis(True, tuned[T.PREC_MIXED])
+    kernel, peak, what = gemm_basis(True, tuned[T.PREC_MIXED], args.plan_mixed)
     x6 = "bf16" in what
+    lu = args.plan_mixed != 7
     out["roofline"] = {"bound": "mfma", "achieved": ach, "peak": peak,
                        "unit": "TFLOP/s", "frac": ach / peak, "peak_basis": what,
-                       "traffic": measured_traffic(x6),
-                       "kernel": "%s (A22 -= L21 U12, K=%d); products under 512 tiles: the "
-                                 "small variant" % (kernel, width_of(T.PREC_MIXED)),
+                       "traffic": measured_traffic(x6) if lu else None,
+                       "kernel": ("%s (A22 -= L21 U12, K=%d); products under 512 tiles: the "
+                                  "small variant" % (kernel, width_of(T.PREC_MIXED)) if lu
+                                  else "%s, K=256" % kernel),
                        "launches": tm_mx["trailing_launches"],
                        "avg_launch_ms": tm_mx["trailing_ms"] / max(1, tm_mx["trailing_launches"]),
                        "measured_in": ("the timed samples" if one else
