@@ -966,7 +966,10 @@ __global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, doubl
                                                     c64* cf)
 {
     __shared__ c64 ex[64];
+    __shared__ double tab[256];  // cos(pi j / 128): k theta_p is a multiple of pi / 128
     const int p = threadIdx.x;
+#pragma unroll
+    for (int j = p; j < 256; j += 64) tab[j] = cospi(j / 128.0);
     const c64 g = scs[blockIdx.x].gamma;
     const double x = D * cospi((p + 0.5) / 64.0);
     double sn, cs;
@@ -976,8 +979,9 @@ __global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, doubl
     __syncthreads();
     if (p >= K) return;
     c64 s{0, 0};
+#pragma unroll 8
     for (int q = 0; q < 64; q++) {
-        const double w = cospi(p * (q + 0.5) / 64.0);
+        const double w = tab[p * (2 * q + 1) & 255];
         s.x = fma(w, ex[q].x, s.x);
         s.y = fma(w, ex[q].y, s.y);
     }

@@ -46,7 +46,6 @@ struct NodalSolver {
     void *tp = nullptr, *op_ = nullptr, *P = nullptr;
     c64 *x = nullptr, *r = nullptr, *b = nullptr, *ysum = nullptr, *dg = nullptr, *cst = nullptr;
     void *v = nullptr, *z = nullptr, *f = nullptr, *y = nullptr, *h = nullptr, *c = nullptr;
-    c64* u = nullptr;
     unsigned long long* norms = nullptr;
     int* active = nullptr;
 

@@ -1015,11 +1015,14 @@ __global__ __launch_bounds__(256) void k_nd_init(NdArgs<T> g, c64* b)
     if (i < g.np) g.f[item * g.np + i] = zero;
 }
 
+// What the host reads, written straight into its pinned copies (one launch in
+// place of a gather and two copies of 4 us each)
 template <typename T>
-__global__ __launch_bounds__(256) void k_nd_pick(NdArgs<T> g, c64* u)
+__global__ __launch_bounds__(256) void k_nd_pick(NdArgs<T> g, c64* u, unsigned long long* norms)
 {
-    const int q = blockIdx.x * 256 + threadIdx.x;
+    const long q = (long)blockIdx.x * 256 + threadIdx.x;
     if (q < g.nb) u[q] = g.x[q * g.N + 2 * g.m + g.inj];
+    if (q < g.nb * g.snorm) norms[q] = g.norms[q];
 }
 
 // ---------------------------------------------------------------------------
@@ -1035,10 +1038,13 @@ __device__ inline void bits_max(unsigned long long& m, double a)
 // node system, its inverse, and `spec` refinement steps, by one work-group, with
 // the operations of the kernels above and the vectors in LDS. The blocks, S^-1
 // and the vectors are left where those kernels take further steps from. As
-// separate launches the same work is 25 of 4 to 6 us each beside two sweeps.
+// separate launches the same work is 25 of 4 to 6 us each beside two sweeps; here
+// 59 us for one sample of 30 segments in complex128 (107 with a pivot at a time
+// and the rows read again for every product), 64 for a hundred in complex64:
+// chains of dependent steps.
 template <typename T>
 __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, long sZ, c64* ball,
-                                                   int spec)
+                                                   int spec, c64* hu, unsigned long long* hnorms)
 {
     const long item = blockIdx.x;
     const int t = threadIdx.x, grp = t >> 8;
@@ -1319,8 +1325,12 @@ __global__ __launch_bounds__(512) void k_nd_small(NdArgs<T> g, const c64* Zall, 
         ro[i] = r[i];
         ball[item * N + i] = c64{i == 2 * m + g.inj ? 1.0 : 0.0, 0.0};
     }
-    for (int i = t; i < g.snorm; i += 512)
-        g.norms[item * g.snorm + i] = i < 4 * (spec + 1) ? nrm[i] : 0;
+    for (int i = t; i < g.snorm; i += 512) {
+        const unsigned long long v = i < 4 * (spec + 1) ? nrm[i] : 0;
+        g.norms[item * g.snorm + i] = v;
+        hnorms[item * g.snorm + i] = v;
+    }
+    if (t == 0) hu[item] = x[2 * m + g.inj];
     if (t < 128) g.v[128 * item + t] = v[t >> 6][t & 63];
     if (t < 64) {
         g.f[64 * item + t] = f[t];
@@ -1380,7 +1390,6 @@ size_t NodalSolver::partition(char* base, int batch)
     y = take(e * np * B);
     h = take(e * np * B);
     c = take(e * np * B);
-    u = (c64*)take(sizeof(c64) * B);
     norms = (unsigned long long*)take(sizeof(unsigned long long) * kNormStride * B);
     active = (int*)take(sizeof(int) * B);
     return off;
@@ -1606,14 +1615,16 @@ int NodalSolver::issue(int nb_, long inj_)
         Timed tm(pr, FAM_SOLVE, st);
         if (f64)
             hipLaunchKernelGGL(k_nd_small<double>, dim3(nb), dim3(512), 0, st,
-                               nd_args<double>(*this, false), (const c64*)Z, sZ, b, step_);
+                               nd_args<double>(*this, false), (const c64*)Z, sZ, b, step_, hu,
+                               hnorms);
         else
             hipLaunchKernelGGL(k_nd_small<float>, dim3(nb), dim3(512), 0, st,
-                               nd_args<float>(*this, false), (const c64*)Z, sZ, b, step_);
+                               nd_args<float>(*this, false), (const c64*)Z, sZ, b, step_, hu,
+                               hnorms);
         TAGS_HIP(hipGetLastError());
         tm.end();
         first_ = true;
-        return queue_results();
+        return 0;
     }
     const long w = std::max(std::max(N, 2 * mp), std::max(np, kNormStride));
     const dim3 gi((unsigned)((w + 255) / 256), nb);
@@ -1653,13 +1664,14 @@ int NodalSolver::queue_spec()
 
 int NodalSolver::queue_results()
 {
-    const dim3 g((nb + 255) / 256);
-    if (f64) hipLaunchKernelGGL(k_nd_pick<double>, g, dim3(256), 0, st, nd_args<double>(*this, false), u);
-    else hipLaunchKernelGGL(k_nd_pick<float>, g, dim3(256), 0, st, nd_args<float>(*this, false), u);
+    const dim3 g((unsigned)(((long)nb * kNormStride + 255) / 256));
+    if (f64)
+        hipLaunchKernelGGL(k_nd_pick<double>, g, dim3(256), 0, st, nd_args<double>(*this, false),
+                           hu, hnorms);
+    else
+        hipLaunchKernelGGL(k_nd_pick<float>, g, dim3(256), 0, st, nd_args<float>(*this, false), hu,
+                           hnorms);
     TAGS_HIP(hipGetLastError());
-    TAGS_HIP(hipMemcpyAsync(hnorms, norms, sizeof(unsigned long long) * kNormStride * nb,
-                            hipMemcpyDeviceToHost, st));
-    TAGS_HIP(hipMemcpyAsync(hu, u, sizeof(c64) * nb, hipMemcpyDeviceToHost, st));
     return 0;
 }
 
