@@ -16,6 +16,7 @@
 #include <complex>
 #include <vector>
 
+#include "dd.h"
 #include "hostcopy.h"
 
 namespace tags {
@@ -137,11 +138,36 @@ static int dft_batch(c64* buf, c64* tmp, const c64* w, long n, long batch, bool 
     return 0;
 }
 
-// w[t] = exp(-2 pi i t / n), t < n. The angle 2 t / n (in units of pi) is
-// reduced to at most 1/4 by symmetries of the integers, exactly; what rounding
-// leaves of the division is put back to first order, so that the values are
-// within an ulp. (In extended precision on the host the table took 3 ms at
-// n = 16,384, more than the transforms.)
+// Double-double products and quotients for the twiddles (a sum hi + lo, |lo|
+// at most half an ulp of hi)
+__device__ inline DD dd_norm(double hi, double lo)
+{
+    const double s = hi + lo;
+    return DD{s, lo - (s - hi)};
+}
+__device__ inline DD dd_mul(DD a, DD b)
+{
+    const double p = a.hi * b.hi;
+    return dd_norm(p, fma(a.hi, b.hi, -p) + fma(a.hi, b.lo, a.lo * b.hi));
+}
+__device__ inline DD dd_div(DD a, double d)
+{
+    const double q = a.hi / d;
+    return dd_norm(q, (fma(-q, d, a.hi) + a.lo) / d);
+}
+__device__ inline DD dd_sum(DD a, DD b)
+{
+    const DD s = dd_plus(a, b);
+    return dd_norm(s.hi, s.lo);
+}
+
+// w[t] = exp(-2 pi i t / n), t < n, rounded from double-double Taylor sums: the
+// table's rounding is part of the transforms' error (a transform pair at n =
+// 16,384: 2.2e-12, against 2.4e-12 with entries only within an ulp), and the
+// kernel takes 6 us. The
+// angle is reduced to at most pi / 4 by symmetries of the integers, exactly. (In
+// extended precision on the host the table took 3 ms there, more than the
+// transforms.)
 __global__ __launch_bounds__(256) void k_twiddles(c64* w, long n)
 {
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
@@ -150,11 +176,17 @@ __global__ __launch_bounds__(256) void k_twiddles(c64* w, long n)
     // pi num / (4 n), |num| <= n
     const long q = (8 * t / n + 1) / 2;
     const long num = 8 * t - 2 * q * n;
-    const double d = 4.0 * (double)n, x = (double)num / d;
-    const double lo = fma(-x, d, (double)num) / d * 3.14159265358979323846;
-    double s, c;
-    sincospi(x, &s, &c);
-    const double s1 = fma(c, lo, s), c1 = fma(-s, lo, c);
+    const DD pi4{0.78539816339744828, 3.0616169978683830e-17};
+    const DD x = dd_mul(dd_div(DD{(double)num, 0.0}, (double)n), pi4), x2 = dd_mul(x, x);
+    DD ts = x, tc{1.0, 0.0}, ss = ts, sc = tc;
+    // |x|^27 / 27! is 1e-31 of x at most
+    for (int k = 1; k <= 12; k++) {
+        tc = dd_div(dd_mul(tc, x2), -(double)((2 * k - 1) * (2 * k)));
+        ts = dd_div(dd_mul(ts, x2), -(double)((2 * k) * (2 * k + 1)));
+        sc = dd_sum(sc, tc);
+        ss = dd_sum(ss, ts);
+    }
+    const double c1 = sc.hi, s1 = ss.hi;
     // rotate by q quarter turns: exp(-i (angle + q pi / 2))
     double re = c1, im = -s1;
     switch (q & 3) {
