@@ -200,3 +200,32 @@ def test_transform_twiddles(nt):
     back = T.inv_laplace_trans(g, s, tmax, nt)
     scale = np.exp(c * k * dt) / (nt * dt)
     assert np.max(np.abs(back - h * scale) / scale) <= 1e-12 * np.abs(h).max()
+
+
+@pytest.mark.parametrize("nt", [7, 1001, 9999])
+def test_transform_twiddles_are_rounded_once(nt):
+    """The table's entries themselves: the direct sum of an impulse at sample 1
+    of height f is f v w^k, v its weight, exactly w^k where f v rounds to a power
+    of two (one of the neighbouring f does; sample k = 0 shows which). Against
+    extended-precision cosines and sines: 0.505 ulp, a correct rounding and what
+    the reference's own 64-bit mantissa and the angle's leave open."""
+    tmax = 1e-4
+    c, dt = np.log(float(nt) ** 2) / tmax, tmax / (nt - 1)
+    f0 = 2.0 ** 10 / (dt * np.exp(-c * dt))
+    f = np.zeros((41, nt))
+    f[:, 1] = f0 * (1.0 + np.arange(-20, 21) * 2.0 ** -52)
+    g, s = T.laplace_trans(f, tmax)
+    exact = np.nonzero(g[:, 0] == 2.0 ** 10)[0]
+    assert len(exact) > 0
+    w = g[exact[0]] * 2.0 ** -10
+    # the angle less the nearest multiple q of a quarter turn, so that its rounding
+    # is relative: pi num / (4 nt)
+    k = np.arange(len(w))
+    q = (8 * k // nt + 1) // 2
+    x = np.longdouble("3.14159265358979323846264338327950288") * (8 * k - 2 * q * nt) / (4 * nt)
+    cs, sn = np.cos(x), np.sin(x)
+    re = np.choose(q % 4, [cs, -sn, -cs, sn])
+    im = np.choose(q % 4, [-sn, -cs, sn, cs])
+    for got, ref in ((w.real, re), (w.imag, im)):
+        ulp = np.spacing(np.abs(ref.astype(float)))
+        assert np.max(np.abs(got - ref) / ulp) <= 0.505

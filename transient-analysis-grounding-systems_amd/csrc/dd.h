@@ -1,4 +1,5 @@
-// Double-double sums for the refinement's residuals.
+// Double-double arithmetic: sums for the refinement's residuals, products and
+// quotients for the transforms' twiddles.
 #pragma once
 
 #include "tags_common.h"
@@ -55,6 +56,32 @@ __device__ inline double dd_sub_from(double b, DD d)
     DD t{b, 0.0};
     dd_add(t, -d.hi);
     return t.hi + (t.lo - d.lo);
+}
+
+// Normalised values (|lo| at most half an ulp of hi)
+__device__ inline DD dd_norm(double hi, double lo)
+{
+#pragma clang fp contract(off)
+    const double s = hi + lo;
+    return DD{s, lo - (s - hi)};
+}
+__device__ inline DD dd_mul(DD a, DD b)
+{
+#pragma clang fp contract(off)
+    const double p = a.hi * b.hi;
+    return dd_norm(p, fma(a.hi, b.hi, -p) + fma(a.hi, b.lo, a.lo * b.hi));
+}
+__device__ inline DD dd_div(DD a, double d)
+{
+#pragma clang fp contract(off)
+    const double q = a.hi / d;
+    return dd_norm(q, (fma(-q, d, a.hi) + a.lo) / d);
+}
+__device__ inline DD dd_sum(DD a, DD b)
+{
+#pragma clang fp contract(off)
+    const DD s = dd_plus(a, b);
+    return dd_norm(s.hi, s.lo);
 }
 
 }  // namespace tags

@@ -138,36 +138,13 @@ static int dft_batch(c64* buf, c64* tmp, const c64* w, long n, long batch, bool 
     return 0;
 }
 
-// Double-double products and quotients for the twiddles (a sum hi + lo, |lo|
-// at most half an ulp of hi)
-__device__ inline DD dd_norm(double hi, double lo)
-{
-    const double s = hi + lo;
-    return DD{s, lo - (s - hi)};
-}
-__device__ inline DD dd_mul(DD a, DD b)
-{
-    const double p = a.hi * b.hi;
-    return dd_norm(p, fma(a.hi, b.hi, -p) + fma(a.hi, b.lo, a.lo * b.hi));
-}
-__device__ inline DD dd_div(DD a, double d)
-{
-    const double q = a.hi / d;
-    return dd_norm(q, (fma(-q, d, a.hi) + a.lo) / d);
-}
-__device__ inline DD dd_sum(DD a, DD b)
-{
-    const DD s = dd_plus(a, b);
-    return dd_norm(s.hi, s.lo);
-}
-
-// w[t] = exp(-2 pi i t / n), t < n, rounded from double-double Taylor sums: the
-// table's rounding is part of the transforms' error (a transform pair at n =
-// 16,384: 2.2e-12, against 2.4e-12 with entries only within an ulp), and the
-// kernel takes 6 us. The
-// angle is reduced to at most pi / 4 by symmetries of the integers, exactly. (In
-// extended precision on the host the table took 3 ms there, more than the
-// transforms.)
+// w[t] = exp(-2 pi i t / n), t < n, rounded from double-double Taylor sums, to
+// the nearest double (0.500 ulp over n = 1001, 9999, 16,383 and 16,384; with the
+// products contracted, whose error terms then count twice, 1.3 ulp): the table's
+// rounding is part of the transforms' error (a transform pair at n = 16,384:
+// 1.9e-12). The angle is reduced to at most pi / 4 by symmetries of the integers,
+// exactly. (In extended precision on the host the table took 3 ms there, more
+// than the transforms.)
 __global__ __launch_bounds__(256) void k_twiddles(c64* w, long n)
 {
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
