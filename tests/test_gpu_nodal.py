@@ -89,3 +89,32 @@ def test_zero_frequency_takes_the_pivoted_factor():
         assert np.array_equal(np.isfinite(u), ok)
         assert np.all(np.abs(u - u0)[ok] <= 1e-8 * np.abs(u0[ok]))
     sw.close()
+
+
+@pytest.mark.parametrize("inflight", [1, 4])
+def test_a_rejected_sample_leaves_the_others_alone(inflight):
+    """Samples around ones that the nodal solve does not accept (zero frequency)
+    answer bit for bit as in a call without them, in both forms, one sample a
+    group and on one slot or several; the rejected ones as the pivoted plan does
+    (1e-9, as the other comparisons with it), whether they share a group or not."""
+    e, nodes = _rod(70)
+    f = np.array([50.0, 0.0, 3e3, 0.0, 1e5, 0.0, 2e6])
+    s = 2j * np.pi * f
+    kap = 2e-3 + s * 12.0 * T.EPS0
+    z = f == 0
+    sw = T.Sweep(e, nodes)
+    sw.set_inflight(inflight)
+    for prec in (T.PREC_FP64, T.PREC_MIXED):
+        sw.set_plan(T.PLAN_ZL_FIRST)
+        p = sw.solve(s, kap, 3, prec)[0]
+        sw.set_plan(T.PLAN_HYBRID)
+        sw.set_batch(1)
+        u, st, x = sw.solve(s, kap, 3, prec, want_x=True)
+        v, sv, y = sw.solve(s[~z], kap[~z], 3, prec, want_x=True)
+        assert np.array_equal(u[~z], v) and np.array_equal(x[~z], y)
+        assert [q["refine_iters"] for q, r in zip(st, z) if not r] == [q["refine_iters"] for q in sv]
+        sw.set_batch(0)
+        w = sw.solve(s, kap, 3, prec)[0]
+        for got in (u, w):
+            assert np.allclose(got[z], p[z], rtol=1e-9, atol=0.0, equal_nan=True)
+    sw.close()

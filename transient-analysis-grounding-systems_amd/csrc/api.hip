@@ -1906,11 +1906,11 @@ struct SweepSlot {
     int cap = 0;
     const tags_sweep* bound = nullptr;  // the sweep whose plans the solver holds
     int bound_kind = -1;                // and its plan kind then
-    long f = -1;            // first sample of the group in flight (-1: idle)
-    int cnt = 0;            // its samples f .. f + cnt - 1
+    std::vector<size_t> at;            // the samples of the group in flight (none: idle)
     std::vector<tags_item_stats> stt;  // their statistics and infos, filled as they finish
     std::vector<int> info;
-    std::vector<double> hz; // their frequencies |s| / 2 pi
+    std::vector<int> spent; // refinement steps of a rejected nodal solve before this one
+    bool busy() const { return !at.empty(); }
     size_t w_cap = 0, rhs_cap = 0;  // allocated elements of W and rhs
     // items [0, static_items) of W hold the frequency-independent part (zero
     // and incidence blocks) of static_sw's layout static_kind: the mixed form
@@ -2021,10 +2021,9 @@ struct tags_sweep {
     tags::LUPlan plan32;
     // TAGS_PLAN_HYBRID: solved by NodalSolver where every segment has two
     // nodes (nodal_ok), in the mixed form at and above nodal_above Hz; a sample
-    // that misses its acceptance rule is factored by ZL_FIRST and, for the rest
-    // of the call, raises the switch to 1.5 times its frequency (mixed) or
-    // turns the nodal solve off (nodal64)
-    bool nodal_ok = true, nodal64 = true;
+    // that misses its acceptance rule is factored by ZL_FIRST and, in the mixed
+    // form, raises the switch to 1.5 times its frequency for the rest of the call
+    bool nodal_ok = true;
     int nd_batch = 1;      // samples per group of the nodal solve
     // device copies of plan and plan32's row orders
     PlanDev plan_dev[2];
@@ -2125,7 +2124,7 @@ static int sweep_nd_batch(const tags_sweep* sw, bool mixed, size_t nfreq)
 static bool sweep_nodal(const tags_sweep* sw, bool mixed, double hz)
 {
     if (sw->plan_kind != TAGS_PLAN_HYBRID || !sw->nodal_ok) return false;
-    return mixed ? hz >= sw->nodal_above : sw->nodal64;
+    return !mixed || hz >= sw->nodal_above;
 }
 
 // The first k slots exist and are allocated for groups of sw->batch samples of
@@ -2583,52 +2582,78 @@ struct SweepCall {
     tags_item_stats* stats;
 };
 
-// Queues the group of samples starting at f on slot `sl`: up to sw->batch
-// consecutive samples that take the same complex64 factor (the hybrid plan
-// chooses per frequency); assembly, right-hand sides and the solve's first
-// half, one set of launches for the group. Returns the samples taken (> 0) or
-// an error.
-static int sweep_issue(tags_sweep* sw, SweepSlot& sl, size_t f, const SweepCall& c)
+// What a call still has to queue: samples from `next` on, and those that the
+// nodal solve did not accept (with the refinement steps it took), which go to
+// the plan's pivoted factor in groups of their own.
+struct SweepTodo {
+    size_t next = 0;
+    struct Rejected {
+        size_t f;
+        int steps;
+    };
+    std::vector<Rejected> rejected;
+    bool left(size_t nfreq) const { return next < nfreq || !rejected.empty(); }
+};
+
+static double sample_hz(const SweepCall& c, size_t q)
+{
+    const c64 sf = from_c(c.s[q]);
+    return std::hypot(sf.x, sf.y) / (2.0 * M_PI);
+}
+
+// Queues the next group of `todo` (which has samples left) on slot `sl`: up to
+// sw->batch consecutive samples that take the same complex64 factor (the hybrid
+// plan chooses per frequency), or rejected ones once they fill a group or
+// nothing else is left; assembly, right-hand sides and the solve's first half,
+// one set of launches for the group.
+static int sweep_issue(tags_sweep* sw, SweepSlot& sl, SweepTodo& todo, const SweepCall& c)
 {
     const long N = sw->N;
     const BlockLayout& L = sw->layout;
     int rc;
-    auto hz_of = [&](size_t q) {
-        const c64 sf = from_c(c.s[q]);
-        return std::hypot(sf.x, sf.y) / (2.0 * M_PI);
-    };
     const bool nodal_plan = sw->plan_kind == TAGS_PLAN_NODAL && c.mixed;
     // the sample's class: 0 the plan's own factor with classic refinement (the
     // hybrid plan's Z_L-first one), 1 a nodal complex64 factor refined by
     // FGMRES, 2 one refined classically, 3 the nodal solve
     auto cls = [&](size_t q) {
-        const double h = hz_of(q);
+        const double h = sample_hz(c, q);
         if (sweep_nodal(sw, c.mixed, h)) return 3;
         return nodal_plan ? (h < sw->gmres_below ? 1 : 2) : 0;
     };
-    const int c0 = cls(f);
-    sl.nodal_path = c0 == 3;
-    const int lim = sl.nodal_path ? sw->nd_batch : sw->batch;
-    int cnt = 0;
-    sl.hz.clear();
-    while (cnt < lim && f + cnt < c.nfreq && cls(f + cnt) == c0) {
-        sl.hz.push_back(hz_of(f + cnt));
-        cnt++;
+    std::vector<size_t> at;
+    std::vector<int> spent;
+    int c0 = 0;
+    auto& rej = todo.rejected;
+    if (!rej.empty() && (rej.size() >= (size_t)sw->batch || todo.next >= c.nfreq)) {
+        const size_t take = std::min(rej.size(), (size_t)sw->batch);
+        for (size_t q = 0; q < take; q++) {
+            at.push_back(rej[q].f);
+            spent.push_back(rej[q].steps);
+        }
+        rej.erase(rej.begin(), rej.begin() + (long)take);
+    } else {
+        c0 = cls(todo.next);
+        const size_t lim = (size_t)(c0 == 3 ? sw->nd_batch : sw->batch);
+        while (at.size() < lim && todo.next < c.nfreq && cls(todo.next) == c0)
+            at.push_back(todo.next++);
+        spent.assign(at.size(), 0);
     }
+    const int cnt = (int)at.size();
+    sl.nodal_path = c0 == 3;
     sl.sv.gmres_k = c0 == 1 ? sw->gmres_steps : 0;
-    // a raised switch, or the nodal solve turned off: buffers made on the way
+    // rejected samples, or a raised switch: buffers made on the way
     if (!sl.nodal_path &&
-        ((rc = sl.init(N, sw->batch)) || (rc = sl.sv.ensure((int)N, c.mixed, sw->batch))))
+        ((rc = sl.init(N, cnt)) || (rc = sl.sv.ensure((int)N, c.mixed, cnt))))
         return rc;
-    sl.f = (long)f;
-    sl.cnt = cnt;
+    sl.at = at;
+    sl.spent = spent;
     sl.stt.assign(cnt, tags_item_stats{});
     for (auto& q : sl.stt)
         for (int i = 0; i < 8; i++) q.refine_hist[i] = -1.0;
     sl.info.assign(cnt, 0);
     hipStream_t st = sl.stream.s;
     for (int z = 0; z < cnt; z++) {
-        const size_t q = f + z;
+        const size_t q = at[z];
         sl.scal.h[z] = sample_scalars(c.s[q], c.kappa[q], c.mur, c.gamma ? &c.gamma[q] : nullptr,
                                       c.ref_l ? &c.ref_l[q] : nullptr,
                                       c.ref_t ? &c.ref_t[q] : nullptr);
@@ -2637,8 +2662,7 @@ static int sweep_issue(tags_sweep* sw, SweepSlot& sl, size_t f, const SweepCall&
         if ((rc = sweep_fill_items(sw, sl.nd.Z, st, &sl.prof, cnt, sl.scal, false, sw->m,
                                    sl.nd.sZ)))
             return rc;
-        rc = sl.nd.issue(cnt, (long)c.inj_node);
-        return rc ? rc : cnt;
+        return sl.nd.issue(cnt, (long)c.inj_node);
     }
     // the zero and incidence blocks stay from the last mixed group of this
     // sweep on this slot unless a factor in FP64 replaced W since
@@ -2656,9 +2680,8 @@ static int sweep_issue(tags_sweep* sw, SweepSlot& sl, size_t f, const SweepCall&
     hipLaunchKernelGGL(k_unit_rhs, dim3((unsigned)((N + 255) / 256), 1, (unsigned)cnt), dim3(256),
                        0, st, sl.rhs.p, N, L.node_off + (long)c.inj_node);
     TAGS_HIP(hipGetLastError());
-    rc = c.mixed ? sl.sv.issue_mixed(sl.W.p, sl.rhs.p, cnt, N * N)
-                 : sl.sv.issue64(sl.W.p, sl.rhs.p, cnt, N * N);
-    return rc ? rc : cnt;
+    return c.mixed ? sl.sv.issue_mixed(sl.W.p, sl.rhs.p, cnt, N * N)
+                   : sl.sv.issue64(sl.W.p, sl.rhs.p, cnt, N * N);
 }
 
 // Backward error of the FP64 form's solution x of sample f (W assembled again
@@ -2687,44 +2710,12 @@ static int sweep_verify64(tags_sweep* sw, SweepSlot& sl, c64* Wz, const c64* xz,
     return 0;
 }
 
-// Sample f, item q of the slot's group, that the nodal solve did not accept:
-// the Z_L-first factor of its assembled W (mixed: complex64 with refinement,
-// then complex128). Waits; its solution replaces the item's x and u.
-static int sweep_nodal_retry(tags_sweep* sw, SweepSlot& sl, int q, size_t f, const SweepCall& c,
-                             tags_item_stats* stt, int* info)
-{
-    const long N = sw->N;
-    int rc;
-    if ((rc = sl.init(N, 1)) || (rc = sl.sv.ensure((int)N, c.mixed, 1))) return rc;
-    slot_bind(sw, sl);
-    sl.static_items = 0;
-    hipStream_t st = sl.stream.s;
-    if ((rc = sweep_fill(sw, sl.W.p, st, sl.scal, c.s[f], c.kappa[f], c.mur,
-                         c.gamma ? &c.gamma[f] : nullptr, c.ref_l ? &c.ref_l[f] : nullptr,
-                         c.ref_t ? &c.ref_t[f] : nullptr)))
-        return rc;
-    hipLaunchKernelGGL(k_unit_rhs, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, sl.rhs.p, N,
-                       sw->layout.node_off + (long)c.inj_node);
-    TAGS_HIP(hipGetLastError());
-    rc = c.mixed ? sl.sv.solve_mixed(sl.W.p, sl.rhs.p, stt) : sl.sv.solve64(sl.W.p, sl.rhs.p, stt);
-    if (rc < 0) return rc;
-    *info = rc;
-    if (!c.mixed && sw->verify && rc == 0 &&
-        (rc = sweep_verify64(sw, sl, sl.W.p, sl.rhs.p, f, c, stt)))
-        return rc;
-    TAGS_HIP(hipMemcpyAsync(sl.nd.x + (long)q * N, sl.rhs.p, sizeof(c64) * N,
-                            hipMemcpyDeviceToDevice, st));
-    TAGS_HIP(hipMemcpyAsync(&sl.nd.hu[q], sl.rhs.p + sw->layout.node_off + c.inj_node, sizeof(c64),
-                            hipMemcpyDeviceToHost, st));
-    TAGS_HIP(hipStreamSynchronize(st));
-    return 0;
-}
-
-// Statistics of a nodal group whose refinement has ended, and the retries.
-static int sweep_nodal_finish(tags_sweep* sw, SweepSlot& sl, const SweepCall& c)
+// Statistics of a nodal group whose refinement has ended; samples that it did
+// not accept go back to `todo`.
+static void sweep_nodal_finish(tags_sweep* sw, SweepSlot& sl, const SweepCall& c, SweepTodo& todo)
 {
     NodalSolver& nd = sl.nd;
-    for (int q = 0; q < sl.cnt; q++) {
+    for (size_t q = 0; q < sl.at.size(); q++) {
         tags_item_stats& t = sl.stt[q];
         sl.info[q] = 0;
         t.info = 0;
@@ -2737,35 +2728,28 @@ static int sweep_nodal_finish(tags_sweep* sw, SweepSlot& sl, const SweepCall& c)
                 for (int i = 0; i < 8; i++) t.refine_hist[i] = nd.hist[8 * q + i];
             continue;
         }
-        int rc = sweep_nodal_retry(sw, sl, q, (size_t)sl.f + q, c, &t, &sl.info[q]);
-        if (rc) return rc;
-        if (c.mixed) {
-            t.refine_iters += nd.steps[q];
-            sw->nodal_above = std::max(sw->nodal_above, 1.5 * sl.hz[q]);
-        } else {
-            sw->nodal64 = false;
-        }
+        todo.rejected.push_back({sl.at[q], nd.steps[q]});
+        if (c.mixed) sw->nodal_above = std::max(sw->nodal_above, 1.5 * sample_hz(c, sl.at[q]));
     }
-    return 0;
 }
 
 // Advances the group in flight on slot `sl`, whose stream has finished what
 // was queued: the mixed form checks its refinement and may queue another step
 // (*complete false); once complete the results are written. A singular sample
 // (info > 0) gets NaN in u_inj and in its block of x_out.
-static int sweep_advance(tags_sweep* sw, SweepSlot& sl, const SweepCall& c, bool* complete)
+static int sweep_advance(tags_sweep* sw, SweepSlot& sl, const SweepCall& c, SweepTodo& todo,
+                         bool* complete)
 {
     const long N = sw->N, n = sw->n, m = sw->m;
     const BlockLayout& L = sw->layout;
-    const size_t f0 = (size_t)sl.f;
-    const int cnt = sl.cnt;
+    const int cnt = (int)sl.at.size();
     std::vector<tags_item_stats>& stt = sl.stt;
     std::vector<int>& info = sl.info;
     *complete = false;
     int rc;
     if (sl.nodal_path) {
         if ((rc = sl.nd.advance(complete)) || !*complete) return rc;
-        if ((rc = sweep_nodal_finish(sw, sl, c))) return rc;
+        sweep_nodal_finish(sw, sl, c, todo);
     } else {
         rc = c.mixed ? sl.sv.advance_mixed(sl.W.p, sl.rhs.p, stt.data(), info.data(), complete)
                      : sl.sv.finish64(stt.data(), info.data());
@@ -2773,13 +2757,14 @@ static int sweep_advance(tags_sweep* sw, SweepSlot& sl, const SweepCall& c, bool
         if (!c.mixed) *complete = true;
         if (!*complete) return 0;
     }
-    sl.f = -1;
+    const std::vector<size_t> at = std::move(sl.at);
+    sl.at.clear();
     hipStream_t st = sl.stream.s;
     if (!sl.nodal_path && !c.mixed && sw->verify)
         for (int z = 0; z < cnt; z++)
             if (info[z] == 0 &&
                 (rc = sweep_verify64(sw, sl, sl.W.p + (long)z * N * N, sl.rhs.p + (long)z * N,
-                                     f0 + z, c, &stt[z])))
+                                     at[z], c, &stt[z])))
                 return rc;
     // the nodal solve has already brought U[inj]
     const bool full = !sl.nodal_path || c.x_out;
@@ -2790,7 +2775,9 @@ static int sweep_advance(tags_sweep* sw, SweepSlot& sl, const SweepCall& c, bool
         TAGS_HIP(hipStreamSynchronize(st));
     }
     for (int z = 0; z < cnt; z++) {
-        const size_t f = f0 + z;
+        const size_t f = at[z];
+        if (sl.nodal_path && !sl.nd.accepted[z]) continue;
+        if (c.mixed) stt[z].refine_iters += sl.spent[z];
         if (c.stats) c.stats[f] = stt[z];
         // a fallback factored this sample's W in FP64
         if (c.mixed && stt[z].precision_used != TAGS_PREC_MIXED) sl.static_items = 0;
@@ -2847,14 +2834,13 @@ int tags_sweep_solve(tags_sweep* sw, size_t nfreq, const TAGS_COMPLEX* s,
     };
     if (tu && mixed && tu->nodal_above >= 0.0) sw->nodal_above = tu->nodal_above;
     if (tu && mixed && tu->gmres_steps > 0) sw->gmres_steps = tu->gmres_steps;
-    sw->nodal64 = true;
     // every slot the call can use is allocated up front (a warm-up call of the
     // same length sets all of them up)
     int rc = sweep_layout(sw);
     const bool nodal = sweep_nodal(sw, mixed, INFINITY);
     const size_t per = (size_t)(nodal ? sw->nd_batch : sw->batch);
-    const int k = (int)std::min<size_t>(tu && tu->inflight > 0 ? tu->inflight : sw->inflight,
-                                        (nfreq + per - 1) / per);
+    const size_t k_max = (size_t)(tu && tu->inflight > 0 ? tu->inflight : sw->inflight);
+    int k = (int)std::min(k_max, (nfreq + per - 1) / per);
     if (!rc) rc = sweep_slots(sw, k, mixed, nodal, !sweep_nodal(sw, mixed, 0.0));
     // after the slots exist: the layout sets every slot's plans
     if (!rc) rc = sweep_layout(sw);
@@ -2864,21 +2850,32 @@ int tags_sweep_solve(tags_sweep* sw, size_t nfreq, const TAGS_COMPLEX* s,
     }
     const SweepCall c{nfreq, s, kappa, gamma, ref_l, ref_t, mur, inj_node, mixed, u_inj, x_out,
                       stats};
-    size_t next = 0;
-    for (int i = 0; i < k && next < nfreq; i++) {
-        const int got = sweep_issue(sw, *sw->slots[i], next, c);
-        if (got < 0) {
-            rc = got;
-            break;
+    SweepTodo todo;
+    // every idle slot takes a group; the groups of rejected samples also slots
+    // that this call did not need so far
+    auto refill = [&]() -> int {
+        const size_t groups = (todo.rejected.size() + sw->batch - 1) / (size_t)sw->batch;
+        if (todo.next >= nfreq && (int)std::min(k_max, groups) > k) {
+            k = (int)std::min(k_max, groups);
+            const int r = sweep_slots(sw, k, mixed, false, false);
+            if (r) return r;
+            for (int i = 0; i < k; i++)
+                if (!sw->slots[i]->busy()) slot_bind(sw, *sw->slots[i]);
         }
-        next += (size_t)got;
-    }
+        for (int i = 0; i < k && todo.left(nfreq); i++)
+            if (!sw->slots[i]->busy()) {
+                const int r = sweep_issue(sw, *sw->slots[i], todo, c);
+                if (r) return r;
+            }
+        return 0;
+    };
+    rc = refill();
     // advance whichever slot's stream is idle; refill a slot whose group is done
     Poll poll;
     while (!rc) {
         int busy = 0, ready = -1;
         for (int i = 0; i < k; i++) {
-            if (sw->slots[i]->f < 0) continue;
+            if (!sw->slots[i]->busy()) continue;
             busy++;
             const hipError_t q = hipStreamQuery(sw->slots[i]->stream.s);
             if (q == hipSuccess) {
@@ -2895,21 +2892,14 @@ int tags_sweep_solve(tags_sweep* sw, size_t nfreq, const TAGS_COMPLEX* s,
         poll.n = 0;
         SweepSlot& sl = *sw->slots[ready];
         bool complete = false;
-        if ((rc = sweep_advance(sw, sl, c, &complete))) break;
-        if (complete && next < nfreq) {
-            const int got = sweep_issue(sw, sl, next, c);
-            if (got < 0) {
-                rc = got;
-                break;
-            }
-            next += (size_t)got;
-        }
+        if ((rc = sweep_advance(sw, sl, c, todo, &complete))) break;
+        if (complete) rc = refill();
     }
     // after an error: let every queued sample end before returning
     restore();
     for (int i = 0; i < k; i++) {
         TAGS_HIP(hipStreamSynchronize(sw->slots[i]->stream.s));
-        sw->slots[i]->f = -1;
+        sw->slots[i]->at.clear();
     }
     return rc;
 }
@@ -3463,7 +3453,7 @@ int tags_cases_solve(tags_cases* cs, int precision)
     std::vector<SweepCall> call(nc);
     std::vector<double> cost(nc), nodal0(nc);
     std::vector<int> gmres0(nc);
-    std::vector<size_t> next(nc, 0);
+    std::vector<SweepTodo> todo(nc);
     for (size_t c = 0; c < nc; c++) {
         tags_sweep* sw = cs->sw[c];
         const tags_case& d = cs->cs[c];
@@ -3477,7 +3467,6 @@ int tags_cases_solve(tags_cases* cs, int precision)
                         ? 1
                         : sweep_batch(sw, mixed);
         sw->nd_batch = sweep_nd_batch(sw, mixed, d.nfreq);
-        sw->nodal64 = true;
         sw->batch_req = batch_req0;
         if (lu_panel_kind() == PANEL_PARTIAL) sw->batch = 1;
         if ((rc = sweep_potentials(sw))) return rc;
@@ -3496,7 +3485,6 @@ int tags_cases_solve(tags_cases* cs, int precision)
     for (size_t c = 0; c < nc; c++) order[c] = c;
     std::stable_sort(order.begin(), order.end(),
                      [&](size_t a, size_t b) { return cost[a] > cost[b]; });
-    size_t qi = 0;  // first case in `order` with samples left
     while ((int)cs->lanes.size() < cs->nlanes) cs->lanes.emplace_back(new SweepSlot());
     // every lane's buffers sized for all cases before any work is queued: a
     // group size chosen by an N^2 budget makes N times the group grow as N
@@ -3547,8 +3535,13 @@ int tags_cases_solve(tags_cases* cs, int precision)
         }
     }
     std::vector<long> lane_case(cs->nlanes, -1);
+    size_t q0 = 0;  // the cases before it in `order` have only rejected samples left, or none
     auto issue = [&](int li) -> int {
-        while (qi < nc && next[order[qi]] >= cs->cs[order[qi]].nfreq) qi++;
+        while (q0 < nc && todo[order[q0]].next >= cs->cs[order[q0]].nfreq) q0++;
+        // (rejected samples are rare: looked for where there are no others)
+        size_t qi = q0;
+        if (qi >= nc)
+            for (qi = 0; qi < nc && todo[order[qi]].rejected.empty();) qi++;
         if (qi >= nc) return 0;
         const size_t c = order[qi];
         tags_sweep* sw = cs->sw[c];
@@ -3561,9 +3554,7 @@ int tags_cases_solve(tags_cases* cs, int precision)
         slot_bind(sw, L);
         // the case's tuned tile shapes and schedule, if any
         TuningScope scope(sw->tuned[mixed ? 1 : 0] ? &sw->ktune[mixed ? 1 : 0] : tuning_current());
-        const int got = sweep_issue(sw, L, next[c], call[c]);
-        if (got < 0) return got;
-        next[c] += (size_t)got;
+        if ((r = sweep_issue(sw, L, todo[c], call[c]))) return r;
         lane_case[li] = (long)c;
         return 0;
     };
@@ -3574,7 +3565,7 @@ int tags_cases_solve(tags_cases* cs, int precision)
     while (!rc) {
         int busy = 0, done = -1;
         for (int li = 0; li < cs->nlanes; li++) {
-            if (cs->lanes[li]->f < 0) continue;
+            if (!cs->lanes[li]->busy()) continue;
             busy++;
             const hipError_t q = hipStreamQuery(cs->lanes[li]->stream.s);
             if (q == hipSuccess) {
@@ -3598,11 +3589,12 @@ int tags_cases_solve(tags_cases* cs, int precision)
             tags_sweep* sw = cs->sw[c];
             TuningScope scope(sw->tuned[mixed ? 1 : 0] ? &sw->ktune[mixed ? 1 : 0]
                                                        : tuning_current());
-            if ((rc = sweep_advance(sw, L, call[c], &complete))) break;
+            if ((rc = sweep_advance(sw, L, call[c], todo[c], &complete))) break;
         }
         if (!complete) continue;
         lane_case[done] = -1;
-        rc = issue(done);
+        for (int li = 0; li < cs->nlanes && !rc; li++)
+            if (!cs->lanes[li]->busy()) rc = issue(li);
     }
     for (size_t c = 0; c < nc; c++) {
         cs->sw[c]->nodal_above = nodal0[c];
@@ -3610,7 +3602,7 @@ int tags_cases_solve(tags_cases* cs, int precision)
     }
     for (auto& l : cs->lanes) {
         TAGS_HIP(hipStreamSynchronize(l->stream.s));
-        l->f = -1;
+        l->at.clear();
     }
     return rc;
 }
