@@ -697,6 +697,12 @@ int tags_device_synchronize(void);
  * calls keep between calls. Safe at any time, from any thread. */
 void tags_release_staging(void);
 
+/* For tests of what a call does where device memory runs out: the nth device
+ * allocation (1, 2, ..) of the calling thread's host-pointer calls and nodal
+ * solves from now on fails as one that does not fit; 0 disarms. Returns what
+ * was left to count, 0 if the last one armed has failed (or none was). */
+long tags_fail_allocation(long nth);
+
 /* GEMM tuning. The trailing update C -= A B of the LU has several MFMA tile
  * variants per precision (precision: tags_precision). Complex64 variants
  * 0-21 and 33 run on the fp32 MFMA cores; 22-32 run on the bf16 MFMA cores,

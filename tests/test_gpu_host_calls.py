@@ -229,3 +229,78 @@ def test_transform_twiddles_are_rounded_once(nt):
     for got, ref in ((w.real, re), (w.imag, im)):
         ulp = np.spacing(np.abs(ref.astype(float)))
         assert np.max(np.abs(got - ref) / ulp) <= 0.505
+
+
+def _failing(call, needed):
+    """call() with its nth device allocation failing, n = 1, 2, .. until it has no
+    more: an error where the call cannot do without it (the first `needed`), the
+    answer from the pivoted route otherwise; and the answer again afterwards."""
+    L = T.lib()
+    n = 0
+    while True:
+        n += 1
+        L.tags_fail_allocation(n)
+        rc = call()
+        left = L.tags_fail_allocation(0)
+        if left:
+            break
+        assert rc == (0 if n > needed else -100), (n, rc)
+    assert rc == 0 and call() == 0
+    return n - 1
+
+
+def test_calls_without_room_for_their_inverses():
+    """The symmetric inverses and the nodal solve need device memory beside what
+    the pivoted factorisation takes: where it does not fit, that one answers."""
+    m, n = 70, 50
+    rng = np.random.default_rng(3)
+    zl0, zt0 = _symmetric(m, 1, True), _symmetric(m, 2, True)
+    A, B = (rng.standard_normal((m, n)) + 0j for _ in range(2))
+    ref = np.linalg.solve(zl0, A), np.linalg.solve(zt0, B)
+    pats = [np.tril(z).T.ravel() for z in (zl0, zt0)]
+
+    def yla_ytb():
+        zl, zt = (p.copy() for p in pats)
+        out = np.zeros(m * n, complex), np.zeros(m * n, complex)
+        rc = T.calculate_yla_ytb(*out, zl, zt, A.T.ravel().copy(), B.T.ravel().copy(), m, n)
+        if rc == 0:
+            for o, r in zip(out, ref):
+                assert np.abs(o.reshape(n, m).T - r).max() <= 1e-12 * np.abs(r).max()
+            for z, z0 in ((zl, zl0), (zt, zt0)):
+                inv = np.linalg.inv(z0)
+                got = z.reshape(m, m).T
+                assert np.abs(np.tril(got) - np.tril(inv)).max() <= 1e-12 * np.abs(inv).max()
+        return rc
+
+    b = rng.standard_normal(m) + 1j * rng.standard_normal(m)
+
+    def admittance():
+        x = b.copy()
+        rc = T.solve_admittance(zl0.T.ravel().copy(), x, m)
+        if rc == 0:
+            assert np.abs(x - np.linalg.solve(zl0, b)).max() <= 1e-12 * np.abs(x).max()
+        return rc
+
+    rc, e, nodes = T.electrode_grid(3, 4, 7.0, 9.0, 4, 3, 5e-3, -0.6)
+    me, ne = len(e), len(nodes)
+    N = ne + 2 * me
+    sc = T.soil_scalars(4e5, 2e-3, 12.0)
+    zl, zt, W = (np.zeros(k, complex) for k in (me * me, me * me, N * N))
+    T.calculate_impedances(zl, zt, e, sc["gamma"], sc["s"], 1.0, sc["kappa"])
+    T.fill_incidence_imm(W, e, nodes)
+    T.fill_impedance_imm(W, zl, zt, me, ne)
+    low = np.tril(W.reshape(N, N).T)
+    c = rng.standard_normal(N) + 1j * rng.standard_normal(N)
+    y = np.linalg.solve(low + np.tril(low, -1).T, c)
+
+    def immittance():
+        x = c.copy()
+        rc = T.solve_immittance(W, x, me, ne)
+        if rc == 0:
+            assert np.abs(x - y).max() <= 1e-9 * np.abs(y).max()
+        return rc
+
+    # the arrays themselves and, for the inverses, A and B in row order
+    assert _failing(yla_ytb, 4) > 4
+    assert _failing(admittance, 2) > 2
+    assert _failing(immittance, 2) > 2

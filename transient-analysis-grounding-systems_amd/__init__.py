@@ -174,7 +174,7 @@ EXPORTED = ["populate_electrode", "segment_electrode", "number_segments", "numbe
             "tags_cases_set_profiling", "tags_cases_get_timers", "tags_cases_destroy",
             "tags_sweep_autotune", "tags_sweep_set_tuning", "tags_sweep_get_tuning",
             "tags_cases_autotune",
-            "tags_sweep_set_gmres", "tags_release_staging"]
+            "tags_sweep_set_gmres", "tags_release_staging", "tags_fail_allocation"]
 
 _lib = None
 
@@ -235,6 +235,7 @@ def lib():
         "tags_version": ([], ctypes.c_char_p),
         "tags_device_synchronize": ([], I),
         "tags_release_staging": ([], None),
+        "tags_fail_allocation": ([ctypes.c_long], ctypes.c_long),
         "tags_gemm_bench": ([I, I, I, I, I, I, ctypes.POINTER(D)], I),
         "tags_gemm_variants": ([I], I),
         "tags_gemm_select": ([I, I, I], I),

@@ -81,13 +81,28 @@ struct Stream {
     ~Stream() { hipStreamDestroy(s); }
 };
 
+static thread_local long g_fail_at = 0;
+hipError_t dev_malloc(void** p, size_t bytes)
+{
+    if (g_fail_at > 0 && --g_fail_at == 0) bytes = (size_t)1 << 60;
+    return hipMalloc(p, bytes);
+}
+
 template <typename X>
 struct DevBuf {
     X* p = nullptr;
     int alloc(size_t n)
     {
-        TAGS_HIP(hipMalloc(&p, sizeof(X) * (n ? n : 1)));
+        TAGS_HIP(dev_malloc((void**)&p, sizeof(X) * (n ? n : 1)));
         return 0;
+    }
+    // false, with nothing left of the error, where it does not fit
+    bool try_alloc(size_t n)
+    {
+        if (dev_malloc((void**)&p, sizeof(X) * (n ? n : 1)) == hipSuccess) return true;
+        p = nullptr;
+        (void)hipGetLastError();
+        return false;
     }
     ~DevBuf() { hipFree(p); }
 };
@@ -624,6 +639,13 @@ using namespace tags;
 extern "C" {
 
 const char* tags_version(void) { return "tags_hip 0.1 (gfx950)"; }
+
+long tags_fail_allocation(long nth)
+{
+    const long left = g_fail_at;
+    g_fail_at = nth;
+    return left;
+}
 
 int tags_device_synchronize(void)
 {
@@ -1336,8 +1358,8 @@ int fill_impedance_imm(TAGS_COMPLEX* wg, const TAGS_COMPLEX* zl, const TAGS_COMP
 // ---------------------------------------------------------------------------
 // The immittance system of a host W (N x N, lower triangle column-major) by the
 // nodal solve: W is on the device in Wd; where it has the structure of the HEM
-// (fill_incidence_imm and fill_impedance_imm's) and the refinement is accepted,
-// x replaces bx and *done is set. (20 x 20 m grid, N = 1185: 8.7 ms by the
+// (fill_incidence_imm and fill_impedance_imm's), the solve's buffers fit beside
+// it and the refinement is accepted, x replaces bx and *done is set. (20 x 20 m grid, N = 1185: 8.7 ms by the
 // pivoted factor of W.)
 static int immittance_nodal(const c64* Wd, c64* bx, long m, long n, hipStream_t st, bool* done)
 {
@@ -1346,7 +1368,7 @@ static int immittance_nodal(const c64* Wd, c64* bx, long m, long n, hipStream_t 
     int rc;
     DevBuf<int> d;
     const size_t ni = 4 * (size_t)m + 1;  // sn, en, their counts, entries out of place
-    if ((rc = d.alloc(ni))) return rc;
+    if (!d.try_alloc(ni)) return 0;
     if ((rc = imm_structure(Wd, N, m, n, d.p, st))) return rc;
     std::vector<int> h(ni);
     if ((rc = copy_out(h.data(), d.p, sizeof(int) * ni, st))) return rc;
@@ -1358,7 +1380,7 @@ static int immittance_nodal(const c64* Wd, c64* bx, long m, long n, hipStream_t 
     bool distinct;
     if (!node_lists(sn, en, n, ptr, seg, &distinct) || !distinct) return 0;
     DevBuf<int> dp, ds;
-    if ((rc = dp.alloc(n + 1)) || (rc = ds.alloc(seg.size()))) return rc;
+    if (!dp.try_alloc(n + 1) || !ds.try_alloc(seg.size())) return 0;
     if ((rc = copy_in(dp.p, ptr.data(), sizeof(int) * (n + 1), st)) ||
         (rc = copy_in(ds.p, seg.data(), sizeof(int) * seg.size(), st)))
         return rc;
@@ -1371,7 +1393,10 @@ static int immittance_nodal(const c64* Wd, c64* bx, long m, long n, hipStream_t 
     op.node_seg = ds.p;
     NodalSolver nd;
     nd.st = st;
-    if ((rc = nd.ensure(op, true, 1))) return rc;
+    if (nd.ensure(op, true, 1)) {
+        (void)hipGetLastError();
+        return 0;
+    }
     if ((rc = imm_blocks(Wd, N, m, n, nd.Z, st))) return rc;
     // the nodal order is [I_L; I_T; U]
     std::vector<c64> b(N);
@@ -1394,8 +1419,8 @@ static int immittance_nodal(const c64* Wd, c64* bx, long m, long n, hipStream_t 
 
 // A dense symmetric system (Wd: n x n with both triangles, on the device; b in
 // bd, replaced by x) by its explicit inverse with refinement; *done unless the
-// refinement does not meet its acceptance rule (a zero pivot or growth without
-// row exchanges among them). (n = 559: 4.4 ms by the pivoted factor.)
+// inverse does not fit beside it or the refinement does not meet its acceptance
+// rule (a zero pivot or growth without row exchanges among the causes). (n = 559: 4.4 ms by the pivoted factor.)
 static int symmetric_solve(const c64* Wd, c64* bd, long n, hipStream_t st, bool* done)
 {
     *done = false;
@@ -1405,9 +1430,9 @@ static int symmetric_solve(const c64* Wd, c64* bd, long n, hipStream_t st, bool*
     DevBuf<char> work;
     DevBuf<unsigned long long> norms;
     constexpr int kSteps = 6;
-    if ((rc = X.alloc((size_t)ld * ld)) || (rc = v.alloc(2 * n)) ||
-        (rc = work.alloc(sym_inverse_bytes(n, 1))) || (rc = norms.alloc(4 * (kSteps + 1))))
-        return rc;
+    if (!X.try_alloc((size_t)ld * ld) || !v.try_alloc(2 * n) ||
+        !work.try_alloc(sym_inverse_bytes(n, 1)) || !norms.try_alloc(4 * (kSteps + 1)))
+        return 0;
     c64 *x = v.p, *r = v.p + n;
     if ((rc = sym_inverse(Wd, n, 0, X.p, n, 1, work.p, st))) return rc;
     if ((rc = fill_c64(x, n, c64{0.0, 0.0}, st)) ||
@@ -1640,75 +1665,78 @@ extern "C" {
 
 // Device copies of the host arrays of one admittance call.
 struct AdmArrays {
-    DevBuf<c64> zl, zt, arm, brm, yla, ytb, yn;
-    DevBuf<c64> z2;  // zl then zt, as uploaded
+    DevBuf<c64> z;         // zl then zt
+    DevBuf<c64> arm, brm;  // A and -B (m x n, row-major)
+    DevBuf<c64> y;         // yla then ytb (m x n, column-major)
+    DevBuf<c64> yn;
 };
 
 // Largest entry of Z X - I for which one Newton step leaves the inverse at
 // working accuracy (its square times m stays far below an ulp).
 constexpr double kInvGate = 1e-10;
 
-// Both inverses without row exchanges, as explicit symmetric inverses X of z2's
-// blocks with a Newton step X + X (I - Z X); *done unless a product Z X is
-// further from I than kInvGate (then nothing of the caller's is touched and the
-// pivoted factorisation follows). Then yla^T = A^T X_L and ytb^T = B^T X_T
-// (row-major n x m: the column-major m x n the caller takes) from a and b as
-// uploaded in arm and brm, and the lower triangles to zl and zt.
+// Both inverses without row exchanges, as explicit symmetric inverses X of d.z's
+// blocks with a Newton step X + X (I - Z X); *done unless its buffers do not fit
+// or a product Z X is further from I than kInvGate (then nothing of the caller's
+// is touched, d.z holds nothing of use and the pivoted factorisation follows).
+// Then yla^T = A^T X_L and ytb^T = B^T X_T (row-major n x m: the column-major
+// m x n the caller takes) from a and b as uploaded in d.y, which they replace,
+// and the lower triangles to zl and zt. About 10 m^2 complex values on the
+// device with n = m, where the pivoted route takes 9.
 // (m = 606, n = 559: 10.6 ms for the whole call by the pivoted factors.)
-static int adm_symmetric(AdmArrays& d, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const c64* av,
-                         const c64* bv, long m, long n, hipStream_t st, bool* done)
+static int adm_symmetric(AdmArrays& d, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, long m, long n,
+                         hipStream_t st, bool* done)
 {
     *done = false;
-    const long ld = (m + 63) / 64 * 64;
+    const long ld = (m + 63) / 64 * 64, mm = m * m, mn = m * n;
     int rc;
-    DevBuf<c64> X, X2, Z, R;
+    DevBuf<c64> X, R;
     DevBuf<char> work;
     DevBuf<unsigned long long> dev;
-    if ((rc = X.alloc((size_t)2 * ld * ld)) || (rc = X2.alloc((size_t)2 * ld * ld)) ||
-        (rc = Z.alloc((size_t)2 * m * m)) || (rc = R.alloc((size_t)2 * m * m)) ||
-        (rc = work.alloc(sym_inverse_bytes(m, 2))) || (rc = dev.alloc(2)))
-        return rc;
-    TAGS_HIP(hipMemcpyAsync(Z.p, d.z2.p, sizeof(c64) * 2 * m * m, hipMemcpyDeviceToDevice, st));
+    if (!X.try_alloc((size_t)2 * ld * ld) || !R.try_alloc((size_t)2 * std::max(mm, mn)) ||
+        !work.try_alloc(sym_inverse_bytes(m, 2)) || !dev.try_alloc(2))
+        return 0;
+    c64* Z = d.z.p;
     for (int i = 0; i < 2; i++)
-        if ((rc = sym_from_upper(Z.p + i * m * m, m, (int)m, st))) return rc;
-    if ((rc = sym_inverse(Z.p, m, m * m, X.p, m, 2, work.p, st))) return rc;
+        if ((rc = sym_from_upper(Z + i * mm, m, (int)m, st))) return rc;
+    if ((rc = sym_inverse(Z, m, mm, X.p, m, 2, work.p, st))) return rc;
     // R = Z X - I
-    GemmArgs<double> g{(int)m, (int)m, (int)m, Z.p, m, nullptr, X.p, ld, nullptr, R.p, m, nullptr, 0};
+    GemmArgs<double> g{(int)m, (int)m, (int)m, Z, m, nullptr, X.p, ld, nullptr, R.p, m, nullptr, 0};
     g.nb = 2;
-    g.sa = m * m;
+    g.sa = mm;
     g.sb = ld * ld;
-    g.sc = m * m;
+    g.sc = mm;
     if ((rc = launch_gemm<double>(g, st))) return rc;
     if ((rc = fill_c64((c64*)dev.p, 1, c64{0.0, 0.0}, st))) return rc;
     if ((rc = sub_identity(R.p, m, 2, dev.p, st))) return rc;
     double h[2];
     if ((rc = copy_out(h, dev.p, sizeof(h), st))) return rc;
     if (!(h[0] <= kInvGate)) return 0;
-    // X2 = X - X R
-    TAGS_HIP(hipMemcpyAsync(X2.p, X.p, sizeof(c64) * 2 * ld * ld, hipMemcpyDeviceToDevice, st));
+    // Z = X - X R
+    for (int i = 0; i < 2; i++)
+        TAGS_HIP(hipMemcpy2DAsync(Z + i * mm, sizeof(c64) * m, X.p + i * ld * ld, sizeof(c64) * ld,
+                                  sizeof(c64) * m, m, hipMemcpyDeviceToDevice, st));
     g.A = X.p;
     g.lda = ld;
     g.sa = ld * ld;
     g.B = R.p;
     g.ldb = m;
-    g.sb = m * m;
-    g.C = X2.p;
-    g.ldc = ld;
-    g.sc = ld * ld;
+    g.sb = mm;
+    g.C = Z;
     g.mode = 1;
     if ((rc = launch_gemm<double>(g, st))) return rc;
     if (n > 0) {
-        GemmArgs<double> p{(int)n, (int)m, (int)m, av, m, nullptr, X2.p, ld, nullptr, d.yla.p, m, nullptr, 0};
+        GemmArgs<double> p{(int)n, (int)m, (int)m, d.y.p, m, nullptr, Z, m, nullptr, R.p, m, nullptr, 0};
+        p.nb = 2;
+        p.sa = p.sc = mn;
+        p.sb = mm;
         if ((rc = launch_gemm<double>(p, st))) return rc;
-        p.A = bv;
-        p.B = X2.p + ld * ld;
-        p.C = d.ytb.p;
-        if ((rc = launch_gemm<double>(p, st))) return rc;
+        std::swap(d.y.p, R.p);
     }
     // the lower triangles (entry (k, i), k >= i, at i m + k of the caller's arrays)
-    c64* packed = Z.p;
+    c64* packed = X.p;
     const long np = m * (m + 1) / 2;
-    if ((rc = sym_pack(X2.p, ld, m, 2, packed, st))) return rc;
+    if ((rc = sym_pack(Z, m, m, 2, packed, st))) return rc;
     for (int i = 0; i < 2; i++) {
         c64* dst = (c64*)(i ? zt : zl);
         rc = copy_out_rows(packed + i * np, m, st, [&](long q, long k, const c64* v, long cnt) {
@@ -1728,35 +1756,34 @@ static int adm_inverses(AdmArrays& d, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const 
 {
     int rc;
     if (m == 0) return 0;
-    if ((rc = d.zl.alloc((size_t)m * m)) || (rc = d.zt.alloc((size_t)m * m)) ||
-        (rc = d.arm.alloc((size_t)m * n)) || (rc = d.brm.alloc((size_t)m * n)) ||
-        (rc = d.yla.alloc((size_t)m * n)) || (rc = d.ytb.alloc((size_t)m * n)))
-        return rc;
     const size_t mm = (size_t)m * m, mn = (size_t)m * n;
-    // a, b (column-major m x n) staged in X order, transposed to row-major
-    DevBuf<c64> ab;
-    if ((rc = ab.alloc(2 * mn)) || (rc = d.z2.alloc(2 * mm))) return rc;
-    if ((rc = copy_in(ab.p, a, sizeof(c64) * mn, st)) ||
-        (rc = copy_in(ab.p + mn, b, sizeof(c64) * mn, st)) ||
-        (rc = copy_in(d.z2.p, zl, sizeof(c64) * mm, st)) ||
-        (rc = copy_in(d.z2.p + mm, zt, sizeof(c64) * mm, st)))
+    if ((rc = d.z.alloc(2 * mm)) || (rc = d.arm.alloc(mn)) || (rc = d.brm.alloc(mn)) ||
+        (rc = d.y.alloc(2 * mn)))
         return rc;
-    if ((rc = transpose(ab.p, m, nullptr, d.arm.p, n, n, m, 1.0, false, st)) ||
-        (rc = transpose(ab.p + mn, m, nullptr, d.brm.p, n, n, m, -1.0, false, st)))
+    // a, b (column-major m x n) staged where yla and ytb go, transposed to row-major
+    if ((rc = copy_in(d.y.p, a, sizeof(c64) * mn, st)) ||
+        (rc = copy_in(d.y.p + mn, b, sizeof(c64) * mn, st)))
         return rc;
+    if ((rc = transpose(d.y.p, m, nullptr, d.arm.p, n, n, m, 1.0, false, st)) ||
+        (rc = transpose(d.y.p + mn, m, nullptr, d.brm.p, n, n, m, -1.0, false, st)))
+        return rc;
+    auto upload = [&]() -> int {
+        const int r = copy_in(d.z.p, zl, sizeof(c64) * mm, st);
+        return r ? r : copy_in(d.z.p + mm, zt, sizeof(c64) * mm, st);
+    };
+    if ((rc = upload())) return rc;
     if (zl != zt) {  // one array for both takes the reference's order of writes
         bool done = false;
-        if ((rc = adm_symmetric(d, zl, zt, ab.p, ab.p + mn, m, n, st, &done)) || done) return rc;
+        if ((rc = adm_symmetric(d, zl, zt, m, n, st, &done)) || done) return rc;
+        if ((rc = upload())) return rc;
     }
-    TAGS_HIP(hipMemcpyAsync(d.zl.p, d.z2.p, sizeof(c64) * mm, hipMemcpyDeviceToDevice, st));
-    TAGS_HIP(hipMemcpyAsync(d.zt.p, d.z2.p + mm, sizeof(c64) * mm, hipMemcpyDeviceToDevice, st));
     LUWork<double> w;
     // Z_L first, written back before Z_T is factored: as with zsytrf/zsytri in
     // the reference, a singular Z_T leaves zl already inverted
-    if ((rc = adm_block(w, d.zl.p, d.arm.p, 1.0, m, n, d.yla.p, st))) return rc;
-    if ((rc = copy_out(zl, d.zl.p, sizeof(c64) * mm, st))) return rc;
-    if ((rc = adm_block(w, d.zt.p, d.brm.p, -1.0, m, n, d.ytb.p, st))) return rc;
-    return copy_out(zt, d.zt.p, sizeof(c64) * mm, st);
+    if ((rc = adm_block(w, d.z.p, d.arm.p, 1.0, m, n, d.y.p, st))) return rc;
+    if ((rc = copy_out(zl, d.z.p, sizeof(c64) * mm, st))) return rc;
+    if ((rc = adm_block(w, d.z.p + mm, d.brm.p, -1.0, m, n, d.y.p + mn, st))) return rc;
+    return copy_out(zt, d.z.p + mm, sizeof(c64) * mm, st);
 }
 
 // yn (n x n column-major) = A^T yla + B^T ytb: as row-major products,
@@ -1770,10 +1797,10 @@ static int adm_products(AdmArrays& d, long m, long n, hipStream_t st)
         TAGS_HIP(hipMemsetAsync(d.yn.p, 0, sizeof(c64) * n * n, st));
         return 0;
     }
-    GemmArgs<double> g{(int)n, (int)n, (int)m, d.yla.p, m, nullptr, d.arm.p, n, nullptr,
+    GemmArgs<double> g{(int)n, (int)n, (int)m, d.y.p, m, nullptr, d.arm.p, n, nullptr,
                        d.yn.p, n, nullptr, 0};
     if ((rc = launch_gemm<double>(g, st))) return rc;
-    g.A = d.ytb.p;
+    g.A = d.y.p + m * n;
     g.B = d.brm.p;
     g.mode = 1;
     return launch_gemm<double>(g, st);
@@ -1800,8 +1827,8 @@ int calculate_yla_ytb(TAGS_COMPLEX* yla, TAGS_COMPLEX* ytb, TAGS_COMPLEX* zl, TA
     AdmArrays d;
     int rc = adm_inverses(d, zl, zt, a, b, m, n, S.s);
     if (rc) return rc;
-    if ((rc = copy_out(yla, d.yla.p, sizeof(c64) * m * n, S.s))) return rc;
-    return copy_out(ytb, d.ytb.p, sizeof(c64) * m * n, S.s);
+    if ((rc = copy_out(yla, d.y.p, sizeof(c64) * m * n, S.s))) return rc;
+    return copy_out(ytb, d.y.p + m * n, sizeof(c64) * m * n, S.s);
 }
 
 int fill_impedance_adm2(TAGS_COMPLEX* yn, TAGS_COMPLEX* yla, TAGS_COMPLEX* ytb, TAGS_COMPLEX* a,
@@ -1814,7 +1841,7 @@ int fill_impedance_adm2(TAGS_COMPLEX* yn, TAGS_COMPLEX* yla, TAGS_COMPLEX* ytb, 
     int rc;
     if (m > 0) {
         if ((rc = d.arm.alloc((size_t)m * n)) || (rc = d.brm.alloc((size_t)m * n)) ||
-            (rc = d.yla.alloc((size_t)m * n)) || (rc = d.ytb.alloc((size_t)m * n)))
+            (rc = d.y.alloc((size_t)2 * m * n)))
             return rc;
         // a and b pass through one staging buffer to their row-major copies
         DevBuf<c64> stage;
@@ -1823,8 +1850,8 @@ int fill_impedance_adm2(TAGS_COMPLEX* yn, TAGS_COMPLEX* yla, TAGS_COMPLEX* ytb, 
         if ((rc = transpose(stage.p, m, nullptr, d.arm.p, n, n, m, 1.0, false, S.s))) return rc;
         if ((rc = copy_in(stage.p, b, sizeof(c64) * m * n, S.s))) return rc;
         if ((rc = transpose(stage.p, m, nullptr, d.brm.p, n, n, m, -1.0, false, S.s))) return rc;
-        if ((rc = copy_in(d.yla.p, yla, sizeof(c64) * m * n, S.s)) ||
-            (rc = copy_in(d.ytb.p, ytb, sizeof(c64) * m * n, S.s)))
+        if ((rc = copy_in(d.y.p, yla, sizeof(c64) * m * n, S.s)) ||
+            (rc = copy_in(d.y.p + m * n, ytb, sizeof(c64) * m * n, S.s)))
             return rc;
     }
     if ((rc = adm_products(d, m, n, S.s))) return rc;

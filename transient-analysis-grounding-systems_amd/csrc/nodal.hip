@@ -1424,7 +1424,7 @@ int NodalSolver::ensure(const HemOp& hem, bool f64_, int batch)
         hipFree(arena);
         arena = nullptr;
         arena_bytes = 0;
-        TAGS_HIP(hipMalloc(&arena, need));
+        TAGS_HIP(dev_malloc((void**)&arena, need));
         arena_bytes = need;
     }
     if (f64) partition<double>(arena, batch);

@@ -111,16 +111,22 @@ enum : int {
     TAGS_ERR_BARRIER = -14,       // a grid barrier timed out (kernel exited early)
 };
 
-// Reports and converts a HIP error; used by every host entry point.
+// Reports and converts a HIP error; used by every host entry point. The runtime's
+// own copy is cleared, or the next call's launch checks would report it again.
 #define TAGS_HIP(call)                                                                  \
     do {                                                                                \
         hipError_t e_ = (call);                                                         \
         if (e_ != hipSuccess) {                                                         \
             std::fprintf(stderr, "tags_hip: %s failed: %s (%s:%d)\n", #call,           \
                          hipGetErrorString(e_), __FILE__, __LINE__);                    \
+            (void)hipGetLastError();                                                    \
             return TAGS_ERR_HIP;                                                        \
         }                                                                               \
     } while (0)
+
+// hipMalloc, except that the allocation armed by tags_fail_allocation fails as
+// one that does not fit.
+hipError_t dev_malloc(void** p, size_t bytes);
 
 // Physical constants with the reference's literal values (src/auxiliary.c:17-21).
 constexpr double kPi = 3.1415926535897932384626433832795029;
