@@ -304,3 +304,10 @@ def test_calls_without_room_for_their_inverses():
     assert _failing(yla_ytb, 4) > 4
     assert _failing(admittance, 2) > 2
     assert _failing(immittance, 2) > 2
+
+
+def test_admittance_size_limit():
+    """65,536 nodes or more stay refused, whichever route would take them."""
+    m, n = 1, 65536
+    a, b, y, z = (np.ones(m * n, complex) for _ in range(4))
+    assert T.calculate_yla_ytb(y, z, np.ones(1, complex), np.ones(1, complex), a, b, m, n) == -13

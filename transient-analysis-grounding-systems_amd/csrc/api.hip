@@ -1756,6 +1756,7 @@ static int adm_inverses(AdmArrays& d, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const 
 {
     int rc;
     if (m == 0) return 0;
+    if (m >= 65536 || n >= 65536) return TAGS_ERR_TOO_LARGE;
     const size_t mm = (size_t)m * m, mn = (size_t)m * n;
     if ((rc = d.z.alloc(2 * mm)) || (rc = d.arm.alloc(mn)) || (rc = d.brm.alloc(mn)) ||
         (rc = d.y.alloc(2 * mn)))
