@@ -248,9 +248,8 @@ __global__ __launch_bounds__(256) void k_gm_update(c64* x, const c64* Z, long sZ
         x[z * n + t] = cadd(o, d);
         a = sqrt(d.x * d.x + d.y * d.y);
     }
-    for (int off = 32; off > 0; off >>= 1) a = fmax(a, __shfl_xor(a, off));
-    if ((threadIdx.x & 63) == 0 && dxn)
-        atomicMax(dxn + z * sn, (unsigned long long)__double_as_longlong(a));
+    const unsigned long long m = wave_max(size_bits(a));
+    if ((threadIdx.x & 63) == 0 && dxn) atomicMax(dxn + z * sn, m);
 }
 
 int GmresWork::alloc(int n_, int kmax_, int cap_)

@@ -1369,7 +1369,7 @@ __global__ __launch_bounds__(256) void k_hem_apply(const c64* W, long ld, HemOp 
     }
     // node rows: sum over the node's segment ends of A^T (x_L) and B^T (x_T)
     const long u = ((long)blockIdx.x - 2 * wg) * 256 + threadIdx.x;
-    double ra = 0, xa = 0, ta = 0;
+    double ra = 0, xa = 0, ta = 0;  // sizes
     if (u < op.n) {
         DD tx{0, 0}, ty{0, 0};
         const int p1 = op.node_ptr[u + 1];
@@ -1395,15 +1395,12 @@ __global__ __launch_bounds__(256) void k_hem_apply(const c64* W, long ld, HemOp 
         }
     }
     if (mode == 0) return;
-    for (int o = 32; o > 0; o >>= 1) {
-        ra = fmax(ra, __shfl_xor(ra, o));
-        xa = fmax(xa, __shfl_xor(xa, o));
-        ta = fmax(ta, __shfl_xor(ta, o));
-    }
+    const unsigned long long rm = wave_max(size_bits(ra)), xm = wave_max(size_bits(xa)),
+                             tm = wave_max(size_bits(ta));
     if ((threadIdx.x & 63) == 0) {
-        atomicMax(&norms[0], (unsigned long long)__double_as_longlong(ra));
-        atomicMax(&norms[1], (unsigned long long)__double_as_longlong(xa));
-        if (want_w) atomicMax(&norms[2], (unsigned long long)__double_as_longlong(ta));
+        atomicMax(&norms[0], rm);
+        atomicMax(&norms[1], xm);
+        if (want_w) atomicMax(&norms[2], tm);
     }
 }
 
@@ -1617,8 +1614,8 @@ __global__ __launch_bounds__(256) void k_update_x(c64* x, const c32* z, const do
         a = sqrt(dx * dx + dy * dy);
     }
     if (!dxn) return;
-    for (int off = 32; off > 0; off >>= 1) a = fmax(a, __shfl_xor(a, off));
-    if ((threadIdx.x & 63) == 0) atomicMax(dxn, (unsigned long long)__double_as_longlong(a));
+    const unsigned long long m = wave_max(size_bits(a));
+    if ((threadIdx.x & 63) == 0) atomicMax(dxn, m);
 }
 
 // t[i] = b[perm[i]]

@@ -911,10 +911,10 @@ __global__ __launch_bounds__(256) void k_nd_node(NdArgs<T> g, int kprev)
     g.f[item * g.np + u] = cx<T>{(T)t.x, (T)t.y};
 }
 
-__device__ inline void dx_max(unsigned long long* p, double a)
+__device__ inline void dx_max(unsigned long long* p, unsigned long long a)
 {
-    for (int o = 32; o > 0; o >>= 1) a = fmax(a, __shfl_xor(a, o));
-    if ((threadIdx.x & 63) == 0) atomicMax(p, (unsigned long long)__double_as_longlong(a));
+    a = wave_max(a);
+    if ((threadIdx.x & 63) == 0) atomicMax(p, a);
 }
 
 // alpha and w (y is replaced by w), u += scale (w + alpha), and the segments'
@@ -947,14 +947,14 @@ __global__ __launch_bounds__(1024) void k_nd_alpha(NdArgs<T> g, int k, int first
     a = wg_sum(a, red);
     if (first) a.x += 1.0;
     const c64 al = cmul(a, g.cst[4 * item + 2]);
-    double dm = 0.0;
+    unsigned long long dm = 0;
     for (long u = threadIdx.x; u < g.n; u += 1024) {
         const cx<T> hu = h[u], yu = yin[u];
         const c64 w = csub(c64{yu.x, yu.y}, cmul(al, c64{hu.x, hu.y}));
         y[u] = cx<T>{(T)w.x, (T)w.y};
         const c64 d = cscale(cadd(w, al), scale);
         x[2 * g.m + u] = first ? d : cadd(x[2 * g.m + u], d);
-        dm = fmax(dm, sqrt(d.x * d.x + d.y * d.y));
+        dm = max(dm, size_bits(sqrt(d.x * d.x + d.y * d.y)));
     }
     dx_max(g.norms + item * g.snorm + 4 * k + 3, dm);
     __syncthreads();
@@ -988,7 +988,7 @@ __global__ __launch_bounds__(256) void k_nd_currents(NdArgs<T> g, int k, int fir
     cx<T> acc[4];
     nd_gemv_rows<T, 2>(g, g.v, item, (int)(mat & 1), row0, acc);
     const int lane = threadIdx.x & 63;
-    double dm = 0.0;
+    unsigned long long dm = 0;
     if (lane < 4 && row0 + lane < g.m) {
         const double s =
             first ? 1.0 : nd_scale(g.norms + item * g.snorm + 4 * (k - 1), sizeof(T) == 4);
@@ -997,7 +997,7 @@ __global__ __launch_bounds__(256) void k_nd_currents(NdArgs<T> g, int k, int fir
         const c64 d{a.x * s, a.y * s};
         c64* xi = g.x + item * g.N + (mat & 1) * g.m + row0 + lane;
         *xi = first ? d : cadd(*xi, d);
-        dm = sqrt(d.x * d.x + d.y * d.y);
+        dm = size_bits(sqrt(d.x * d.x + d.y * d.y));
     }
     dx_max(g.norms + item * g.snorm + 4 * k + 3, dm);
 }
@@ -1028,11 +1028,7 @@ __global__ __launch_bounds__(256) void k_nd_pick(NdArgs<T> g, c64* u, unsigned l
 // ---------------------------------------------------------------------------
 // Small systems (at most 64 segments and 64 nodes) in one launch
 // ---------------------------------------------------------------------------
-// the larger of two values >= 0 as bits (a NaN is larger than all)
-__device__ inline void bits_max(unsigned long long& m, double a)
-{
-    m = max(m, (unsigned long long)__double_as_longlong(a));
-}
+__device__ inline void bits_max(unsigned long long& m, double a) { m = max(m, size_bits(a)); }
 
 // Everything of a sample after the fill: both inverses (256 threads each), the
 // node system, its inverse, and `spec` refinement steps, by one work-group, with
@@ -1836,15 +1832,9 @@ __global__ __launch_bounds__(256) void k_sub_identity(c64* R, long m, long total
             v.x -= 1.0;
             R[e] = v;
         }
-        // as bit patterns: a NaN counts as larger than any number
-        const unsigned long long b =
-            (unsigned long long)__double_as_longlong(fabs(v.x) + fabs(v.y));
-        a = b > a ? b : a;
+        a = max(a, size_bits(fabs(v.x) + fabs(v.y)));
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long b = __shfl_xor(a, o);
-        a = b > a ? b : a;
-    }
+    a = wave_max(a);
     if ((threadIdx.x & 63) == 0) atomicMax(dmax, a);
 }
 int sub_identity(c64* R, long m, int items, unsigned long long* dmax, hipStream_t st)

@@ -163,6 +163,18 @@ struct BlockLayout {
     long node_off, zl_off, zt_off;
 };
 
+// Norms are reduced as the bits of values >= 0, which order as the values do and
+// put a NaN above every number (fmax would drop it).
+__device__ inline unsigned long long size_bits(double a)
+{
+    return (unsigned long long)__double_as_longlong(a);
+}
+__device__ inline unsigned long long wave_max(unsigned long long a)
+{
+    for (int o = 32; o > 0; o >>= 1) a = max(a, (unsigned long long)__shfl_xor(a, o));
+    return a;
+}
+
 // ---- fill.hip ----
 int gl_tables_init();
 int launch_pairs_dropin(double* zl, double* zt, bool alias, SegSoA e, long m,
