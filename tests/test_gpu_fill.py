@@ -75,3 +75,70 @@ def test_group_fill_matches_single_samples(m, nf):
         res.append(sw.solve(s, kap, 0, T.PREC_FP64)[0])
     sw.close()
     assert np.max(np.abs(res[0] - res[1]) / np.abs(res[1])) <= 1e-12
+
+
+def _unit_integral(S, R, g):
+    """int int e^{-g r} / r over the unit square in extended precision: 24-point
+    Gauss rules on two panels a side (a segment apart or more: below 1e-17)."""
+    x, w = np.polynomial.legendre.leggauss(24)
+    x, w = (x.astype(np.longdouble) + 1) / 4, w.astype(np.longdouble) / 4
+    # one Newton step on P_24 from the 64-bit nodes, and their weights
+    z = 4 * x - 1
+    p0, p1 = np.ones_like(z), np.zeros_like(z)
+    for k in range(1, 25):
+        p0, p1 = ((2 * k - 1) * z * p0 - (k - 1) * p1) / k, p0
+    dp = 24 * (z * p0 - p1) / (z * z - 1)
+    z = z - p0 / dp
+    p0, p1 = np.ones_like(z), np.zeros_like(z)
+    for k in range(1, 25):
+        p0, p1 = ((2 * k - 1) * z * p0 - (k - 1) * p1) / k, p0
+    dp = 24 * (z * p0 - p1) / (z * z - 1)
+    x, w = (z + 1) / 4, 2 / ((1 - z * z) * dp * dp) / 4
+    t, wt = np.concatenate([x, x + np.longdouble(0.5)]), np.concatenate([w, w])
+    a, b, c, d = (np.asarray(v, np.longdouble) for v in (*S, *R))
+    p, q = a + t[:, None] * (b - a), c + t[:, None] * (d - c)
+    r = np.sqrt(((p[:, None] - q[None]) ** 2).sum(axis=2))
+    f = np.exp(-g * r) / r
+    return (wt[:, None] * wt[None] * f).sum()
+
+
+# gamma = (1 + 0 j or 1 j) re, exactly: its square is kappa with s = 1 and s mu = 1
+@pytest.mark.parametrize("re,im", [(2.0, 0), (3.625, 0), (5.0, 0), (7.25, 0), (1.75, 1), (2.5, 1),
+                                   (3.5, 1), (4.9375, 1), (6.0, 1)])
+def test_fill_keeps_the_direct_rules_digits(re, im):
+    """Far pairs (3 to 20 lengths) of 40 segments of 0.3 to 1 m in random
+    directions 12 m deep, with their images, on all sides of the moment rule's
+    limits. Against extended precision: 2e-14 of both parts' sizes. (The direct
+    rule's rounding and remainder stay below 1e-14 there, largest at |gamma| = 7,
+    where the phase of the farthest pair is 140. Below |gamma| = 1 the remainder of
+    its orders, not rounding, decides: up to 2.5e-12.)"""
+    rng = np.random.default_rng(11)
+    m, depth = 40, 12.0
+    c = rng.uniform(-7, 7, (m, 3))
+    d = rng.standard_normal((m, 3))
+    d *= rng.uniform(0.15, 0.5, (m, 1)) / np.linalg.norm(d, axis=1, keepdims=True)
+    d[0] *= 0.5 / np.linalg.norm(d[0])
+    e = np.zeros(m, T.ELECTRODE_DTYPE)
+    for i in range(m):
+        e[i] = T.populate_electrode(c[i] - d[i] - [0, 0, depth], c[i] + d[i] - [0, 0, depth], 5e-3)[1][0]
+    nodes = np.concatenate([e["start_point"], e["end_point"]])
+    g = re * (1 + im * 1j)
+    kap = 2j * re * re if im else re * re + 0j
+    mur = [v for v in 1 / T.MU0 + np.arange(-4, 5) * np.spacing(1 / T.MU0) if T.MU0 * v == 1.0][0]
+    pairs = [(i, k) for i in range(m) for k in range(i) if np.linalg.norm(c[i] - c[k]) >= 4.0]
+    pairs = [pairs[j] for j in rng.choice(len(pairs), 60, replace=False)]
+    n = len(nodes)
+    i, k = np.array(pairs).T
+    sw = T.Sweep(e, nodes)
+    got = -sw.assemble_entries(1.0, kap, n + m + i, n + m + k, mur=mur)
+    sw.close()
+    img = T.images_of(e)
+    kl = np.clongdouble(kap)
+    eps = np.longdouble(T.EPS0)
+    for z, (p, q) in zip(got, pairs):
+        d, r = (_unit_integral((e[q]["start_point"], e[q]["end_point"]),
+                               (x[p]["start_point"], x[p]["end_point"]), np.clongdouble(g))
+                for x in (e, img))
+        r *= (kl - eps) / (kl + eps)
+        err = abs(z * np.longdouble(T.FOUR_PI) * kl - (d + r))
+        assert err <= 2e-14 * (abs(d) + abs(r)), (p, q, float(err / (abs(d) + abs(r))))

@@ -2287,10 +2287,11 @@ static int sweep_fill_items(tags_sweep* sw, c64* W, hipStream_t st, Profiler* pr
     Timed tm(prof, FAM_FILL, st);
     int rc;
     TAGS_HIP(hipMemcpyAsync(sb.d, sb.h, sizeof(PairScalars) * nb, hipMemcpyHostToDevice, st));
-    double gabs = 0.0;
+    double gabs = 0.0, gre = 0.0;
     for (int z = 0; z < nb; z++) {
         const double g = std::hypot(sb.h[z].gamma.x, sb.h[z].gamma.y);
         gabs = g > gabs || g != g ? g : gabs;
+        gre = std::max(gre, std::fabs(sb.h[z].gamma.x));
     }
     if (fill_static && (rc = launch_fill_static(W, N, sw->layout, sw->sn, sw->en, st, nb, sW)))
         return rc;
@@ -2301,9 +2302,9 @@ static int sweep_fill_items(tags_sweep* sw, c64* W, hipStream_t st, Profiler* pr
                                    sw->pot + mm, sw->pot + 2 * mm, sw->pot + 3 * mm, sb.d, st, nb,
                                    sW)))
             return rc;
-    } else if (sw->dmax > 0.0 && fill_terms(gabs * sw->dmax) > 0) {
+    } else if (sw->dmax > 0.0 && fill_terms(gabs * sw->dmax, gre * sw->dmax) > 0) {
         if ((rc = launch_fill_moments(W, N, L, sw->e.soa(), sw->img.soa(), sb.d, sb.cf, nb, sW,
-                                      sw->dmax, gabs, st)))
+                                      sw->dmax, gabs, gre, st)))
             return rc;
     } else if ((rc = launch_fill_zblocks(W, N, L, sw->e.soa(), sw->img.soa(), sb.d, st, nb, sW))) {
         return rc;

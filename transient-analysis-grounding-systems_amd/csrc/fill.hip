@@ -38,27 +38,29 @@ __constant__ int g_gloff[kNumOrders];
 static bool g_gl_ready = false;
 static std::mutex g_gl_mutex;
 
-// Legendre nodes by Newton iteration on P_n from the Chebyshev-like guess.
+// Legendre nodes by Newton iteration on P_n from the Chebyshev-like guess, in
+// extended precision: in 64 bits the weights of the nodes near the ends, where
+// 1 - z^2 cancels, were several ulps off.
 void gauss_legendre(int n, double* x, double* w)
 {
     for (int i = 0; i < n; i++) {
-        double z = std::cos(kPi * (i + 0.75) / (n + 0.5));
-        double dp = 0;
+        long double z = std::cos(kPi * (i + 0.75) / (n + 0.5));
+        long double dp = 0;
         for (int it = 0; it < 100; it++) {
-            double p0 = 1.0, p1 = 0.0;
+            long double p0 = 1.0L, p1 = 0.0L;
             for (int k = 1; k <= n; k++) {
-                double p2 = p1;
+                long double p2 = p1;
                 p1 = p0;
-                p0 = ((2.0 * k - 1.0) * z * p1 - (k - 1.0) * p2) / k;
+                p0 = ((2.0L * k - 1.0L) * z * p1 - (k - 1.0L) * p2) / k;
             }
-            dp = n * (z * p0 - p1) / (z * z - 1.0);
-            double dz = p0 / dp;
+            dp = n * (z * p0 - p1) / (z * z - 1.0L);
+            long double dz = p0 / dp;
             z -= dz;
-            if (std::fabs(dz) < 1e-16) break;
+            if (std::fabs(dz) < 1e-19L) break;
         }
         // map [-1, 1] -> [0, 1]
-        x[i] = 0.5 * (1.0 - z);
-        w[i] = 1.0 / ((1.0 - z * z) * dp * dp);
+        x[i] = (double)(0.5L * (1.0L - z));
+        w[i] = (double)(1.0L / ((1.0L - z * z) * dp * dp));
     }
 }
 
@@ -638,8 +640,16 @@ int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
 // direct rule would take, then one complex exponential and 2 K multiply-adds
 // per sample, where the direct rule takes a square root, an exponential and a
 // sine and cosine at every point of every sample. The Chebyshev tail beyond K
-// terms is below 1e-17 for |gamma| D <= 7.3 (K = 32, see fill_terms); larger
-// ones keep the direct rule (k_fill_zblocks).
+// terms is below 1e-17 (see fill_terms).
+//
+// Rounding. The coefficients grow as e^{|Re gamma| D} while J is governed by the r
+// near R, so the sum cancels by up to that factor; and the one phase gamma R has
+// the rounding that the direct rule spreads over its points, so its products'
+// rounding errors are carried (rotor). With |Re gamma| D <= 2 and |gamma| D <= 5
+// the error is the direct rule's (worst of 160 pairs far, near and touching, R to
+// 60 D, arg gamma 0 .. 90 degrees, against 113 bits: 2.5e-15 against 3e-15 at
+// |gamma| D = 2, 1.5e-14 against 1.2e-14 at 5); beyond, up to 3e-13 against 8e-15,
+// so those keep the direct rule (k_fill_zblocks).
 //
 // One thread per pair of a TS x TS tile on or below the diagonal, work-groups
 // of one tile and a range of the samples (so that few segments still fill the
@@ -726,6 +736,18 @@ __device__ inline void mom_duffy(Moments<K>& M, V3 p, V3 q, bool w_on_p, int lan
             hi += hi;
         }
     }
+}
+
+// e^{-g R} with the rounding errors of both products g R taken along
+__device__ inline c64 rotor(c64 g, double R)
+{
+    const double ph = -g.y * R, pl = fma(-g.y, R, -ph);
+    const double ea = -g.x * R, el = fma(-g.x, R, -ea);
+    double sn, cs;
+    sincos(ph, &sn, &cs);
+    double mag = exp(ea);
+    mag = fma(mag, el, mag);
+    return c64{mag * fma(-pl, sn, cs), mag * fma(pl, cs, sn)};
 }
 
 // Moments of a pair by one wave (touching, or closer than two lengths)
@@ -910,13 +932,8 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
                 ix = fma(q.x, mi[j], ix);
                 iy = fma(q.y, mi[j], iy);
             }
-            double sn, cs;
-            sincos(-sc.gamma.y * rd, &sn, &cs);
-            double mag = exp(-sc.gamma.x * rd);
-            const c64 jd = cmul(c64{mag * cs, mag * sn}, c64{dx, dy});
-            sincos(-sc.gamma.y * ri, &sn, &cs);
-            mag = exp(-sc.gamma.x * ri);
-            const c64 ji = cmul(c64{mag * cs, mag * sn}, c64{ix, iy});
+            const c64 jd = cmul(rotor(sc.gamma, rd), c64{dx, dy});
+            const c64 ji = cmul(rotor(sc.gamma, ri), c64{ix, iy});
             // the formulas of k_fill_zblocks, J the integral over L_r L_s
             if (k == i) {
                 vl = cscale(sc.zl_dir, self);
@@ -988,20 +1005,22 @@ __global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, doubl
     cf[(long)blockIdx.x * K + p] = cscale(s, (p == 0 ? 1.0 : 2.0) / 64.0);
 }
 
-// Chebyshev terms for |gamma| D = z: 2 (z / 2)^K / K! <= 1e-17, the size of the
-// first coefficient left out; 0 beyond the largest table entry
-int fill_terms(double z)
+// Chebyshev terms for |gamma| D = z, |Re gamma| D = re: 2 (z / 2)^K / K! <= 1e-17,
+// the size of the first coefficient left out (which 32 terms keep to z = 7.3); 0
+// where the sum's rounding passes the direct rule's
+int fill_terms(double z, double re)
 {
-    return z <= 0.38 ? 12 : z <= 1.13 ? 16 : z <= 3.7 ? 24 : z <= 7.3 ? kFillTermsMax : 0;
+    if (!(re <= 2.0)) return 0;
+    return z <= 0.38 ? 12 : z <= 1.13 ? 16 : z <= 3.7 ? 24 : z <= 5.0 ? kFillTermsMax : 0;
 }
 
 int launch_fill_moments(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
                         const PairScalars* scs, c64* cf, int nb, long sw, double D, double gabs,
-                        hipStream_t st)
+                        double gre, hipStream_t st)
 {
     const long m = L.m;
     if (m <= 0 || nb <= 0) return 0;
-    const int K = fill_terms(gabs * D);
+    const int K = fill_terms(gabs * D, gre * D);
     if (K == 0 || !(D > 0.0) || !scs || !cf) return TAGS_ERR_ARG;
     int rc = gl_tables_init();
     if (rc) return rc;

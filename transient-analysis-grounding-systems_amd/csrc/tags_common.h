@@ -193,14 +193,14 @@ int launch_fill_mhem(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA im
 int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
                         const PairScalars* scs, hipStream_t st, int nb, long sw);
 // The impedance blocks of nb samples from Chebyshev moments (k_fill_moments):
-// D the longest segment (by its end points), gabs the largest |gamma| of the
-// samples, fill_terms(gabs D) > 0; scs in device memory, cf nb kFillTermsMax
-// values of scratch.
+// D the longest segment (by its end points), gabs and gre the largest |gamma| and
+// |Re gamma| of the samples, fill_terms(gabs D, gre D) > 0; scs in device memory,
+// cf nb kFillTermsMax values of scratch.
 constexpr int kFillTermsMax = 32;
-int fill_terms(double z);
+int fill_terms(double z, double re);
 int launch_fill_moments(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
                         const PairScalars* scs, c64* cf, int nb, long sw, double D, double gabs,
-                        hipStream_t st);
+                        double gre, hipStream_t st);
 int launch_fill_static(c64* W, long ldw, const BlockLayout& L, const int* seg_start_node,
                        const int* seg_end_node, hipStream_t st, int nb = 1, long sw = 0);
 int launch_single_pair(SegSoA e, SegSoA r, c64 gamma, int type, double* out4, hipStream_t st);
