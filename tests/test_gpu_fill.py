@@ -142,3 +142,33 @@ def test_fill_keeps_the_direct_rules_digits(re, im):
         r *= (kl - eps) / (kl + eps)
         err = abs(z * np.longdouble(T.FOUR_PI) * kl - (d + r))
         assert err <= 2e-14 * (abs(d) + abs(r)), (p, q, float(err / (abs(d) + abs(r))))
+
+
+@pytest.mark.parametrize("m", [9, 17, 257])
+def test_a_sample_does_not_see_its_group(m):
+    """Samples of every class of the moment rule and of the direct one, in rising
+    and in shuffled order, solved in one group, in groups of three and one at a
+    time, on one slot and several: the same bits, and W alone the same as W in any
+    company (through x)."""
+    rc, e, nodes = T.segment_electrode([0, 0, -0.5], [3.0 * m, 0, -0.5], m, 7e-3)
+    f = np.concatenate([[50.0], 10.0 ** np.linspace(4, 8, 33)])
+    s = 2j * np.pi * f
+    kap = 1e-3 + s * 10.0 * T.EPS0
+    z = np.abs(np.sqrt(s * T.MU0 * kap)) * 3.0
+    assert [np.sum((z > a) & (z <= b)) > 0 for a, b in
+            ((0, 0.38), (0.38, 1), (1, 2), (2, 3.7), (3.7, 5), (5, 1e9))] == [True] * 6
+    mix = np.random.default_rng(m).permutation(len(f))
+    sw = T.Sweep(e, nodes)
+    for prec in (T.PREC_FP64, T.PREC_MIXED):
+        ref = None
+        for batch, inflight, order in ((1, 1, np.arange(len(f))), (0, 4, np.arange(len(f))),
+                                       (0, 1, mix), (3, 2, mix)):
+            sw.set_batch(batch)
+            sw.set_inflight(inflight)
+            u, st, x = sw.solve(s[order], kap[order], 0, prec, want_x=True)
+            assert all(q["precision_used"] == prec for q in st)
+            back = np.argsort(order)
+            if ref is None:
+                ref = x[back]
+            assert np.array_equal(x[back], ref)
+    sw.close()

@@ -113,6 +113,7 @@ static PairScalars make_scalars(c64 gamma, c64 s, double mur, c64 kappa, c64 ref
     PairScalars sc;
     sc.gamma = gamma;
     sc.intg_type = type;
+    sc.item = 0;
     if (type == INTG_NONE || type == INTG_MHEM) {
         sc.zl_dir = sc.zt_dir = sc.zl_img = sc.zt_img = c64{1.0, 0.0};
         return sc;
@@ -2273,6 +2274,25 @@ static PairScalars sample_scalars(TAGS_COMPLEX s_, TAGS_COMPLEX kappa_, double m
     return make_scalars(gf, sf, mur, kf, rl, rt, INTG_DOUBLE);
 }
 
+// The scalars of items 0 .. nb - 1 by the class of their |gamma| D (those that keep
+// the direct rule last), each naming its item, and the classes' counts.
+static void sort_by_class(PairScalars* h, int nb, double D, int (&count)[kFillClasses + 1])
+{
+    std::vector<int> cls(nb), at(kFillClasses + 2, 0);
+    bool sorted = true;
+    for (int z = 0; z < nb; z++) {
+        h[z].item = z;
+        const c64 g = h[z].gamma;
+        cls[z] = D > 0.0 ? fill_class(std::hypot(g.x, g.y) * D, std::fabs(g.x) * D) : kFillClasses;
+        count[cls[z]]++;
+        sorted = sorted && (z == 0 || cls[z] >= cls[z - 1]);
+    }
+    if (sorted) return;
+    for (int c = 0; c <= kFillClasses; c++) at[c + 1] = at[c] + count[c];
+    const std::vector<PairScalars> was(h, h + nb);
+    for (int z = 0; z < nb; z++) h[at[cls[z]]++] = was[z];
+}
+
 // Assembly of nb samples' W (item z at W + z N^2) in the sweep's block layout:
 // their scalars in sb.h (uploaded here).
 static int sweep_fill_items(tags_sweep* sw, c64* W, hipStream_t st, Profiler* prof, int nb,
@@ -2286,28 +2306,26 @@ static int sweep_fill_items(tags_sweep* sw, c64* W, hipStream_t st, Profiler* pr
     else sW = N * N;
     Timed tm(prof, FAM_FILL, st);
     int rc;
+    const bool hem = sw->formulation != TAGS_FORM_MHEM;
+    int count[kFillClasses + 1] = {};
+    if (hem) sort_by_class(sb.h, nb, sw->dmax, count);
     TAGS_HIP(hipMemcpyAsync(sb.d, sb.h, sizeof(PairScalars) * nb, hipMemcpyHostToDevice, st));
-    double gabs = 0.0, gre = 0.0;
-    for (int z = 0; z < nb; z++) {
-        const double g = std::hypot(sb.h[z].gamma.x, sb.h[z].gamma.y);
-        gabs = g > gabs || g != g ? g : gabs;
-        gre = std::max(gre, std::fabs(sb.h[z].gamma.x));
-    }
     if (fill_static && (rc = launch_fill_static(W, N, sw->layout, sw->sn, sw->en, st, nb, sW)))
         return rc;
-    if (sw->formulation == TAGS_FORM_MHEM) {
+    if (!hem) {
         if (!sw->pot) return TAGS_ERR_ARG;
         const size_t mm = (size_t)sw->m * sw->m;
         if ((rc = launch_fill_mhem(W, N, L, sw->e.soa(), sw->img.soa(), sw->pot,
                                    sw->pot + mm, sw->pot + 2 * mm, sw->pot + 3 * mm, sb.d, st, nb,
                                    sW)))
             return rc;
-    } else if (sw->dmax > 0.0 && fill_terms(gabs * sw->dmax, gre * sw->dmax) > 0) {
-        if ((rc = launch_fill_moments(W, N, L, sw->e.soa(), sw->img.soa(), sb.d, sb.cf, nb, sW,
-                                      sw->dmax, gabs, gre, st)))
+    } else {
+        const int nd = count[kFillClasses];
+        if ((rc = launch_fill_moments(W, N, L, sw->e.soa(), sw->img.soa(), sb.d, sb.cf, count, sW,
+                                      sw->dmax, st)) ||
+            (rc = launch_fill_zblocks(W, N, L, sw->e.soa(), sw->img.soa(), sb.d + nb - nd, st, nd,
+                                      sW)))
             return rc;
-    } else if ((rc = launch_fill_zblocks(W, N, L, sw->e.soa(), sw->img.soa(), sb.d, st, nb, sW))) {
-        return rc;
     }
     tm.end();
     return 0;

@@ -513,7 +513,7 @@ __global__ __launch_bounds__(256) void k_fill_zblocks(c64* W, long ldw, long zl_
 {
     // item blockIdx.z of a batch: its own W and frequency-sample scalars
     const PairScalars sc = scs[blockIdx.z];
-    W += (long)blockIdx.z * sw;
+    W += (long)sc.item * sw;
     // triangular tile index -> (ti >= tk)
     const long b = blockIdx.x;
     long ti = (long)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
@@ -636,11 +636,13 @@ int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
 // so that the pair integral of every sample is
 //   J(gamma) = e^{-gamma R} sum_{k < K} c_k(gamma) M_k,
 //   M_k = int int T_k((r - R) / D) / r over the unit square:
-// K real moments per pair and group of samples, on the quadrature points the
+// K real moments per pair and class of samples, on the quadrature points the
 // direct rule would take, then one complex exponential and 2 K multiply-adds
 // per sample, where the direct rule takes a square root, an exponential and a
-// sine and cosine at every point of every sample. The Chebyshev tail beyond K
-// terms is below 1e-17 (see fill_terms).
+// sine and cosine at every point of every sample. The number of terms and the
+// quadrature orders follow the sample's own |gamma| in steps (fill_class), so that
+// what it is solved with does not show in its entries; the Chebyshev tail beyond
+// K terms is below 1e-17.
 //
 // Rounding. The coefficients grow as e^{|Re gamma| D} while J is governed by the r
 // near R, so the sum cancels by up to that factor; and the one phase gamma R has
@@ -652,8 +654,8 @@ int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
 // so those keep the direct rule (k_fill_zblocks).
 //
 // One thread per pair of a TS x TS tile on or below the diagonal, work-groups
-// of one tile and a range of the samples (so that few segments still fill the
-// device). Pairs that touch or are closer than two lengths, which need the
+// of one tile and a range of the samples of one class (so that few segments still
+// fill the device). Pairs that touch or are closer than two lengths, which need the
 // Duffy rule or 144 points and more, are listed in LDS and taken by whole
 // waves, the lanes sharing the points; moments pass through LDS, so that few
 // of them are live in registers at a time. TS is 16, or 8 for few segments (a
@@ -796,13 +798,34 @@ __device__ inline bool pair_near(const DSeg& S, const DSeg& R, double* rho)
 }
 
 constexpr int fill_waves(int ts) { return ts == 8 ? 8 : 4; }
-template <int K, int TS>
+
+// The classes of samples by |gamma| D (in ascending order): Chebyshev terms and the
+// bound that the class's quadrature orders are chosen for. Terms: 2 (z / 2)^K / K!,
+// the size of the first coefficient left out, is at most 1e-17 (12 to z = 0.38, 16
+// to 1.13, 24 to 3.7, 32 to 7.3); bounds where geometric_order steps.
+constexpr int kFillTerms[kFillClasses] = {12, 16, 24, 24, 32};
+constexpr double kFillBound[kFillClasses] = {0.38, 1.0, 2.0, 3.7, 5.0};
+__device__ inline double fill_bound(int c)
+{
+    return c == 0 ? kFillBound[0] : c == 1 ? kFillBound[1] : c == 2 ? kFillBound[2]
+         : c == 3 ? kFillBound[3] : kFillBound[4];
+}
+
+// Samples by class: class c's are first[c] .. first[c + 1] - 1, in work-groups
+// (blockIdx.y) chunk[c] .. chunk[c + 1] - 1 of `per` samples.
+struct FillGroups {
+    int first[kFillClasses + 1], chunk[kFillClasses + 1], per;
+};
+
+// One kernel for all classes: the terms of the widest one decide the registers,
+// but two waves per SIMD is what every one of them allows (170 .. 256).
+template <int TS>
 __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __restrict__ W, long ldw,
                                                        long zl_off, long zt_off, long m, SegSoA e,
                                                        SegSoA img,
                                                        const PairScalars* __restrict__ scs, long sw,
-                                                       const c64* __restrict__ cf, int nf, int per,
-                                                       double D, double gabs)
+                                                       const c64* __restrict__ cf, FillGroups grp,
+                                                       double D)
 {
     const long b = blockIdx.x;
     long ti = (long)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
@@ -823,7 +846,7 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
     // every pair's moments of one kind or both while they are formed; then the
     // tiles being transposed
     union Stage {
-        double mom[KINDS][K][NP];
+        double mom[KINDS][kFillTermsMax][NP];
         c64 tile[2][2][TS][TS + 1];
     };
     __shared__ Stage stage;
@@ -849,6 +872,13 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
         return DSeg{V3{geo[side][0][s], geo[side][1][s], geo[side][2][s]},
                     V3{geo[side][3][s], geo[side][4][s], geo[side][5][s]}, geo[side][6][s]};
     };
+    int cls = 0;
+    while (cls + 1 < kFillClasses && (int)blockIdx.y >= grp.chunk[cls + 1]) cls++;
+    const double gabs = fill_bound(cls) / D;
+    const int f0 = grp.first[cls] + ((int)blockIdx.y - grp.chunk[cls]) * grp.per;
+    const int f1 = min(grp.first[cls + 1], f0 + grp.per);
+    auto fill = [&](auto terms) {
+    constexpr int K = decltype(terms)::value;
     double md[K], mi[K];  // direct, image
     double rd = 0.0, ri = 0.0, cost = 0.0, cosi = 0.0, ll = 1.0;
     // far pairs by a lane each (with 8 x 8 tiles a wave to each kind) ..
@@ -917,10 +947,9 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
         ll = S.len * R.len;
     }
     const double self = in && k == i ? self_integral_dev(geo[1][6][a], geo[1][7][a]) : 0.0;
-    const int f0 = blockIdx.y * per, f1 = min(nf, f0 + per);
     for (int f = f0 + (TS == 8 ? wave : 0); f < f1; f += TS == 8 ? NW : 1) {
         const PairScalars& sc = scs[f];
-        const c64* cq = cf + (long)f * K;
+        const c64* cq = cf + (long)f * kFillTermsMax;
         c64 vl{0, 0}, vt{0, 0};
         if (in) {
             double dx = 0, dy = 0, ix = 0, iy = 0;
@@ -947,7 +976,7 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
                 vl = cadd(vl, cscale(cmul(sc.zl_img, ji), cosi));
             vl = c64{-vl.x, -vl.y};
             vt = c64{-vt.x, -vt.y};
-            c64* Wf = W + (long)f * sw;
+            c64* Wf = W + (long)sc.item * sw;
             Wf[(zl_off + i) * ldw + zl_off + k] = vl;
             Wf[(zt_off + i) * ldw + zt_off + k] = vt;
         }
@@ -958,7 +987,7 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
             const c64 ot{__shfl(vt.x, from), __shfl(vt.y, from)};
             const long ko = k0 + a, io = i0 + c;
             if (io < m && ko < io) {
-                c64* Wf = W + (long)f * sw;
+                c64* Wf = W + (long)sc.item * sw;
                 Wf[(zl_off + ko) * ldw + zl_off + io] = ol;
                 Wf[(zt_off + ko) * ldw + zt_off + io] = ot;
             }
@@ -969,18 +998,24 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
             __syncthreads();
             const long ko = k0 + a, io = i0 + c;  // entry (ko, io) of the other triangle
             if (io < m && ko < io) {
-                c64* Wf = W + (long)f * sw;
+                c64* Wf = W + (long)sc.item * sw;
                 Wf[(zl_off + ko) * ldw + zl_off + io] = stage.tile[h][0][c][a];
                 Wf[(zt_off + ko) * ldw + zt_off + io] = stage.tile[h][1][c][a];
             }
         }
+    }    };
+    switch (cls) {
+    case 0: fill(std::integral_constant<int, kFillTerms[0]>()); break;
+    case 1: fill(std::integral_constant<int, kFillTerms[1]>()); break;
+    case 2:
+    case 3: fill(std::integral_constant<int, kFillTerms[3]>()); break;
+    default: fill(std::integral_constant<int, kFillTerms[4]>()); break;
     }
 }
 
 // c_k(gamma_f) = (2 - [k = 0]) / P sum_p cos(k theta_p) e^{-gamma D cos theta_p},
 // theta_p = pi (p + 1/2) / P, P = 64; one wave per sample
-__global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, double D, int K,
-                                                    c64* cf)
+__global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, double D, c64* cf)
 {
     __shared__ c64 ex[64];
     __shared__ double tab[256];  // cos(pi j / 128): k theta_p is a multiple of pi / 128
@@ -994,7 +1029,7 @@ __global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, doubl
     const double mag = exp(-g.x * x);
     ex[p] = c64{mag * cs, mag * sn};
     __syncthreads();
-    if (p >= K) return;
+    if (p >= kFillTermsMax) return;
     c64 s{0, 0};
 #pragma unroll 8
     for (int q = 0; q < 64; q++) {
@@ -1002,51 +1037,51 @@ __global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, doubl
         s.x = fma(w, ex[q].x, s.x);
         s.y = fma(w, ex[q].y, s.y);
     }
-    cf[(long)blockIdx.x * K + p] = cscale(s, (p == 0 ? 1.0 : 2.0) / 64.0);
+    cf[(long)blockIdx.x * kFillTermsMax + p] = cscale(s, (p == 0 ? 1.0 : 2.0) / 64.0);
 }
 
-// Chebyshev terms for |gamma| D = z, |Re gamma| D = re: 2 (z / 2)^K / K! <= 1e-17,
-// the size of the first coefficient left out (which 32 terms keep to z = 7.3); 0
-// where the sum's rounding passes the direct rule's
-int fill_terms(double z, double re)
+// Class of a sample with |gamma| D = z, |Re gamma| D = re; kFillClasses where the
+// sum's rounding passes the direct rule's (or nothing is known of z)
+int fill_class(double z, double re)
 {
-    if (!(re <= 2.0)) return 0;
-    return z <= 0.38 ? 12 : z <= 1.13 ? 16 : z <= 3.7 ? 24 : z <= 5.0 ? kFillTermsMax : 0;
+    if (re <= 2.0)
+        for (int c = 0; c < kFillClasses; c++)
+            if (z <= kFillBound[c]) return c;
+    return kFillClasses;
 }
 
 int launch_fill_moments(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
-                        const PairScalars* scs, c64* cf, int nb, long sw, double D, double gabs,
-                        double gre, hipStream_t st)
+                        const PairScalars* scs, c64* cf, const int* count, long sw, double D,
+                        hipStream_t st)
 {
     const long m = L.m;
+    int nb = 0;
+    for (int c = 0; c < kFillClasses; c++) nb += count[c];
     if (m <= 0 || nb <= 0) return 0;
-    const int K = fill_terms(gabs * D, gre * D);
-    if (K == 0 || !(D > 0.0) || !scs || !cf) return TAGS_ERR_ARG;
+    if (!(D > 0.0) || !scs || !cf) return TAGS_ERR_ARG;
     int rc = gl_tables_init();
     if (rc) return rc;
-    hipLaunchKernelGGL(k_fill_coefs, dim3(nb), dim3(64), 0, st, scs, D, K, cf);
+    hipLaunchKernelGGL(k_fill_coefs, dim3(nb), dim3(64), 0, st, scs, D, cf);
     const bool small = m <= 256;
     const long T = small ? (m + 7) / 8 : (m + 15) / 16, tiles = T * (T + 1) / 2;
-    // samples per work-group: all of them once the tiles alone give every CU
+    // samples per work-group: all of a class once the tiles alone give every CU
     // four work-groups (8 x 8 tiles: two, of eight samples at least), else fewer
     // (the moments are then formed more often)
     const long chunks = std::max(1L, std::min(small ? (nb + 7L) / 8 : (long)nb,
                                               (small ? 512 : 1024) / tiles));
-    const int per = (int)((nb + chunks - 1) / chunks);
-    const dim3 g((unsigned)tiles, (unsigned)((nb + per - 1) / per));
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, g, dim3(small ? 512 : 256), 0, st, W, ldw, L.zl_off, L.zt_off, m, e, img, scs,
-                           sw, (const c64*)cf, nb, per, D, gabs);
-    };
-    auto terms = [&](auto kt) {
-        constexpr int k = decltype(kt)::value;
-        if (small) go(k_fill_moments<k, 8>);
-        else go(k_fill_moments<k, 16>);
-    };
-    if (K == 12) terms(std::integral_constant<int, 12>());
-    else if (K == 16) terms(std::integral_constant<int, 16>());
-    else if (K == 24) terms(std::integral_constant<int, 24>());
-    else terms(std::integral_constant<int, kFillTermsMax>());
+    FillGroups g{};
+    g.per = (int)((nb + chunks - 1) / chunks);
+    for (int c = 0; c < kFillClasses; c++) {
+        g.first[c + 1] = g.first[c] + count[c];
+        g.chunk[c + 1] = g.chunk[c] + (count[c] + g.per - 1) / g.per;
+    }
+    const dim3 grid((unsigned)tiles, (unsigned)g.chunk[kFillClasses]);
+    if (small)
+        hipLaunchKernelGGL(k_fill_moments<8>, grid, dim3(512), 0, st, W, ldw, L.zl_off, L.zt_off, m,
+                           e, img, scs, sw, (const c64*)cf, g, D);
+    else
+        hipLaunchKernelGGL(k_fill_moments<16>, grid, dim3(256), 0, st, W, ldw, L.zl_off, L.zt_off,
+                           m, e, img, scs, sw, (const c64*)cf, g, D);
     TAGS_HIP(hipGetLastError());
     return 0;
 }

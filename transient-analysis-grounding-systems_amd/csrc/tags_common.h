@@ -153,6 +153,7 @@ struct PairScalars {
     c64 zl_dir, zt_dir;   // s mu / 4 pi and 1 / (4 pi kappa)
     c64 zl_img, zt_img;   // ref_l s mu / 4 pi and ref_t / (4 pi kappa)
     int intg_type;        // INTG_DOUBLE, INTG_MHEM or INTG_NONE
+    int item;             // fills of several samples: which W of the batch is its
 };
 
 // Placement of the three unknown blocks of the immittance system (row and
@@ -185,22 +186,21 @@ int launch_pairs_packed(c64* zl, c64* zt, SegSoA e, SegSoA img, long m, const Pa
 void gauss_legendre(int n, double* x, double* w);
 int launch_mhem_potentials(double* pl, double* pt, double* pli, double* pti, long m, SegSoA e,
                            SegSoA img, hipStream_t st);
-// Fills of nb frequency samples at once: W of item z at W + z sw, its scalars
-// scs[z] in device memory.
+// Fills of nb frequency samples at once, their scalars scs[z] in device memory: W
+// of item z at W + z sw (mHEM: scs in item order; else scs[z] names its item).
 int launch_fill_mhem(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
                      const double* pl, const double* pt, const double* pli, const double* pti,
                      const PairScalars* scs, hipStream_t st, int nb, long sw);
 int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
                         const PairScalars* scs, hipStream_t st, int nb, long sw);
-// The impedance blocks of nb samples from Chebyshev moments (k_fill_moments):
-// D the longest segment (by its end points), gabs and gre the largest |gamma| and
-// |Re gamma| of the samples, fill_terms(gabs D, gre D) > 0; scs in device memory,
-// cf nb kFillTermsMax values of scratch.
-constexpr int kFillTermsMax = 32;
-int fill_terms(double z, double re);
+// The impedance blocks of samples from Chebyshev moments (k_fill_moments): D the
+// longest segment (by its end points), count[c] samples of each class in class
+// order; scs in device memory, cf kFillTermsMax values of scratch per sample.
+constexpr int kFillTermsMax = 32, kFillClasses = 5;
+int fill_class(double z, double re);
 int launch_fill_moments(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
-                        const PairScalars* scs, c64* cf, int nb, long sw, double D, double gabs,
-                        double gre, hipStream_t st);
+                        const PairScalars* scs, c64* cf, const int* count, long sw, double D,
+                        hipStream_t st);
 int launch_fill_static(c64* W, long ldw, const BlockLayout& L, const int* seg_start_node,
                        const int* seg_end_node, hipStream_t st, int nb = 1, long sw = 0);
 int launch_single_pair(SegSoA e, SegSoA r, c64 gamma, int type, double* out4, hipStream_t st);
