@@ -311,3 +311,25 @@ def test_admittance_size_limit():
     m, n = 1, 65536
     a, b, y, z = (np.ones(m * n, complex) for _ in range(4))
     assert T.calculate_yla_ytb(y, z, np.ones(1, complex), np.ones(1, complex), a, b, m, n) == -13
+
+
+@pytest.mark.parametrize("counts", [(8, 5), (4, 40, 30)])
+def test_solve_immittance_of_separate_conductors(counts):
+    """Conductors that no segment joins, a full right-hand side, against numpy on
+    the same W (1e-9: cond ~ 1e5)."""
+    rods = [T.segment_electrode([0, 7 * k, -0.5 - k], [3 + c, 7 * k, -0.5 - k], c, 7e-3)[1:]
+            for k, c in enumerate(counts)]
+    e, nodes = (np.concatenate(v) for v in zip(*rods))
+    m, n = len(e), len(nodes)
+    N = n + 2 * m
+    sc = T.soil_scalars(4e5, 2e-3, 12.0)
+    zl, zt, W = (np.zeros(k, complex) for k in (m * m, m * m, N * N))
+    T.calculate_impedances(zl, zt, e, sc["gamma"], sc["s"], 1.0, sc["kappa"])
+    assert T.fill_incidence_imm(W, e, nodes) == 0 and T.fill_impedance_imm(W, zl, zt, m, n) == 0
+    low = np.tril(W.reshape(N, N).T)
+    rng = np.random.default_rng(m)
+    b = rng.standard_normal(N) + 1j * rng.standard_normal(N)
+    x = b.copy()
+    assert T.solve_immittance(W, x, m, n) == 0
+    ref = np.linalg.solve(low + np.tril(low, -1).T, b)
+    assert np.abs(x - ref).max() <= 1e-9 * np.abs(ref).max()

@@ -118,3 +118,49 @@ def test_a_rejected_sample_leaves_the_others_alone(inflight):
         for got in (u, w):
             assert np.allclose(got[z], p[z], rtol=1e-9, atol=0.0, equal_nan=True)
     sw.close()
+
+
+def _conductors(rods):
+    """Separate straight conductors (start, end, segments), their nodes shuffled."""
+    e, nodes = zip(*[T.segment_electrode(a, b, k, 7e-3)[1:] for a, b, k in rods])
+    e, nodes = np.concatenate(e), np.concatenate(nodes)
+    return e, nodes[np.random.default_rng(len(e)).permutation(len(nodes))]
+
+
+_RODS = [([0, 0, -0.5], [15, 0, -0.5]), ([0, 20, -0.5], [12, 20, -0.5]), ([30, 0, -0.5], [30, 0, -3.5]),
+         ([3, 1, -0.6], [3, 9, -0.6])]
+
+
+# (segments of each): few and small, past 64 nodes, beyond the 128- and 256-column steps;
+# single segments, which a part's root and one more node make up
+@pytest.mark.parametrize("counts", [(3, 2), (30, 24), (30, 24, 6), (1, 1, 1, 1), (60, 50, 6, 20),
+                                    (20, 150, 9), (210, 90, 12)])
+@pytest.mark.parametrize("mhem", [False, True])
+def test_separate_conductors(counts, mhem):
+    """Several conductors that no segment joins, injected at a root, at another
+    node of a part and at the largest part: as one conductor is, and refined in the
+    steps that one takes. Without their constants taken out, two rods contract by
+    0.03 to 0.1 a step at 60 Hz and the mixed form needs 10 steps and more; one
+    conductor of 30 segments needs the three that are always done, a longer one
+    at most two more (1e-2 a step is the slowest that the node system is known
+    for, 1e-10 the goal)."""
+    e, nodes = _conductors([(a, b, k) for (a, b), k in zip(_RODS, counts)])
+    f = [60.0, 1e4, 3e6]
+    _compare(e, nodes, f, mhem=mhem)
+    s = 2j * np.pi * np.asarray(f)
+    kap = 2e-3 + s * 12.0 * T.EPS0
+    sw = T.Sweep(e, nodes)
+    if mhem:
+        sw.set_formulation(T.FORM_MHEM)
+    for end in ([0, 0, -0.5], [0, 20, -0.5], [12, 20, -0.5]):
+        inj = int(np.argmin(np.linalg.norm(nodes - end, axis=1)))
+        sw.set_plan(T.PLAN_ZL_FIRST)
+        u0, _, x0 = sw.solve(s, kap, inj, T.PREC_FP64, want_x=True)
+        sw.set_plan(T.PLAN_HYBRID)
+        scale = np.abs(x0).max(axis=1, keepdims=True)
+        for prec, tol in ((T.PREC_FP64, 1e-9), (T.PREC_MIXED, 1e-8)):
+            u, st, x = sw.solve(s, kap, inj, prec, want_x=True)
+            assert np.max(np.abs(u - u0) / np.abs(u0)) <= tol
+            assert np.max(np.abs(x - x0) / scale) <= 1e-8
+            assert all(q["precision_used"] == prec and q["refine_iters"] <= 5 for q in st), st
+    sw.close()

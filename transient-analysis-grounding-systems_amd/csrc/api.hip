@@ -1246,6 +1246,64 @@ static bool node_lists(const std::vector<int>& sn, const std::vector<int>& en, l
     return true;
 }
 
+// The parts of the node graph that no segment joins (see HemOp): how many, and
+// where there are several the lists part (n), root (parts), pseg_ptr (parts + 1),
+// pseg (m), pnode_ptr (parts + 1) and pnode (n), one after the other.
+struct Parts {
+    int count = 1;
+    std::vector<int> lists;
+    Parts(const std::vector<int>& sn, const std::vector<int>& en, long n)
+    {
+        const long m = (long)sn.size();
+        std::vector<int> up(n);
+        for (long u = 0; u < n; u++) up[u] = (int)u;
+        auto top = [&](int u) {
+            while (up[u] != u) u = up[u] = up[up[u]];
+            return u;
+        };
+        for (long s = 0; s < m; s++) {
+            const int a = top(sn[s]), b = top(en[s]);
+            up[std::max(a, b)] = std::min(a, b);  // (a part's top is its first node)
+        }
+        std::vector<int> root, size(n, 0), of(n);
+        for (long u = 0; u < n; u++) {
+            const int t = top((int)u);
+            if (t == u) root.push_back((int)u);
+            size[t]++;
+        }
+        count = (int)root.size();
+        if (count <= 1) return;
+        std::swap(root[0], *std::max_element(root.begin(), root.end(), [&](int a, int b) {
+            return size[a] < size[b];
+        }));
+        for (int j = 0; j < count; j++) of[root[j]] = j;
+        std::vector<int> part(n), pseg(m), pnode(n), sp(count + 1, 0), np(count + 1, 0);
+        for (long u = 0; u < n; u++) np[(part[u] = of[top((int)u)]) + 1]++;
+        for (long s = 0; s < m; s++) sp[part[sn[s]] + 1]++;
+        for (int j = 0; j < count; j++) {
+            sp[j + 1] += sp[j];
+            np[j + 1] += np[j];
+        }
+        std::vector<int> sat(sp), nat(np);
+        for (long u = 0; u < n; u++) pnode[nat[part[u]]++] = (int)u;
+        for (long s = 0; s < m; s++) pseg[sat[part[sn[s]]]++] = (int)s;
+        for (const std::vector<int>* v : {&part, &root, &sp, &pseg, &np, &pnode})
+            lists.insert(lists.end(), v->begin(), v->end());
+    }
+    // sets the lists of a HemOp whose m and n are set from their device copy
+    void bind(HemOp& op, const int* d) const
+    {
+        op.parts = count;
+        if (count <= 1) return;
+        op.part = d;
+        op.root = op.part + op.n;
+        op.pseg_ptr = op.root + count;
+        op.pseg = op.pseg_ptr + count + 1;
+        op.pnode_ptr = op.pseg + op.m;
+        op.pnode = op.pnode_ptr + count + 1;
+    }
+};
+
 // Calls put(segment, node, end) for every match.
 template <typename F>
 static void incidence_each(const Incidence& inc, F put)
@@ -1380,10 +1438,13 @@ static int immittance_nodal(const c64* Wd, c64* bx, long m, long n, hipStream_t 
     std::vector<int> ptr, seg;
     bool distinct;
     if (!node_lists(sn, en, n, ptr, seg, &distinct) || !distinct) return 0;
-    DevBuf<int> dp, ds;
-    if (!dp.try_alloc(n + 1) || !ds.try_alloc(seg.size())) return 0;
+    const Parts parts(sn, en, n);
+    DevBuf<int> dp, ds, dl;
+    if (!dp.try_alloc(n + 1) || !ds.try_alloc(seg.size()) || !dl.try_alloc(parts.lists.size()))
+        return 0;
     if ((rc = copy_in(dp.p, ptr.data(), sizeof(int) * (n + 1), st)) ||
-        (rc = copy_in(ds.p, seg.data(), sizeof(int) * seg.size(), st)))
+        (rc = copy_in(ds.p, seg.data(), sizeof(int) * seg.size(), st)) ||
+        (rc = copy_in(dl.p, parts.lists.data(), sizeof(int) * parts.lists.size(), st)))
         return rc;
     HemOp op;
     op.m = m;
@@ -1392,6 +1453,7 @@ static int immittance_nodal(const c64* Wd, c64* bx, long m, long n, hipStream_t 
     op.en = d.p + m;
     op.node_ptr = dp.p;
     op.node_seg = ds.p;
+    parts.bind(op, dl.p);
     NodalSolver nd;
     nd.st = st;
     if (nd.ensure(op, true, 1)) {
@@ -2072,6 +2134,7 @@ struct tags_sweep {
     // structure of W in the current layout, for the refinement's products
     int* node_ptr = nullptr;
     int* node_seg = nullptr;
+    int* part_lists = nullptr;  // see Parts
     tags::HemOp hem{};
     std::vector<std::unique_ptr<SweepSlot>> slots;
     bool profiling = false;
@@ -2141,7 +2204,7 @@ static int sweep_nd_batch(const tags_sweep* sw, bool mixed, size_t nfreq)
     if (sw->batch_req > 0) {
         lim = (size_t)sw->batch_req;
     } else if (sw->N < kBatchOneAbove) {
-        const double per = (double)NodalSolver::bytes(sw->m, sw->n, !mixed, 1);
+        const double per = (double)NodalSolver::bytes(sw->m, sw->n, sw->hem.parts, !mixed, 1);
         lim = (size_t)std::max(1.0, std::min((double)kNdBatchMax, std::floor(kBatchBytes / per)));
     }
     const size_t groups = std::max<size_t>(1, (nfreq + lim - 1) / lim);
@@ -2426,6 +2489,15 @@ int tags_sweep_create(tags_sweep** out, const Electrode* electrodes, const Elect
     TAGS_HIP(hipMemcpy(hen.data(), sw->en, sizeof(int) * m, hipMemcpyDeviceToHost));
     std::vector<int> ptr, seg;
     if (!node_lists(hsn, hen, n, ptr, seg, &sw->nodal_ok)) return TAGS_ERR_ARG;
+    const Parts parts(hsn, hen, n);
+    if (parts.count > 1) {
+        const size_t nb = sizeof(int) * parts.lists.size();
+        TAGS_HIP(hipMalloc(&sw->part_lists, nb));
+        TAGS_HIP(hipMemcpy(sw->part_lists, parts.lists.data(), nb, hipMemcpyHostToDevice));
+    }
+    sw->hem.m = m;
+    sw->hem.n = n;
+    parts.bind(sw->hem, sw->part_lists);
     TAGS_HIP(hipMalloc(&sw->node_ptr, sizeof(int) * (n + 1)));
     TAGS_HIP(hipMalloc(&sw->node_seg, sizeof(int) * std::max<size_t>(1, seg.size())));
     TAGS_HIP(hipMemcpy(sw->node_ptr, ptr.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice));
@@ -2589,6 +2661,7 @@ void tags_sweep_destroy(tags_sweep* sw)
     hipFree(sw->en);
     hipFree(sw->node_ptr);
     hipFree(sw->node_seg);
+    hipFree(sw->part_lists);
     hipFree(sw->pot);
     hipStream_t st = sw->st;
     delete sw;
@@ -3317,7 +3390,7 @@ int tags_sweep_autotune(tags_sweep* sw, int precision, size_t nprobe, const TAGS
         // device's memory
         size_t mem_free = 0, mem_total = 0;
         if (hipMemGetInfo(&mem_free, &mem_total) != hipSuccess) mem_total = 0;
-        const double per = nodal ? (double)NodalSolver::bytes(sw->m, sw->n, !mixed, 1)
+        const double per = nodal ? (double)NodalSolver::bytes(sw->m, sw->n, sw->hem.parts, !mixed, 1)
                                  : (double)sw->N * (double)sw->N * (mixed ? 24.0 : 16.0);
         const int k = cur.inflight > 0 ? cur.inflight : sw->inflight;
         for (int b = 2; b <= 4; b++) {
@@ -3572,7 +3645,7 @@ int tags_cases_solve(tags_cases* cs, int precision)
             for (size_t c = 0; c < nc; c++) {
                 const tags_sweep* sw = cs->sw[c];
                 if (!sweep_nodal(sw, mixed, INFINITY)) continue;
-                const size_t nbytes = NodalSolver::bytes(sw->m, sw->n, !mixed, sw->nd_batch);
+                const size_t nbytes = NodalSolver::bytes(sw->m, sw->n, sw->hem.parts, !mixed, sw->nd_batch);
                 if (nbytes > most) {
                     most = nbytes;
                     big = sw;

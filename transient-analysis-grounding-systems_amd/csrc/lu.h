@@ -491,6 +491,15 @@ struct HemOp {
     const int* en = nullptr;        // end node (device, m)
     const int* node_ptr = nullptr;  // device, n + 1
     const int* node_seg = nullptr;  // device, node_ptr[n]
+    // The nodal solve's view of separate conductors (parts of the node graph that
+    // no segment joins), null where there is one: each node's part, the first node
+    // of each part (its root), and the segments and nodes of each part. Part 0 is
+    // the one with the most nodes.
+    int parts = 1;
+    const int* part = nullptr;                               // n
+    const int* root = nullptr;                               // parts
+    const int *pseg_ptr = nullptr, *pseg = nullptr;          // parts + 1, m
+    const int *pnode_ptr = nullptr, *pnode = nullptr;        // parts + 1, n
 };
 
 // norms[0..1] (and [2] with want_wnorm) receive |r|, |x| (|W|) as max-reductions;

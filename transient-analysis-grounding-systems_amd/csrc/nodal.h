@@ -31,6 +31,7 @@ struct NodalSolver {
     int cap = 0, nb = 0;
     long inj = 0;
     HemOp op;  // node lists and offsets of the compact storage
+    int parts = 1;  // parts that the solve in flight tells apart
 
     char* arena = nullptr;
     size_t arena_bytes = 0;
@@ -50,7 +51,7 @@ struct NodalSolver {
     int* active = nullptr;
 
     // bytes of `batch` items (without allocating)
-    static size_t bytes(long m, long n, bool f64, int batch);
+    static size_t bytes(long m, long n, int parts, bool f64, int batch);
     int ensure(const HemOp& hem, bool f64, int batch);
     void release();
     ~NodalSolver() { release(); }
