@@ -156,7 +156,7 @@ def test_a_sample_does_not_see_its_group(m):
     kap = 1e-3 + s * 10.0 * T.EPS0
     z = np.abs(np.sqrt(s * T.MU0 * kap)) * 3.0
     assert [np.sum((z > a) & (z <= b)) > 0 for a, b in
-            ((0, 0.38), (0.38, 1), (1, 2), (2, 3.7), (3.7, 5), (5, 1e9))] == [True] * 6
+            ((0, 0.5), (0.5, 1), (1, 2), (2, 3.7), (3.7, 5), (5, 1e9))] == [True] * 6
     mix = np.random.default_rng(m).permutation(len(f))
     sw = T.Sweep(e, nodes)
     for prec in (T.PREC_FP64, T.PREC_MIXED):

@@ -789,6 +789,32 @@ __device__ inline void mom_wave(Moments<K>& M, const DSeg& S, const DSeg& R, dou
         }
 }
 
+// The sums of K <= 32 values over a wave's lanes, folded: each halving of the lanes
+// halves the sums that a lane holds, 17 or 32 exchanges instead of 6 K (a group
+// forms its near pairs' moments once per class). The lane has sum *j (32: none).
+template <int K>
+__device__ inline double fold_sums(const double (&m)[K], int lane, int* j)
+{
+    constexpr int L = K <= 16 ? 4 : 5, P = 1 << L;
+    double f[P];
+#pragma unroll
+    for (int q = 0; q < P; q++) f[q] = q < K ? m[q] : 0.0;
+    int id = 0;
+#pragma unroll
+    for (int l = 0; l < L; l++) {
+        const int o = 32 >> l, h = P >> (l + 1);
+        const bool up = lane & o;
+        id += up ? h : 0;
+#pragma unroll
+        for (int q = 0; q < h; q++)
+            f[q] = (up ? f[q + h] : f[q]) + __shfl_xor(up ? f[q] : f[q + h], o);
+    }
+#pragma unroll
+    for (int o = 32 >> L; o > 0; o >>= 1) f[0] += __shfl_xor(f[0], o);
+    *j = lane & ((64 >> L) - 1) ? 32 : id;
+    return f[0];
+}
+
 // Whether a pair goes to the waves: shared end points, or closer than two lengths
 __device__ inline bool pair_near(const DSeg& S, const DSeg& R, double* rho)
 {
@@ -799,12 +825,13 @@ __device__ inline bool pair_near(const DSeg& S, const DSeg& R, double* rho)
 
 constexpr int fill_waves(int ts) { return ts == 8 ? 8 : 4; }
 
-// The classes of samples by |gamma| D (in ascending order): Chebyshev terms and the
-// bound that the class's quadrature orders are chosen for. Terms: 2 (z / 2)^K / K!,
-// the size of the first coefficient left out, is at most 1e-17 (12 to z = 0.38, 16
-// to 1.13, 24 to 3.7, 32 to 7.3); bounds where geometric_order steps.
-constexpr int kFillTerms[kFillClasses] = {12, 16, 24, 24, 32};
-constexpr double kFillBound[kFillClasses] = {0.38, 1.0, 2.0, 3.7, 5.0};
+// The classes of samples by |gamma| D (in ascending order): the bound that the
+// class's quadrature orders are chosen for, which is where geometric_order steps
+// (a group forms its moments once per class it holds, so there is no class between
+// two steps), and its Chebyshev terms: 2 (z / 2)^K / K!, the size of the first
+// coefficient left out at the bound, is at most 1e-17.
+constexpr int kFillTerms[kFillClasses] = {13, 16, 20, 24, 28};
+constexpr double kFillBound[kFillClasses] = {0.5, 1.0, 2.0, 3.7, 5.0};
 __device__ inline double fill_bound(int c)
 {
     return c == 0 ? kFillBound[0] : c == 1 ? kFillBound[1] : c == 2 ? kFillBound[2]
@@ -907,12 +934,9 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
         M.invd = 1.0 / D;
         M.rc = vnorm(vsub(vmid(S), vmid(R)));
         mom_wave(M, S, R, gabs, lane);
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            double v = M.m[j];
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-            if (lane == 0) stage.mom[KINDS == 2 ? kind : 0][j][w] = v;
-        }
+        int j;
+        const double v = fold_sums(M.m, lane, &j);
+        if (j < K) stage.mom[KINDS == 2 ? kind : 0][j][w] = v;
     };
     if constexpr (KINDS == 2) {
         if (wave < 2) far(wave);
@@ -1007,7 +1031,7 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
     switch (cls) {
     case 0: fill(std::integral_constant<int, kFillTerms[0]>()); break;
     case 1: fill(std::integral_constant<int, kFillTerms[1]>()); break;
-    case 2:
+    case 2: fill(std::integral_constant<int, kFillTerms[2]>()); break;
     case 3: fill(std::integral_constant<int, kFillTerms[3]>()); break;
     default: fill(std::integral_constant<int, kFillTerms[4]>()); break;
     }
