@@ -697,6 +697,13 @@ int tags_device_synchronize(void);
  * calls keep between calls. Safe at any time, from any thread. */
 void tags_release_staging(void);
 
+/* How often the calling thread's calls took a symmetric route and how often they
+ * left it to the pivoted factorisation, since the thread began (pairs taken, left):
+ * [0, 1] samples of the hybrid plan's nodal solve, [2, 3] solve_immittance, [4, 5]
+ * solve_admittance, [6, 7] calculate_yla_ytb and fill_impedance_adm. Answers and
+ * statistics do not tell the routes apart. */
+void tags_route_counts(unsigned long long counts[8]);
+
 /* For tests of what a call does where device memory runs out: the nth device
  * allocation (1, 2, ..) of the calling thread's host-pointer calls and nodal
  * solves from now on fails as one that does not fit; 0 disarms. Returns what

@@ -117,18 +117,25 @@ def _symmetric(m, seed, definite):
 
 
 @pytest.mark.parametrize("m", [1, 2, 63, 64, 65, 128, 129, 200])
-@pytest.mark.parametrize("kind", ["dominant", "indefinite", "zero_pivot"])
+@pytest.mark.parametrize("kind", ["dominant", "indefinite", "zero_pivot", "zero_block"])
 def test_symmetric_inverse_and_its_fallback(m, kind):
     """solve_admittance and calculate_yla_ytb on matrices that the inverse
     without row exchanges takes, on ones whose growth without them its checks
-    have to see, and on ones with an exactly zero first pivot: against numpy,
-    1e-11 of the largest entry times cond (a stable solve's normwise bound at
-    these orders, with a factor of about 100 to spare)."""
+    have to see, on ones with an exactly zero first pivot (which the 2 x 2 pivots
+    take) and with a zero first 2 x 2 block (which nothing without row exchanges
+    does): against numpy, 1e-14 of the largest entry times cond (a stable solve's
+    normwise bound at these orders, with a factor of about 100 to spare). The
+    counts tell that the first kind stays on the route and the last leaves it."""
     if kind == "zero_pivot" and m == 1:
         pytest.skip("a singular 1 x 1 matrix")
     a = _symmetric(m, 5 + m, kind == "dominant")
+    if kind == "zero_block" and m < 5:
+        pytest.skip("a singular matrix")
     if kind == "zero_pivot":
         a[0, 0] = 0.0
+    if kind == "zero_block":
+        a[:2, :2] = 0.0
+    routes = T.route_counts()
     cond = np.linalg.cond(a)
     rng = np.random.default_rng(m)
     b = rng.standard_normal(m) + 1j * rng.standard_normal(m)
@@ -147,6 +154,10 @@ def test_symmetric_inverse_and_its_fallback(m, kind):
     got = zl.reshape(m, m).T
     assert np.abs(np.tril(got) - np.tril(inv)).max() <= tol
     assert np.all(got[np.triu_indices(m, 1)] == 0)
+    if kind in ("dominant", "zero_block"):
+        for call in ("symmetric", "admittance"):
+            was, now = routes[call], T.route_counts()[call]
+            assert (now[0] - was[0], now[1] - was[1]) == ((1, 0) if kind == "dominant" else (0, 1))
 
 
 def test_solve_immittance_structure():
@@ -178,7 +189,10 @@ def test_solve_immittance_structure():
         full = low + np.tril(low, -1).T
         x = b.copy()
         keep = W.copy()
+        was = T.route_counts()["immittance"]
         assert T.solve_immittance(W, x, m, n) == 0
+        now = T.route_counts()["immittance"]
+        assert (now[0] - was[0], now[1] - was[1]) == ((0, 1) if change else (1, 0))
         assert np.array_equal(W, keep)
         ref = np.linalg.solve(full, b)
         assert np.abs(x - ref).max() <= 1e-9 * np.abs(ref).max()
@@ -330,6 +344,8 @@ def test_solve_immittance_of_separate_conductors(counts):
     rng = np.random.default_rng(m)
     b = rng.standard_normal(N) + 1j * rng.standard_normal(N)
     x = b.copy()
+    was = T.route_counts()["immittance"]
     assert T.solve_immittance(W, x, m, n) == 0
+    assert T.route_counts()["immittance"] == (was[0] + 1, was[1])
     ref = np.linalg.solve(low + np.tril(low, -1).T, b)
     assert np.abs(x - ref).max() <= 1e-9 * np.abs(ref).max()

@@ -20,6 +20,14 @@ T = tags_pkg.load()
 pytestmark = pytest.mark.gpu
 
 
+def _routes(kind, taken, left, before):
+    """The route counts since `before`: a sample that the solve under test leaves to
+    the pivoted factor would be answered by what it is compared with."""
+    now = T.route_counts()[kind]
+    assert (now[0] - before[0], now[1] - before[1]) == (taken, left)
+    return now
+
+
 def _rod(m):
     rc, e, nodes = T.segment_electrode([0, 0, -0.5], [0.5 * m, 0, -0.5], m, 7e-3)
     return e, nodes
@@ -45,7 +53,9 @@ def _compare(e, nodes, f, groups=(0,), mhem=False):
     for g in groups:
         sw.set_batch(g)
         for prec, tol in ((T.PREC_FP64, 1e-9), (T.PREC_MIXED, 1e-8)):
+            r0 = T.route_counts()["nodal"]
             u, st, x = sw.solve(s, kap, inj, prec, want_x=True)
+            _routes("nodal", len(s), 0, r0)
             assert all(q["info"] == 0 and q["precision_used"] == prec for q in st), (prec, st)
             assert np.max(np.abs(u - u0) / np.abs(u0)) <= tol, (prec, g)
             assert np.max(np.abs(x - x0) / scale) <= 1e-8, (prec, g)
@@ -83,7 +93,9 @@ def test_zero_frequency_takes_the_pivoted_factor():
     u0, st0 = sw.solve(s, kap, 0, T.PREC_FP64)
     sw.set_plan(T.PLAN_HYBRID)
     for prec in (T.PREC_FP64, T.PREC_MIXED):
+        r0 = T.route_counts()["nodal"]
         u, st = sw.solve(s, kap, 0, prec)
+        _routes("nodal", 1, 1, r0)
         assert [q["info"] for q in st] == [q["info"] for q in st0]
         ok = np.isfinite(u0)
         assert np.array_equal(np.isfinite(u), ok)
@@ -109,7 +121,9 @@ def test_a_rejected_sample_leaves_the_others_alone(inflight):
         p = sw.solve(s, kap, 3, prec)[0]
         sw.set_plan(T.PLAN_HYBRID)
         sw.set_batch(1)
+        r0 = T.route_counts()["nodal"]
         u, st, x = sw.solve(s, kap, 3, prec, want_x=True)
+        _routes("nodal", 4, 3, r0)
         v, sv, y = sw.solve(s[~z], kap[~z], 3, prec, want_x=True)
         assert np.array_equal(u[~z], v) and np.array_equal(x[~z], y)
         assert [q["refine_iters"] for q, r in zip(st, z) if not r] == [q["refine_iters"] for q in sv]

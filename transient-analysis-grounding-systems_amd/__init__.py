@@ -174,7 +174,8 @@ EXPORTED = ["populate_electrode", "segment_electrode", "number_segments", "numbe
             "tags_cases_set_profiling", "tags_cases_get_timers", "tags_cases_destroy",
             "tags_sweep_autotune", "tags_sweep_set_tuning", "tags_sweep_get_tuning",
             "tags_cases_autotune",
-            "tags_sweep_set_gmres", "tags_release_staging", "tags_fail_allocation"]
+            "tags_sweep_set_gmres", "tags_release_staging", "tags_fail_allocation",
+            "tags_route_counts"]
 
 _lib = None
 
@@ -236,6 +237,7 @@ def lib():
         "tags_device_synchronize": ([], I),
         "tags_release_staging": ([], None),
         "tags_fail_allocation": ([ctypes.c_long], ctypes.c_long),
+        "tags_route_counts": ([P], None),
         "tags_gemm_bench": ([I, I, I, I, I, I, ctypes.POINTER(D)], I),
         "tags_gemm_variants": ([I], I),
         "tags_gemm_select": ([I, I, I], I),
@@ -542,6 +544,16 @@ def gemm_run(a, b, c, precision, variant, arow=None, brow=None, crow=None, mode=
     if rc:
         raise RuntimeError("tags_gemm_run failed: %d" % rc)
     return c
+
+
+def route_counts():
+    """How often this thread's calls took a symmetric route and how often they left
+    it to the pivoted factorisation: {"nodal": (taken, left), "immittance": ..,
+    "symmetric": .., "admittance": ..} (tags_route_counts)."""
+    c = np.zeros(8, np.uint64)
+    lib().tags_route_counts(_p(c))
+    return {k: (int(c[2 * i]), int(c[2 * i + 1]))
+            for i, k in enumerate(("nodal", "immittance", "symmetric", "admittance"))}
 
 
 def set_panel(kind):

@@ -81,6 +81,10 @@ struct Stream {
     ~Stream() { hipStreamDestroy(s); }
 };
 
+// see tags_route_counts
+enum Route { NODAL_TAKEN, NODAL_LEFT, IMM_TAKEN, IMM_LEFT, SYM_TAKEN, SYM_LEFT, ADM_TAKEN, ADM_LEFT };
+static thread_local unsigned long long g_routes[8];
+
 static thread_local long g_fail_at = 0;
 hipError_t dev_malloc(void** p, size_t bytes)
 {
@@ -640,6 +644,11 @@ using namespace tags;
 extern "C" {
 
 const char* tags_version(void) { return "tags_hip 0.1 (gfx950)"; }
+
+void tags_route_counts(unsigned long long counts[8])
+{
+    std::memcpy(counts, g_routes, sizeof(g_routes));
+}
 
 long tags_fail_allocation(long nth)
 {
@@ -1542,6 +1551,7 @@ static int dense_solve_host(const c64* a, c64* bx, long n, int precision, bool s
         bool done = false;
         if (imm_m > 0 && n > 2 * imm_m) {
             if ((rc = immittance_nodal(W.p, bx, imm_m, n - 2 * imm_m, S.s, &done))) return rc;
+            g_routes[done ? IMM_TAKEN : IMM_LEFT]++;
             if (done) return 0;
         }
         if ((rc = copy_in(bv.p, bx, sizeof(c64) * n, S.s)) ||
@@ -1549,6 +1559,7 @@ static int dense_solve_host(const c64* a, c64* bx, long n, int precision, bool s
             return rc;
         if (imm_m < 0) {
             if ((rc = symmetric_solve(W.p, bv.p, n, S.s, &done))) return rc;
+            g_routes[done ? SYM_TAKEN : SYM_LEFT]++;
             if (done) return copy_out(bx, bv.p, sizeof(c64) * n, S.s);
         }
     } else if ((rc = copy_in(bv.p, bx, sizeof(c64) * n, S.s))) {
@@ -1838,7 +1849,9 @@ static int adm_inverses(AdmArrays& d, TAGS_COMPLEX* zl, TAGS_COMPLEX* zt, const 
     if ((rc = upload())) return rc;
     if (zl != zt) {  // one array for both takes the reference's order of writes
         bool done = false;
-        if ((rc = adm_symmetric(d, zl, zt, m, n, st, &done)) || done) return rc;
+        if ((rc = adm_symmetric(d, zl, zt, m, n, st, &done))) return rc;
+        g_routes[done ? ADM_TAKEN : ADM_LEFT]++;
+        if (done) return 0;
         if ((rc = upload())) return rc;
     }
     LUWork<double> w;
@@ -2839,6 +2852,7 @@ static void sweep_nodal_finish(tags_sweep* sw, SweepSlot& sl, const SweepCall& c
         tags_item_stats& t = sl.stt[q];
         sl.info[q] = 0;
         t.info = 0;
+        g_routes[nd.accepted[q] ? NODAL_TAKEN : NODAL_LEFT]++;
         if (nd.accepted[q]) {
             t.precision_used = c.mixed ? TAGS_PREC_MIXED : TAGS_PREC_FP64;
             t.refine_iters = c.mixed ? nd.steps[q] : 0;
