@@ -41,12 +41,15 @@ struct StageRef {
 // bytes of `src` (host) to `dst` on st, in stream order; `src` may change once
 // it returns. Up to 8 MiB through the stage (a pageable copy of 0.25 MB takes
 // 127 us, staged 20), larger ones by the runtime's own pageable path (35 GB/s
-// at 17 MB, where one thread's copy into the stage runs at 30).
+// at 17 MB, where one thread's copy into the stage runs at 30), waited for: from
+// memory that the caller has pinned the runtime's copy is still under way when it
+// returns.
 inline int copy_in(void* dst, const void* src, size_t bytes, hipStream_t st)
 {
     if (bytes == 0) return 0;
     if (bytes > 2 * PinnedStage::kChunk) {
         TAGS_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
+        TAGS_HIP(hipStreamSynchronize(st));
         return 0;
     }
     StageRef r;
