@@ -349,3 +349,18 @@ def test_solve_immittance_of_separate_conductors(counts):
     assert T.route_counts()["immittance"] == (was[0] + 1, was[1])
     ref = np.linalg.solve(low + np.tril(low, -1).T, b)
     assert np.abs(x - ref).max() <= 1e-9 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("gamma", [np.inf, 1e30 + 1e30j, 1e20j, complex(np.nan, 1.0), complex(0.1, np.inf)])
+def test_gamma_without_end_of_panels(gamma):
+    """A gamma that is infinite, not a number, or so large that its panels could
+    not be told from each other: NaN, and at once."""
+    rc, e, nodes = T.segment_electrode([0, 0, -0.5], [2, 0, -0.5], 4, 7e-3)
+    pts = np.array([[0.3, 0.4, 0.0], [9.0, 2.0, 0.0]])
+    il = it = np.ones((1, 4), complex)
+    for v in T.fields(pts, e, il, it, gamma, 1j, 1e-3 + 0j):
+        assert np.all(np.isnan(v))
+    zl, zt = np.zeros(16, complex), np.zeros(16, complex)
+    assert T.calculate_impedances(zl, zt, e, gamma, 1j, 1.0, 1e-3 + 0j, integration_type=T.INTG_SINGLE) == 0
+    off = np.triu(np.ones((4, 4), bool), 1).ravel()
+    assert np.all(np.isnan(zt[off])) and np.all(np.isfinite(zt[::5]))

@@ -119,7 +119,9 @@ __device__ void segment_kernels(const double P[3], const double a[3], const doub
     const double ga = sqrt(g.x * g.x + g.y * g.y);
     const double wmax = ga * L > 2.0 ? 2.0 / (ga * L) : 1.0;
     ks = c64{0.0, 0.0};
-    kf[0] = kf[1] = kf[2] = c64{0.0, 0.0};
+    if (!(ga * L <= kPanelLimit)) ks = c64{NAN, NAN};
+    kf[0] = kf[1] = kf[2] = ks;
+    if (!(ga * L <= kPanelLimit)) return;
     int off = 0;
     // (r >= 1e-7 keeps clear of the DBL_EPSILON floors below)
     const int n = dist2 >= 1e-14 && dd > 0.0 ? field_order(wmin, ga * L, &off) : 0;

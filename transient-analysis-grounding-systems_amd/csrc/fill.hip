@@ -348,6 +348,7 @@ __device__ c64 single_unit(const DSeg& S, V3 M, c64 g)
     const double L = dd > 0.0 ? sqrt(dd) : S.len;
     const double wmin = fmax(vnorm(vsub(vadd(S.a, vmul(d, t0)), M)) / L, 1e-14);
     const double ga = sqrt(g.x * g.x + g.y * g.y);
+    if (!(ga * L <= kPanelLimit)) return c64{NAN, NAN};
     const double wmax = ga * L > 2.0 ? 2.0 / (ga * L) : 1.0;
     double sx = 0.0, sy = 0.0;
     for (int side = 0; side < 2; side++) {

@@ -135,6 +135,12 @@ constexpr double kFourPi = 12.5663706143591729538505735331;
 constexpr double kMu0 = 1.256637061435917e-6;
 constexpr double kEps0 = 8.854187817620e-12;
 
+// |gamma| L up to which a segment is integrated by panels of at most 2 / (|gamma| L)
+// of its length (half a million): beyond, or with a gamma that is not a number,
+// the integral is NaN, where the panels' count has no end (their width falls
+// below the rounding of the position, or is zero).
+constexpr double kPanelLimit = 1048576.0;
+
 // Segment geometry in structure-of-arrays form on the device.
 struct SegSoA {
     const double* ax;  // start point
