@@ -702,8 +702,12 @@ __device__ inline void mom_gl(Moments<K>& M, const DSeg& S, const DSeg& R, int o
     for (int i = p0; i < q * q; i += step) {
         const int a = i / q, b = i - a * q;
         const V3 d = vsub(vadd(R.a, vmul(dr, g_glx[off + a])), vadd(S.a, vmul(ds, g_glx[off + b])));
-        const double r = vnorm(d);
-        M.add(r, scale * g_glw[off + a] * g_glw[off + b] / r);
+        // (one reciprocal root in place of a root and a division; r to half an ulp,
+        // as it is multiplied by gamma)
+        const double r2 = vdot(d, d), ri = rsqrt(r2);
+        double r = r2 * ri;
+        r = fma(0.5 * ri, fma(-r, r, r2), r);
+        M.add(r, scale * g_glw[off + a] * g_glw[off + b] * ri);
     }
 }
 
