@@ -436,8 +436,8 @@ int tags_sweep_set_formulation(tags_sweep *sw, int formulation);
  * hybrid plan's nodal solve refines classically at every frequency): a
  * sample at |s| / 2 pi < below_hz (default 2e4 Hz) refines by FGMRES in FP64
  * right-preconditioned by the complex64 factor, `steps` (1 .. 32, default 6)
- * Arnoldi steps per refinement step (GMRES-based refinement), where the classic correction from the factor alone converges
- * slowly or not at all (the node block's Schur complement is dominated by
+ * Arnoldi steps per refinement step (GMRES-based refinement), where the
+ * classic correction from the factor alone converges slowly or not at all (the node block's Schur complement is dominated by
  * A^T Z_L^-1 A, whose complex64 rounding swamps the grounding terms at low
  * frequency); a higher one refines classically. No counterpart in the
  * reference. Returns 0, or TAGS_ERR_ARG. */
@@ -461,9 +461,10 @@ int tags_sweep_set_nodal_above(tags_sweep *sw, double hz);
  * grid per sample, side by side), so that mid-size systems fill the device.
  * Consecutive samples form a group; the hybrid plan starts a new group where
  * its choice of complex64 factor changes. Each sample's arithmetic is its own:
- * results agree with one-sample groups to rounding (the GEMM tile shape is
- * chosen by the size of the whole launch), and are independent of the
- * samples in flight. Grounded plans in the mixed form and the partial-
+ * the hybrid plan's nodal solve gives the bits of one-sample groups, the
+ * factorisations agree with them to rounding (the GEMM tile shape is chosen by
+ * the size of the whole launch), and both are independent of the samples in
+ * flight. Grounded plans in the mixed form and the partial-
  * pivoting panel take one sample at a time. No counterpart in the reference. */
 int tags_sweep_set_batch(tags_sweep *sw, int samples);
 
@@ -532,10 +533,10 @@ int tags_sweep_set_verify(tags_sweep *sw, int on);
  * The calling
  * thread queues a group on every slot, then finishes them in issue order,
  * queuing the next group on each slot as it frees up, so that one group's
- * trailing updates keep the GPU busy while another waits on its panel chain. Results do not depend on the count, except
- * where TAGS_PLAN_HYBRID raises its switch during a call: samples already in
- * flight keep the factor they were issued with (both answers meet the same
- * acceptance rule). */
+ * trailing updates keep the GPU busy while another waits on its panel chain.
+ * Results do not depend on the count, except where TAGS_PLAN_HYBRID raises its
+ * switch during a call in the mixed form: samples already in flight keep the
+ * factor they were issued with (both answers meet the same acceptance rule). */
 int tags_sweep_set_inflight(tags_sweep *sw, int samples);
 
 /* Assembles W for one frequency sample on the GPU exactly as tags_sweep_solve

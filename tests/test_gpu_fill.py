@@ -1,12 +1,12 @@
-"""GPU test of the sweep's impedance fill on both sides of each of its rules:
-the number of Chebyshev terms (12, 16, 24 or 32 by |gamma| times the longest
-segment) and the direct rule beyond them, on a geometry with touching
-segments (in line, at a right angle, at 10 degrees, of very different
-lengths), segments closer than two lengths down to a tenth of one, far ones,
-and images of shallow segments. Against the oracle's adaptive integrals
-(relative tolerance 1e-11): 1e-9 of each entry, the bar of the assembly
-tests; groups of several samples against single ones bit for bit in what they
-share (the terms of the group's largest |gamma| may differ): 1e-12."""
+"""GPU test of the sweep's impedance fill: over the range of its classes by |gamma|
+times the longest segment (13 to 32 Chebyshev terms up to 7.3) and the direct rule
+beyond them, on a geometry with touching segments (in line, at a right angle, at 10
+degrees, of very different lengths), segments closer than two lengths down to a
+tenth of one, far ones, and images of shallow segments. Against the oracle's
+adaptive integrals (relative tolerance 1e-11): 1e-9 of each entry, the bar of the
+assembly tests. Far pairs against extended precision: 2e-14. Groups of several
+samples against single ones: 1e-12 over tiles and sample ranges, bit for bit where
+every class meets every other."""
 import numpy as np
 import pytest
 
@@ -36,8 +36,10 @@ def _geometry():
     return e, nodes
 
 
-# |gamma| on either side of 0.38, 1.13, 3.7 and 7.3 over the longest segment (1 m)
-@pytest.mark.parametrize("glen", [0.02, 0.37, 0.39, 1.12, 1.14, 3.6, 3.8, 7.2, 7.4, 12.0])
+# |gamma| times the longest segment (1 m) in every class of the moment rule (they end
+# at 0.5, 1, 2, 3.7 and 7.3, or where gamma's real part is too large: here at 5) and in
+# the direct rule
+@pytest.mark.parametrize("glen", [0.02, 0.37, 0.39, 0.7, 1.12, 1.14, 3.6, 3.8, 4.9, 7.2, 7.4, 12.0])
 def test_fill_terms_vs_oracle(glen):
     e, nodes = _geometry()
     m, n = len(e), len(nodes)
@@ -156,7 +158,7 @@ def test_a_sample_does_not_see_its_group(m):
     kap = 1e-3 + s * 10.0 * T.EPS0
     z = np.abs(np.sqrt(s * T.MU0 * kap)) * 3.0
     assert [np.sum((z > a) & (z <= b)) > 0 for a, b in
-            ((0, 0.5), (0.5, 1), (1, 2), (2, 3.7), (3.7, 5), (5, 1e9))] == [True] * 6
+            ((0, 0.5), (0.5, 1), (1, 2), (2, 3.7), (3.7, 7.3), (7.3, 1e9))] == [True] * 6
     mix = np.random.default_rng(m).permutation(len(f))
     sw = T.Sweep(e, nodes)
     for prec in (T.PREC_FP64, T.PREC_MIXED):

@@ -648,11 +648,12 @@ int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
 // Rounding. The coefficients grow as e^{|Re gamma| D} while J is governed by the r
 // near R, so the sum cancels by up to that factor; and the one phase gamma R has
 // the rounding that the direct rule spreads over its points, so its products'
-// rounding errors are carried (rotor). With |Re gamma| D <= 2 and |gamma| D <= 5
-// the error is the direct rule's (worst of 160 pairs far, near and touching, R to
-// 60 D, arg gamma 0 .. 90 degrees, against 113 bits: 2.5e-15 against 3e-15 at
-// |gamma| D = 2, 1.5e-14 against 1.2e-14 at 5); beyond, up to 3e-13 against 8e-15,
-// so those keep the direct rule (k_fill_zblocks).
+// rounding errors are carried (rotor). With |Re gamma| D <= 2, from |gamma| D = 5 on
+// 1.3, the error is the direct rule's (worst of 120 pairs far, near and touching, R
+// to 60 D, arg gamma 0 .. 90 degrees, against 113 bits: 2.7e-15 against 3.0e-15 at
+// |gamma| D = 2, 1.5e-14 against 1.1e-14 at 5; rms of 320 pairs at 7.3, 80 degrees and
+// more: 1.9e-15 both); beyond, up to 6e-13 against 8e-15, so those keep the direct rule
+// (k_fill_zblocks).
 //
 // One thread per pair of a TS x TS tile on or below the diagonal, work-groups
 // of one tile and a range of the samples of one class (so that few segments still
@@ -835,8 +836,8 @@ constexpr int fill_waves(int ts) { return ts == 8 ? 8 : 4; }
 // (a group forms its moments once per class it holds, so there is no class between
 // two steps), and its Chebyshev terms: 2 (z / 2)^K / K!, the size of the first
 // coefficient left out at the bound, is at most 1e-17.
-constexpr int kFillTerms[kFillClasses] = {13, 16, 20, 24, 28};
-constexpr double kFillBound[kFillClasses] = {0.5, 1.0, 2.0, 3.7, 5.0};
+constexpr int kFillTerms[kFillClasses] = {13, 16, 20, 24, 32};
+constexpr double kFillBound[kFillClasses] = {0.5, 1.0, 2.0, 3.7, 7.3};
 __device__ inline double fill_bound(int c)
 {
     return c == 0 ? kFillBound[0] : c == 1 ? kFillBound[1] : c == 2 ? kFillBound[2]
@@ -1073,7 +1074,7 @@ __global__ __launch_bounds__(64) void k_fill_coefs(const PairScalars* scs, doubl
 // sum's rounding passes the direct rule's (or nothing is known of z)
 int fill_class(double z, double re)
 {
-    if (re <= 2.0)
+    if (re <= (z <= 5.0 ? 2.0 : 1.3))
         for (int c = 0; c < kFillClasses; c++)
             if (z <= kFillBound[c]) return c;
     return kFillClasses;

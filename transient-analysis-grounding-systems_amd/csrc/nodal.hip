@@ -18,7 +18,7 @@
 // incidence products with Y are gathers of four entries; and every solve of
 // the refinement is a matrix-vector product at memory speed, where triangular
 // solves are a chain of dependent blocks. For a 60 x 60 m grid (m = 7,440,
-// n = 6,541) that is 3.7e12 operations per sample, against 8.7e12 for the
+// n = 6,541) that is 4.4e12 operations per sample, against 8.7e12 for the
 // block elimination with the node columns carried along and 1.84e13 for the
 // pivoted elimination.
 //

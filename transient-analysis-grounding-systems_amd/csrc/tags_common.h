@@ -202,7 +202,7 @@ int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
 // The impedance blocks of samples from Chebyshev moments (k_fill_moments): D the
 // longest segment (by its end points), count[c] samples of each class in class
 // order; scs in device memory, cf kFillTermsMax values of scratch per sample.
-constexpr int kFillTermsMax = 28, kFillClasses = 5;
+constexpr int kFillTermsMax = 32, kFillClasses = 5;
 int fill_class(double z, double re);
 int launch_fill_moments(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA img,
                         const PairScalars* scs, c64* cf, const int* count, long sw, double D,
