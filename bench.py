@@ -249,7 +249,7 @@ def transient_bench(T, nt=2 ** 14):
            "N": len(nodes) + 2 * len(e), "inj_node": inj, "nt": nt, "samples": len(s)}
     res = {}
     for name, prec in (("fp64", T.PREC_FP64), ("mixed", T.PREC_MIXED)):
-        sw.solve(s[:4], kap[:4], inj, prec)
+        sw.solve(s[:512], kap[:512], inj, prec)
         L.tags_device_synchronize()
         t0 = time.perf_counter()
         zh, st = sw.solve(s, kap, inj, prec)
@@ -354,7 +354,7 @@ def sweep_config(T, e, nodes, inj, s, kap, plan=7, tuning=("table", TUNING_TABLE
     ps = probe_step(sw.N)
     for name, prec in (("mixed", T.PREC_MIXED), ("fp64", T.PREC_FP64)):
         tu = apply_tuning(T, sw, prec, s[::ps], kap[::ps], inj, tuning[0], tuning[1])
-        sw.solve(s[:2], kap[:2], inj, prec)  # allocations
+        sw.solve(s, kap, inj, prec)  # allocations, which follow the number of samples
         (u, st), dt = _timed_solve(T, sw, prec, s, kap, inj)
         sw.set_profiling(True)
         sw.solve(s, kap, inj, prec)
@@ -669,7 +669,8 @@ def main():
         group = 1
         if isinstance(tu, dict):
             inflight = tu["inflight"] if tu["inflight"] > 0 else args.inflight
-            group = max(1, tu["batch"])
+            # (by default two samples of the hybrid plan, at most)
+            group = tu["batch"] if tu["batch"] > 0 else 2
             if one_at_a_time:
                 sw.set_tuning(prec, dict(tu, inflight=1))
             else:

@@ -661,9 +661,11 @@ int launch_fill_zblocks(c64* W, long ldw, const BlockLayout& L, SegSoA e, SegSoA
 // Duffy rule or 144 points and more, are listed in LDS and taken by whole
 // waves, the lanes sharing the points; moments pass through LDS, so that few
 // of them are live in registers at a time. TS is 16, or 8 for few segments (a
-// fourth of the listed pairs per work-group, whose four waves then take a
-// sample each). Bound: the samples' exponentials and sines (FP64 VALU, about
-// 300 instructions per pair and sample), then the writes of both triangles.
+// fourth of the listed pairs per work-group, whose eight waves then take a
+// sample each: 34 us at m = 30; 96 samples of m = 1320 in three classes 3.3 ms).
+// Bound: the samples' exponentials and sines (FP64 VALU, about 300 instructions per
+// pair and sample) and, for few samples, the points; then the writes of both
+// triangles.
 // ---------------------------------------------------------------------------
 template <int K>
 struct Moments {
@@ -911,129 +913,130 @@ __global__ __launch_bounds__(fill_waves(TS) * 64, 2) void k_fill_moments(c64* __
     const int f0 = grp.first[cls] + ((int)blockIdx.y - grp.chunk[cls]) * grp.per;
     const int f1 = min(grp.first[cls + 1], f0 + grp.per);
     auto fill = [&](auto terms) {
-    constexpr int K = decltype(terms)::value;
-    double md[K], mi[K];  // direct, image
-    double rd = 0.0, ri = 0.0, cost = 0.0, cosi = 0.0, ll = 1.0;
-    // far pairs by a lane each (with 8 x 8 tiles a wave to each kind) ..
-    auto far = [&](int kind) {
-        Moments<K> M;
-        M.zero();
-        double rho;
-        if (in && (kind || k != i)) {
-            const DSeg S = seg(0, c), R = seg(1 + kind, a);
-            if (pair_near(S, R, &rho)) {
-                near_at[kind][atomicAdd(&near_n[kind], 1)] = pr;
-            } else {
-                M.rc = vnorm(vsub(vmid(S), vmid(R)));
-                M.invd = 1.0 / D;
-                mom_gl(M, S, R, geometric_order(rho, gabs * fmax(S.len, R.len)), 0, 1, 1.0);
+        constexpr int K = decltype(terms)::value;
+        double md[K], mi[K];  // direct, image
+        double rd = 0.0, ri = 0.0, cost = 0.0, cosi = 0.0, ll = 1.0;
+        // far pairs by a lane each (with 8 x 8 tiles a wave to each kind) ..
+        auto far = [&](int kind) {
+            Moments<K> M;
+            M.zero();
+            double rho;
+            if (in && (kind || k != i)) {
+                const DSeg S = seg(0, c), R = seg(1 + kind, a);
+                if (pair_near(S, R, &rho)) {
+                    near_at[kind][atomicAdd(&near_n[kind], 1)] = pr;
+                } else {
+                    M.rc = vnorm(vsub(vmid(S), vmid(R)));
+                    M.invd = 1.0 / D;
+                    mom_gl(M, S, R, geometric_order(rho, gabs * fmax(S.len, R.len)), 0, 1, 1.0);
+                }
             }
-        }
 #pragma unroll
-        for (int j = 0; j < K; j++) stage.mom[KINDS == 2 ? kind : 0][j][pr] = M.m[j];
-    };
-    // .. and near ones by a wave each
-    auto near = [&](int kind, int w) {
-        const DSeg S = seg(0, w % TS), R = seg(1 + kind, w / TS);
-        Moments<K> M;
-        M.zero();
-        M.invd = 1.0 / D;
-        M.rc = vnorm(vsub(vmid(S), vmid(R)));
-        mom_wave(M, S, R, gabs, lane);
-        int j;
-        const double v = fold_sums(M.m, lane, &j);
-        if (j < K) stage.mom[KINDS == 2 ? kind : 0][j][w] = v;
-    };
-    if constexpr (KINDS == 2) {
-        if (wave < 2) far(wave);
-        __syncthreads();
-        const int n0 = near_n[0], nn = n0 + near_n[1];
-        for (int q = wave; q < nn; q += NW) near(q >= n0, near_at[q >= n0][q >= n0 ? q - n0 : q]);
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            md[j] = stage.mom[0][j][pr];
-            mi[j] = stage.mom[KINDS - 1][j][pr];
-        }
-    } else {
-#pragma unroll
-        for (int kind = 0; kind < 2; kind++) {
-            far(kind);
+            for (int j = 0; j < K; j++) stage.mom[KINDS == 2 ? kind : 0][j][pr] = M.m[j];
+        };
+        // .. and near ones by a wave each
+        auto near = [&](int kind, int w) {
+            const DSeg S = seg(0, w % TS), R = seg(1 + kind, w / TS);
+            Moments<K> M;
+            M.zero();
+            M.invd = 1.0 / D;
+            M.rc = vnorm(vsub(vmid(S), vmid(R)));
+            mom_wave(M, S, R, gabs, lane);
+            int j;
+            const double v = fold_sums(M.m, lane, &j);
+            if (j < K) stage.mom[KINDS == 2 ? kind : 0][j][w] = v;
+        };
+        if constexpr (KINDS == 2) {
+            if (wave < 2) far(wave);
             __syncthreads();
-            const int nn = near_n[kind];
-            for (int q = wave; q < nn; q += NW) near(kind, near_at[kind][q]);
+            const int n0 = near_n[0], nn = n0 + near_n[1];
+            for (int q = wave; q < nn; q += NW)
+                near(q >= n0, near_at[q >= n0][q >= n0 ? q - n0 : q]);
             __syncthreads();
-#pragma unroll
-            for (int j = 0; j < K; j++) (kind ? mi[j] : md[j]) = stage.mom[0][j][pr];
-            __syncthreads();
-        }
-    }
-    if (in) {
-        const DSeg S = seg(0, c), R = seg(1, a), Ri = seg(2, a);
-        rd = vnorm(vsub(vmid(S), vmid(R)));
-        ri = vnorm(vsub(vmid(S), vmid(Ri)));
-        cost = abs_dot(S, R);
-        cosi = abs_dot(S, Ri);
-        ll = S.len * R.len;
-    }
-    const double self = in && k == i ? self_integral_dev(geo[1][6][a], geo[1][7][a]) : 0.0;
-    for (int f = f0 + (TS == 8 ? wave : 0); f < f1; f += TS == 8 ? NW : 1) {
-        const PairScalars& sc = scs[f];
-        const c64* cq = cf + (long)f * kFillTermsMax;
-        c64 vl{0, 0}, vt{0, 0};
-        if (in) {
-            double dx = 0, dy = 0, ix = 0, iy = 0;
 #pragma unroll
             for (int j = 0; j < K; j++) {
-                const c64 q = cq[j];
-                dx = fma(q.x, md[j], dx);
-                dy = fma(q.y, md[j], dy);
-                ix = fma(q.x, mi[j], ix);
-                iy = fma(q.y, mi[j], iy);
-            }
-            const c64 jd = cmul(rotor(sc.gamma, rd), c64{dx, dy});
-            const c64 ji = cmul(rotor(sc.gamma, ri), c64{ix, iy});
-            // the formulas of k_fill_zblocks, J the integral over L_r L_s
-            if (k == i) {
-                vl = cscale(sc.zl_dir, self);
-                vt = cscale(sc.zt_dir, self / ll);
-            } else {
-                vt = cmul(sc.zt_dir, jd);
-                if (!(cost < 2.220446049250313e-16)) vl = cscale(cmul(sc.zl_dir, jd), cost);
-            }
-            vt = cadd(vt, cmul(sc.zt_img, ji));
-            if (cosi > 2.220446049250313e-16)
-                vl = cadd(vl, cscale(cmul(sc.zl_img, ji), cosi));
-            vl = c64{-vl.x, -vl.y};
-            vt = c64{-vt.x, -vt.y};
-            c64* Wf = W + (long)sc.item * sw;
-            Wf[(zl_off + i) * ldw + zl_off + k] = vl;
-            Wf[(zt_off + i) * ldw + zt_off + k] = vt;
-        }
-        if constexpr (TS == 8) {
-            // the other triangle's entry (k0 + a, i0 + c) is lane (c, a)'s
-            const int from = c * 8 + a;
-            const c64 ol{__shfl(vl.x, from), __shfl(vl.y, from)};
-            const c64 ot{__shfl(vt.x, from), __shfl(vt.y, from)};
-            const long ko = k0 + a, io = i0 + c;
-            if (io < m && ko < io) {
-                c64* Wf = W + (long)sc.item * sw;
-                Wf[(zl_off + ko) * ldw + zl_off + io] = ol;
-                Wf[(zt_off + ko) * ldw + zt_off + io] = ot;
+                md[j] = stage.mom[0][j][pr];
+                mi[j] = stage.mom[KINDS - 1][j][pr];
             }
         } else {
-            const int h = f & 1;
-            stage.tile[h][0][a][c] = vl;
-            stage.tile[h][1][a][c] = vt;
-            __syncthreads();
-            const long ko = k0 + a, io = i0 + c;  // entry (ko, io) of the other triangle
-            if (io < m && ko < io) {
-                c64* Wf = W + (long)sc.item * sw;
-                Wf[(zl_off + ko) * ldw + zl_off + io] = stage.tile[h][0][c][a];
-                Wf[(zt_off + ko) * ldw + zt_off + io] = stage.tile[h][1][c][a];
+#pragma unroll
+            for (int kind = 0; kind < 2; kind++) {
+                far(kind);
+                __syncthreads();
+                const int nn = near_n[kind];
+                for (int q = wave; q < nn; q += NW) near(kind, near_at[kind][q]);
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < K; j++) (kind ? mi[j] : md[j]) = stage.mom[0][j][pr];
+                __syncthreads();
             }
         }
-    }    };
+        if (in) {
+            const DSeg S = seg(0, c), R = seg(1, a), Ri = seg(2, a);
+            rd = vnorm(vsub(vmid(S), vmid(R)));
+            ri = vnorm(vsub(vmid(S), vmid(Ri)));
+            cost = abs_dot(S, R);
+            cosi = abs_dot(S, Ri);
+            ll = S.len * R.len;
+        }
+        const double self = in && k == i ? self_integral_dev(geo[1][6][a], geo[1][7][a]) : 0.0;
+        for (int f = f0 + (TS == 8 ? wave : 0); f < f1; f += TS == 8 ? NW : 1) {
+            const PairScalars& sc = scs[f];
+            const c64* cq = cf + (long)f * kFillTermsMax;
+            c64 vl{0, 0}, vt{0, 0};
+            if (in) {
+                double dx = 0, dy = 0, ix = 0, iy = 0;
+#pragma unroll
+                for (int j = 0; j < K; j++) {
+                    const c64 q = cq[j];
+                    dx = fma(q.x, md[j], dx);
+                    dy = fma(q.y, md[j], dy);
+                    ix = fma(q.x, mi[j], ix);
+                    iy = fma(q.y, mi[j], iy);
+                }
+                const c64 jd = cmul(rotor(sc.gamma, rd), c64{dx, dy});
+                const c64 ji = cmul(rotor(sc.gamma, ri), c64{ix, iy});
+                // the formulas of k_fill_zblocks, J the integral over L_r L_s
+                if (k == i) {
+                    vl = cscale(sc.zl_dir, self);
+                    vt = cscale(sc.zt_dir, self / ll);
+                } else {
+                    vt = cmul(sc.zt_dir, jd);
+                    if (!(cost < 2.220446049250313e-16)) vl = cscale(cmul(sc.zl_dir, jd), cost);
+                }
+                vt = cadd(vt, cmul(sc.zt_img, ji));
+                if (cosi > 2.220446049250313e-16)
+                    vl = cadd(vl, cscale(cmul(sc.zl_img, ji), cosi));
+                vl = c64{-vl.x, -vl.y};
+                vt = c64{-vt.x, -vt.y};
+                c64* Wf = W + (long)sc.item * sw;
+                Wf[(zl_off + i) * ldw + zl_off + k] = vl;
+                Wf[(zt_off + i) * ldw + zt_off + k] = vt;
+            }
+            if constexpr (TS == 8) {
+                // the other triangle's entry (k0 + a, i0 + c) is lane (c, a)'s
+                const int from = c * 8 + a;
+                const c64 ol{__shfl(vl.x, from), __shfl(vl.y, from)};
+                const c64 ot{__shfl(vt.x, from), __shfl(vt.y, from)};
+                const long ko = k0 + a, io = i0 + c;
+                if (io < m && ko < io) {
+                    c64* Wf = W + (long)sc.item * sw;
+                    Wf[(zl_off + ko) * ldw + zl_off + io] = ol;
+                    Wf[(zt_off + ko) * ldw + zt_off + io] = ot;
+                }
+            } else {
+                const int h = f & 1;
+                stage.tile[h][0][a][c] = vl;
+                stage.tile[h][1][a][c] = vt;
+                __syncthreads();
+                const long ko = k0 + a, io = i0 + c;  // entry (ko, io) of the other triangle
+                if (io < m && ko < io) {
+                    c64* Wf = W + (long)sc.item * sw;
+                    Wf[(zl_off + ko) * ldw + zl_off + io] = stage.tile[h][0][c][a];
+                    Wf[(zt_off + ko) * ldw + zt_off + io] = stage.tile[h][1][c][a];
+                }
+            }
+        }    };
     switch (cls) {
     case 0: fill(std::integral_constant<int, kFillTerms[0]>()); break;
     case 1: fill(std::integral_constant<int, kFillTerms[1]>()); break;
