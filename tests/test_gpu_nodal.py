@@ -178,3 +178,29 @@ def test_separate_conductors(counts, mhem):
             assert np.max(np.abs(x - x0) / scale) <= 1e-8
             assert all(q["precision_used"] == prec and q["refine_iters"] <= 5 for q in st), st
     sw.close()
+
+
+@pytest.mark.parametrize("lanes", [1, 3])
+def test_cases_with_rejected_samples_and_separate_conductors(lanes):
+    """Many cases over lanes, each lane's solver serving one and several parts in
+    turn, with samples that the nodal solve rejects: every case as its own sweep
+    gives it, accepted samples bit for bit."""
+    f = np.array([50.0, 0.0, 2e4, 1e6])
+    s = 2j * np.pi * f
+    kap = 2e-3 + s * 12.0 * T.EPS0
+    geo = [_rod(20), _conductors([(a, b, k) for (a, b), k in zip(_RODS, (30, 24, 6))]), _rod(90),
+           _conductors([(a, b, k) for (a, b), k in zip(_RODS, (3, 2))]), _rod(70)]
+    descs = [dict(electrodes=e, nodes=nodes, s=s, kappa=kap, inj_node=1) for e, nodes in geo]
+    cs = T.Cases(descs)
+    cs.set_lanes(lanes)
+    for prec in (T.PREC_FP64, T.PREC_MIXED):
+        r0 = T.route_counts()["nodal"]
+        got, _ = cs.solve(prec)
+        _routes("nodal", 3 * len(geo), len(geo), r0)
+        for u, (e, nodes) in zip(got, geo):
+            sw = T.Sweep(e, nodes)
+            v = sw.solve(s, kap, 1, prec)[0]
+            sw.close()
+            assert np.array_equal(u[f > 0], v[f > 0])
+            assert np.allclose(u, v, rtol=1e-9, atol=0.0, equal_nan=True)
+    cs.close()
